@@ -1,18 +1,17 @@
 // engine.hip -- gfx950 kernels of the 3D FFT path and their launchers.
 //
-//  k_x_r2c / k_x_c2r : transforms along the contiguous X axis.  Two real rows
-//                      are packed into one complex row (x_a + i x_b) and run
-//                      through one complex FFT; the two half spectra are
+//  k_x_r2c_ct / k_x_c2r_ct : transforms along the contiguous X axis.  Two real
+//                      rows are packed into one complex row (x_a + i x_b) and
+//                      run through one complex FFT; the two half spectra are
 //                      separated (r2c) or merged (c2r) in LDS.  Replaces the
 //                      FFTW r2c/c2r plans of build/fft_exec.F90:495-540,298-342.
-//  k_col             : transform along a strided axis (Y or Z) of a 3D view.
-//                      A workgroup owns TX adjacent inner columns of one outer
-//                      index; loads are coalesced along the inner axis (or along
-//                      the transform axis for the STRIDE1 layout), the pruning
+//  k_colio_ct / k_col_ct : transform along a strided axis (Y or Z) of a 3D view.
+//                      A workgroup owns TX adjacent inner columns; the pruning
 //                      index maps and zero fills of build/module.F90:502-706 are
 //                      applied in the load/store indexing, and DCT-I / DST-I are
-//                      run as complex FFTs of the even / odd extension built in
-//                      LDS (build/fft_exec.F90:646-701, 866-921).
+//                      run as complex FFTs of the even / odd extension
+//                      (build/fft_exec.F90:646-701, 866-921).
+//  Lengths without these compile-time kernels run those of engine_gen.hip.
 //  k_gen_tw          : FP64 twiddle generation (sincospi), stored as double2 or
 //                      as hi+lo float pairs.
 //  k_cheby           : Chebyshev derivative recurrence (build/ftran.F90:408-451)
@@ -26,6 +25,7 @@
 
 #include "engine.hpp"
 #include "engine_ct.hpp"
+#include "engine_gen.hpp"
 
 namespace p3amd {
 
@@ -52,127 +52,6 @@ __device__ __forceinline__ int tile_of(int rev, int xcd = 1) {
   return rev ? (int)gridDim.x - 1 - t : t;
 }
 
-// ---------------------------------------------------------------------------
-// Stockham stages over an LDS tile.  COL layout: element e of sequence b at
-// lds[e*B + b] (B sequences side by side, sequence index fastest).  ROW layout:
-// lds[b*n + e].
-// ---------------------------------------------------------------------------
-template <class T, int R, bool FWD, bool COL, int NT, int EPT>
-__device__ __forceinline__ void stage_r(cpx<T>* lds, const LenDesc& L, int s, int B, FDiv dB,
-                                        const typename TwT<T>::type* tw) {
-  constexpr int IT = EPT / R;
-  static_assert(IT >= 1, "radix larger than the per-thread element budget");
-  const int n = L.n, nR = n / R, Ns = L.ns[s];
-  const int total = B * nR;
-  cpx<T> v[IT][R];
-#pragma unroll
-  for (int m = 0; m < IT; m++) {
-    const int it = threadIdx.x + m * NT;
-    if (it < total) {
-      int b, j;
-      if (COL) { j = fdiv(it, dB); b = it - j * B; }
-      else { b = fdiv(it, L.dnr[s]); j = it - b * nR; }
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        const int e = j + r * nR;
-        v[m][r] = lds[COL ? e * B + b : b * n + e];
-      }
-      if (s > 0) {
-        const int k = j - fdiv(j, L.dns[s]) * Ns;
-        const typename TwT<T>::type* w = tw + L.twoff[s] + k * (R - 1);
-#pragma unroll
-        for (int r = 1; r < R; r++) v[m][r] = twmul<FWD>(v[m][r], w[r - 1]);
-      }
-      dft<R, FWD>(v[m]);
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int m = 0; m < IT; m++) {
-    const int it = threadIdx.x + m * NT;
-    if (it < total) {
-      int b, j;
-      if (COL) { j = fdiv(it, dB); b = it - j * B; }
-      else { b = fdiv(it, L.dnr[s]); j = it - b * nR; }
-      const int k = j - fdiv(j, L.dns[s]) * Ns;
-      const int base = (j - k) * R + k;
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        const int e = base + r * Ns;
-        lds[COL ? e * B + b : b * n + e] = v[m][r];
-      }
-    }
-  }
-  __syncthreads();
-}
-
-// Any radix (used for prime factors above 13): one output per work item,
-// y = sum_r x_r W_{Ns R}^{r (k + q Ns)}, twiddles from the full table W_n^e.
-template <class T, bool FWD, bool COL, int NT, int EPT>
-__device__ __forceinline__ void stage_g(cpx<T>* lds, const LenDesc& L, int s, int B, FDiv dB,
-                                        const typename TwT<T>::type* tw) {
-  const int n = L.n, R = L.radix[s], nR = n / R, Ns = L.ns[s], M = Ns * R, step = n / M;
-  const int total = B * n;
-  const typename TwT<T>::type* wf = tw + L.fulloff;
-  cpx<T> v[EPT];
-#pragma unroll
-  for (int m = 0; m < EPT; m++) {
-    const int it = threadIdx.x + m * NT;
-    if (it < total) {
-      int b, jq;
-      if (COL) { jq = fdiv(it, dB); b = it - jq * B; }
-      else { b = fdiv(it, L.dn); jq = it - b * n; }
-      const int q = fdiv(jq, L.dnr[s]);
-      const int j = jq - q * nR;
-      const int k = j - fdiv(j, L.dns[s]) * Ns;
-      const int inc = k + q * Ns;
-      int e = 0;
-      cpx<T> acc = mk<T>(0, 0);
-      for (int r = 0; r < R; r++) {
-        const int ee = j + r * nR;
-        acc = add(acc, twmul<FWD>(lds[COL ? ee * B + b : b * n + ee], wf[e * step]));
-        e += inc;
-        if (e >= M) e -= M;
-      }
-      v[m] = acc;
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int m = 0; m < EPT; m++) {
-    const int it = threadIdx.x + m * NT;
-    if (it < total) {
-      int b, jq;
-      if (COL) { jq = fdiv(it, dB); b = it - jq * B; }
-      else { b = fdiv(it, L.dn); jq = it - b * n; }
-      const int q = fdiv(jq, L.dnr[s]);
-      const int j = jq - q * nR;
-      const int k = j - fdiv(j, L.dns[s]) * Ns;
-      const int e = (j - k) * R + k + q * Ns;
-      lds[COL ? e * B + b : b * n + e] = v[m];
-    }
-  }
-  __syncthreads();
-}
-
-template <class T, bool FWD, bool COL, int NT, int EPT>
-__device__ void run_fft(cpx<T>* lds, const LenDesc& L, int B, FDiv dB, const typename TwT<T>::type* tw) {
-  for (int s = 0; s < L.nst; s++) {
-    switch (L.radix[s]) {
-      case 2: stage_r<T, 2, FWD, COL, NT, EPT>(lds, L, s, B, dB, tw); break;
-      case 3: stage_r<T, 3, FWD, COL, NT, EPT>(lds, L, s, B, dB, tw); break;
-      case 4: stage_r<T, 4, FWD, COL, NT, EPT>(lds, L, s, B, dB, tw); break;
-      case 5: stage_r<T, 5, FWD, COL, NT, EPT>(lds, L, s, B, dB, tw); break;
-      case 7: stage_r<T, 7, FWD, COL, NT, EPT>(lds, L, s, B, dB, tw); break;
-      case 8: stage_r<T, 8, FWD, COL, NT, EPT>(lds, L, s, B, dB, tw); break;
-      case 11: stage_r<T, 11, FWD, COL, NT, EPT>(lds, L, s, B, dB, tw); break;
-      case 13: stage_r<T, 13, FWD, COL, NT, EPT>(lds, L, s, B, dB, tw); break;
-      case 16: stage_r<T, 16, FWD, COL, NT, EPT>(lds, L, s, B, dB, tw); break;
-      default: stage_g<T, FWD, COL, NT, EPT>(lds, L, s, B, dB, tw); break;
-    }
-  }
-}
-
 // copy the twiddle table into LDS behind the data tile
 template <class T, int NT>
 __device__ __forceinline__ const typename TwT<T>::type* stage_twiddles(unsigned char* smem, size_t off,
@@ -187,6 +66,11 @@ __device__ __forceinline__ const typename TwT<T>::type* stage_twiddles(unsigned 
 // ---------------------------------------------------------------------------
 // X kernels
 // ---------------------------------------------------------------------------
+// a length as the specialised kernels see it
+struct CtLenArg {
+  int n, twcount;
+};
+
 struct XArgs {
   const void* in;
   void* out;
@@ -194,7 +78,7 @@ struct XArgs {
   int nxo;     // r2c: kept modes; c2r: valid input modes
   int B;       // row pairs per workgroup
   FDiv dnxo;
-  LenDesc L;
+  CtLenArg L;
   const void* tw;
   int tw_lds;  // twiddles staged in LDS
   int tw_off;  // byte offset of the staged twiddles
@@ -205,69 +89,6 @@ struct XArgs {
 };
 
 extern __shared__ __align__(16) unsigned char g_smem[];
-
-template <class T, int NT, int EPT>
-__global__ __launch_bounds__(NT) void k_x_r2c(XArgs a) {
-  typedef typename TwT<T>::type TwL;
-  cpx<T>* lds = (cpx<T>*)g_smem;
-  const int n = a.L.n, B = a.B;
-  const TwL* tw = (const TwL*)a.tw;
-  if (a.tw_lds) tw = stage_twiddles<T, NT>(g_smem, a.tw_off, tw, a.L.twcount);
-  const long long pair0 = (long long)tile_of(a.rev) * B;
-  const T* in = (const T*)a.in;
-  for (int q = threadIdx.x; q < B * n; q += NT) {
-    const int b = fdiv(q, a.L.dn), j = q - b * n;
-    const long long ra = 2 * (pair0 + b), rb = ra + 1;
-    const T xa = ra < a.nrows ? in[ra * a.si_row + j] : (T)0;
-    const T xb = rb < a.nrows ? in[rb * a.si_row + j] : (T)0;
-    lds[b * n + j] = mk<T>(xa, xb);
-  }
-  __syncthreads();
-  run_fft<T, true, false, NT, EPT>(lds, a.L, B, FDiv{0, 1}, tw);
-  cpx<T>* out = (cpx<T>*)a.out;
-  const T h = (T)0.5;
-  for (int q = threadIdx.x; q < B * a.nxo; q += NT) {
-    const int b = fdiv(q, a.dnxo), k = q - b * a.nxo;
-    const cpx<T> zk = lds[b * n + k], zn = lds[b * n + (k == 0 ? 0 : n - k)];
-    const long long ra = 2 * (pair0 + b), rb = ra + 1;
-    if (ra < a.nrows) out[ra * a.so_row + k] = mk<T>((zk.x + zn.x) * h, (zk.y - zn.y) * h);
-    if (rb < a.nrows) out[rb * a.so_row + k] = mk<T>((zk.y + zn.y) * h, (zn.x - zk.x) * h);
-  }
-}
-
-template <class T, int NT, int EPT>
-__global__ __launch_bounds__(NT) void k_x_c2r(XArgs a) {
-  typedef typename TwT<T>::type TwL;
-  cpx<T>* lds = (cpx<T>*)g_smem;
-  const int n = a.L.n, B = a.B, h = n / 2;
-  const TwL* tw = (const TwL*)a.tw;
-  if (a.tw_lds) tw = stage_twiddles<T, NT>(g_smem, a.tw_off, tw, a.L.twcount);
-  const long long pair0 = (long long)tile_of(a.rev) * B;
-  const cpx<T>* in = (const cpx<T>*)a.in;
-  for (int q = threadIdx.x; q < B * n; q += NT) {
-    const int b = fdiv(q, a.L.dn), k = q - b * n;
-    const long long ra = 2 * (pair0 + b), rb = ra + 1;
-    const int kk = k <= h ? k : n - k;
-    cpx<T> A = mk<T>(0, 0), Bv = mk<T>(0, 0);
-    if (kk < a.nxo) {
-      if (ra < a.nrows) A = in[ra * a.si_row + kk];
-      if (rb < a.nrows) Bv = in[rb * a.si_row + kk];
-    }
-    // FFTW c2r: the imaginary parts of k=0 and k=n/2 (n even) do not contribute
-    if (kk == 0 || 2 * kk == n) { A.y = 0; Bv.y = 0; }
-    lds[b * n + k] = (k == kk) ? mk<T>(A.x - Bv.y, A.y + Bv.x) : mk<T>(A.x + Bv.y, Bv.x - A.y);
-  }
-  __syncthreads();
-  run_fft<T, false, false, NT, EPT>(lds, a.L, B, FDiv{0, 1}, tw);
-  T* out = (T*)a.out;
-  for (int q = threadIdx.x; q < B * n; q += NT) {
-    const int b = fdiv(q, a.L.dn), j = q - b * n;
-    const long long ra = 2 * (pair0 + b), rb = ra + 1;
-    const cpx<T> z = lds[b * n + j];
-    if (ra < a.nrows) out[ra * a.so_row + j] = z.x;
-    if (rb < a.nrows) out[rb * a.so_row + j] = z.y;
-  }
-}
 
 // ---------------------------------------------------------------------------
 // column kernel
@@ -284,8 +105,7 @@ struct ColArgs {
   int nst, st_lo, st_shift;
   int ld_lenfast, st_lenfast;
   FDiv dnld, dnst;
-  int nrows_lds;  // rows of the LDS tile
-  LenDesc L;
+  CtLenArg L;
   const void* tw;
   int tw_lds, tw_off;
   int rev;  // walk the tiles from the last one
@@ -308,69 +128,8 @@ struct ColArgs {
   int mirror;
 };
 
-template <class T, bool FWD, int NT, int EPT>
-__global__ __launch_bounds__(NT) void k_col(ColArgs a) {
-  typedef typename TwT<T>::type TwL;
-  cpx<T>* lds = (cpx<T>*)g_smem;
-  const int TX = a.TX;
-  const int t = xcd_tile(blockIdx.x, gridDim.x);
-  const int o = t / a.tiles;
-  const int ti = t - o * a.tiles;
-  const long long i0 = (long long)ti * TX;
-  const int nb = (int)((long long)a.n_inner - i0 < TX ? (long long)a.n_inner - i0 : TX);
-  const cpx<T>* in = (const cpx<T>*)a.in + i0 * a.si_in + (long long)o * a.so_in;
-  cpx<T>* out = (cpx<T>*)a.out + i0 * a.si_out + (long long)o * a.so_out;
-  const TwL* tw = (const TwL*)a.tw;
-  if (a.tw_lds) tw = stage_twiddles<T, NT>(g_smem, a.tw_off, tw, a.L.twcount);
-  const int off = (a.kind == COL_DST1) ? 1 : 0;
-  for (int q = threadIdx.x; q < TX * a.nld; q += NT) {
-    int b, e;
-    if (a.ld_lenfast) { b = fdiv(q, a.dnld); e = q - b * a.nld; }
-    else { e = fdiv(q, a.dTX); b = q - e * TX; }
-    cpx<T> v = mk<T>(0, 0);
-    if (b < nb) {
-      const int src = e < a.ld_lo ? e : (e >= a.ld_hi ? e - a.ld_shift : -1);
-      if (src >= 0) v = in[(long long)b * a.si_in + (long long)src * a.sl_in];
-    }
-    lds[(e + off) * TX + b] = v;
-  }
-  __syncthreads();
-  if (a.kind == COL_DCT1) {
-    // even extension of length m = 2(nld-1): row e <- row m-e
-    const int m = a.L.n;
-    for (int q = threadIdx.x; q < TX * (m - a.nld); q += NT) {
-      const int r = fdiv(q, a.dTX), b = q - r * TX, e = a.nld + r;
-      lds[e * TX + b] = lds[(m - e) * TX + b];
-    }
-    __syncthreads();
-  } else if (a.kind == COL_DST1) {
-    // odd extension of length m = 2(nld+1): rows 0 and nld+1 zero, row e <- -row m-e
-    const int m = a.L.n;
-    for (int q = threadIdx.x; q < TX * (m - a.nld - 1); q += NT) {
-      const int r = fdiv(q, a.dTX), b = q - r * TX, e = a.nld + 1 + r;
-      if (e == a.nld + 1) lds[e * TX + b] = mk<T>(0, 0);
-      else { const cpx<T> u = lds[(m - e) * TX + b]; lds[e * TX + b] = mk<T>(-u.x, -u.y); }
-    }
-    for (int b = threadIdx.x; b < TX; b += NT) lds[b] = mk<T>(0, 0);
-    __syncthreads();
-  }
-  if (a.kind != COL_COPY) run_fft<T, FWD, true, NT, EPT>(lds, a.L, TX, a.dTX, tw);
-  for (int q = threadIdx.x; q < TX * a.nst; q += NT) {
-    int b, e;
-    if (a.st_lenfast) { b = fdiv(q, a.dnst); e = q - b * a.nst; }
-    else { e = fdiv(q, a.dTX); b = q - e * TX; }
-    if (b < nb) {
-      const int p = e < a.st_lo ? e : e + a.st_shift;
-      cpx<T> v;
-      if (a.kind == COL_DST1) { const cpx<T> u = lds[(p + 1) * TX + b]; v = mk<T>(-u.y, u.x); }
-      else v = lds[p * TX + b];
-      out[(long long)b * a.si_out + (long long)e * a.sl_out] = v;
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
-// compile-time specialised kernels (same arguments and semantics as above).
+// compile-time specialised kernels.
 // TWL: the twiddle table is staged in LDS (decided per length at compile
 // time, so twiddle reads are LDS reads).  Addresses are a wave-uniform 64-bit
 // tile base plus 32-bit byte offsets (the host checks that they fit).
@@ -1630,9 +1389,9 @@ static FDiv make_fdiv(int d) {
   return f;
 }
 
-// stage radices: radix 8 as far as possible (two 4s instead of an 8 and a 2),
-// then 3, 5, 7, 11, 13, then any remaining prime (generic stage)
-static std::vector<int> factorize(int n) {
+// stage radices of the specialised lengths: radix 8 as far as possible (two 4s
+// instead of an 8 and a 2), then 3 and 5
+static std::vector<int> ct_factors(int n) {
   // 2048 with radix 16: three stages (two LDS exchanges instead of three),
   // the share-mode length-2048 stages 4-10% faster; radix 16 for 256, 384
   // and 1024 measured no faster (kernel trace of 384^3 FP32: 505 against
@@ -1646,82 +1405,92 @@ static std::vector<int> factorize(int n) {
   else if (rem == 1) f.push_back(2);
   else if (rem == 2) f.push_back(4);
   for (int i = 0; i < n8; i++) f.insert(f.begin(), 8);
-  for (int p : {3, 5, 7, 11, 13})
+  for (int p : {3, 5})
     while (m % p == 0) { f.push_back(p); m /= p; }
-  for (int p = 17; (long long)p * p <= m; p += 2)
-    while (m % p == 0) { f.push_back(p); m /= p; }
-  if (m > 1) f.push_back(m);
   return f;
-}
-
-static bool is_templated(int r) {
-  return r == 2 || r == 3 || r == 4 || r == 5 || r == 7 || r == 8 || r == 11 || r == 13 || r == 16;
 }
 
 static std::mutex g_len_mu;
 static std::map<int, Len1D> g_lens;
 static std::vector<tw_t*> g_retired_tw;
 static void prep_kernels(const Len1D& L);
+static bool has_ct_schedule(int n);
 
-std::vector<int> default_factors(int n) { return n > 1 ? factorize(n) : std::vector<int>{}; }
+// the device table of the twiddles exp(-2 pi i x / y), one per entry
+static tw_t* gen_table(const std::vector<int2>& idx) {
+  if (idx.empty()) return nullptr;
+  const int cnt = (int)idx.size();
+  int2* didx = nullptr;
+  tw_t* tw = nullptr;
+  check_hip(hipMalloc(&didx, cnt * sizeof(int2)), "hipMalloc(twiddle index)");
+  check_hip(hipMemcpy(didx, idx.data(), cnt * sizeof(int2), hipMemcpyHostToDevice), "hipMemcpy");
+  check_hip(hipMalloc(&tw, cnt * sizeof(Tw)), "hipMalloc(twiddles)");
+  k_gen_tw<Tw><<<(cnt + 255) / 256, 256>>>(didx, cnt, tw);
+  check_hip(hipGetLastError(), "k_gen_tw launch");
+  check_hip(hipDeviceSynchronize(), "k_gen_tw");
+  check_hip(hipFree(didx), "hipFree");
+  return tw;
+}
 
-// plan of length n with the radix schedule f (stage s has radix f[s]):
-// stage descriptors and the FP64-generated twiddle table
-static Len1D build_len(int n, const std::vector<int>& f) {
-  Len1D L;
-  std::memset(&L.d, 0, sizeof(L.d));
-  L.d.n = n;
+std::vector<int> default_factors(int n) { return has_ct_schedule(n) ? ct_factors(n) : gen_factors(n); }
+
+// stage descriptor of the radix schedule f and its FP64-generated twiddle
+// table: stage s > 0 has W_{Ns R}^{k r}, k < Ns, r = 1..R-1, a prime stage of
+// the run-time kernels also W_R^j, j < R
+static LenDesc build_desc(int n, const std::vector<int>& f, tw_t** tw) {
+  LenDesc d;
+  std::memset(&d, 0, sizeof(d));
+  d.n = n;
   long long prod = 1;
   for (int r : f) prod *= r;
-  if ((n > 1 && prod != n) || (n <= 1 && !f.empty())) throw Error{"radix schedule does not multiply to the length", -1};
+  if (prod != n) throw Error{"radix schedule does not multiply to the length", -1};
   if ((int)f.size() > kMaxStages) throw Error{"transform length has too many factors", -1};
   std::vector<int2> idx;
   int ns = 1;
   for (size_t s = 0; s < f.size(); s++) {
     const int R = f[s];
-    L.d.radix[s] = R;
-    L.d.ns[s] = ns;
-    L.d.twoff[s] = (int)idx.size();
-    L.d.dns[s] = make_fdiv(ns);
-    L.d.dnr[s] = make_fdiv(n / R);
-    if (!is_templated(R)) L.has_generic = true;
-    if (s > 0 && is_templated(R))
+    d.radix[s] = R;
+    d.ns[s] = ns;
+    d.twoff[s] = (int)idx.size();
+    if (s > 0)
       for (int k = 0; k < ns; k++)
         for (int r = 1; r < R; r++) idx.push_back(make_int2(k * r, ns * R));
+    if (gen_is_prime_stage(R))
+      for (int j = 0; j < R; j++) idx.push_back(make_int2(j, R));
     ns *= R;
   }
-  L.d.nst = (int)f.size();
-  L.d.dn = make_fdiv(n);
-  L.d.fulloff = (int)idx.size();
-  if (L.has_generic)
-    for (int e = 0; e < n; e++) idx.push_back(make_int2(e, n));
-  L.d.twcount = (int)idx.size();
+  d.nst = (int)f.size();
+  d.twcount = (int)idx.size();
+  *tw = gen_table(idx);
+  return d;
+}
+
+// plan of length n with the radix schedule f: the specialised kernels' (and
+// the run-time kernels' where they have its radices)
+static Len1D build_len(int n, const std::vector<int>& f0) {
+  Len1D L;
+  const std::vector<int> f = has_ct_schedule(n) ? f0 : gen_wrap(f0);
+  L.d = build_desc(n, f, &L.tw);
+  bool runtime = !f.empty();
+  for (int r : f) runtime = runtime && (gen_in_registers(r) || gen_is_prime_stage(r));
+  if (runtime && has_ct_schedule(n)) runtime = gen_wrap(f) == f;
+  L.gtw = L.tw;
+  L.gd = L.d;
+  if (!runtime) L.gd = build_desc(n, gen_factors(n), &L.gtw);
   if (n == 512) {
     // the wave kernels' table W_512^e
     std::vector<int2> fidx(n);
     for (int e = 0; e < n; e++) fidx[e] = make_int2(e, n);
-    int2* didx = nullptr;
-    check_hip(hipMalloc(&didx, n * sizeof(int2)), "hipMalloc(twiddle index)");
-    check_hip(hipMemcpy(didx, fidx.data(), n * sizeof(int2), hipMemcpyHostToDevice), "hipMemcpy");
-    check_hip(hipMalloc(&L.twf, n * sizeof(Tw)), "hipMalloc(twiddles)");
-    k_gen_tw<Tw><<<(n + 255) / 256, 256>>>(didx, n, L.twf);
-    check_hip(hipGetLastError(), "k_gen_tw launch");
-    check_hip(hipDeviceSynchronize(), "k_gen_tw");
-    check_hip(hipFree(didx), "hipFree");
-  }
-  if (!idx.empty()) {
-    int2* didx = nullptr;
-    check_hip(hipMalloc(&didx, idx.size() * sizeof(int2)), "hipMalloc(twiddle index)");
-    check_hip(hipMemcpy(didx, idx.data(), idx.size() * sizeof(int2), hipMemcpyHostToDevice), "hipMemcpy");
-    check_hip(hipMalloc(&L.tw, idx.size() * sizeof(Tw)), "hipMalloc(twiddles)");
-    const int cnt = (int)idx.size();
-    k_gen_tw<Tw><<<(cnt + 255) / 256, 256>>>(didx, cnt, L.tw);
-    check_hip(hipGetLastError(), "k_gen_tw launch");
-    check_hip(hipDeviceSynchronize(), "k_gen_tw");
-    check_hip(hipFree(didx), "hipFree");
+    L.twf = gen_table(fidx);
   }
   prep_kernels(L);
   return L;
+}
+
+static void retire(Len1D& L, std::vector<tw_t*>& to) {
+  if (L.tw) to.push_back(L.tw);
+  if (L.gtw && L.gtw != L.tw) to.push_back(L.gtw);
+  if (L.twf) to.push_back(L.twf);
 }
 
 const Len1D& get_len(int n) {
@@ -1745,48 +1514,21 @@ void set_len_plan(int n, const std::vector<int>& factors, bool ct_ok, int tile_b
   }
   // the old table is retired, not freed: launches captured earlier (graphs)
   // may still read it; retired tables are freed with the plans
-  if (it->second.tw) g_retired_tw.push_back(it->second.tw);
-  if (it->second.twf) g_retired_tw.push_back(it->second.twf);
+  retire(it->second, g_retired_tw);
   it->second = L;  // same map node: references to the entry stay valid
 }
 
 void free_lens() {
   std::lock_guard<std::mutex> lk(g_len_mu);
   (void)hipDeviceSynchronize();
-  for (auto& kv : g_lens) {
-    if (kv.second.tw) (void)hipFree(kv.second.tw);
-    if (kv.second.twf) (void)hipFree(kv.second.twf);
-  }
+  for (auto& kv : g_lens) retire(kv.second, g_retired_tw);
   for (tw_t* t : g_retired_tw) (void)hipFree(t);
   g_retired_tw.clear();
   g_lens.clear();
 }
 
-// Per-thread element budget of every stage (registers hold EPT complex values)
-// and the workgroup sizes the kernels are built for.
-static const int kEPT = 16;
-static const int kNTs[] = {64, 128, 256, 512, 1024};
 static constexpr size_t kLdsMax = 160 * 1024;
-// data bytes per tile the tile-shape heuristics aim for (two tiles per CU)
-static const size_t kTileBytes = 64 * 1024;
-
 int max_len() { return 8192; }
-
-// elements one thread can own in every stage of this length
-static int len_cap_per_thread(const Len1D& L) {
-  int c = kEPT;
-  for (int s = 0; s < L.d.nst; s++) {
-    const int R = L.d.radix[s];
-    if (is_templated(R)) c = std::min(c, R * (kEPT / R));
-  }
-  return c;
-}
-
-static int pick_nt(long long elems, int cpt) {
-  for (int nt : kNTs)
-    if (elems <= (long long)nt * cpt) return nt;
-  throw Error{"transform tile exceeds the 1024-thread workgroup capacity", -1};
-}
 
 // dynamic LDS up to the CU's 160 KiB less the kernel's static LDS
 template <class K>
@@ -1796,60 +1538,6 @@ static void allow_big_lds(K kernel) {
   if (hipFuncGetAttributes(&fa, (const void*)kernel) == hipSuccess) stat = fa.sharedSizeBytes;
   (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kLdsMax - stat));
   (void)hipGetLastError();  // a refused attribute leaves the default limit, not a pending error
-}
-
-// choose where twiddles live; returns LDS bytes
-static size_t lds_layout(size_t data_bytes, const Len1D& L, int* tw_lds, int* tw_off) {
-  size_t off = (data_bytes + 15) & ~(size_t)15;
-  size_t twb = (size_t)L.d.twcount * sizeof(Tw);
-  if (L.d.twcount > 0 && off + twb <= 96 * 1024) {
-    *tw_lds = 1;
-    *tw_off = (int)off;
-    return off + twb;
-  }
-  *tw_lds = 0;
-  *tw_off = 0;
-  return data_bytes;
-}
-
-constexpr int kEPTc = 16;
-
-// launch functors: one per kernel family, instantiated per workgroup size
-struct GoXr2c {
-  template <int NT>
-  static void go(const XArgs& a, unsigned g, size_t b, hipStream_t s) {
-    k_x_r2c<real_t, NT, kEPTc><<<g, NT, b, s>>>(a);
-  }
-  template <int NT>
-  static void prep() { allow_big_lds(k_x_r2c<real_t, NT, kEPTc>); }
-};
-struct GoXc2r {
-  template <int NT>
-  static void go(const XArgs& a, unsigned g, size_t b, hipStream_t s) {
-    k_x_c2r<real_t, NT, kEPTc><<<g, NT, b, s>>>(a);
-  }
-  template <int NT>
-  static void prep() { allow_big_lds(k_x_c2r<real_t, NT, kEPTc>); }
-};
-template <bool FWD>
-struct GoCol {
-  template <int NT>
-  static void go(const ColArgs& a, unsigned g, size_t b, hipStream_t s) {
-    k_col<real_t, FWD, NT, kEPTc><<<g, NT, b, s>>>(a);
-  }
-  template <int NT>
-  static void prep() { allow_big_lds(k_col<real_t, FWD, NT, kEPTc>); }
-};
-
-template <class F, class A>
-static void dispatch_nt(int nt, const A& a, unsigned g, size_t b, hipStream_t s) {
-  switch (nt) {
-    case 64: F::template go<64>(a, g, b, s); break;
-    case 128: F::template go<128>(a, g, b, s); break;
-    case 256: F::template go<256>(a, g, b, s); break;
-    case 512: F::template go<512>(a, g, b, s); break;
-    default: F::template go<1024>(a, g, b, s); break;
-  }
 }
 
 // ---- compile-time specialised lengths ----------------------------------
@@ -2090,18 +1778,24 @@ struct CtLen {
   }
 };
 
-// Specialised kernel set for a length, if one exists and its radix schedule
-// matches the length plan (the twiddle tables are laid out by that schedule).
-static const CtInfo* find_ct(const Len1D& L) {
-  if (!L.ct_ok) return nullptr;
+// the lengths that have specialised kernels
+static const std::map<int, CtInfo>& ct_table() {
   static const std::map<int, CtInfo> tab = {
       {32, CtLen<8, 4>::info()},       {48, CtLen<4, 4, 3>::info()},    {64, CtLen<8, 8>::info()},
       {96, CtLen<8, 4, 3>::info()},    {128, CtLen<8, 4, 4>::info()},   {160, CtLen<8, 4, 5>::info()},
       {192, CtLen<8, 8, 3>::info()},   {256, CtLen<8, 8, 4>::info()},   {320, CtLen<8, 8, 5>::info()},
       {384, CtLen<8, 4, 4, 3>::info()}, {512, CtLen<8, 8, 8>::info()},  {1024, CtLen<8, 8, 4, 4>::info()},
       {2048, CtLen<16, 16, 8>::info()}};
-  auto it = tab.find(L.d.n);
-  if (it == tab.end()) return nullptr;
+  return tab;
+}
+static bool has_ct_schedule(int n) { return ct_table().count(n) != 0; }
+
+// Specialised kernel set for a length, if one exists and its radix schedule
+// matches the length plan (the twiddle tables are laid out by that schedule).
+static const CtInfo* find_ct(const Len1D& L) {
+  if (!L.ct_ok) return nullptr;
+  auto it = ct_table().find(L.d.n);
+  if (it == ct_table().end()) return nullptr;
   const CtInfo& c = it->second;
   if (c.nr != L.d.nst) return nullptr;
   for (int i = 0; i < c.nr; i++)
@@ -2109,32 +1803,18 @@ static const CtInfo* find_ct(const Len1D& L) {
   return &c;
 }
 
-bool len_has_ct(int n) {
-  Len1D probe;
-  std::memset(&probe.d, 0, sizeof(probe.d));
-  const std::vector<int> f = default_factors(n);
-  probe.d.n = n;
-  probe.d.nst = (int)f.size();
-  for (size_t i = 0; i < f.size() && i < (size_t)kMaxStages; i++) probe.d.radix[i] = f[i];
-  return find_ct(probe) != nullptr;
-}
+bool len_has_ct(int n) { return has_ct_schedule(n); }
 
 std::string len_describe(int n) {
   const Len1D& L = get_len(n);
-  std::string r = "radix ";
-  for (int s = 0; s < L.d.nst; s++) r += (s ? "x" : "") + std::to_string(L.d.radix[s]);
-  if (find_ct(L)) return r + ", specialised";
-  return r + ", generic, tile " + std::to_string(L.tile_bytes / 1024) + " KiB, segment " +
+  auto radices = [](const LenDesc& d) {
+    std::string r = "radix ";
+    for (int s = 0; s < d.nst; s++) r += (s ? "x" : "") + std::to_string(d.radix[s]);
+    return r;
+  };
+  if (find_ct(L)) return radices(L.d) + ", specialised";
+  return radices(L.gd) + ", run-time, tile " + std::to_string(L.tile_bytes / 1024) + " KiB, segment " +
          std::to_string(L.col_seg) + " B";
-}
-
-template <class F>
-static void prep_generic_nt() {
-  F::template prep<64>();
-  F::template prep<128>();
-  F::template prep<256>();
-  F::template prep<512>();
-  F::template prep<1024>();
 }
 
 // Kernel attributes (the dynamic-LDS limit) are set when a length is first
@@ -2142,15 +1822,12 @@ static void prep_generic_nt() {
 // transform, which is what stream capture into a graph requires.
 static void prep_plane_kernels(int n);
 static void prep_kernels(const Len1D& L) {
-  static bool generic_done = false;
-  if (!generic_done) {
-    prep_generic_nt<GoXr2c>();
-    prep_generic_nt<GoXc2r>();
-    prep_generic_nt<GoCol<true>>();
-    prep_generic_nt<GoCol<false>>();
+  static bool spectrum_done = false;
+  if (!spectrum_done) {
     allow_big_lds(k_spectrum<real_t>);
-    generic_done = true;
+    spectrum_done = true;
   }
+  gen_prep_kernels();
   if (const CtInfo* c = find_ct(L)) c->prep();
   prep_plane_kernels(L.d.n);
 }
@@ -2188,32 +1865,6 @@ void set_tile_order(bool alternate) { g_alt_order = alternate; }
 bool tile_order_alternate() { return g_alt_order; }
 void set_specialised(bool on) { g_use_ct = on; }
 
-// row-pair count per X tile
-static long long x_pairs_per_tile(const Len1D& L, int nx, long long pairs) {
-  const long long tgt = (long long)(L.tile_bytes / sizeof(cplx_t));
-  long long B = std::max<long long>(1, tgt / nx);
-  // keep at least ~2048 workgroups in flight when the problem allows
-  B = std::min<long long>(B, std::max<long long>(1, pairs / 2048));
-  return B;
-}
-
-static void x_setup(XArgs& a, const Len1D& L, long long nrows, int nx, size_t* bytes, int* nt, unsigned* nwg) {
-  const long long pairs = (nrows + 1) / 2;
-  long long B = x_pairs_per_tile(L, nx, pairs);
-  const int cpt = len_cap_per_thread(L);
-  while (B > 1 && B * nx > 1024LL * cpt) B--;
-  a.B = (int)B;
-  a.L = L.d;
-  a.tw = L.tw;
-  const long long elems = B * nx;
-  *bytes = lds_layout((size_t)elems * sizeof(cplx_t), L, &a.tw_lds, &a.tw_off);
-  if (*bytes > kLdsMax) throw Error{"X transform does not fit in LDS", -1};
-  *nt = pick_nt(elems, cpt);
-  const long long g = (pairs + B - 1) / B;
-  if (g > 0x7fffffffLL) throw Error{"grid too large", -1};
-  *nwg = (unsigned)g;
-}
-
 // LDS bytes of a specialised tile of `data` bytes; sets the twiddle placement
 static size_t ct_lds(size_t data, bool twl, const CtInfo& c, int* tw_lds, int* tw_off) {
   const size_t d16 = (size_t)round16((long long)data);
@@ -2229,7 +1880,7 @@ static bool x_setup_ct(XArgs& a, const Len1D& L, const CtInfo& c, long long nrow
   if (span >= (1LL << 32)) return false;
   const long long pairs = (nrows + 1) / 2;
   a.B = c.BX;
-  a.L = L.d;
+  a.L = CtLenArg{L.d.n, L.d.twcount};
   a.tw = L.tw;
   *bytes = ct_lds((size_t)(c.BX + 1) * L.d.n * sizeof(cplx_t), c.twl_x, c, &a.tw_lds, &a.tw_off);
   const long long g = (pairs + c.BX - 1) / c.BX;
@@ -2281,10 +1932,7 @@ void launch_x_r2c(const real_t* in, cplx_t* out, long long nrows, long long si_r
       return;
     }
   }
-  size_t bytes; int nt; unsigned nwg;
-  x_setup(a, L, nrows, nx, &bytes, &nt, &nwg);
-  dispatch_nt<GoXr2c>(nt, a, nwg, bytes, st);
-  check_hip(hipGetLastError(), "k_x_r2c launch");
+  gen_launch_x_r2c(L, in, out, nrows, si_row, so_row, nxo, rev, st);
 }
 
 bool launch_x_r2c_tab(const real_t* in, cplx_t* out, long long nrows, int nx, int nxo, const int2* xt,
@@ -2347,10 +1995,7 @@ void launch_x_c2r(const cplx_t* in, real_t* out, long long nrows, long long si_r
       return;
     }
   }
-  size_t bytes; int nt; unsigned nwg;
-  x_setup(a, L, nrows, nx, &bytes, &nt, &nwg);
-  dispatch_nt<GoXc2r>(nt, a, nwg, bytes, st);
-  check_hip(hipGetLastError(), "k_x_c2r launch");
+  gen_launch_x_c2r(L, in, out, nrows, si_row, so_row, nxi, rev, st);
 }
 
 // Plane kernels (k_xy_plane_fwd / k_yx_plane_bwd) for the (nx, ny) pairs
@@ -2491,7 +2136,7 @@ bool launch_col_tab(const ColSpec& c, const int2* ltab, const int2* stab, hipStr
   a.TX = TX;
   a.dTX = make_fdiv(TX);
   a.tiles = (c.n_inner + TX - 1) / TX;
-  a.L = L.d;
+  a.L = CtLenArg{L.d.n, L.d.twcount};
   a.tw = L.tw;
   if (g_col_pipe && ct->pipe) {
     size_t pb = ct_lds((size_t)TX * c.n * sizeof(cplx_t), ct->twl_pipe_tab, *ct, &a.tw_lds, &a.tw_off);
@@ -2548,7 +2193,6 @@ bool launch_col(const ColSpec& c, hipStream_t st) {
     nfft = m;
   }
   const int rows = std::max(nfft, c.nld + (c.kind == COL_DST1 ? 2 : 0));
-  a.nrows_lds = rows;
   a.ld_lenfast = (c.sl_in == 1 && c.si_in != 1) ? 1 : 0;
   a.st_lenfast = (c.sl_out == 1 && c.si_out != 1) ? 1 : 0;
   a.dnld = make_fdiv(c.nld);
@@ -2561,7 +2205,7 @@ bool launch_col(const ColSpec& c, hipStream_t st) {
     a.TX = TX;
     a.dTX = make_fdiv(TX);
     a.tiles = (c.n_inner + TX - 1) / TX;
-    a.L = L->d;
+    a.L = CtLenArg{L->d.n, L->d.twcount};
     a.tw = L->tw;
     const size_t bytes = ct_lds((size_t)TX * rows * sizeof(cplx_t), ct->twl_col, *ct, &a.tw_lds, &a.tw_off);
     if (bytes > kLdsMax) throw Error{"column transform does not fit in LDS", -1};
@@ -2612,34 +2256,7 @@ bool launch_col(const ColSpec& c, hipStream_t st) {
     check_hip(hipGetLastError(), "k_col_ct launch");
     return a.cheby != 0;
   }
-  const int cpt = L ? len_cap_per_thread(*L) : kEPT;
-  // tile width: one segment of adjacent columns (128 bytes unless the plan
-  // says otherwise) per row where capacity allows
-  int TX = std::max(1, (int)((L ? L->col_seg : 128) / (int)sizeof(cplx_t)));
-  const long long tgt = (long long)((L ? (size_t)L->tile_bytes : kTileBytes) / sizeof(cplx_t));
-  while (TX > 1 && (long long)TX * rows > std::max<long long>(tgt, rows)) TX /= 2;
-  while (TX > 1 && (long long)TX * rows > 1024LL * cpt) TX /= 2;
-  while (TX > 1 && TX / 2 >= c.n_inner) TX /= 2;
-  a.TX = TX;
-  a.dTX = make_fdiv(TX);
-  a.tiles = (c.n_inner + TX - 1) / TX;
-  const long long nwg = (long long)a.tiles * c.n_outer;
-  if (nwg > 0x7fffffffLL) throw Error{"grid too large", -1};
-  const long long elems = (long long)TX * rows;
-  size_t bytes;
-  if (L) {
-    a.L = L->d;
-    a.tw = L->tw;
-    bytes = lds_layout((size_t)elems * sizeof(cplx_t), *L, &a.tw_lds, &a.tw_off);
-  } else {
-    a.L.n = nfft;
-    bytes = (size_t)elems * sizeof(cplx_t);
-  }
-  if (bytes > kLdsMax) throw Error{"column transform does not fit in LDS", -1};
-  const int nt = pick_nt(elems, cpt);
-  if (fwd) dispatch_nt<GoCol<true>>(nt, a, (unsigned)nwg, bytes, st);
-  else dispatch_nt<GoCol<false>>(nt, a, (unsigned)nwg, bytes, st);
-  check_hip(hipGetLastError(), "k_col launch");
+  gen_launch_col(L, c, a.xcd, st);
   return false;
 }
 
@@ -2658,7 +2275,7 @@ bool launch_zsolve(cplx_t* spec, int nxh, int ny, int nz, double scale, hipStrea
   const int TX = ct->TX;
   a.TX = TX;
   a.tiles = (int)((ninner + TX - 1) / TX);
-  a.L = L.d;
+  a.L = CtLenArg{L.d.n, L.d.twcount};
   a.tw = L.tw;
   if ((ninner + (long long)nz * ninner + TX) * (long long)sizeof(cplx_t) >= (1LL << 32)) return false;
   const size_t bytes = ct_lds((size_t)TX * nz * sizeof(cplx_t), ct->twl_col, *ct, &a.tw_lds, &a.tw_off);
@@ -2781,7 +2398,7 @@ GroupBatch* group_batch_create(int mode, int n, const int* shapes, real_t* const
         a.nxo = nxh;
         a.dnxo = make_fdiv(nxh);
         a.B = ct->BX;
-        a.L = L.d;
+        a.L = CtLenArg{L.d.n, L.d.twcount};
         a.tw = L.tw;
         h.s.bytes = ct_lds((size_t)(ct->BX + 1) * len * sizeof(cplx_t), ct->twl_x, *ct, &a.tw_lds, &a.tw_off);
       } else {
@@ -2789,7 +2406,7 @@ GroupBatch* group_batch_create(int mode, int n, const int* shapes, real_t* const
         a.kind = COL_C2C;
         a.TX = ct->TX;
         a.dTX = make_fdiv(ct->TX);
-        a.L = L.d;
+        a.L = CtLenArg{L.d.n, L.d.twcount};
         a.tw = L.tw;
         h.s.bytes = ct_lds((size_t)ct->TX * len * sizeof(cplx_t), ct->twl_col, *ct, &a.tw_lds, &a.tw_off);
       }

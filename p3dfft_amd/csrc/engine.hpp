@@ -32,9 +32,12 @@ void check_hip(hipError_t e, const char* what);
 // A 1D length with its stage schedule and device twiddle table.
 struct Len1D {
   LenDesc d;
-  tw_t* tw = nullptr;  // device table: stage twiddles then (if needed) W_n^e
+  tw_t* tw = nullptr;  // device table of the stage twiddles
+  // schedule and table of the run-time kernels (engine_gen.hip): d and tw,
+  // unless those hold a radix only the specialised kernels have
+  LenDesc gd;
+  tw_t* gtw = nullptr;
   tw_t* twf = nullptr; // W_n^e, e < n, for the wave kernels of n = 512
-  bool has_generic = false;
   // plan choices (plan-time measurement may change them): specialised
   // kernels allowed; data bytes per tile and bytes of adjacent columns per
   // row segment of the run-time-generic kernels

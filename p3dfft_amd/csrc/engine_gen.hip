@@ -1,0 +1,916 @@
+// engine_gen.hip -- gfx950 kernels for transform lengths whose radix schedule
+// is a run-time value.
+//
+// A length n = R_0 R_1 ... R_{S-1} (radices up to 16, the composite ones as
+// prime-factor butterflies in registers) is run in place over an LDS tile of
+// B sequences.  Position p of the tile is written in mixed radix with R_0 the
+// fastest digit; stage s combines the R_s values a stride Ns = R_0 ... R_{s-1}
+// apart:
+//   forward order (decimation in time): twiddle W_{Ns R}^{k r}, then the
+//     butterfly, stages 0 .. S-1; input index e sits at the digit-reversed
+//     position, the result is in natural order;
+//   reverse order (decimation in frequency): butterfly, then the twiddle,
+//     stages S-1 .. 0; natural order in, digit-reversed out.
+// Both use one twiddle table.  A butterfly writes the positions it read, so
+// a stage needs one barrier, one butterfly's registers and one tile, and the
+// number of butterflies per thread is a run-time loop.  The digit reversal
+// costs nothing on the side that addresses memory by rows: stage 0 there reads
+// (or writes) global memory itself, one 128-byte row segment per value, and
+// the reversal is one division per butterfly.
+//
+// A prime radix above 16 runs as a stage over LDS by the symmetric pairs
+// v_i +- v_{R-i} (half the multiplications of the direct sum), its outputs
+// held in registers across a barrier.
+//
+// What bounds the passes: with 128-byte row segments they move each byte once
+// per pass and run at 3-5 TB/s; the rest is the instruction issue of the
+// butterflies and the compensated twiddles.
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <mutex>
+#include <type_traits>
+
+#include "engine_gen.hpp"
+
+namespace p3amd {
+
+typedef TwT<real_t>::type Tw;
+static constexpr size_t kLdsMax = 160 * 1024;
+
+struct GenStage {
+  int R, Ns, tw;    // radix, product of the earlier radices, twiddle offset
+  unsigned mNs;     // ceil(2^32 / Ns) (see gdiv)
+  unsigned mR;
+};
+constexpr int kGenStages = 16;
+// bytes before the twiddles that hold the columns' offsets (length-fastest views)
+constexpr int kColTab = 32 * sizeof(unsigned long long);
+struct GenDesc {
+  int n, nst;
+  GenStage st[kGenStages];
+  int twcount;
+};
+
+// x / d for x, d < 2^16 with m = ceil(2^32 / d); d is uniform
+__device__ __forceinline__ int gdiv(int x, unsigned m, int d) {
+  return d == 1 ? x : (int)__umulhi((unsigned)x, m);
+}
+
+// address of position p: blocks of R_0 positions BP apart, the blocks R_0 BP +
+// skew apart
+struct GenTile {
+  int BP, P0, skew, R0;
+  unsigned mR0;
+};
+
+template <class F>
+__device__ __forceinline__ void with_radix(int R, F f) {
+#define P3_CASE(N)                                                            \
+  case N:                                                                     \
+    if constexpr (N <= kGenMaxRadix) f(std::integral_constant<int, N>{});     \
+    break;
+  switch (R) {
+    P3_CASE(1) P3_CASE(2) P3_CASE(3) P3_CASE(4) P3_CASE(5) P3_CASE(6) P3_CASE(7) P3_CASE(8)
+    P3_CASE(9) P3_CASE(10) P3_CASE(11) P3_CASE(12) P3_CASE(13) P3_CASE(14) P3_CASE(15) P3_CASE(16)
+    default: break;
+  }
+#undef P3_CASE
+}
+
+// input index of stage 0's butterfly j (its R_0 values are n / R_0 apart)
+__device__ __forceinline__ int gen_rev(const GenDesc& L, int j) {
+  int acc = 0;
+  for (int s = 1; s + 1 < L.nst; s++) {
+    const int q = gdiv(j, L.st[s].mR, L.st[s].R);
+    acc = acc * L.st[s].R + (j - q * L.st[s].R);
+    j = q;
+  }
+  return L.nst > 1 ? acc * L.st[L.nst - 1].R + j : 0;
+}
+
+// the butterfly j whose input index is e (the inverse of gen_rev)
+__device__ __forceinline__ int gen_unrev(const GenDesc& L, int e) {
+  int acc = 0;
+  for (int s = L.nst - 1; s > 1; s--) {
+    const int q = gdiv(e, L.st[s].mR, L.st[s].R);
+    acc = acc * L.st[s].R + (e - q * L.st[s].R);
+    e = q;
+  }
+  return L.nst > 1 ? acc * L.st[1].R + e : 0;
+}
+
+// address of the first value of stage s's butterfly (block g, offset k) and
+// the stride of its values
+__device__ __forceinline__ int gen_base(const GenTile& t, const GenStage& st, int g, int k, int SP) {
+  int a = g * st.R * SP + k * t.BP;
+  if (t.skew) a += gdiv(k, t.mR0, t.R0) * t.skew;
+  return a;
+}
+__device__ __forceinline__ int gen_stride(const GenTile& t, const GenStage& st) {
+  return gdiv(st.Ns, t.mR0, t.R0) * t.P0;
+}
+
+// a stage with a prime radix above 16: outputs by symmetric pairs
+constexpr int kPrimeItems = 8;
+template <class T, bool FWD, bool DIF>
+__device__ __forceinline__ void gen_prime(cpx<T>* lds, const GenDesc& L, const GenStage& st, const GenTile& t, int B,
+                                          unsigned mB, const typename TwT<T>::type* tw) {
+  typedef typename TwT<T>::type TwL;
+  const int NT = blockDim.x, R = st.R, H = (R - 1) / 2;
+  const int nj = gdiv(L.n, st.mR, R), nb = B * nj, SP = gen_stride(t, st);
+  const unsigned mb = nb > 1 ? (unsigned)((0x100000000ull + nb - 1) / nb) : 0;
+  // v_i, v_{R-i} -> their sum and difference, in place
+  for (int it = threadIdx.x; it < nb * H; it += NT) {
+    const int i0 = gdiv(it, mb, nb), w = it - i0 * nb, i = i0 + 1;
+    const int j = gdiv(w, mB, B), b = w - j * B;
+    const int g = gdiv(j, st.mNs, st.Ns), k = j - g * st.Ns;
+    const int p = gen_base(t, st, g, k, SP) + b;
+    cpx<T> u = lds[p + i * SP], v = lds[p + (R - i) * SP];
+    if constexpr (!DIF) {
+      const TwL* q = tw + st.tw + k * (R - 1);
+      u = twmul<FWD>(u, q[i - 1]);
+      v = twmul<FWD>(v, q[R - i - 1]);
+    }
+    lds[p + i * SP] = add(u, v);
+    lds[p + (R - i) * SP] = sub(u, v);
+  }
+  __syncthreads();
+  const TwL* wr = tw + st.tw + st.Ns * (R - 1);  // W_R^j
+  cpx<T> ya[kPrimeItems], yb[kPrimeItems];
+#pragma unroll
+  for (int m = 0; m < kPrimeItems; m++) {
+    const int it = threadIdx.x + m * NT;
+    if (it < nb * (H + 1)) {
+      const int q = gdiv(it, mb, nb), w = it - q * nb;
+      const int j = gdiv(w, mB, B), b = w - j * B;
+      const int g = gdiv(j, st.mNs, st.Ns), k = j - g * st.Ns;
+      const int p = gen_base(t, st, g, k, SP) + b;
+      cpx<T> c = lds[p], d = mk<T>(0, 0);
+      int e = 0;
+      for (int i = 1; i <= H; i++) {
+        e += q;
+        if (e >= R) e -= R;
+        // cos and sin of 2 pi i q / R times the pair's sum and difference
+        const TwL x = wr[e];
+        const cpx<T> s = lds[p + i * SP], f = lds[p + (R - i) * SP];
+        if constexpr (sizeof(T) == 4) {
+          c.x = fmaf(s.x, x.x, fmaf(s.x, x.z, c.x));
+          c.y = fmaf(s.y, x.x, fmaf(s.y, x.z, c.y));
+          d.x = fmaf(f.x, -x.y, fmaf(f.x, -x.w, d.x));
+          d.y = fmaf(f.y, -x.y, fmaf(f.y, -x.w, d.y));
+        } else {
+          c.x = fma(s.x, x.x, c.x);
+          c.y = fma(s.y, x.x, c.y);
+          d.x = fma(f.x, -x.y, d.x);
+          d.y = fma(f.y, -x.y, d.y);
+        }
+      }
+      d = rot<FWD>(d);
+      ya[m] = add(c, d);
+      yb[m] = sub(c, d);
+      if constexpr (DIF) {
+        const TwL* w2 = tw + st.tw + k * (R - 1);
+        if (q > 0) {
+          ya[m] = twmul<FWD>(ya[m], w2[q - 1]);
+          yb[m] = twmul<FWD>(yb[m], w2[R - q - 1]);
+        }
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < kPrimeItems; m++) {
+    const int it = threadIdx.x + m * NT;
+    if (it < nb * (H + 1)) {
+      const int q = gdiv(it, mb, nb), w = it - q * nb;
+      const int j = gdiv(w, mB, B), b = w - j * B;
+      const int g = gdiv(j, st.mNs, st.Ns), k = j - g * st.Ns;
+      const int p = gen_base(t, st, g, k, SP) + b;
+      lds[p + q * SP] = ya[m];
+      if (q > 0) lds[p + (R - q) * SP] = yb[m];
+    }
+  }
+  __syncthreads();
+}
+
+// an in-place stage over the tile; b: this thread's sequence, jt, js: its
+// first butterfly and their stride
+template <class T, bool FWD, bool DIF>
+__device__ __forceinline__ void gen_mid(cpx<T>* lds, const GenDesc& L, int s, const GenTile& t, int B, unsigned mB,
+                                        int b, int jt, int js, const typename TwT<T>::type* tw) {
+  const GenStage st = L.st[s];
+  if (st.R > kGenMaxRadix) {
+    gen_prime<T, FWD, DIF>(lds, L, st, t, B, mB, tw);
+    return;
+  }
+  const int nj = gdiv(L.n, st.mR, st.R), SP = gen_stride(t, st);
+  with_radix(st.R, [&](auto rc) {
+    constexpr int R = decltype(rc)::value;
+    for (int j = jt; j < nj; j += js) {
+      const int g = gdiv(j, st.mNs, st.Ns), k = j - g * st.Ns;
+      cpx<T>* p = lds + gen_base(t, st, g, k, SP) + b;
+      cpx<T> v[R];
+#pragma unroll
+      for (int r = 0; r < R; r++) v[r] = p[r * SP];
+      const typename TwT<T>::type* w = tw + st.tw + k * (R - 1);
+      if constexpr (!DIF) {
+#pragma unroll
+        for (int r = 1; r < R; r++) v[r] = twmul<FWD>(v[r], w[r - 1]);
+      }
+      dft<R, FWD>(v);
+      if constexpr (DIF) {
+#pragma unroll
+        for (int r = 1; r < R; r++) v[r] = twmul<FWD>(v[r], w[r - 1]);
+      }
+#pragma unroll
+      for (int r = 0; r < R; r++) p[r * SP] = v[r];
+    }
+  });
+  __syncthreads();
+}
+
+extern __shared__ __align__(16) unsigned char gen_smem[];
+
+// the twiddle table, copied into LDS behind the tile where it fits (complete
+// at the next barrier)
+template <class T>
+__device__ __forceinline__ const typename TwT<T>::type* gen_twiddles(const void* tw, int in_lds, int off, int count) {
+  typedef typename TwT<T>::type TwL;
+  const TwL* g = (const TwL*)tw;
+  if (!in_lds) return g;
+  TwL* l = (TwL*)(gen_smem + off);
+  for (int i = threadIdx.x; i < count; i += blockDim.x) l[i] = g[i];
+  return l;
+}
+
+// workgroup id -> tile: each XCD (id mod 8) owns a contiguous range
+__device__ __forceinline__ int gen_tile_of(int rev, int xcd) {
+  const int n = (int)gridDim.x, bid = (int)blockIdx.x;
+  int t = bid;
+  if (xcd) {
+    const int q = n >> 3, rm = n & 7, x = bid & 7;
+    t = x * q + (x < rm ? x : rm) + (bid >> 3);
+  }
+  return rev ? n - 1 - t : t;
+}
+
+// ---------------------------------------------------------------------------
+// columns
+// ---------------------------------------------------------------------------
+struct GColArgs {
+  const void* in;
+  void* out;
+  long long si_in, sl_in, so_in, si_out, sl_out, so_out;
+  long long ncol;
+  int n_inner;
+  int lB;             // log2 of the columns per tile
+  int kind, rows;     // ColKind, logical rows of a column
+  int nld, ld_lo, ld_hi, ld_shift, nst, st_lo, st_shift;
+  FDiv dld, dst;      // length-fastest sides: divide by the rows loaded / stored
+  GenTile t;
+  GenDesc L;
+  const void* tw;
+  int tw_lds, tw_off;
+  int rev, xcd;
+};
+
+// input row of FFT row e (-1: zero); neg: with its sign changed
+__device__ __forceinline__ int gen_src(const GColArgs& a, int e, bool& neg) {
+  neg = false;
+  int i = e;
+  if (a.kind == COL_DCT1) {
+    if (e >= a.rows) i = a.L.n - e;
+  } else if (a.kind == COL_DST1) {
+    if (e == 0 || e == a.rows + 1) return -1;
+    neg = e > a.rows;
+    i = neg ? a.L.n - e - 1 : e - 1;
+  }
+  if (i >= a.nld) return -1;
+  return i < a.ld_lo ? i : (i >= a.ld_hi ? i - a.ld_shift : -1);
+}
+// output row of FFT row p (-1: not stored)
+__device__ __forceinline__ int gen_dst(const GColArgs& a, int p) {
+  const int i = a.kind == COL_DST1 ? p - 1 : p;
+  const int e = i < a.st_lo ? i : (i >= a.st_lo + a.st_shift ? i - a.st_shift : -1);
+  return e < a.nst ? e : -1;
+}
+template <class T>
+__device__ __forceinline__ cpx<T> gen_out(const GColArgs& a, cpx<T> v) {
+  return a.kind == COL_DST1 ? mk<T>(-v.y, v.x) : v;
+}
+
+// MAP: pruned rows, DCT-I / DST-I extensions.  LF: 0 rows on both sides, 1 the
+// input is length-fastest (decimation in frequency), 2 the output is.  Off: the
+// type of the byte offsets from the tile's first column.
+template <class T, bool FWD, bool MAP, int LF, class Off>
+__global__ __launch_bounds__(1024) void k_gcol(GColArgs a) {
+  typedef cpx<T> C;
+  constexpr long long E = sizeof(C);
+  C* lds = (C*)gen_smem;
+  const auto* tw = gen_twiddles<T>(a.tw, a.tw_lds, a.tw_off, a.L.twcount);
+  const int B = 1 << a.lB, NT = blockDim.x, S = a.L.nst;
+  const unsigned mB = a.lB ? 1u << (32 - a.lB) : 0u;
+  const int b = threadIdx.x & (B - 1), jt = threadIdx.x >> a.lB, js = NT >> a.lB;
+  const long long c0 = (long long)gen_tile_of(a.rev, a.xcd) * B;
+  const int nb = (int)(a.ncol - c0 < B ? a.ncol - c0 : B);
+  const unsigned n_in = (unsigned)a.n_inner;
+  const unsigned o0 = (unsigned)c0 / n_in, i0 = (unsigned)c0 - o0 * n_in;
+  const char* in = (const char*)a.in + ((long long)o0 * a.so_in + (long long)i0 * a.si_in) * E;
+  char* out = (char*)a.out + ((long long)o0 * a.so_out + (long long)i0 * a.si_out) * E;
+  // columns past the last one repeat it and are not stored
+  const unsigned c = (unsigned)c0 + (b < nb ? b : nb - 1);
+  const unsigned o = c / n_in, i = c - o * n_in;
+  const Off lin = (Off)((((long long)o - o0) * a.so_in + ((long long)i - i0) * a.si_in) * E);
+  const Off lout = (Off)((((long long)o - o0) * a.so_out + ((long long)i - i0) * a.si_out) * E);
+  const Off sin = (Off)(a.sl_in * E), sout = (Off)(a.sl_out * E);
+  const bool valid = b < nb;
+  const GenStage s0 = a.L.st[0];
+  const int n0 = gdiv(a.L.n, s0.mR, s0.R);
+  // values of a finished butterfly: FFT rows p0 + r * dp
+  auto store = [&](auto rc, C* v, int p0, int dp) {
+    constexpr int R = decltype(rc)::value;
+    if (!valid) return;
+    if constexpr (MAP) {
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const int e = gen_dst(a, p0 + r * dp);
+        if (e >= 0) *(C*)(out + (lout + (Off)e * sout)) = gen_out(a, v[r]);
+      }
+    } else {
+      Off q = lout + (Off)p0 * sout;
+      const Off dq = (Off)dp * sout;
+#pragma unroll
+      for (int r = 0; r < R; r++, q += dq) *(C*)(out + q) = v[r];
+    }
+  };
+  if constexpr (LF == 1) {
+    // natural order into the tile, the lanes along the length
+    const int m = a.L.n;
+    unsigned long long* colb = (unsigned long long*)(gen_smem + a.tw_off - kColTab);
+    if (threadIdx.x < B) colb[threadIdx.x] = (unsigned long long)lin;
+    __syncthreads();
+    for (int q = threadIdx.x; q < B * m; q += NT) {
+      const int bb = fdiv(q, a.dld), e = q - bb * m;
+      bool neg;
+      const int src = gen_src(a, e, neg);
+      C v = mk<T>(0, 0);
+      if (src >= 0) v = *(const C*)(in + (colb[bb] + (unsigned long long)src * (unsigned long long)sin));
+      lds[e * a.t.BP + bb] = neg ? mk<T>(-v.x, -v.y) : v;
+    }
+    __syncthreads();
+    for (int s = S - 1; s > 0; s--) gen_mid<T, FWD, true>(lds, a.L, s, a.t, B, mB, b, jt, js, tw);
+    with_radix(s0.R, [&](auto rc) {
+      constexpr int R = decltype(rc)::value;
+      for (int j = jt; j < n0; j += js) {
+        C v[R];
+        const C* p = lds + j * a.t.P0 + b;
+#pragma unroll
+        for (int r = 0; r < R; r++) v[r] = p[r * a.t.BP];
+        dft<R, FWD>(v);
+        store(rc, v, gen_rev(a.L, j), n0);
+      }
+    });
+    return;
+  }
+  with_radix(s0.R, [&](auto rc) {
+    constexpr int R = decltype(rc)::value;
+    for (int j = jt; j < n0; j += js) {
+      const int e0 = gen_rev(a.L, j);
+      C v[R];
+      if constexpr (MAP) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+          bool neg;
+          const int src = gen_src(a, e0 + r * n0, neg);
+          // a row that is zero reads the column's first row instead, so no
+          // load sits under a branch
+          const C u = *(const C*)(in + (lin + (Off)(src >= 0 ? src : 0) * sin));
+          v[r].x = src >= 0 ? (neg ? -u.x : u.x) : (T)0;
+          v[r].y = src >= 0 ? (neg ? -u.y : u.y) : (T)0;
+        }
+      } else {
+        Off q = lin + (Off)e0 * sin;
+        const Off dq = (Off)n0 * sin;
+#pragma unroll
+        for (int r = 0; r < R; r++, q += dq) v[r] = *(const C*)(in + q);
+      }
+      dft<R, FWD>(v);
+      if (S == 1 && LF == 0) {
+        store(rc, v, 0, 1);
+      } else {
+        C* p = lds + j * a.t.P0 + b;
+#pragma unroll
+        for (int r = 0; r < R; r++) p[r * a.t.BP] = v[r];
+      }
+    }
+  });
+  if (S == 1 && LF == 0) return;
+  __syncthreads();
+  const int last = LF == 2 ? S : S - 1;
+  for (int s = 1; s < last; s++) gen_mid<T, FWD, false>(lds, a.L, s, a.t, B, mB, b, jt, js, tw);
+  if constexpr (LF == 2) {
+    unsigned long long* colb = (unsigned long long*)(gen_smem + a.tw_off - kColTab);
+    if (threadIdx.x < B) colb[threadIdx.x] = (unsigned long long)lout;
+    __syncthreads();
+    for (int q = threadIdx.x; q < nb * a.nst; q += NT) {
+      const int bb = fdiv(q, a.dst), e = q - bb * a.nst;
+      const int p = (e < a.st_lo ? e : e + a.st_shift) + (a.kind == COL_DST1 ? 1 : 0);
+      *(C*)(out + (colb[bb] + (unsigned long long)e * (unsigned long long)sout)) = gen_out(a, lds[p * a.t.BP + bb]);
+    }
+  } else {
+    const GenStage st = a.L.st[S - 1];
+    const int SP = gen_stride(a.t, st);
+    with_radix(st.R, [&](auto rc) {
+      constexpr int R = decltype(rc)::value;
+      for (int j = jt; j < st.Ns; j += js) {
+        C v[R];
+        const C* p = lds + gen_base(a.t, st, 0, j, SP) + b;
+#pragma unroll
+        for (int r = 0; r < R; r++) v[r] = p[r * SP];
+        const auto* w = tw + st.tw + j * (R - 1);
+#pragma unroll
+        for (int r = 1; r < R; r++) v[r] = twmul<FWD>(v[r], w[r - 1]);
+        dft<R, FWD>(v);
+        store(rc, v, j, st.Ns);
+      }
+    });
+  }
+}
+
+// rows moved without a transform (row maps and the length-fastest layout),
+// through an LDS tile so that both sides are read and written along their
+// contiguous index
+template <class T>
+__global__ __launch_bounds__(256) void k_gcopy(GColArgs a) {
+  typedef cpx<T> C;
+  C* lds = (C*)gen_smem;
+  const int B = 1 << a.lB, NT = blockDim.x;
+  const long long c0 = (long long)gen_tile_of(a.rev, a.xcd) * B;
+  const int nb = (int)(a.ncol - c0 < B ? a.ncol - c0 : B);
+  const bool lf_in = a.sl_in == 1 && a.si_in != 1, lf_out = a.sl_out == 1 && a.si_out != 1;
+  const unsigned n_in = (unsigned)a.n_inner;
+  auto col = [&](int b, long long si, long long so) {
+    const unsigned c = (unsigned)c0 + b, o = c / n_in, i = c - o * n_in;
+    return (long long)o * so + (long long)i * si;
+  };
+  for (int q = threadIdx.x; q < B * a.nld; q += NT) {
+    int b, e;
+    if (lf_in) { b = fdiv(q, a.dld); e = q - b * a.nld; }
+    else { e = q >> a.lB; b = q & (B - 1); }
+    const int src = e < a.ld_lo ? e : (e >= a.ld_hi ? e - a.ld_shift : -1);
+    C v = mk<T>(0, 0);
+    if (b < nb && src >= 0) v = ((const C*)a.in)[col(b, a.si_in, a.so_in) + (long long)src * a.sl_in];
+    lds[e * a.t.BP + b] = v;
+  }
+  __syncthreads();
+  for (int q = threadIdx.x; q < B * a.nst; q += NT) {
+    int b, e;
+    if (lf_out) { b = fdiv(q, a.dst); e = q - b * a.nst; }
+    else { e = q >> a.lB; b = q & (B - 1); }
+    if (b < nb) {
+      const int p = e < a.st_lo ? e : e + a.st_shift;
+      ((C*)a.out)[col(b, a.si_out, a.so_out) + (long long)e * a.sl_out] = lds[p * a.t.BP + b];
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// rows along X: two real rows as one complex row (x_a + i x_b)
+// ---------------------------------------------------------------------------
+struct GXArgs {
+  const void* in;
+  void* out;
+  long long nrows, si_row, so_row;
+  int nk;         // r2c: kept modes; c2r: valid input modes
+  int lB, lBL;    // log2 of the row pairs per tile, and of those side by side in a wave
+  FDiv dnk, dn0;  // divide by the modes, by n / R_0
+  GenTile t;
+  GenDesc L;
+  const void* tw;
+  int tw_lds, tw_off;
+  int rev;
+};
+
+// r2c: stage 0 reads the rows (lanes along the row), in-place stages, and the
+// two half spectra separated from the natural-order result as they are stored
+template <class T>
+__global__ __launch_bounds__(1024) void k_gx_r2c(GXArgs a) {
+  typedef cpx<T> C;
+  C* lds = (C*)gen_smem;
+  const auto* tw = gen_twiddles<T>(a.tw, a.tw_lds, a.tw_off, a.L.twcount);
+  const int B = 1 << a.lB, NT = blockDim.x, S = a.L.nst, n = a.L.n;
+  const long long pair0 = (long long)gen_tile_of(a.rev, 1) * B;
+  const int nr = (int)(a.nrows - 2 * pair0 < 2 * B ? a.nrows - 2 * pair0 : 2 * B);
+  const char* in = (const char*)a.in + 2 * pair0 * a.si_row * (long long)sizeof(T);
+  const unsigned si = (unsigned)(a.si_row * sizeof(T));
+  const GenStage s0 = a.L.st[0];
+  const int n0 = gdiv(n, s0.mR, s0.R);
+  with_radix(s0.R, [&](auto rc) {
+    constexpr int R = decltype(rc)::value;
+    for (int it = threadIdx.x; it < B * n0; it += NT) {
+      const int u = it >> a.lBL, bh = fdiv(u, a.dn0), e0 = u - bh * n0;
+      const int b = (it & ((1 << a.lBL) - 1)) + (bh << a.lBL);
+      const bool oka = 2 * b < nr, okb = 2 * b + 1 < nr;
+      // rows past the last one read the tile's first row and are zeroed
+      const char* pa = in + ((oka ? (unsigned)(2 * b) * si : 0u) + (unsigned)e0 * (unsigned)sizeof(T));
+      const char* pb = in + ((okb ? (unsigned)(2 * b + 1) * si : 0u) + (unsigned)e0 * (unsigned)sizeof(T));
+      C v[R];
+      const unsigned d = (unsigned)n0 * (unsigned)sizeof(T);
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        v[r].x = *(const T*)(pa + (unsigned)r * d);
+        v[r].y = *(const T*)(pb + (unsigned)r * d);
+      }
+      if (!oka) {
+#pragma unroll
+        for (int r = 0; r < R; r++) v[r].x = (T)0;
+      }
+      if (!okb) {
+#pragma unroll
+        for (int r = 0; r < R; r++) v[r].y = (T)0;
+      }
+      dft<R, true>(v);
+      C* p = lds + gen_unrev(a.L, e0) * a.t.P0 + b;
+#pragma unroll
+      for (int r = 0; r < R; r++) p[r * a.t.BP] = v[r];
+    }
+  });
+  __syncthreads();
+  const int b0 = threadIdx.x & (B - 1), jt = threadIdx.x >> a.lB, js = NT >> a.lB;
+  const unsigned mB = a.lB ? 1u << (32 - a.lB) : 0u;
+  for (int s = 1; s < S; s++)
+    gen_mid<T, true, false>(lds, a.L, s, a.t, B, mB, b0, jt, js, tw);
+  char* out = (char*)a.out + 2 * pair0 * a.so_row * (long long)sizeof(C);
+  const unsigned so = (unsigned)(a.so_row * sizeof(C));
+  const T h = (T)0.5;
+  for (int q = threadIdx.x; q < B * a.nk; q += NT) {
+    const int b = fdiv(q, a.dnk), k = q - b * a.nk;
+    const C zk = lds[k * a.t.BP + b], zn = lds[(k == 0 ? 0 : n - k) * a.t.BP + b];
+    const unsigned off = (unsigned)(2 * b) * so + (unsigned)k * (unsigned)sizeof(C);
+    if (2 * b < nr) *(C*)(out + off) = mk<T>((zk.x + zn.x) * h, (zk.y - zn.y) * h);
+    if (2 * b + 1 < nr) *(C*)(out + off + so) = mk<T>((zk.y + zn.y) * h, (zn.x - zk.x) * h);
+  }
+}
+
+// c2r: the mirror image: natural order in, decimation in frequency, stage 0
+// stores the rows
+template <class T>
+__global__ __launch_bounds__(1024) void k_gx_c2r(GXArgs a) {
+  typedef cpx<T> C;
+  C* lds = (C*)gen_smem;
+  const auto* tw = gen_twiddles<T>(a.tw, a.tw_lds, a.tw_off, a.L.twcount);
+  const int B = 1 << a.lB, NT = blockDim.x, S = a.L.nst, n = a.L.n, K = n / 2 + 1;
+  const long long pair0 = (long long)gen_tile_of(a.rev, 1) * B;
+  const int nr = (int)(a.nrows - 2 * pair0 < 2 * B ? a.nrows - 2 * pair0 : 2 * B);
+  const char* in = (const char*)a.in + 2 * pair0 * a.si_row * (long long)sizeof(C);
+  const unsigned si = (unsigned)(a.si_row * sizeof(C));
+  for (int q = threadIdx.x; q < B * K; q += NT) {
+    const int b = fdiv(q, a.dnk), k = q - b * K;
+    const bool oka = k < a.nk && 2 * b < nr, okb = k < a.nk && 2 * b + 1 < nr;
+    const unsigned off = (unsigned)(2 * b) * si + (unsigned)k * (unsigned)sizeof(C);
+    C A = *(const C*)(in + (oka ? off : 0u)), Bv = *(const C*)(in + (okb ? off + si : 0u));
+    if (!oka) A = mk<T>(0, 0);
+    if (!okb) Bv = mk<T>(0, 0);
+    // FFTW c2r: the imaginary parts of k = 0 and k = n/2 (n even) do not
+    // contribute; there both forms are the same value
+    if (k == 0 || 2 * k == n) { A.y = 0; Bv.y = 0; }
+    lds[k * a.t.BP + b] = mk<T>(A.x - Bv.y, A.y + Bv.x);
+    lds[(k == 0 ? 0 : n - k) * a.t.BP + b] = mk<T>(A.x + Bv.y, Bv.x - A.y);
+  }
+  __syncthreads();
+  const int b0 = threadIdx.x & (B - 1), jt = threadIdx.x >> a.lB, js = NT >> a.lB;
+  const unsigned mB = a.lB ? 1u << (32 - a.lB) : 0u;
+  for (int s = S - 1; s > 0; s--)
+    gen_mid<T, false, true>(lds, a.L, s, a.t, B, mB, b0, jt, js, tw);
+  char* out = (char*)a.out + 2 * pair0 * a.so_row * (long long)sizeof(T);
+  const unsigned so = (unsigned)(a.so_row * sizeof(T));
+  const GenStage s0 = a.L.st[0];
+  const int n0 = gdiv(n, s0.mR, s0.R);
+  with_radix(s0.R, [&](auto rc) {
+    constexpr int R = decltype(rc)::value;
+    for (int it = threadIdx.x; it < B * n0; it += NT) {
+      const int u = it >> a.lBL, bh = fdiv(u, a.dn0), e0 = u - bh * n0;
+      const int b = (it & ((1 << a.lBL) - 1)) + (bh << a.lBL);
+      C v[R];
+      const C* p = lds + gen_unrev(a.L, e0) * a.t.P0 + b;
+#pragma unroll
+      for (int r = 0; r < R; r++) v[r] = p[r * a.t.BP];
+      dft<R, false>(v);
+      char* pa = out + ((unsigned)(2 * b) * so + (unsigned)e0 * (unsigned)sizeof(T));
+      const unsigned d = (unsigned)n0 * (unsigned)sizeof(T);
+      if (2 * b < nr) {
+#pragma unroll
+        for (int r = 0; r < R; r++) *(T*)(pa + (unsigned)r * d) = v[r].x;
+      }
+      if (2 * b + 1 < nr) {
+#pragma unroll
+        for (int r = 0; r < R; r++) *(T*)(pa + so + (unsigned)r * d) = v[r].y;
+      }
+    }
+  });
+}
+
+// ---------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------
+// instructions of a butterfly of radix r per value, and of a stage's
+// twiddles, addresses and LDS accesses per value, in units of one FP32
+// instruction: the schedule with the smallest sum is taken
+static double radix_cost(int r) {
+  static const double c[17] = {0, 0, 4, 12, 16, 34, 36, 66, 56, 90, 88, 160, 96, 220, 160, 162, 170};
+  return r <= 16 ? c[r] / r : 8.0 * r;
+}
+constexpr double kStageCost = 16;
+
+static void search(int m, int maxr, std::vector<int>& cur, double cost, std::vector<int>& best, double& bc) {
+  if (cost >= bc) return;
+  if (m == 1) {
+    bc = cost;
+    best = cur;
+    return;
+  }
+  for (int r = std::min(maxr, m); r >= 2; r--) {
+    if (m % r) continue;
+    cur.push_back(r);
+    search(m / r, r, cur, cost + radix_cost(r) + kStageCost, best, bc);
+    cur.pop_back();
+  }
+}
+
+std::vector<int> gen_factors(int n) {
+  std::vector<int> big;
+  int m = n;
+  for (int p = 11; p <= m; p++) {
+    bool prime = true;
+    for (int q = 2; (long long)q * q <= p; q++)
+      if (p % q == 0) { prime = false; break; }
+    if (prime && !gen_in_registers(p))
+      while (m % p == 0) { big.push_back(p); m /= p; }
+  }
+  std::vector<int> cur, best;
+  double bc = 1e30;
+  search(m, kGenMaxRadix, cur, 0, best, bc);
+  // the factors in registers, largest first; the large primes in between
+  best.insert(best.begin() + (best.empty() ? 0 : 1), big.begin(), big.end());
+  return gen_wrap(best);
+}
+
+std::vector<int> gen_wrap(const std::vector<int>& f) {
+  std::vector<int> g = f;
+  if (g.empty() || !gen_in_registers(g.front())) g.insert(g.begin(), 1);
+  if (!gen_in_registers(g.back())) g.push_back(1);
+  return g;
+}
+
+static unsigned magic(int d) { return d > 1 ? (unsigned)(((1ull << 32) + d - 1) / d) : 0u; }
+static FDiv make_fdiv(int d) {
+  FDiv f;
+  f.d = d;
+  f.m = ((1ULL << 32) + (uint64_t)d - 1) / (uint64_t)d;
+  return f;
+}
+
+static GenDesc make_desc(const Len1D& L) {
+  GenDesc g;
+  std::memset(&g, 0, sizeof(g));
+  g.n = L.gd.n;
+  g.nst = L.gd.nst;
+  if (g.nst > kGenStages) throw Error{"transform length has too many factors", -1};
+  for (int s = 0; s < g.nst; s++) {
+    GenStage& t = g.st[s];
+    t.R = L.gd.radix[s];
+    t.Ns = L.gd.ns[s];
+    t.tw = L.gd.twoff[s];
+    t.mNs = magic(t.Ns);
+    t.mR = magic(t.R);
+  }
+  g.twcount = L.gd.twcount;
+  return g;
+}
+
+static int log2i(int x) {
+  int l = 0;
+  while ((1 << (l + 1)) <= x) l++;
+  return l;
+}
+
+// LDS bytes of a tile of `data` bytes and its twiddle table, which joins the
+// tile where that leaves room for as many workgroups per CU or at least two
+static size_t place_twiddles(size_t data, const Len1D& L, int* tw_lds, int* tw_off) {
+  const size_t off = (data + 15) & ~(size_t)15, twb = (size_t)L.gd.twcount * sizeof(Tw);
+  *tw_off = (int)off;
+  *tw_lds = L.gd.twcount > 0 && (off + twb <= 80 * 1024 || (off > 80 * 1024 && off + twb <= kLdsMax)) ? 1 : 0;
+  return *tw_lds ? off + twb : off;
+}
+
+// threads of a workgroup: the count that finishes most tiles per unit of
+// time, a butterfly of radix R counted as R + 3 and a CU as holding as many
+// workgroups as the LDS, 16 waves (128 registers per lane) and the number of
+// tiles allow
+static int pick_threads(const Len1D& L, int B, size_t lds, long long tiles) {
+  double best = -1;
+  int bn = 64;
+  for (int nt = 64; nt <= 1024; nt += 64) {
+    long long wg = std::min<long long>((long long)(kLdsMax / std::max<size_t>(lds, 1)), 1024 / nt);
+    wg = std::max<long long>(1, std::min<long long>(wg, (tiles + 255) / 256));
+    double t = 0;
+    bool ok = true;
+    for (int s = 0; s < L.gd.nst; s++) {
+      const int R = L.gd.radix[s];
+      const long long nb = (long long)B * (L.gd.n / R);
+      if (gen_in_registers(R)) {
+        t += (double)((nb + nt - 1) / nt) * (R + 3);
+      } else {
+        const long long items = nb * ((R + 1) / 2);
+        if (items > (long long)nt * kPrimeItems) ok = false;
+        t += (double)((items + nt - 1) / nt) * 2 * R;
+      }
+    }
+    if (!ok) continue;
+    const double rate = (double)wg / t;
+    if (rate > best * 1.02) { best = rate; bn = nt; }
+  }
+  if (best < 0) throw Error{"transform tile exceeds the 1024-thread workgroup capacity", -1};
+  return bn;
+}
+
+static bool has_prime_stage(const Len1D& L) {
+  for (int s = 0; s < L.gd.nst; s++)
+    if (!gen_in_registers(L.gd.radix[s])) return true;
+  return false;
+}
+
+template <bool FWD, bool MAP, int LF, class Off>
+static void go_col(const GColArgs& a, unsigned g, int nt, size_t bytes, hipStream_t st) {
+  k_gcol<real_t, FWD, MAP, LF, Off><<<g, nt, bytes, st>>>(a);
+}
+
+void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, hipStream_t st) {
+  const long long ncol = (long long)c.n_inner * c.n_outer;
+  if (ncol > 0x7fffffffLL) throw Error{"grid too large", -1};
+  GColArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.in = c.in; a.out = c.out;
+  a.si_in = c.si_in; a.sl_in = c.sl_in; a.so_in = c.so_in;
+  a.si_out = c.si_out; a.sl_out = c.sl_out; a.so_out = c.so_out;
+  a.ncol = ncol;
+  a.n_inner = c.n_inner;
+  a.kind = c.kind;
+  a.rows = c.n;
+  a.nld = c.nld; a.ld_lo = c.ld_lo; a.ld_hi = c.ld_hi; a.ld_shift = c.ld_shift;
+  a.nst = c.nst; a.st_lo = c.st_lo; a.st_shift = c.st_shift;
+  a.rev = c.rev ? 1 : 0;
+  a.xcd = xcd;
+  const bool lf_in = c.sl_in == 1 && c.si_in != 1, lf_out = c.sl_out == 1 && c.si_out != 1;
+  const bool lf = lf_in || lf_out;
+  const int m = L ? L->gd.n : c.nld;
+  const long long E = sizeof(cplx_t);
+  // columns per tile: a 128-byte row segment (plan-time measurement may choose
+  // another) while the tile stays within the plan's bytes, segments of 64
+  // bytes as long as the tile fits at all; halved while there is not a tile
+  // for every CU
+  const long long want = L ? L->tile_bytes : 64 * 1024;
+  int B = 1;
+  while (B * 2 * E <= (L ? L->col_seg : 128)) B *= 2;
+  auto bytes_of = [&](int b) { return ((long long)m * (lf && b > 1 ? b + 1 : b) + b) * E + 256; };
+  while (B > 1 && ((bytes_of(B) > want + want / 8 && B * E > 64) || bytes_of(B) > (long long)kLdsMax)) B /= 2;
+  // a prime stage holds its outputs in registers, kPrimeItems pairs a thread
+  while (B > 1 && L && has_prime_stage(*L) && (long long)B * m > 1024LL * (2 * kPrimeItems - 1)) B /= 2;
+  while (B * E > 32 && (ncol + B - 1) / B < 256) B /= 2;
+  a.lB = log2i(B);
+  const bool cross = lf && B > 1;
+  a.t.BP = cross ? B + 1 : B;
+  const int R0 = L ? L->gd.radix[0] : 1;
+  a.t.R0 = R0;
+  a.t.mR0 = magic(R0);
+  // fewer columns than one LDS access covers: blocks an odd multiple of B apart
+  a.t.skew = !lf && B * E < 128 && R0 % 2 == 0 ? B : 0;
+  a.t.P0 = R0 * a.t.BP + a.t.skew;
+  const long long nwg = (ncol + B - 1) / B;
+  if (nwg > 0x7fffffffLL) throw Error{"grid too large", -1};
+  size_t data = (size_t)((long long)m * a.t.BP + (long long)(m / R0) * a.t.skew) * E;
+  if (!L) {
+    if (data > kLdsMax) throw Error{"column copy does not fit in LDS", -1};
+    a.dld = make_fdiv(c.nld);
+    a.dst = make_fdiv(c.nst);
+    k_gcopy<real_t><<<(unsigned)nwg, 256, data, st>>>(a);
+    check_hip(hipGetLastError(), "k_gcopy launch");
+    return;
+  }
+  a.L = make_desc(*L);
+  a.tw = L->gtw;
+  a.dld = make_fdiv(m);
+  a.dst = make_fdiv(std::max(c.nst, 1));
+  if (lf) data = ((data + 15) & ~(size_t)15) + kColTab;
+  const size_t bytes = place_twiddles(data, *L, &a.tw_lds, &a.tw_off);
+  if (bytes > kLdsMax) throw Error{"column transform does not fit in LDS", -1};
+  const int nt = pick_threads(*L, B, bytes, nwg);
+  const bool fwd = c.fwd || c.kind == COL_DCT1 || c.kind == COL_DST1;
+  const bool ld_id = c.nld == m && (c.ld_lo >= m || (c.ld_hi <= c.ld_lo && c.ld_shift == 0));
+  const bool st_id = c.nst == m && (c.st_lo >= m || c.st_shift == 0);
+  const bool map = c.kind != COL_C2C || !(ld_id && st_id);
+  const long long nout = B / std::max(c.n_inner, 1) + 2;
+  auto span = [&](long long si, long long sl, long long so) {
+    return (nout * so + (long long)c.n_inner * si + (long long)(std::max(c.nld, c.nst) + 1) * sl) * E;
+  };
+  const bool fits = span(c.si_in, c.sl_in, c.so_in) < (1LL << 32) && span(c.si_out, c.sl_out, c.so_out) < (1LL << 32);
+  typedef unsigned U32;
+  typedef unsigned long long U64;
+  const unsigned g = (unsigned)nwg;
+  if (fwd) {
+    if (lf_in) go_col<true, true, 1, U64>(a, g, nt, bytes, st);
+    else if (lf_out) go_col<true, true, 2, U64>(a, g, nt, bytes, st);
+    else if (!fits) go_col<true, true, 0, U64>(a, g, nt, bytes, st);
+    else if (map) go_col<true, true, 0, U32>(a, g, nt, bytes, st);
+    else go_col<true, false, 0, U32>(a, g, nt, bytes, st);
+  } else {
+    if (lf_in) go_col<false, true, 1, U64>(a, g, nt, bytes, st);
+    else if (lf_out) go_col<false, true, 2, U64>(a, g, nt, bytes, st);
+    else if (!fits) go_col<false, true, 0, U64>(a, g, nt, bytes, st);
+    else if (map) go_col<false, true, 0, U32>(a, g, nt, bytes, st);
+    else go_col<false, false, 0, U32>(a, g, nt, bytes, st);
+  }
+  check_hip(hipGetLastError(), "k_gcol launch");
+}
+
+// tile of the X kernels; returns the LDS bytes
+static size_t x_tile(GXArgs& a, const Len1D& L, long long nrows, long long row, int* nt, unsigned* nwg) {
+  const long long pairs = (nrows + 1) / 2, E = sizeof(cplx_t);
+  const int n = L.gd.n;
+  int B = 16;
+  while (B > 1 && ((long long)n * (B + 1) * E > L.tile_bytes || (2LL * B + 1) * row * E >= (1LL << 32))) B /= 2;
+  while (B > 2 && (pairs + B - 1) / B < 512) B /= 2;
+  a.lB = log2i(B);
+  a.lBL = std::min(2, a.lB);
+  a.t.BP = B > 1 ? B + 1 : 1;
+  a.t.R0 = L.gd.radix[0];
+  a.t.mR0 = magic(a.t.R0);
+  a.t.P0 = a.t.R0 * a.t.BP;
+  a.L = make_desc(L);
+  a.tw = L.gtw;
+  a.dn0 = make_fdiv(n / a.t.R0);
+  const size_t bytes = place_twiddles((size_t)n * a.t.BP * E, L, &a.tw_lds, &a.tw_off);
+  if (bytes > kLdsMax) throw Error{"X transform does not fit in LDS", -1};
+  const long long g = (pairs + B - 1) / B;
+  if (g > 0x7fffffffLL) throw Error{"grid too large", -1};
+  *nwg = (unsigned)g;
+  *nt = pick_threads(L, B, bytes, g);
+  return bytes;
+}
+
+void gen_launch_x_r2c(const Len1D& L, const real_t* in, cplx_t* out, long long nrows, long long si_row,
+                      long long so_row, int nxo, bool rev, hipStream_t st) {
+  GXArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.in = in; a.out = out; a.nrows = nrows; a.si_row = si_row; a.so_row = so_row;
+  a.nk = nxo; a.dnk = make_fdiv(nxo);
+  a.rev = rev ? 1 : 0;
+  int nt;
+  unsigned g;
+  const size_t bytes = x_tile(a, L, nrows, std::max(si_row, so_row), &nt, &g);
+  k_gx_r2c<real_t><<<g, nt, bytes, st>>>(a);
+  check_hip(hipGetLastError(), "k_gx_r2c launch");
+}
+
+void gen_launch_x_c2r(const Len1D& L, const cplx_t* in, real_t* out, long long nrows, long long si_row,
+                      long long so_row, int nxi, bool rev, hipStream_t st) {
+  GXArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.in = in; a.out = out; a.nrows = nrows; a.si_row = si_row; a.so_row = so_row;
+  a.nk = nxi; a.dnk = make_fdiv(L.gd.n / 2 + 1);
+  a.rev = rev ? 1 : 0;
+  int nt;
+  unsigned g;
+  const size_t bytes = x_tile(a, L, nrows, std::max(si_row, so_row), &nt, &g);
+  k_gx_c2r<real_t><<<g, nt, bytes, st>>>(a);
+  check_hip(hipGetLastError(), "k_gx_c2r launch");
+}
+
+template <class K>
+static void allow_big_lds(K kernel) {
+  (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax);
+  (void)hipGetLastError();  // a refused attribute leaves the default limit, not a pending error
+}
+template <bool FWD>
+static void prep_dir() {
+  typedef unsigned U32;
+  typedef unsigned long long U64;
+  allow_big_lds(k_gcol<real_t, FWD, false, 0, U32>);
+  allow_big_lds(k_gcol<real_t, FWD, true, 0, U32>);
+  allow_big_lds(k_gcol<real_t, FWD, true, 0, U64>);
+  allow_big_lds(k_gcol<real_t, FWD, true, 1, U64>);
+  allow_big_lds(k_gcol<real_t, FWD, true, 2, U64>);
+}
+void gen_prep_kernels() {
+  static std::once_flag once;
+  std::call_once(once, [] {
+    prep_dir<true>();
+    prep_dir<false>();
+    allow_big_lds(k_gcopy<real_t>);
+    allow_big_lds(k_gx_r2c<real_t>);
+    allow_big_lds(k_gx_c2r<real_t>);
+  });
+}
+
+}  // namespace p3amd

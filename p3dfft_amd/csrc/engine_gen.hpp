@@ -1,0 +1,34 @@
+// engine_gen.hpp -- transforms of any length up to max_len() whose radix
+// schedule is a run-time value (lengths without compile-time specialised
+// kernels); the kernels are in engine_gen.hip.
+#pragma once
+#include "engine.hpp"
+
+namespace p3amd {
+
+// the radix schedule of a length: factors of at most 16 where the length has
+// such a form, a prime above 16 otherwise stands between two factors (1 if
+// there is none), since the first and the last stage hold a whole butterfly
+// in registers
+std::vector<int> gen_factors(int n);
+// the same for factors in a given order (a plan-time candidate)
+std::vector<int> gen_wrap(const std::vector<int>& f);
+#ifndef P3_RM
+#define P3_RM 10
+#endif
+constexpr int kGenMaxRadix = P3_RM;
+inline bool gen_in_registers(int r) { return r <= kGenMaxRadix; }
+// a prime radix above that (the specialised schedules also hold 16)
+inline bool gen_is_prime_stage(int r) { return r > kGenMaxRadix && r % 2 == 1; }
+
+// the launchers of engine.hpp for these kernels
+void gen_launch_x_r2c(const Len1D& L, const real_t* in, cplx_t* out, long long nrows, long long si_row,
+                      long long so_row, int nxo, bool rev, hipStream_t st);
+void gen_launch_x_c2r(const Len1D& L, const cplx_t* in, real_t* out, long long nrows, long long si_row,
+                      long long so_row, int nxi, bool rev, hipStream_t st);
+// L: the plan of the transform length (null: COL_COPY)
+void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, hipStream_t st);
+// raise the kernels' dynamic-LDS limits (once, when a length is planned)
+void gen_prep_kernels();
+
+}  // namespace p3amd

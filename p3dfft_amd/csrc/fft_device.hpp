@@ -228,12 +228,83 @@ __device__ __forceinline__ void dftp(cpx<T>* v) {
 }
 
 template <int R, bool FWD, class T>
+__device__ __forceinline__ void dft(cpx<T>* v);
+
+// 9 points as 3 x 3, twiddles W9^(n1 k1)
+template <bool FWD, class T>
+__device__ __forceinline__ void dft9(cpx<T>* v) {
+  constexpr double C[5] = {1.0, 0.76604444311897803520, 0.17364817766693034885, -0.5, -0.93969262078590838405};
+  constexpr double S[5] = {0.0, 0.64278760968653932632, 0.98480775301220805937, 0.86602540378443864676,
+                           0.34202014332566873304};
+  cpx<T> y[3][3];
+#pragma unroll
+  for (int n1 = 0; n1 < 3; n1++) {
+    cpx<T> t[3] = {v[n1], v[n1 + 3], v[n1 + 6]};
+    dft3<FWD>(t);
+#pragma unroll
+    for (int k1 = 0; k1 < 3; k1++) {
+      const int m = n1 * k1;
+      if (m == 0) {
+        y[n1][k1] = t[k1];
+      } else {
+        const T c = (T)C[m], sy = FWD ? -(T)S[m] : (T)S[m];
+        y[n1][k1] = mk<T>(t[k1].x * c - t[k1].y * sy, t[k1].x * sy + t[k1].y * c);
+      }
+    }
+  }
+#pragma unroll
+  for (int k1 = 0; k1 < 3; k1++) {
+    cpx<T> t[3] = {y[0][k1], y[1][k1], y[2][k1]};
+    dft3<FWD>(t);
+#pragma unroll
+    for (int k2 = 0; k2 < 3; k2++) v[k1 + 3 * k2] = t[k2];
+  }
+}
+
+// N1 x N2 points, N1 and N2 coprime, without twiddles (the prime-factor
+// algorithm of Good and Thomas: the input index runs over N2 n1 + N1 n2, the
+// output index is recovered by the Chinese remainder theorem)
+constexpr int inv_mod(int a, int m) {
+  for (int x = 1; x < m; x++)
+    if (a % m * x % m == 1) return x;
+  return 0;
+}
+template <int N1, int N2, bool FWD, class T>
+__device__ __forceinline__ void dft_pfa(cpx<T>* v) {
+  constexpr int N = N1 * N2;
+  constexpr int E1 = N2 * inv_mod(N2, N1), E2 = N1 * inv_mod(N1, N2);
+  cpx<T> y[N1][N2];
+#pragma unroll
+  for (int n1 = 0; n1 < N1; n1++) {
+#pragma unroll
+    for (int n2 = 0; n2 < N2; n2++) y[n1][n2] = v[(N2 * n1 + N1 * n2) % N];
+    dft<N2, FWD>(y[n1]);
+  }
+#pragma unroll
+  for (int k2 = 0; k2 < N2; k2++) {
+    cpx<T> t[N1];
+#pragma unroll
+    for (int n1 = 0; n1 < N1; n1++) t[n1] = y[n1][k2];
+    dft<N1, FWD>(t);
+#pragma unroll
+    for (int k1 = 0; k1 < N1; k1++) v[(E1 * k1 + E2 * k2) % N] = t[k1];
+  }
+}
+
+template <int R, bool FWD, class T>
 __device__ __forceinline__ void dft(cpx<T>* v) {
-  if constexpr (R == 2) dft2<FWD>(v);
+  if constexpr (R == 1) return;
+  else if constexpr (R == 2) dft2<FWD>(v);
   else if constexpr (R == 3) dft3<FWD>(v);
   else if constexpr (R == 4) dft4<FWD>(v);
   else if constexpr (R == 5) dft5<FWD>(v);
+  else if constexpr (R == 6) dft_pfa<2, 3, FWD>(v);
   else if constexpr (R == 8) dft8<FWD>(v);
+  else if constexpr (R == 9) dft9<FWD>(v);
+  else if constexpr (R == 10) dft_pfa<2, 5, FWD>(v);
+  else if constexpr (R == 12) dft_pfa<4, 3, FWD>(v);
+  else if constexpr (R == 14) dft_pfa<2, 7, FWD>(v);
+  else if constexpr (R == 15) dft_pfa<3, 5, FWD>(v);
   else if constexpr (R == 16) dft16<FWD>(v);
   else dftp<R, FWD>(v);
 }
@@ -251,7 +322,7 @@ __device__ __forceinline__ int fdiv(int x, const FDiv& f) {
 }
 
 // ---------------------------------------------------------------------------
-// length descriptor (host builds it; passed by value in kernel arguments)
+// length descriptor (built by the host)
 // ---------------------------------------------------------------------------
 constexpr int kMaxStages = 24;
 struct LenDesc {
@@ -260,11 +331,7 @@ struct LenDesc {
   int radix[kMaxStages];   // radix of each stage
   int ns[kMaxStages];      // product of the radices of earlier stages
   int twoff[kMaxStages];   // offset of each stage's twiddles in the table
-  FDiv dns[kMaxStages];    // divide by ns
-  FDiv dnr[kMaxStages];    // divide by n / radix
-  FDiv dn;                 // divide by n
-  int fulloff;             // offset of the full table W_n^e, e = 0..n-1
-  int twcount;             // total entries (stage tables + full table)
+  int twcount;             // total entries
 };
 
 }  // namespace p3amd
