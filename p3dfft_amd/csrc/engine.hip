@@ -2065,7 +2065,11 @@ static const PlaneInfo* find_plane(int nx, int ny) {
   return it == tab.end() ? nullptr : &it->second;
 }
 
-bool launch_xy_plane(bool fwd, const void* in, void* out, int nx, int ny, int nz, hipStream_t st) {
+static size_t plane_bytes(const PlaneInfo& p, const Len1D& Lx, const Len1D& Ly) {
+  return (size_t)p.data + (size_t)(Lx.d.twcount + (Lx.d.n == Ly.d.n ? 0 : Ly.d.twcount)) * sizeof(Tw);
+}
+
+bool xy_plane_applies(int nx, int ny, int nz) {
   if (g_plane_mode == 0 || !g_use_ct || nz <= 0) return false;
   if (g_plane_mode == 2 &&
       ((long long)nx * ny * nz > (1LL << 22) || (nz < 64 && (long long)nx * ny > 64 * 64)))
@@ -2075,16 +2079,19 @@ bool launch_xy_plane(bool fwd, const void* in, void* out, int nx, int ny, int nz
   const Len1D& Lx = get_len(nx);
   const Len1D& Ly = get_len(ny);
   // the kernels' radix schedules must be the plans' (the twiddle layout)
-  if (!find_ct(Lx) || !find_ct(Ly)) return false;
+  return find_ct(Lx) && find_ct(Ly) && plane_bytes(*p, Lx, Ly) <= kLdsMax;
+}
+
+void launch_xy_plane(bool fwd, const void* in, void* out, int nx, int ny, int nz, hipStream_t st) {
+  const PlaneInfo* p = find_plane(nx, ny);
+  const Len1D& Lx = get_len(nx);
+  const Len1D& Ly = get_len(ny);
   PlaneArgs a;
   a.in = in; a.out = out;
   a.twx = Lx.tw; a.twy = Ly.tw;
   a.ntwx = Lx.d.twcount; a.ntwy = nx == ny ? 0 : Ly.d.twcount;
-  const size_t bytes = (size_t)p->data + (size_t)(a.ntwx + a.ntwy) * sizeof(Tw);
-  if (bytes > kLdsMax) return false;
-  p->go(fwd, a, nz, bytes, st);
+  p->go(fwd, a, nz, plane_bytes(*p, Lx, Ly), st);
   check_hip(hipGetLastError(), fwd ? "k_xy_plane_fwd launch" : "k_yx_plane_bwd launch");
-  return true;
 }
 
 // The byte offsets of a column tile relative to its first column stay below

@@ -92,9 +92,11 @@ bool launch_x_c2r_tab(const cplx_t* in, real_t* out, long long nrows, int nx, in
 // X and Y transforms of whole z-planes in one launch (one workgroup per
 // plane, the plane kept in LDS), for small grids of the (nx, ny) pairs that
 // have such kernels: forward real (nx, ny, nz) -> half spectrum (nx/2+1, ny,
-// nz), backward the reverse (Im of the DC and Nyquist modes ignored).  False
-// when the grid does not qualify (the caller runs the separate passes).
-bool launch_xy_plane(bool fwd, const void* in, void* out, int nx, int ny, int nz, hipStream_t st);
+// nz), backward the reverse (Im of the DC and Nyquist modes ignored).  Only
+// for grids that xy_plane_applies names (the caller runs the separate passes
+// on the others).
+bool xy_plane_applies(int nx, int ny, int nz);
+void launch_xy_plane(bool fwd, const void* in, void* out, int nx, int ny, int nz, hipStream_t st);
 // 0: never; 1: wherever they apply; 2 (default): on small grids only.
 void set_plane_kernels(int mode);
 // X rows of 512 points through the wave kernels (one wavefront per row pair,

@@ -14,6 +14,7 @@ namespace p3amd {
 struct Pending {
   int slot;
   hipEvent_t a, b;
+  bool own_a;  // a belongs to this entry (else it is the b of the one before)
 };
 
 // The reference's module variables (build/module.F90:101-176) for one setup.
@@ -51,6 +52,11 @@ struct State {
   double timers[12] = {0};
   bool timing = true;
   hipEvent_t open[12] = {};
+  bool open_own[12] = {};
+  // the end of the last timed stage of the current call and its stream: the
+  // start of the next one (null: the next stage records its own)
+  hipEvent_t chain = nullptr;
+  hipStream_t chain_stream = nullptr;
   std::vector<Pending> pend;
   std::vector<hipEvent_t> evpool;
 };
