@@ -117,7 +117,7 @@ struct ColArgs {
   int xcd;
   const int2* ltab;  // table-addressed rows (see ColIO)
   const int2* stab;
-  int tab_off;       // byte offset of the LDS copy of the row tables
+  int tab_off;       // byte offset of the LDS copy of the row tables (length-fastest views: of the columns' offsets)
   // Chebyshev recurrence fused into a DCT-I column pass (k_col_ct): applied
   // to the output rows in LDS before they are stored; cheby_off: byte offset
   // of its per-wave sums behind the tile
@@ -1088,6 +1088,21 @@ __global__ __launch_bounds__(NT, W) void k_col_ct(ColArgs a) {
   }
 }
 
+// C2C columns with a length-fastest ("STRIDE1") input (IN) or output
+template <class T, bool FWD, bool IN, int TX, int NT, class RL, int W, bool TWL>
+__global__ __launch_bounds__(NT, W) void k_collf_ct(ColArgs a) {
+  cpx<T>* lds = (cpx<T>*)g_smem;
+  const auto* tw = ct_twiddles<T, NT, TWL>(a.tw, a.tw_off, a.L.twcount);
+  const long long ncol = (long long)a.n_inner * a.n_outer;
+  const long long c0 = (long long)tile_of(a.rev, a.xcd) * TX;
+  const int nb = (int)(ncol - c0 < TX ? ncol - c0 : TX);
+  const ColIO io = col_io<T, TX>(a, c0, nb);
+  unsigned long long* colb = (unsigned long long*)(g_smem + a.tab_off);
+  if (threadIdx.x < TX) colb[threadIdx.x] = IN ? io.lane_in : io.lane_out;
+  if constexpr (IN) __syncthreads();  // else the first stage's barrier
+  run_fft_lenfast<T, FWD, TX, NT, IN>(lds, tw, io, colb, RL{});
+}
+
 // fused Z-solve: the Z column of a spectrum (nxh, ny, nz), forward FFT,
 // -scale/|k|^2, inverse FFT, in place
 template <class T, int TX, int NT, class RL, int W, bool TWL>
@@ -1628,6 +1643,8 @@ struct CtInfo {
   void (*col)(bool, const ColArgs&, unsigned, size_t, hipStream_t);
   void (*colio)(bool, bool, bool, const ColArgs&, unsigned, size_t, hipStream_t);
   void (*colpipe)(bool, bool, const ColArgs&, unsigned, size_t, hipStream_t);
+  void (*collf)(bool, bool, const ColArgs&, unsigned, size_t, hipStream_t);
+  bool twl_lf;          // twiddles in LDS in the length-fastest kernels
   void (*xr2c)(const XArgs&, unsigned, size_t, hipStream_t);
   void (*xc2r)(const XArgs&, unsigned, size_t, hipStream_t);
   void (*zsolve)(const ColArgs&, double, int, int, unsigned, size_t, hipStream_t);
@@ -1672,6 +1689,11 @@ struct CtLen {
   // CU; the table-addressed form keeps both row tables (2 N int2) in LDS
   static constexpr bool PIPE = DC > kCtLdsTw;
   static constexpr bool TWLP = TWLC && round16(DC + TWB) + 2 * N * (long long)sizeof(int2) <= (long long)kLdsMax;
+  // the length-fastest kernels' tile, its columns' offsets behind it
+  static constexpr long long DF = DC + 8 * (TX + TX % 2);
+  static constexpr bool TWLF =
+      TWB > 0 && (DF + TWB <= kCtLdsTw || (DF > kCtLdsTw && DF + TWB <= (long long)kLdsMax));
+  static constexpr int WF = ct_waves(DF + (TWLF ? TWB : 0), NTC);
   // waves per SIMD the LDS footprint allows: the register budget of each kernel
   static constexpr int WC = ct_waves(DC + (TWLC ? TWB : 0), NTC);
   static constexpr int WX = ct_waves(DX + (TWLX ? TWB : 0), NTX);
@@ -1719,6 +1741,16 @@ struct CtLen {
       }
     }
   }
+  // in: the input is length-fastest, else the output
+  static void collf(bool fwd, bool in, const ColArgs& a, unsigned g, size_t bytes, hipStream_t s) {
+    if (fwd) {
+      if (in) go(k_collf_ct<real_t, true, true, TX, NTC, RL, WF, TWLF>, g, NTC, bytes, s, a);
+      else go(k_collf_ct<real_t, true, false, TX, NTC, RL, WF, TWLF>, g, NTC, bytes, s, a);
+    } else {
+      if (in) go(k_collf_ct<real_t, false, true, TX, NTC, RL, WF, TWLF>, g, NTC, bytes, s, a);
+      else go(k_collf_ct<real_t, false, false, TX, NTC, RL, WF, TWLF>, g, NTC, bytes, s, a);
+    }
+  }
   static void xr2c(const XArgs& a, unsigned g, size_t bytes, hipStream_t s) {
     if (a.xt) gox(k_x_r2c_ct<real_t, BX, NTX, RL, WX, TWLX, true>, g, NTX, bytes, s, a);
     else gox(k_x_r2c_ct<real_t, BX, NTX, RL, WX, TWLX, false>, g, NTX, bytes, s, a);
@@ -1740,6 +1772,8 @@ struct CtLen {
     allow_big_lds(k_colio_ct<real_t, FWD, TX, NTC, RL, WC, TWLC, true, unsigned>);
     allow_big_lds(k_colio_ct<real_t, FWD, TX, NTC, RL, WC, TWLC, false, unsigned long long>);
     allow_big_lds(k_colio_ct<real_t, FWD, TX, NTC, RL, WC, TWLC, false, unsigned>);
+    allow_big_lds(k_collf_ct<real_t, FWD, true, TX, NTC, RL, WF, TWLF>);
+    allow_big_lds(k_collf_ct<real_t, FWD, false, TX, NTC, RL, WF, TWLF>);
     if constexpr (PIPE) {
       allow_big_lds(k_colio_pipe<real_t, FWD, TX, NTC, RL, WC, TWLP, TabRows>);
       allow_big_lds(k_colio_pipe<real_t, FWD, TX, NTC, RL, WC, TWLC, unsigned>);
@@ -1778,7 +1812,7 @@ struct CtLen {
     c.nr = (int)sizeof...(Rs);
     for (int i = 0; i < c.nr; i++) c.radix[i] = rs[i];
     c.twl_col = TWLC; c.twl_x = TWLX; c.twl_tab = TWLT; c.twb = TWB;
-    c.pipe = PIPE; c.twl_pipe_tab = TWLP;
+    c.pipe = PIPE; c.twl_pipe_tab = TWLP; c.twl_lf = TWLF; c.collf = &collf;
     c.col = &col; c.colio = &colio; c.colpipe = &colpipe; c.xr2c = &xr2c; c.xc2r = &xc2r; c.zsolve = &zsolve; c.prep = &prep;
     c.xgrp = &xgrp; c.cgrp = &cgrp; c.zgrp = &zgrp;
     return c;
@@ -2104,12 +2138,13 @@ void launch_xy_plane(bool fwd, const void* in, void* out, int nx, int ny, int nz
 // The byte offsets of a column tile relative to its first column stay below
 // 2^32: lanes span at most TX/n_inner + 2 outer indices and n_inner inner
 // ones, plus `rows` rows.
-static bool col_fits32(const ColSpec& c, int TX, int rows) {
+static bool col_side_fits32(const ColSpec& c, bool in, int TX, int rows) {
   const long long nout = TX / std::max(c.n_inner, 1) + 2;
-  auto span = [&](long long si, long long sl, long long so) {
-    return (nout * so + (long long)c.n_inner * si + (long long)rows * sl + 1) * (long long)sizeof(cplx_t);
-  };
-  return span(c.si_in, c.sl_in, c.so_in) < (1LL << 32) && span(c.si_out, c.sl_out, c.so_out) < (1LL << 32);
+  const long long si = in ? c.si_in : c.si_out, sl = in ? c.sl_in : c.sl_out, so = in ? c.so_in : c.so_out;
+  return (nout * so + (long long)c.n_inner * si + (long long)rows * sl + 1) * (long long)sizeof(cplx_t) < (1LL << 32);
+}
+static bool col_fits32(const ColSpec& c, int TX, int rows) {
+  return col_side_fits32(c, true, TX, rows) && col_side_fits32(c, false, TX, rows);
 }
 
 // Persistent column kernels (k_colio_pipe) for the lengths whose tile takes
@@ -2239,6 +2274,25 @@ bool launch_col(const ColSpec& c, hipStream_t st) {
       ct->colio(fwd, pr, !fits, a, (unsigned)((ncol + TX - 1) / TX), bytes, st);
       check_hip(hipGetLastError(), "k_colio_ct launch");
       return false;
+    }
+    // one side length-fastest, the other one unpruned rows; the row side's
+    // stride decides the tile order as in a Z pass (XCD-aware -> dispatch, us,
+    // forward: FP64 256^3 82 -> 68, FP32 512x512x256 134 -> 111 where the rule
+    // says dispatch; FP64 256x252x256 56 -> 64, FP32 126x64x2048 35 -> 42 where
+    // it does not).  Against the LDS pass with bank conflicts (k_col_ct),
+    // forward / backward: FP32 256^3 54 / 42 -> 25 / 28 us, 384^3 184 / 145 ->
+    // 98 / 115; FP64 384^3 225 / 213 -> 189 / 211
+    if (c.kind == COL_C2C && a.ld_lenfast != a.st_lenfast && (a.ld_lenfast ? st_id : ld_id) && c.nld == nfft &&
+        col_side_fits32(c, !a.ld_lenfast, TX, rows) && !g_wide_offsets) {
+      size_t lf = (size_t)round16((long long)TX * nfft * (long long)sizeof(cplx_t));
+      a.tab_off = (int)lf;
+      lf = ct_lds(lf + 8 * (size_t)(TX + TX % 2), ct->twl_lf, *ct, &a.tw_lds, &a.tw_off);
+      if (lf <= kLdsMax) {
+        a.xcd = flat_dispatch_order(c) ? 0 : 1;
+        ct->collf(fwd, a.ld_lenfast != 0, a, (unsigned)((ncol + TX - 1) / TX), lf, st);
+        check_hip(hipGetLastError(), "k_collf_ct launch");
+        return false;
+      }
     }
     // DCT-I without the fused Chebyshev recurrence: the direct-load kernel
     // reads the even extension's mirrored rows from the input itself (no LDS

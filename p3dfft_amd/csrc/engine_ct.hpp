@@ -27,6 +27,16 @@ struct RProd<A> {
   static constexpr int value = A;
 };
 
+// element `row` of sequence b in a tile of B sequences: rows BP elements apart,
+// or (BP = 0) rows of B elements rotated by the row, so that lanes along the
+// rows and lanes along the sequences both meet distinct LDS banks without
+// padding
+template <int B, int BP>
+__device__ __forceinline__ int lds_at(int row, int b) {
+  if constexpr (BP == 0) return row * B + ((b + row) & (B - 1));
+  else return row * BP + b;
+}
+
 // One stage: radix R, Ns = product of the earlier radices, twiddles at Off.
 template <class T, int R, bool FWD, int N, int B, int BP, int NT, int Ns, int Off>
 __device__ __forceinline__ void stage_ct(cpx<T>* lds, const typename TwT<T>::type* tw) {
@@ -40,7 +50,7 @@ __device__ __forceinline__ void stage_ct(cpx<T>* lds, const typename TwT<T>::typ
     if ((total % NT) == 0 || it < total) {
       const int j = it / B, b = it % B;
 #pragma unroll
-      for (int r = 0; r < R; r++) v[m][r] = lds[(j + r * nR) * BP + b];
+      for (int r = 0; r < R; r++) v[m][r] = lds[lds_at<B, BP>(j + r * nR, b)];
       if constexpr (Ns > 1) {
         const int k = j % Ns;
         const typename TwT<T>::type* w = tw + Off + k * (R - 1);
@@ -59,7 +69,7 @@ __device__ __forceinline__ void stage_ct(cpx<T>* lds, const typename TwT<T>::typ
       const int k = j % Ns;
       const int base = (j - k) * R + k;
 #pragma unroll
-      for (int r = 0; r < R; r++) lds[(base + r * Ns) * BP + b] = v[m][r];
+      for (int r = 0; r < R; r++) lds[lds_at<B, BP>(base + r * Ns, b)] = v[m][r];
     }
   }
   __syncthreads();
@@ -193,7 +203,7 @@ __device__ __forceinline__ void stage0_put(cpx<T>* lds, Stage0Regs<T, R, N, B, N
 // that every load of the tile is issued back to back: composed of the two
 // steps, the compiler interleaved them with address arithmetic and waited
 // before the last one)
-template <class T, int R, bool FWD, int N, int B, int NT, bool PR, class Off>
+template <class T, int R, bool FWD, int N, int B, int NT, bool PR, class Off, int BP = B>
 __device__ __forceinline__ void stage0_global(cpx<T>* lds, const ColIO& io) {
   static_assert(NT % B == 0, "one column per thread");
   constexpr bool TB = std::is_same<Off, TabRows>::value;
@@ -236,14 +246,14 @@ __device__ __forceinline__ void stage0_global(cpx<T>* lds, const ColIO& io) {
       const int j = it / B, b = it % B;
       dft<R, FWD>(v[m]);
 #pragma unroll
-      for (int r = 0; r < R; r++) lds[(j * R + r) * B + b] = v[m][r];
+      for (int r = 0; r < R; r++) lds[lds_at<B, BP>(j * R + r, b)] = v[m][r];
     }
   }
   __syncthreads();
 }
 
 // last stage: Ns * R == N, so every butterfly index j < Ns and k == j
-template <class T, int R, bool FWD, int N, int B, int NT, int Ns, int TwOff, bool PR, class Off>
+template <class T, int R, bool FWD, int N, int B, int BP, int NT, int Ns, int TwOff, bool PR, class Off>
 __device__ __forceinline__ void stageL_global(const cpx<T>* lds, const typename TwT<T>::type* tw,
                                               const ColIO& io) {
   static_assert(Ns * R == N, "last stage");
@@ -259,7 +269,7 @@ __device__ __forceinline__ void stageL_global(const cpx<T>* lds, const typename 
       const int j = it / B, b = it % B;
       cpx<T> v[R];
 #pragma unroll
-      for (int r = 0; r < R; r++) v[r] = lds[(j + r * Ns) * B + b];
+      for (int r = 0; r < R; r++) v[r] = lds[lds_at<B, BP>(j + r * Ns, b)];
       const typename TwT<T>::type* w = tw + TwOff + j * (R - 1);
 #pragma unroll
       for (int r = 1; r < R; r++) v[r] = twmul<FWD>(v[r], w[r - 1]);
@@ -295,13 +305,13 @@ __device__ __forceinline__ void stageL_global(const cpx<T>* lds, const typename 
   }
 }
 
-template <class T, bool FWD, int N, int B, int NT, int Ns, int TwOff, bool PR, class Off, int R, int... Rest>
+template <class T, bool FWD, int N, int B, int BP, int NT, int Ns, int TwOff, bool PR, class Off, int R, int... Rest>
 __device__ __forceinline__ void mid_and_last(cpx<T>* lds, const typename TwT<T>::type* tw, const ColIO& io) {
   if constexpr (sizeof...(Rest) == 0) {
-    stageL_global<T, R, FWD, N, B, NT, Ns, TwOff, PR, Off>(lds, tw, io);
+    stageL_global<T, R, FWD, N, B, BP, NT, Ns, TwOff, PR, Off>(lds, tw, io);
   } else {
-    stage_ct<T, R, FWD, N, B, B, NT, Ns, TwOff>(lds, tw);
-    mid_and_last<T, FWD, N, B, NT, Ns * R, (Ns > 1 ? TwOff + Ns * (R - 1) : TwOff), PR, Off, Rest...>(lds, tw, io);
+    stage_ct<T, R, FWD, N, B, BP, NT, Ns, TwOff>(lds, tw);
+    mid_and_last<T, FWD, N, B, BP, NT, Ns * R, (Ns > 1 ? TwOff + Ns * (R - 1) : TwOff), PR, Off, Rest...>(lds, tw, io);
   }
 }
 
@@ -311,7 +321,7 @@ __device__ __forceinline__ void run_fft_io(cpx<T>* lds, const typename TwT<T>::t
   static_assert(sizeof...(Rs) >= 1, "at least two stages");
   constexpr int N = R0 * RProd<Rs...>::value;
   stage0_global<T, R0, FWD, N, B, NT, PR, Off>(lds, io);
-  mid_and_last<T, FWD, N, B, NT, R0, 0, PR, Off, Rs...>(lds, tw, io);
+  mid_and_last<T, FWD, N, B, B, NT, R0, 0, PR, Off, Rs...>(lds, tw, io);
 }
 
 // run_fft_io over the tiles t0, t0 + dt, ... below t1 of one workgroup: the
@@ -334,7 +344,7 @@ __device__ __forceinline__ void run_fft_io_pipe(cpx<T>* lds, const typename TwT<
       io = make_io(t + dt);
       stage0_load<T, R0, N, B, NT, PR, Off>(rg, io);
     }
-    mid_and_last<T, FWD, N, B, NT, R0, 0, PR, Off, Rs...>(lds, tw, cur);
+    mid_and_last<T, FWD, N, B, B, NT, R0, 0, PR, Off, Rs...>(lds, tw, cur);
     // the last stage's LDS reads before the next tile's first-stage writes
     __syncthreads();
   }
@@ -367,7 +377,7 @@ __device__ __forceinline__ void run_fft_io_tab(cpx<T>* lds, int2* tl, const type
   for (int i = threadIdx.x; i < N; i += NT) tl[i] = stab[i];
   __syncthreads();
   io.stab = tl;
-  mid_and_last<T, FWD, N, B, NT, R0, 0, false, TabRows, Rs...>(lds, tw, io);
+  mid_and_last<T, FWD, N, B, B, NT, R0, 0, false, TabRows, Rs...>(lds, tw, io);
 }
 
 // Spectral solve along the column: forward FFT, per-mode multiply by
@@ -398,7 +408,51 @@ __device__ __forceinline__ void run_fft_solve(cpx<T>* lds, const typename TwT<T>
     lds[q] = mk<T>((T)(v.x * f), (T)(v.y * f));
   }
   __syncthreads();
-  mid_and_last<T, false, N, B, NT, 1, 0, false, unsigned, R0, Rs...>(lds, tw, io);
+  mid_and_last<T, false, N, B, B, NT, 1, 0, false, unsigned, R0, Rs...>(lds, tw, io);
+}
+
+// Columns whose input (IN) or output is length-fastest, the other side being
+// rows, through a tile with rotated rows (a padded one costs the FP64 lengths
+// 256 and 1024 a workgroup per CU: 256^3 82.4 us against 74.6 us of the kernel
+// that met bank conflicts).  colb[b]:
+// byte offset of column b of the length-fastest side from the tile's first.
+template <class T, bool FWD, int B, int NT, bool IN, int R0, int... Rs>
+__device__ __forceinline__ void run_fft_lenfast(cpx<T>* lds, const typename TwT<T>::type* tw, const ColIO& io,
+                                                const unsigned long long* colb, RList<R0, Rs...>) {
+  static_assert(sizeof...(Rs) >= 1, "at least two stages");
+  constexpr int N = R0 * RProd<Rs...>::value, BP = 0;
+  constexpr int LI = (B * N + NT - 1) / NT;
+  if constexpr (IN) {
+    cpx<T> v[LI];
+#pragma unroll
+    for (int u = 0; u < LI; u++) {
+      const int q = threadIdx.x + u * NT, b = q / N, e = q % N;
+      const int src = e < io.ld_lo ? e : (e >= io.ld_hi ? e - io.ld_shift : -1);
+      const bool ok = ((B * N) % NT == 0 || q < B * N) && b < io.nb && src >= 0;
+      // items outside the tile load its first element (always valid) and are
+      // zeroed, so no load sits under a branch
+      const cpx<T> t = *(const cpx<T>*)(io.in + (ok ? colb[b] + (unsigned)src * (unsigned)sizeof(cpx<T>) : 0ull));
+      v[u] = ok ? t : mk<T>(0, 0);
+    }
+#pragma unroll
+    for (int u = 0; u < LI; u++) {
+      const int q = threadIdx.x + u * NT;
+      if ((B * N) % NT == 0 || q < B * N) lds[lds_at<B, BP>(q % N, q / N)] = v[u];
+    }
+    __syncthreads();
+    mid_and_last<T, FWD, N, B, BP, NT, 1, 0, false, unsigned, R0, Rs...>(lds, tw, io);
+  } else {
+    stage0_global<T, R0, FWD, N, B, NT, false, unsigned, BP>(lds, io);
+    stages_ct<T, FWD, N, B, BP, NT, R0, 0, Rs...>(lds, tw);
+#pragma unroll
+    for (int u = 0; u < LI; u++) {
+      const int q = threadIdx.x + u * NT, b = q / N, p = q % N;
+      const int e = p < io.st_lo ? p : p - io.st_shift;
+      const bool kept = p < io.st_lo || (p >= io.st_lo + io.st_shift && e < io.nst);
+      if (((B * N) % NT == 0 || q < B * N) && b < io.nb && kept)
+        *(cpx<T>*)(io.out + (colb[b] + (unsigned)e * (unsigned)sizeof(cpx<T>))) = lds[lds_at<B, BP>(p, b)];
+    }
+  }
 }
 
 // Twiddle table entries used by a radix list (all stages after the first).
