@@ -75,6 +75,56 @@ __device__ __forceinline__ void stage_ct(cpx<T>* lds, const typename TwT<T>::typ
   __syncthreads();
 }
 
+// The same stage in place: positions in mixed radix, the first radix the
+// fastest digit, so a butterfly writes the positions it read (see the first
+// stage's Rev): one barrier, nothing held across it.
+template <class T, int R, bool FWD, int N, int B, int BP, int NT, int Ns, int Off>
+__device__ __forceinline__ void stage_ip(cpx<T>* lds, const typename TwT<T>::type* tw) {
+  constexpr int total = B * (N / R);
+  constexpr int IT = (total + NT - 1) / NT;
+#pragma unroll
+  for (int m = 0; m < IT; m++) {
+    const int it = threadIdx.x + m * NT;
+    if ((total % NT) == 0 || it < total) {
+      const int j = it / B, b = it % B;
+      const int k = j % Ns, base = (j - k) * R + k;
+      cpx<T> v[R];
+#pragma unroll
+      for (int r = 0; r < R; r++) v[r] = lds[lds_at<B, BP>(base + r * Ns, b)];
+      const typename TwT<T>::type* w = tw + Off + k * (R - 1);
+#pragma unroll
+      for (int r = 1; r < R; r++) v[r] = twmul<FWD>(v[r], w[r - 1]);
+      dft<R, FWD>(v);
+#pragma unroll
+      for (int r = 0; r < R; r++) lds[lds_at<B, BP>(base + r * Ns, b)] = v[r];
+    }
+  }
+  __syncthreads();
+}
+
+template <class T, bool FWD, int N, int B, int BP, int NT, int Ns, int Off, int R, int... Rest>
+__device__ __forceinline__ void stages_ip(cpx<T>* lds, const typename TwT<T>::type* tw) {
+  stage_ip<T, R, FWD, N, B, BP, NT, Ns, Off>(lds, tw);
+  if constexpr (sizeof...(Rest) > 0)
+    stages_ip<T, FWD, N, B, BP, NT, Ns * R, Off + Ns * (R - 1), Rest...>(lds, tw);
+}
+
+// Input row of the first stage's butterfly j: j itself for the autosort
+// stages; for the in-place ones the digits of j over the later radices
+// (Rs..., the first of them the fastest digit of j) in reverse.
+struct RowNatural {
+  static __device__ __forceinline__ int at(int j) { return j; }
+};
+template <int... Rs>
+struct RowRev {
+  template <int R, int... Rest>
+  static __device__ __forceinline__ int step(int j, int acc) {
+    if constexpr (sizeof...(Rest) == 0) return acc * R + j;
+    else return step<Rest...>(j / R, acc * R + j % R);
+  }
+  static __device__ __forceinline__ int at(int j) { return step<Rs...>(j, 0); }
+};
+
 template <class T, bool FWD, int N, int B, int BP, int NT, int Ns, int Off, int R, int... Rest>
 __device__ __forceinline__ void stages_ct(cpx<T>* lds, const typename TwT<T>::type* tw) {
   stage_ct<T, R, FWD, N, B, BP, NT, Ns, Off>(lds, tw);
@@ -144,7 +194,7 @@ struct Stage0Regs {
 };
 
 // first stage, loads: the tile's values of every butterfly of this thread
-template <class T, int R, int N, int B, int NT, bool PR, class Off>
+template <class T, int R, int N, int B, int NT, bool PR, class Off, class Row>
 __device__ __forceinline__ void stage0_load(Stage0Regs<T, R, N, B, NT>& rg, const ColIO& io) {
   static_assert(NT % B == 0, "one column per thread");
   constexpr bool TB = std::is_same<Off, TabRows>::value;
@@ -154,7 +204,7 @@ __device__ __forceinline__ void stage0_load(Stage0Regs<T, R, N, B, NT>& rg, cons
   for (int m = 0; m < S::IT; m++) {
     const int it = threadIdx.x + m * NT;
     if ((S::total % NT) == 0 || it < S::total) {
-      const int j = it / B;
+      const int j = Row::at(it / B);
 #pragma unroll
       for (int r = 0; r < R; r++) {
         const int e = j + r * S::nR;
@@ -203,7 +253,7 @@ __device__ __forceinline__ void stage0_put(cpx<T>* lds, Stage0Regs<T, R, N, B, N
 // that every load of the tile is issued back to back: composed of the two
 // steps, the compiler interleaved them with address arithmetic and waited
 // before the last one)
-template <class T, int R, bool FWD, int N, int B, int NT, bool PR, class Off, int BP = B>
+template <class T, int R, bool FWD, int N, int B, int NT, bool PR, class Off, class Row, int BP = B>
 __device__ __forceinline__ void stage0_global(cpx<T>* lds, const ColIO& io) {
   static_assert(NT % B == 0, "one column per thread");
   constexpr bool TB = std::is_same<Off, TabRows>::value;
@@ -214,7 +264,7 @@ __device__ __forceinline__ void stage0_global(cpx<T>* lds, const ColIO& io) {
   for (int m = 0; m < S::IT; m++) {
     const int it = threadIdx.x + m * NT;
     if ((S::total % NT) == 0 || it < S::total) {
-      const int j = it / B;
+      const int j = Row::at(it / B);
 #pragma unroll
       for (int r = 0; r < R; r++) {
         const int e = j + r * S::nR;
@@ -305,13 +355,18 @@ __device__ __forceinline__ void stageL_global(const cpx<T>* lds, const typename 
   }
 }
 
-template <class T, bool FWD, int N, int B, int BP, int NT, int Ns, int TwOff, bool PR, class Off, int R, int... Rest>
+// the stages from Ns on, the last one stored; IP: in place (after a first
+// stage with RowRev), else autosort
+template <class T, bool FWD, int N, int B, int BP, int NT, int Ns, int TwOff, bool PR, class Off, bool IP, int R,
+          int... Rest>
 __device__ __forceinline__ void mid_and_last(cpx<T>* lds, const typename TwT<T>::type* tw, const ColIO& io) {
   if constexpr (sizeof...(Rest) == 0) {
     stageL_global<T, R, FWD, N, B, BP, NT, Ns, TwOff, PR, Off>(lds, tw, io);
   } else {
-    stage_ct<T, R, FWD, N, B, BP, NT, Ns, TwOff>(lds, tw);
-    mid_and_last<T, FWD, N, B, BP, NT, Ns * R, (Ns > 1 ? TwOff + Ns * (R - 1) : TwOff), PR, Off, Rest...>(lds, tw, io);
+    if constexpr (IP) stage_ip<T, R, FWD, N, B, BP, NT, Ns, TwOff>(lds, tw);
+    else stage_ct<T, R, FWD, N, B, BP, NT, Ns, TwOff>(lds, tw);
+    mid_and_last<T, FWD, N, B, BP, NT, Ns * R, (Ns > 1 ? TwOff + Ns * (R - 1) : TwOff), PR, Off, IP, Rest...>(lds, tw,
+                                                                                                            io);
   }
 }
 
@@ -320,8 +375,8 @@ __device__ __forceinline__ void run_fft_io(cpx<T>* lds, const typename TwT<T>::t
                                            RList<R0, Rs...>) {
   static_assert(sizeof...(Rs) >= 1, "at least two stages");
   constexpr int N = R0 * RProd<Rs...>::value;
-  stage0_global<T, R0, FWD, N, B, NT, PR, Off>(lds, io);
-  mid_and_last<T, FWD, N, B, B, NT, R0, 0, PR, Off, Rs...>(lds, tw, io);
+  stage0_global<T, R0, FWD, N, B, NT, PR, Off, RowRev<Rs...>>(lds, io);
+  mid_and_last<T, FWD, N, B, B, NT, R0, 0, PR, Off, true, Rs...>(lds, tw, io);
 }
 
 // run_fft_io over the tiles t0, t0 + dt, ... below t1 of one workgroup: the
@@ -336,15 +391,15 @@ __device__ __forceinline__ void run_fft_io_pipe(cpx<T>* lds, const typename TwT<
   if (t0 >= t1) return;
   Stage0Regs<T, R0, N, B, NT> rg;
   ColIO io = make_io(t0);
-  stage0_load<T, R0, N, B, NT, PR, Off>(rg, io);
+  stage0_load<T, R0, N, B, NT, PR, Off, RowRev<Rs...>>(rg, io);
   for (int t = t0; t < t1; t += dt) {
     stage0_put<T, R0, FWD, N, B, NT>(lds, rg);
     const ColIO cur = io;
     if (t + dt < t1) {
       io = make_io(t + dt);
-      stage0_load<T, R0, N, B, NT, PR, Off>(rg, io);
+      stage0_load<T, R0, N, B, NT, PR, Off, RowRev<Rs...>>(rg, io);
     }
-    mid_and_last<T, FWD, N, B, B, NT, R0, 0, PR, Off, Rs...>(lds, tw, cur);
+    mid_and_last<T, FWD, N, B, B, NT, R0, 0, PR, Off, true, Rs...>(lds, tw, cur);
     // the last stage's LDS reads before the next tile's first-stage writes
     __syncthreads();
   }
@@ -358,8 +413,8 @@ __device__ __forceinline__ void run_fft_in_io(cpx<T>* lds, const typename TwT<T>
                                               RList<R0, Rs...>) {
   static_assert(sizeof...(Rs) >= 1, "at least two stages");
   constexpr int N = R0 * RProd<Rs...>::value;
-  stage0_global<T, R0, true, N, B, NT, true, Off>(lds, io);
-  stages_ct<T, true, N, B, B, NT, R0, 0, Rs...>(lds, tw);
+  stage0_global<T, R0, true, N, B, NT, true, Off, RowRev<Rs...>>(lds, io);
+  stages_ip<T, true, N, B, B, NT, R0, 0, Rs...>(lds, tw);
 }
 
 // Table-addressed rows (Off = TabRows) with the row tables staged in LDS at
@@ -373,11 +428,11 @@ __device__ __forceinline__ void run_fft_io_tab(cpx<T>* lds, int2* tl, const type
   for (int i = threadIdx.x; i < N; i += NT) tl[i] = ltab[i];
   __syncthreads();
   io.ltab = tl;
-  stage0_global<T, R0, FWD, N, B, NT, false, TabRows>(lds, io);
+  stage0_global<T, R0, FWD, N, B, NT, false, TabRows, RowRev<Rs...>>(lds, io);
   for (int i = threadIdx.x; i < N; i += NT) tl[i] = stab[i];
   __syncthreads();
   io.stab = tl;
-  mid_and_last<T, FWD, N, B, B, NT, R0, 0, false, TabRows, Rs...>(lds, tw, io);
+  mid_and_last<T, FWD, N, B, B, NT, R0, 0, false, TabRows, true, Rs...>(lds, tw, io);
 }
 
 // Spectral solve along the column: forward FFT, per-mode multiply by
@@ -393,8 +448,8 @@ __device__ __forceinline__ void run_fft_solve(cpx<T>* lds, const typename TwT<T>
                                               long long i0, const SolveCtx& sc, RList<R0, Rs...>) {
   static_assert(sizeof...(Rs) >= 1, "at least two stages");
   constexpr int N = R0 * RProd<Rs...>::value;
-  stage0_global<T, R0, true, N, B, NT, false, unsigned>(lds, io);
-  stages_ct<T, true, N, B, B, NT, R0, 0, Rs...>(lds, tw);
+  stage0_global<T, R0, true, N, B, NT, false, unsigned, RowRev<Rs...>>(lds, io);
+  stages_ip<T, true, N, B, B, NT, R0, 0, Rs...>(lds, tw);
   for (int q = threadIdx.x; q < B * N; q += NT) {
     const int e = q / B, b = q % B;
     const long long i = i0 + b;
@@ -408,7 +463,7 @@ __device__ __forceinline__ void run_fft_solve(cpx<T>* lds, const typename TwT<T>
     lds[q] = mk<T>((T)(v.x * f), (T)(v.y * f));
   }
   __syncthreads();
-  mid_and_last<T, false, N, B, B, NT, 1, 0, false, unsigned, R0, Rs...>(lds, tw, io);
+  mid_and_last<T, false, N, B, B, NT, 1, 0, false, unsigned, false, R0, Rs...>(lds, tw, io);
 }
 
 // Columns whose input (IN) or output is length-fastest, the other side being
@@ -440,10 +495,10 @@ __device__ __forceinline__ void run_fft_lenfast(cpx<T>* lds, const typename TwT<
       if ((B * N) % NT == 0 || q < B * N) lds[lds_at<B, BP>(q % N, q / N)] = v[u];
     }
     __syncthreads();
-    mid_and_last<T, FWD, N, B, BP, NT, 1, 0, false, unsigned, R0, Rs...>(lds, tw, io);
+    mid_and_last<T, FWD, N, B, BP, NT, 1, 0, false, unsigned, false, R0, Rs...>(lds, tw, io);
   } else {
-    stage0_global<T, R0, FWD, N, B, NT, false, unsigned, BP>(lds, io);
-    stages_ct<T, FWD, N, B, BP, NT, R0, 0, Rs...>(lds, tw);
+    stage0_global<T, R0, FWD, N, B, NT, false, unsigned, RowRev<Rs...>, BP>(lds, io);
+    stages_ip<T, FWD, N, B, BP, NT, R0, 0, Rs...>(lds, tw);
 #pragma unroll
     for (int u = 0; u < LI; u++) {
       const int q = threadIdx.x + u * NT, b = q / N, p = q % N;
