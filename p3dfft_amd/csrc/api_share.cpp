@@ -223,7 +223,7 @@ int p3dfft_share_ftran_y(const p3amd::real_t* recv1, p3amd::real_t* send2, void*
     y.in = (const cplx_t*)recv1; y.out = (cplx_t*)send2;
     y.n_inner = g.iisize; y.n_outer = g.kjsize; y.n = g.ny; y.kind = COL_C2C; y.fwd = true;
     tstart(g, 7, st);
-    const bool done = launch_col_tab(y, g.sg.d_yt, g.sg.d_ysf, st);
+    const bool done = launch_col_tab(y, g.sg.d_yt, g.sg.d_ysf, g.sg.all_rows, g.sg.sep_f, st);
     tstop(g, 7, st);
     if (done) return 0;
   }
@@ -327,7 +327,7 @@ int p3dfft_share_btran_y(const p3amd::real_t* recv, p3amd::real_t* send, void* s
     y.in = (const cplx_t*)recv; y.out = (cplx_t*)send;
     y.n_inner = g.iisize; y.n_outer = g.kjsize; y.n = g.ny; y.kind = COL_C2C; y.fwd = false;
     tstart(g, 10, st);
-    const bool done = launch_col_tab(y, g.sg.d_ylb, g.sg.d_yt, st);
+    const bool done = launch_col_tab(y, g.sg.d_ylb, g.sg.d_yt, g.sg.all_rows, g.sg.sep_b, st);
     tstop(g, 10, st);
     if (done) return 0;
   }

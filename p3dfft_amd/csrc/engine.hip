@@ -117,6 +117,8 @@ struct ColArgs {
   int xcd;
   const int2* ltab;  // table-addressed rows (see ColIO)
   const int2* stab;
+  int tab_all;       // no row of either table is missing
+  ColTabSep sep;     // sep.ok: the separable form of the tables
   int tab_off;       // byte offset of the LDS copy of the row tables (length-fastest views: of the columns' offsets)
   // Chebyshev recurrence fused into a DCT-I column pass (k_col_ct): applied
   // to the output rows in LDS before they are stored; cheby_off: byte offset
@@ -831,12 +833,14 @@ __global__ __launch_bounds__(NT) void k_yx_plane_bwd(PlaneArgs a) {
 // column index c = o * n_inner + i, element (o, i, row e) at
 // o*so + i*si + e*sl.  The tile base is column c0's address; lane offsets are
 // relative to it and non-negative (so >= n_inner * si).
-template <class T, int B>
+// CL: lanes past the last column repeat it.
+template <class T, int B, bool CL = false>
 __device__ __forceinline__ ColIO col_io(const ColArgs& a, long long c0, int nb) {
   ColIO io;
   const unsigned n_in = (unsigned)a.n_inner;
   const unsigned o0 = (unsigned)c0 / n_in, i0 = (unsigned)c0 - o0 * n_in;
-  const unsigned c = (unsigned)c0 + threadIdx.x % B;
+  const int b = threadIdx.x % B;
+  const unsigned c = (unsigned)c0 + (CL && b >= nb ? nb - 1 : b);
   const unsigned o = c / n_in, i = c - o * n_in;
   constexpr long long E = sizeof(cpx<T>);
   io.in = (const char*)a.in + ((long long)o0 * a.so_in + (long long)i0 * a.si_in) * E;
@@ -870,34 +874,65 @@ __global__ __launch_bounds__(NT, W) void k_colio_ct(ColArgs a) {
   const long long c0 = (long long)tile_of(a.rev, a.xcd) * TX;
   const int nb = (int)(ncol - c0 < TX ? ncol - c0 : TX);
   const ColIO io = col_io<T, TX>(a, c0, nb);
-  if constexpr (std::is_same<Off, TabRows>::value)
-    run_fft_io_tab<T, FWD, TX, NT>(lds, (int2*)(g_smem + a.tab_off), tw, io, a.ltab, a.stab, RL{});
+  if constexpr (is_tab<Off>)
+    run_fft_io_tab<T, FWD, TX, NT, Off>(lds, (int2*)(g_smem + a.tab_off), tw, io, a.ltab, a.stab, RL{});
   else
     run_fft_io<T, FWD, TX, NT, PR, Off>(lds, tw, io, RL{});
 }
+
+// the rows of a thread's first-stage butterflies (their first values) and of
+// its last-stage ones in k_colio_pipe: item `it` of a tile of TX columns
+template <class RL, int TX, int NT>
+struct PipeRows;
+template <int R0, int... Rs, int TX, int NT>
+struct PipeRows<RList<R0, Rs...>, TX, NT> {
+  static constexpr int N = R0 * RProd<Rs...>::value;
+  static constexpr int rlast() {
+    int l = 0;
+    for (int r : {Rs...}) l = r;
+    return l;
+  }
+  static constexpr int IT0 = (TX * (N / R0) + NT - 1) / NT, ITL = (TX * (N / rlast()) + NT - 1) / NT;
+  static __device__ __forceinline__ int row0(int it) { return RowRev<Rs...>::at(it / TX); }
+  static __device__ __forceinline__ int rowL(int it) { return it / TX; }
+};
 
 // Persistent form of k_colio_ct (unpruned rows, 32-bit offsets or the
 // table-addressed rows) for tiles that take more than half the LDS, i.e. one
 // workgroup per CU: gridDim.x workgroups, the 8 XCDs (workgroup w on XCD
 // w mod 8) each owning a contiguous range of tiles that its workgroups
-// share out round robin (a.xcd; else workgroup w takes tiles w, w + G, ...),
+// share out round robin (a.xcd; else workgroup w takes tiles w, w + G, ...)
+// in whole rounds, the columns left after those as one round of narrower tiles,
 // and each workgroup keeping its next tile's loads in flight while the
-// current tile computes.  The row tables (TabRows) are the
+// current tile computes.  The row tables (TabRows, TabAll) are the
 // same for every tile and stay in LDS, load table then store table, at
 // tab_off.
 template <class T, bool FWD, int TX, int NT, class RL, int W, bool TWL, class Off>
 __global__ __launch_bounds__(NT, W) void k_colio_pipe(ColArgs a) {
   constexpr int N = RL_N<RL>::value;
-  constexpr bool TB = std::is_same<Off, TabRows>::value;
+  constexpr bool TB = is_tab<Off>, SP = std::is_same<Off, TabSep>::value;
   cpx<T>* lds = (cpx<T>*)g_smem;
   // the twiddle staging is completed by the barrier at the end of the first stage
   const auto* tw = ct_twiddles<T, NT, TWL>(a.tw, a.tw_off, a.L.twcount);
   const long long ncol = (long long)a.n_inner * a.n_outer;
   const int ntiles = (int)((ncol + TX - 1) / TX);
-  const int G = (int)gridDim.x, x = (int)(blockIdx.x & 7), slot = (int)(blockIdx.x >> 3);
-  const int nslot = G / 8 + (x < G % 8 ? 1 : 0);
-  const int q = ntiles / 8, rm = ntiles % 8;
-  const int lo = x * q + (x < rm ? x : rm), cnt = q + (x < rm ? 1 : 0);
+  // this XCD's tiles [lo, lo + cnt) and workgroups (dispatch order: all of
+  // them, so that the tiles running at once form one contiguous range)
+  const int G = (int)gridDim.x, x = a.xcd ? (int)(blockIdx.x & 7) : 0;
+  const int slot = a.xcd ? (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+  const int nslot = a.xcd ? G / 8 + (x < G % 8 ? 1 : 0) : G;
+  const int q = a.xcd ? ntiles / 8 : ntiles, rm = a.xcd ? ntiles % 8 : 0;
+  const int lo0 = x * q + (x < rm ? x : rm), cnt = q + (x < rm ? 1 : 0);
+  const int lo = a.rev ? ntiles - lo0 - cnt : lo0;
+  // whole rounds of tiles of TX columns, then the remaining columns as one
+  // round of narrower tiles over all the workgroups
+  const int nfull = cnt / nslot * nslot;
+  const long long tail0 = (long long)(a.rev ? lo : lo + nfull) * TX;
+  const long long tail_end = (long long)(lo + cnt - (a.rev ? nfull : 0)) * TX;
+  const int tail = (int)((tail_end < ncol ? tail_end : ncol) - tail0);
+  constexpr int WMIN = sizeof(cpx<T>) < 16 ? 16 / (int)sizeof(cpx<T>) : 1;  // at least 16 bytes of a row
+  const int wt0 = (tail + nslot - 1) / nslot, wt = wt0 < WMIN ? WMIN : wt0;
+  const int nt = nfull + (tail > 0 ? (tail + wt - 1) / wt : 0);
   int2* tl = (int2*)(g_smem + a.tab_off);
   if constexpr (TB) {
     for (int i = threadIdx.x; i < N; i += NT) {
@@ -906,19 +941,40 @@ __global__ __launch_bounds__(NT, W) void k_colio_pipe(ColArgs a) {
     }
     __syncthreads();
   }
+  // separable rows: this thread's parts (the same for every tile)
+  unsigned sa_in[kSepIT] = {}, sa_out[kSepIT] = {};
+  if constexpr (SP) {
+    typedef PipeRows<RL, TX, NT> P;
+    static_assert(P::IT0 <= kSepIT && P::ITL <= kSepIT, "separable rows");
+#pragma unroll
+    for (int m = 0; m < P::IT0; m++) sa_in[m] = (unsigned)a.ltab[P::row0(threadIdx.x + m * NT)].x * (unsigned)sizeof(cpx<T>);
+#pragma unroll
+    for (int m = 0; m < P::ITL; m++) sa_out[m] = (unsigned)a.stab[P::rowL(threadIdx.x + m * NT)].x * (unsigned)sizeof(cpx<T>);
+  }
   auto make_io = [&](int t) -> ColIO {
-    const long long c0 = (long long)(a.rev ? ntiles - 1 - t : t) * TX;
-    const int nb = (int)(ncol - c0 < TX ? ncol - c0 : TX);
-    ColIO io = col_io<T, TX>(a, c0, nb);
+    const bool full = t < nfull;
+    const int ft = a.rev ? lo + cnt - 1 - t : lo + t;
+    const long long c0 = full ? (long long)ft * TX : tail0 + (long long)(t - nfull) * wt;
+    const long long end = full ? ncol : tail0 + tail;
+    const int w = full ? TX : wt;
+    const int nb = (int)(end - c0 < w ? end - c0 : w);
+    ColIO io = col_io<T, TX, true>(a, c0, nb);
     if constexpr (TB) {
       io.ltab = tl;
       io.stab = tl + N;
     }
+    if constexpr (SP) {
+      constexpr unsigned E = sizeof(cpx<T>);
+      io.lane_in = (io.lane_o * (unsigned)a.sep.y_in + io.lane_i) * E;
+      io.lane_out = (io.lane_o * (unsigned)a.sep.y_out + io.lane_i) * E;
+#pragma unroll
+      for (int m = 0; m < kSepIT; m++) { io.sa_in[m] = sa_in[m]; io.sa_out[m] = sa_out[m]; }
+#pragma unroll
+      for (int r = 0; r < kSepR; r++) { io.sb_in[r] = a.sep.b_in[r]; io.sb_out[r] = a.sep.b_out[r]; }
+    }
     return io;
   };
-  if (a.xcd) run_fft_io_pipe<T, FWD, TX, NT, false, Off>(lds, tw, lo + slot, lo + cnt, nslot, make_io, RL{});
-  // dispatch order: the tiles running at once form one contiguous range
-  else run_fft_io_pipe<T, FWD, TX, NT, false, Off>(lds, tw, (int)blockIdx.x, ntiles, G, make_io, RL{});
+  run_fft_io_pipe<T, FWD, TX, NT, Off>(lds, tw, slot, nt, nslot, make_io, RL{});
 }
 
 // Chebyshev derivative recurrence (build/ftran.F90:408-451) on the output
@@ -1715,8 +1771,13 @@ struct CtLen {
     typedef unsigned U32;
     typedef unsigned long long U64;
     if (a.ltab) {
-      if (fwd) go(k_colio_ct<real_t, true, TX, NTC, RL, WC, TWLT, false, TabRows>, g, NTC, bytes, s, a);
-      else go(k_colio_ct<real_t, false, TX, NTC, RL, WC, TWLT, false, TabRows>, g, NTC, bytes, s, a);
+      if (a.tab_all) {
+        if (fwd) go(k_colio_ct<real_t, true, TX, NTC, RL, WC, TWLT, false, TabAll>, g, NTC, bytes, s, a);
+        else go(k_colio_ct<real_t, false, TX, NTC, RL, WC, TWLT, false, TabAll>, g, NTC, bytes, s, a);
+      } else {
+        if (fwd) go(k_colio_ct<real_t, true, TX, NTC, RL, WC, TWLT, false, TabRows>, g, NTC, bytes, s, a);
+        else go(k_colio_ct<real_t, false, TX, NTC, RL, WC, TWLT, false, TabRows>, g, NTC, bytes, s, a);
+      }
       return;
     }
     if (fwd) {
@@ -1732,7 +1793,13 @@ struct CtLen {
   // tab: table-addressed rows (a.ltab), else unpruned rows at 32-bit offsets
   static void colpipe(bool fwd, bool tab, const ColArgs& a, unsigned g, size_t bytes, hipStream_t s) {
     if constexpr (PIPE) {
-      if (tab) {
+      if (tab && a.sep.ok) {
+        if (fwd) go(k_colio_pipe<real_t, true, TX, NTC, RL, WC, TWLC, TabSep>, g, NTC, bytes, s, a);
+        else go(k_colio_pipe<real_t, false, TX, NTC, RL, WC, TWLC, TabSep>, g, NTC, bytes, s, a);
+      } else if (tab && a.tab_all) {
+        if (fwd) go(k_colio_pipe<real_t, true, TX, NTC, RL, WC, TWLP, TabAll>, g, NTC, bytes, s, a);
+        else go(k_colio_pipe<real_t, false, TX, NTC, RL, WC, TWLP, TabAll>, g, NTC, bytes, s, a);
+      } else if (tab) {
         if (fwd) go(k_colio_pipe<real_t, true, TX, NTC, RL, WC, TWLP, TabRows>, g, NTC, bytes, s, a);
         else go(k_colio_pipe<real_t, false, TX, NTC, RL, WC, TWLP, TabRows>, g, NTC, bytes, s, a);
       } else {
@@ -1769,6 +1836,7 @@ struct CtLen {
   static void prep_dir() {
     allow_big_lds(k_col_ct<real_t, FWD, TX, NTC, RL, WC, TWLC>);
     allow_big_lds(k_colio_ct<real_t, FWD, TX, NTC, RL, WC, TWLT, false, TabRows>);
+    allow_big_lds(k_colio_ct<real_t, FWD, TX, NTC, RL, WC, TWLT, false, TabAll>);
     allow_big_lds(k_colio_ct<real_t, FWD, TX, NTC, RL, WC, TWLC, true, unsigned>);
     allow_big_lds(k_colio_ct<real_t, FWD, TX, NTC, RL, WC, TWLC, false, unsigned long long>);
     allow_big_lds(k_colio_ct<real_t, FWD, TX, NTC, RL, WC, TWLC, false, unsigned>);
@@ -1776,6 +1844,8 @@ struct CtLen {
     allow_big_lds(k_collf_ct<real_t, FWD, false, TX, NTC, RL, WF, TWLF>);
     if constexpr (PIPE) {
       allow_big_lds(k_colio_pipe<real_t, FWD, TX, NTC, RL, WC, TWLP, TabRows>);
+      allow_big_lds(k_colio_pipe<real_t, FWD, TX, NTC, RL, WC, TWLP, TabAll>);
+      allow_big_lds(k_colio_pipe<real_t, FWD, TX, NTC, RL, WC, TWLC, TabSep>);
       allow_big_lds(k_colio_pipe<real_t, FWD, TX, NTC, RL, WC, TWLC, unsigned>);
     }
   }
@@ -2155,17 +2225,45 @@ static bool col_fits32(const ColSpec& c, int TX, int rows) {
 static int g_col_pipe = 1;
 void set_col_pipe(int on) { g_col_pipe = on ? 1 : 0; }
 
-// workgroups of a persistent launch: one per CU of the current device, and
-// at least min(ntiles, 8), so that each XCD's share of the tiles has a
-// workgroup (k_colio_pipe)
-static unsigned pipe_grid(long long ntiles) {
+// workgroups of a persistent launch over ncol columns: one per CU of the
+// current device, fewer only where columns of at least 16 bytes a row run out
+// (k_colio_pipe; every XCD that owns a tile then still has a workgroup)
+static unsigned pipe_grid(long long ncol) {
   int dev = 0, ncu = 0;
   check_hip(hipGetDevice(&dev), "hipGetDevice");
   check_hip(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute");
-  return (unsigned)std::max<long long>(1, std::min<long long>(ntiles, std::max(ncu, 8)));
+  const long long wmin = sizeof(cplx_t) < 16 ? 16 / (long long)sizeof(cplx_t) : 1;
+  return (unsigned)std::max<long long>(1, std::min<long long>((ncol + wmin - 1) / wmin, std::max(ncu, 8)));
 }
 
-bool launch_col_tab(const ColSpec& c, const int2* ltab, const int2* stab, hipStream_t st) {
+ColTabSep col_tab_separable(int n, const std::vector<int2>& ltab, const std::vector<int2>& stab, long long elems) {
+  ColTabSep s;
+  std::memset(&s, 0, sizeof(s));
+  const CtInfo* ct = g_use_ct && n <= max_len() ? find_ct(get_len(n)) : nullptr;
+  if (!ct || !ct->pipe || ct->radix[0] > kSepR || ct->radix[ct->nr - 1] > kSepR ||
+      elems * (long long)sizeof(cplx_t) >= (1LL << 32))
+    return s;
+  auto split = [&](const std::vector<int2>& t, int R, int* y, unsigned* b) {
+    const int q = n / R;
+    *y = t[0].y;
+    for (int r = 0; r < R; r++) {
+      const long long d = (long long)t[(size_t)r * q].x - t[0].x;
+      b[r] = (unsigned)(d * (long long)sizeof(cplx_t));
+      for (int e = 0; e < q; e++) {
+        const int2 v = t[(size_t)r * q + e];
+        if (v.x < 0 || v.y != *y || (long long)v.x - t[e].x != d) return false;
+      }
+    }
+    return true;
+  };
+  s.r0 = ct->radix[0];
+  s.rl = ct->radix[ct->nr - 1];
+  s.ok = split(ltab, s.r0, &s.y_in, s.b_in) && split(stab, s.rl, &s.y_out, s.b_out) ? 1 : 0;
+  return s;
+}
+
+bool launch_col_tab(const ColSpec& c, const int2* ltab, const int2* stab, bool all_rows, const ColTabSep& sep,
+                    hipStream_t st) {
   if (c.n_inner <= 0 || c.n_outer <= 0) return true;
   if (c.kind != COL_C2C || !g_use_ct || c.n > max_len()) return false;
   const Len1D& L = get_len(c.n);
@@ -2179,6 +2277,7 @@ bool launch_col_tab(const ColSpec& c, const int2* ltab, const int2* stab, hipStr
   a.n_inner = c.n_inner; a.n_outer = c.n_outer;
   a.kind = COL_C2C;
   a.ltab = ltab; a.stab = stab;
+  a.tab_all = all_rows ? 1 : 0;
   a.rev = c.rev ? 1 : 0;
   a.xcd = 1;  // table-addressed rows: tiles share lines across peer blocks
   const int TX = ct->TX;
@@ -2187,12 +2286,19 @@ bool launch_col_tab(const ColSpec& c, const int2* ltab, const int2* stab, hipStr
   a.tiles = (c.n_inner + TX - 1) / TX;
   a.L = CtLenArg{L.d.n, L.d.twcount};
   a.tw = L.tw;
+  if (g_col_pipe && ct->pipe && sep.ok && sep.r0 == ct->radix[0] && sep.rl == ct->radix[ct->nr - 1]) {
+    a.sep = sep;
+    const size_t pb = ct_lds((size_t)TX * c.n * sizeof(cplx_t), ct->twl_col, *ct, &a.tw_lds, &a.tw_off);
+    ct->colpipe(c.fwd, true, a, pipe_grid(ncol), pb, st);
+    check_hip(hipGetLastError(), "k_colio_pipe (separable table) launch");
+    return true;
+  }
   if (g_col_pipe && ct->pipe) {
     size_t pb = ct_lds((size_t)TX * c.n * sizeof(cplx_t), ct->twl_pipe_tab, *ct, &a.tw_lds, &a.tw_off);
     a.tab_off = (int)round16((long long)pb);
     pb = (size_t)a.tab_off + 2 * (size_t)c.n * sizeof(int2);
     if (pb <= kLdsMax) {
-      ct->colpipe(c.fwd, true, a, pipe_grid((ncol + TX - 1) / TX), pb, st);
+      ct->colpipe(c.fwd, true, a, pipe_grid(ncol), pb, st);
       check_hip(hipGetLastError(), "k_colio_pipe (table) launch");
       return true;
     }
@@ -2266,7 +2372,7 @@ bool launch_col(const ColSpec& c, hipStream_t st) {
     const bool pr = !(ld_id && st_id);
     const bool fits = col_fits32(c, TX, rows) && !g_wide_offsets;
     if (c.kind == COL_C2C && !a.ld_lenfast && !a.st_lenfast && fits && !pr && g_col_pipe && ct->pipe) {
-      ct->colpipe(fwd, false, a, pipe_grid((ncol + TX - 1) / TX), bytes, st);
+      ct->colpipe(fwd, false, a, pipe_grid(ncol), bytes, st);
       check_hip(hipGetLastError(), "k_colio_pipe launch");
       return false;
     }

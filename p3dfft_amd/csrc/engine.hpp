@@ -134,12 +134,24 @@ void launch_col_long(const ColSpec& c, int m, hipStream_t st);
 // nk = nxo (r2c) or nxi (c2r)
 void launch_x_long(bool r2c, const void* in, void* out, long long nrows, long long si_row, long long so_row, int nx,
                    int nk, hipStream_t st);
+// Row tables that are the sum of a part per butterfly and a part per value of
+// the persistent column kernel's first (load) and last (store) stages, with one
+// outer stride: x(e0 + r n/R) = x(e0) + b[r] / sizeof(complex)
+struct ColTabSep {
+  int ok, r0, rl;  // rl, r0: the radices it was built for
+  int y_in, y_out;
+  unsigned b_in[16], b_out[16];  // bytes
+};
+// the separable form of a load and a store table of n rows (host copies) into
+// arrays of `elems` elements; ok = 0 where they have none
+ColTabSep col_tab_separable(int n, const std::vector<int2>& ltab, const std::vector<int2>& stab, long long elems);
 // C2C column transform of n_inner x n_outer columns of length n whose rows
 // are table-addressed: row e of column (o, i) at element ltab[e].x + o *
 // ltab[e].y + i of c.in (zero when ltab[e].x < 0), FFT row p stored at
-// stab[p] likewise in c.out (skipped when < 0).  False when n has no
-// specialised kernel.
-bool launch_col_tab(const ColSpec& c, const int2* ltab, const int2* stab, hipStream_t st);
+// stab[p] likewise in c.out (skipped when < 0); all_rows: neither table has a
+// negative entry; sep: their separable form, if any.  False when n has no specialised kernel.
+bool launch_col_tab(const ColSpec& c, const int2* ltab, const int2* stab, bool all_rows, const ColTabSep& sep,
+                    hipStream_t st);
 
 // Consecutive passes over one buffer walk their tiles in opposite orders, so
 // a pass starts on what the previous pass wrote last (still in the

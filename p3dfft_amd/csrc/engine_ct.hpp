@@ -79,12 +79,12 @@ __device__ __forceinline__ void stage_ct(cpx<T>* lds, const typename TwT<T>::typ
 // fastest digit, so a butterfly writes the positions it read (see the first
 // stage's Rev): one barrier, nothing held across it.
 template <class T, int R, bool FWD, int N, int B, int BP, int NT, int Ns, int Off>
-__device__ __forceinline__ void stage_ip(cpx<T>* lds, const typename TwT<T>::type* tw) {
+__device__ __forceinline__ void stage_ip(cpx<T>* lds, const typename TwT<T>::type* tw, int tid = threadIdx.x) {
   constexpr int total = B * (N / R);
   constexpr int IT = (total + NT - 1) / NT;
 #pragma unroll
   for (int m = 0; m < IT; m++) {
-    const int it = threadIdx.x + m * NT;
+    const int it = tid + m * NT;
     if ((total % NT) == 0 || it < total) {
       const int j = it / B, b = it % B;
       const int k = j % Ns, base = (j - k) * R + k;
@@ -149,6 +149,7 @@ __device__ __forceinline__ void run_fft_ct(cpx<T>* lds, const typename TwT<T>::t
 // remapped on load (pruning zero-fill) and on store (pruning selection);
 // without it both maps are the identity.
 // ---------------------------------------------------------------------------
+constexpr int kSepIT = 2, kSepR = 16;
 struct ColIO {
   const char* in;             // input tile base
   char* out;                  // output tile base
@@ -164,10 +165,21 @@ struct ColIO {
   const int2* ltab;
   const int2* stab;
   unsigned lane_o, lane_i;    // this lane's outer and inner column index
+  // separable rows (Off = TabSep): row e0 + r n/R of this lane's column at
+  // byte lane_in + sa_in[m] + sb_in[r], e0 the first row of this thread's m-th
+  // first-stage butterfly; FFT row j + r Ns likewise at lane_out + sa_out[m] +
+  // sb_out[r]
+  unsigned sa_in[kSepIT], sa_out[kSepIT], sb_in[kSepR], sb_out[kSepR];
 };
 
-// offset type selecting the table-addressed rows
+// offset types selecting the table-addressed rows: some rows missing, none
+// missing, or none missing and the table a sum of a part per butterfly and a
+// part per value (peers with equal blocks), which needs no table in LDS
 struct TabRows {};
+struct TabAll {};
+struct TabSep {};
+template <class Off>
+constexpr bool is_tab = std::is_same<Off, TabRows>::value || std::is_same<Off, TabAll>::value;
 
 template <int R, int N, int B, int NT>
 struct Stage0 {
@@ -193,38 +205,36 @@ struct Stage0Regs {
   cpx<T> v[Stage0<R, N, B, NT>::IT][R];
 };
 
-// first stage, loads: the tile's values of every butterfly of this thread
-template <class T, int R, int N, int B, int NT, bool PR, class Off, class Row>
-__device__ __forceinline__ void stage0_load(Stage0Regs<T, R, N, B, NT>& rg, const ColIO& io) {
+// first stage, loads: the tile's values of every butterfly of this thread.
+// Lanes past the tile's last column repeat it (col_io with CL), so a loaded
+// value is left alone until the butterflies: a select on it would wait for it
+// where it is issued.
+template <class T, int R, int N, int B, int NT, class Off, class Row>
+__device__ __forceinline__ void stage0_load(Stage0Regs<T, R, N, B, NT>& rg, const ColIO& io, int tid) {
   static_assert(NT % B == 0, "one column per thread");
-  constexpr bool TB = std::is_same<Off, TabRows>::value;
   typedef Stage0<R, N, B, NT> S;
-  const bool valid = (int)(threadIdx.x % B) < io.nb;
+  static_assert(!std::is_same<Off, TabSep>::value || (S::IT <= kSepIT && R <= kSepR), "separable rows");
 #pragma unroll
   for (int m = 0; m < S::IT; m++) {
-    const int it = threadIdx.x + m * NT;
+    const int it = tid + m * NT;
     if ((S::total % NT) == 0 || it < S::total) {
       const int j = Row::at(it / B);
 #pragma unroll
       for (int r = 0; r < R; r++) {
         const int e = j + r * S::nR;
-        // items outside the tile load its first element (always valid) and
-        // are zeroed, so no load sits under a branch
-        if constexpr (TB) {
+        if constexpr (std::is_same<Off, TabSep>::value) {
+          rg.v[m][r] = ld_at<T, unsigned>(io.in, (unsigned)io.lane_in + io.sa_in[m] + io.sb_in[r]);
+        } else if constexpr (is_tab<Off>) {
           const int2 t = io.ltab[e];
-          const bool ok = valid && t.x >= 0;
-          const unsigned el = ok ? (unsigned)t.x + io.lane_o * (unsigned)t.y + io.lane_i : 0u;
-          const cpx<T> u = ((const cpx<T>*)io.in)[el];
-          rg.v[m][r] = ok ? u : mk<T>(0, 0);
-        } else if constexpr (PR) {
-          const int src = io.mirror ? (e < io.mirror ? e : 2 * (io.mirror - 1) - e)
-                                    : (e < io.ld_lo ? e : (e >= io.ld_hi ? e - io.ld_shift : -1));
-          const bool ok = valid && src >= 0;
-          const cpx<T> u = ld_at<T, Off>(io.in, ok ? (Off)io.lane_in + (Off)src * (Off)io.sl_in : (Off)0);
-          rg.v[m][r] = ok ? u : mk<T>(0, 0);
+          const unsigned el = (unsigned)t.x + io.lane_o * (unsigned)t.y + io.lane_i;
+          if constexpr (std::is_same<Off, TabAll>::value) {
+            rg.v[m][r] = ((const cpx<T>*)io.in)[el];
+          } else {
+            const cpx<T> u = ((const cpx<T>*)io.in)[t.x >= 0 ? el : 0u];
+            rg.v[m][r] = t.x >= 0 ? u : mk<T>(0, 0);
+          }
         } else {
-          const cpx<T> u = ld_at<T, Off>(io.in, valid ? (Off)io.lane_in + (Off)e * (Off)io.sl_in : (Off)0);
-          rg.v[m][r] = valid ? u : mk<T>(0, 0);
+          rg.v[m][r] = ld_at<T, Off>(io.in, (Off)io.lane_in + (Off)e * (Off)io.sl_in);
         }
       }
     }
@@ -233,11 +243,11 @@ __device__ __forceinline__ void stage0_load(Stage0Regs<T, R, N, B, NT>& rg, cons
 
 // first stage, butterflies (no twiddles) and results into the LDS tile
 template <class T, int R, bool FWD, int N, int B, int NT>
-__device__ __forceinline__ void stage0_put(cpx<T>* lds, Stage0Regs<T, R, N, B, NT>& rg) {
+__device__ __forceinline__ void stage0_put(cpx<T>* lds, Stage0Regs<T, R, N, B, NT>& rg, int tid) {
   typedef Stage0<R, N, B, NT> S;
 #pragma unroll
   for (int m = 0; m < S::IT; m++) {
-    const int it = threadIdx.x + m * NT;
+    const int it = tid + m * NT;
     if ((S::total % NT) == 0 || it < S::total) {
       const int j = it / B, b = it % B;
       dft<R, FWD>(rg.v[m]);
@@ -256,7 +266,7 @@ __device__ __forceinline__ void stage0_put(cpx<T>* lds, Stage0Regs<T, R, N, B, N
 template <class T, int R, bool FWD, int N, int B, int NT, bool PR, class Off, class Row, int BP = B>
 __device__ __forceinline__ void stage0_global(cpx<T>* lds, const ColIO& io) {
   static_assert(NT % B == 0, "one column per thread");
-  constexpr bool TB = std::is_same<Off, TabRows>::value;
+  constexpr bool TB = is_tab<Off>;
   typedef Stage0<R, N, B, NT> S;
   const bool valid = (int)(threadIdx.x % B) < io.nb;
   cpx<T> v[S::IT][R];
@@ -272,7 +282,7 @@ __device__ __forceinline__ void stage0_global(cpx<T>* lds, const ColIO& io) {
         // are zeroed, so no load sits under a branch
         if constexpr (TB) {
           const int2 t = io.ltab[e];
-          const bool ok = valid && t.x >= 0;
+          const bool ok = valid && (std::is_same<Off, TabAll>::value || t.x >= 0);
           const unsigned el = ok ? (unsigned)t.x + io.lane_o * (unsigned)t.y + io.lane_i : 0u;
           const cpx<T> u = ((const cpx<T>*)io.in)[el];
           v[m][r] = ok ? u : mk<T>(0, 0);
@@ -302,19 +312,21 @@ __device__ __forceinline__ void stage0_global(cpx<T>* lds, const ColIO& io) {
   __syncthreads();
 }
 
-// last stage: Ns * R == N, so every butterfly index j < Ns and k == j
-template <class T, int R, bool FWD, int N, int B, int BP, int NT, int Ns, int TwOff, bool PR, class Off>
+// last stage: Ns * R == N, so every butterfly index j < Ns and k == j.  CL:
+// lanes past the last column repeat it and store its values again, so that no
+// store sits under a branch
+template <class T, int R, bool FWD, int N, int B, int BP, int NT, int Ns, int TwOff, bool PR, class Off, bool CL>
 __device__ __forceinline__ void stageL_global(const cpx<T>* lds, const typename TwT<T>::type* tw,
-                                              const ColIO& io) {
+                                              const ColIO& io, int tid) {
   static_assert(Ns * R == N, "last stage");
   static_assert(NT % B == 0, "one column per thread");
-  constexpr bool TB = std::is_same<Off, TabRows>::value;
+  constexpr bool TB = is_tab<Off>;
   constexpr int total = B * Ns;
   constexpr int IT = (total + NT - 1) / NT;
-  const bool valid = (int)(threadIdx.x % B) < io.nb;
+  const bool valid = CL || (int)(tid % B) < io.nb;
 #pragma unroll
   for (int m = 0; m < IT; m++) {
-    const int it = threadIdx.x + m * NT;
+    const int it = tid + m * NT;
     if ((total % NT) == 0 || it < total) {
       const int j = it / B, b = it % B;
       cpx<T> v[R];
@@ -333,14 +345,16 @@ __device__ __forceinline__ void stageL_global(const cpx<T>* lds, const typename 
         for (int r = 0; r < R; r++) {
           const int2 t = io.stab[j + r * Ns];
           el[r] = (unsigned)t.x + io.lane_o * (unsigned)t.y + io.lane_i;
-          st[r] = t.x >= 0;
+          st[r] = std::is_same<Off, TabAll>::value || t.x >= 0;
         }
       }
       if (valid) {
 #pragma unroll
         for (int r = 0; r < R; r++) {
           const int p = j + r * Ns;
-          if constexpr (TB) {
+          if constexpr (std::is_same<Off, TabSep>::value) {
+            st_at<T, unsigned>(io.out, (unsigned)io.lane_out + io.sa_out[m] + io.sb_out[r], v[r]);
+          } else if constexpr (TB) {
             if (st[r]) ((cpx<T>*)io.out)[el[r]] = v[r];
           } else if constexpr (PR) {
             const int e = p < io.st_lo ? p : p - io.st_shift;
@@ -357,16 +371,17 @@ __device__ __forceinline__ void stageL_global(const cpx<T>* lds, const typename 
 
 // the stages from Ns on, the last one stored; IP: in place (after a first
 // stage with RowRev), else autosort
-template <class T, bool FWD, int N, int B, int BP, int NT, int Ns, int TwOff, bool PR, class Off, bool IP, int R,
-          int... Rest>
-__device__ __forceinline__ void mid_and_last(cpx<T>* lds, const typename TwT<T>::type* tw, const ColIO& io) {
+template <class T, bool FWD, int N, int B, int BP, int NT, int Ns, int TwOff, bool PR, class Off, bool IP, bool CL,
+          int R, int... Rest>
+__device__ __forceinline__ void mid_and_last(cpx<T>* lds, const typename TwT<T>::type* tw, const ColIO& io,
+                                             int tid = threadIdx.x) {
   if constexpr (sizeof...(Rest) == 0) {
-    stageL_global<T, R, FWD, N, B, BP, NT, Ns, TwOff, PR, Off>(lds, tw, io);
+    stageL_global<T, R, FWD, N, B, BP, NT, Ns, TwOff, PR, Off, CL>(lds, tw, io, tid);
   } else {
-    if constexpr (IP) stage_ip<T, R, FWD, N, B, BP, NT, Ns, TwOff>(lds, tw);
+    if constexpr (IP) stage_ip<T, R, FWD, N, B, BP, NT, Ns, TwOff>(lds, tw, tid);
     else stage_ct<T, R, FWD, N, B, BP, NT, Ns, TwOff>(lds, tw);
-    mid_and_last<T, FWD, N, B, BP, NT, Ns * R, (Ns > 1 ? TwOff + Ns * (R - 1) : TwOff), PR, Off, IP, Rest...>(lds, tw,
-                                                                                                            io);
+    mid_and_last<T, FWD, N, B, BP, NT, Ns * R, (Ns > 1 ? TwOff + Ns * (R - 1) : TwOff), PR, Off, IP, CL, Rest...>(
+        lds, tw, io, tid);
   }
 }
 
@@ -376,14 +391,17 @@ __device__ __forceinline__ void run_fft_io(cpx<T>* lds, const typename TwT<T>::t
   static_assert(sizeof...(Rs) >= 1, "at least two stages");
   constexpr int N = R0 * RProd<Rs...>::value;
   stage0_global<T, R0, FWD, N, B, NT, PR, Off, RowRev<Rs...>>(lds, io);
-  mid_and_last<T, FWD, N, B, B, NT, R0, 0, PR, Off, true, Rs...>(lds, tw, io);
+  mid_and_last<T, FWD, N, B, B, NT, R0, 0, PR, Off, true, false, Rs...>(lds, tw, io);
 }
 
 // run_fft_io over the tiles t0, t0 + dt, ... below t1 of one workgroup: the
 // next tile's first-stage loads are issued before the current tile's later
-// stages and its stores, so they are in flight while those run.  make_io(t)
-// gives tile t's addressing.
-template <class T, bool FWD, int B, int NT, bool PR, class Off, class MakeIO, int R0, int... Rs>
+// stages and its stores, so they are in flight while those run.  The loop is
+// turned so that the wait for them stands behind the stores in straight-line
+// code: the memory counter retires in order, so it then waits for the loads
+// only and the stores drain during the next tile.  make_io(t) gives tile t's
+// addressing (lanes past the last column clamped).
+template <class T, bool FWD, int B, int NT, class Off, class MakeIO, int R0, int... Rs>
 __device__ __forceinline__ void run_fft_io_pipe(cpx<T>* lds, const typename TwT<T>::type* tw, int t0, int t1,
                                                 int dt, MakeIO make_io, RList<R0, Rs...>) {
   static_assert(sizeof...(Rs) >= 1, "at least two stages");
@@ -391,18 +409,27 @@ __device__ __forceinline__ void run_fft_io_pipe(cpx<T>* lds, const typename TwT<
   if (t0 >= t1) return;
   Stage0Regs<T, R0, N, B, NT> rg;
   ColIO io = make_io(t0);
-  stage0_load<T, R0, N, B, NT, PR, Off, RowRev<Rs...>>(rg, io);
-  for (int t = t0; t < t1; t += dt) {
-    stage0_put<T, R0, FWD, N, B, NT>(lds, rg);
-    const ColIO cur = io;
-    if (t + dt < t1) {
-      io = make_io(t + dt);
-      stage0_load<T, R0, N, B, NT, PR, Off, RowRev<Rs...>>(rg, io);
-    }
-    mid_and_last<T, FWD, N, B, B, NT, R0, 0, PR, Off, true, Rs...>(lds, tw, cur);
+  int tid = threadIdx.x;
+  stage0_load<T, R0, N, B, NT, Off, RowRev<Rs...>>(rg, io, tid);
+  stage0_put<T, R0, FWD, N, B, NT>(lds, rg, tid);
+  for (int t = t0 + dt; t < t1; t += dt) {
+    // the thread index is opaque in the loop: hoisted out of it, the LDS and
+    // row addresses take the registers the loads in flight need
+    asm volatile("" : "+v"(tid));
+    __builtin_assume(tid >= 0 && tid < NT);
+    const ColIO nx = make_io(t);
+    stage0_load<T, R0, N, B, NT, Off, RowRev<Rs...>>(rg, nx, tid);
+    // the scheduler would sink the loads to save registers, and lift the first
+    // butterflies (and their wait for the loads) above the later stages
+    __builtin_amdgcn_sched_barrier(0);
+    mid_and_last<T, FWD, N, B, B, NT, R0, 0, false, Off, true, true, Rs...>(lds, tw, io, tid);
     // the last stage's LDS reads before the next tile's first-stage writes
     __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    stage0_put<T, R0, FWD, N, B, NT>(lds, rg, tid);
+    io = nx;
   }
+  mid_and_last<T, FWD, N, B, B, NT, R0, 0, false, Off, true, true, Rs...>(lds, tw, io, tid);
 }
 
 // Forward FFT of a tile whose first stage is fed from global memory (with
@@ -417,10 +444,10 @@ __device__ __forceinline__ void run_fft_in_io(cpx<T>* lds, const typename TwT<T>
   stages_ip<T, true, N, B, B, NT, R0, 0, Rs...>(lds, tw);
 }
 
-// Table-addressed rows (Off = TabRows) with the row tables staged in LDS at
+// Table-addressed rows (Off = TabRows or TabAll) with the row tables staged in LDS at
 // `tl` (n int2): the load table before the first stage, the store table
 // after it, so every table read is an LDS read.
-template <class T, bool FWD, int B, int NT, int R0, int... Rs>
+template <class T, bool FWD, int B, int NT, class Off, int R0, int... Rs>
 __device__ __forceinline__ void run_fft_io_tab(cpx<T>* lds, int2* tl, const typename TwT<T>::type* tw, ColIO io,
                                                const int2* ltab, const int2* stab, RList<R0, Rs...>) {
   static_assert(sizeof...(Rs) >= 1, "at least two stages");
@@ -428,11 +455,11 @@ __device__ __forceinline__ void run_fft_io_tab(cpx<T>* lds, int2* tl, const type
   for (int i = threadIdx.x; i < N; i += NT) tl[i] = ltab[i];
   __syncthreads();
   io.ltab = tl;
-  stage0_global<T, R0, FWD, N, B, NT, false, TabRows, RowRev<Rs...>>(lds, io);
+  stage0_global<T, R0, FWD, N, B, NT, false, Off, RowRev<Rs...>>(lds, io);
   for (int i = threadIdx.x; i < N; i += NT) tl[i] = stab[i];
   __syncthreads();
   io.stab = tl;
-  mid_and_last<T, FWD, N, B, B, NT, R0, 0, false, TabRows, true, Rs...>(lds, tw, io);
+  mid_and_last<T, FWD, N, B, B, NT, R0, 0, false, Off, true, false, Rs...>(lds, tw, io);
 }
 
 // Spectral solve along the column: forward FFT, per-mode multiply by
@@ -463,7 +490,7 @@ __device__ __forceinline__ void run_fft_solve(cpx<T>* lds, const typename TwT<T>
     lds[q] = mk<T>((T)(v.x * f), (T)(v.y * f));
   }
   __syncthreads();
-  mid_and_last<T, false, N, B, B, NT, 1, 0, false, unsigned, false, R0, Rs...>(lds, tw, io);
+  mid_and_last<T, false, N, B, B, NT, 1, 0, false, unsigned, false, false, R0, Rs...>(lds, tw, io);
 }
 
 // Columns whose input (IN) or output is length-fastest, the other side being
@@ -495,7 +522,7 @@ __device__ __forceinline__ void run_fft_lenfast(cpx<T>* lds, const typename TwT<
       if ((B * N) % NT == 0 || q < B * N) lds[lds_at<B, BP>(q % N, q / N)] = v[u];
     }
     __syncthreads();
-    mid_and_last<T, FWD, N, B, BP, NT, 1, 0, false, unsigned, false, R0, Rs...>(lds, tw, io);
+    mid_and_last<T, FWD, N, B, BP, NT, 1, 0, false, unsigned, false, false, R0, Rs...>(lds, tw, io);
   } else {
     stage0_global<T, R0, FWD, N, B, NT, false, unsigned, RowRev<Rs...>, BP>(lds, io);
     stages_ip<T, FWD, N, B, BP, NT, R0, 0, Rs...>(lds, tw);

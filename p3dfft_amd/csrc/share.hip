@@ -339,6 +339,11 @@ void share_build_tables(ShareGeom& s, const std::vector<int>& iist, const std::v
       if (hy[yh] >= 0) ysf[hy[yh]] = make_int2((int)ha[yh], (int)hb[yh]);
     for (int y = 0; y < s.ny; y++)
       if (yh_of[y] >= 0) ylb[y] = make_int2((int)ha[yh_of[y]], (int)hb[yh_of[y]]);
+    s.all_rows = true;
+    for (int y = 0; y < s.ny; y++) s.all_rows = s.all_rows && ysf[y].x >= 0 && ylb[y].x >= 0;
+    const long long elems = (long long)s.iisize * s.ny * s.kjsize;
+    s.sep_f = col_tab_separable(s.ny, yt, ysf, elems);
+    s.sep_b = col_tab_separable(s.ny, ylb, yt, elems);
     s.d_yt = upload_vec(yt); s.d_ysf = upload_vec(ysf); s.d_ylb = upload_vec(ylb);
   }
   if ((long long)s.nxhpc * unit_x < (1LL << 31)) {

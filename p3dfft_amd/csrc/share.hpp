@@ -45,6 +45,8 @@ struct ShareGeom {
   int2* d_yt = nullptr;
   int2* d_ysf = nullptr;
   int2* d_ylb = nullptr;
+  ColTabSep sep_f{}, sep_b{};  // separable forms (forward: d_yt -> d_ysf, backward: d_ylb -> d_yt)
+  bool all_rows = false;  // every row of the column exchange's blocks is written and read (no cut of Y)
 };
 
 // Build (and upload) the address tables from the 0-based splits.
