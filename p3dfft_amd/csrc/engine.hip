@@ -980,44 +980,46 @@ __global__ __launch_bounds__(NT, W) void k_colio_pipe(ColArgs a) {
 // Chebyshev derivative recurrence (build/ftran.F90:408-451) on the output
 // rows of an LDS column tile: output row e of column b sits in LDS row
 // p(e) = e (e < st_lo) or e + st_shift.  As in k_cheby, two interleaved
-// suffix sums: thread (chunk q, column b), b fastest, owns a chunk of at
-// most RM rows of its column, held in registers; chunk sums by parity, then
-// the sums of the later chunks (inside a wave by shuffles at a stride of TX
-// lanes, across waves through LDS at `wt`), then each chunk walked from its
-// top with that carry.  Columns fastest keep the lanes of one LDS access on
-// different banks; every LDS access of a thread is issued as a batch.
-constexpr int kChebyRM = 8;
+// suffix sums: thread (chunk q, column b), b fastest, owns the RM rows from
+// q RM on, held in registers; chunk sums by parity, then the sums of the later
+// chunks (inside a wave by shuffles at a stride of TX lanes, across waves
+// through LDS at `wt`), then each chunk walked from its top with that carry.
+// The top row N-1 is no chunk's: its term goes into every chunk's carry and
+// its output is zero, so the 2^k rows below it divide evenly and, RM being
+// even, a row's parity is its position's (256x256x257 FP64: 4 rows a thread
+// instead of 5 in 8 guarded positions, the pass 98 -> 93 us, cheby and its
+// backward transform 337 -> 328 us).  Columns fastest
+// keep the lanes of one LDS access on different banks; every LDS access of a
+// thread is issued as a batch.
+template <int N2, int P>
+constexpr int cheby_rows = ((N2 / 2 + P - 1) / P + 1) / 2 * 2;
 // Each thread stores its output rows straight to `out` (column b of the tile
 // at out + b*si_out, row e at + e*sl_out; columns b >= nb are not stored).
-template <class T, int TX, int NT>
+template <class T, int TX, int NT, int RM>
 __device__ __forceinline__ void cheby_tile(cpx<T>* lds, double* wt, const ColArgs& a, cpx<T>* out, int nb) {
-  static_assert(64 % TX == 0 && NT % 64 == 0, "whole column groups per wave");
-  constexpr int P = NT / TX, CW = 64 / TX, NW = NT / 64, RM = kChebyRM;
-  const int N = a.nst;
+  static_assert(64 % TX == 0 && NT % 64 == 0 && RM % 2 == 0, "whole column groups per wave");
+  constexpr int CW = 64 / TX, NW = NT / 64, P = NT / TX;
+  const int N = a.nst;  // at most RM * P + 1 (checked by the host)
   const int b = threadIdx.x % TX, q = threadIdx.x / TX;
   const int c = q % CW, w = q / CW;  // chunk within the wave, wave
-  const int R = (N + P - 1) / P;     // <= RM (checked by the host)
-  const int lo = q * R, hi = min(N, lo + R);
+  const int lo = q * RM, hi = min(N - 1, lo + RM);
   const double scale = a.cheby_scale, L = a.cheby_L;
+  auto at = [&](int e) { return (e < a.st_lo ? e : e + a.st_shift) * TX + b; };
   cpx<T> t[RM];
-  int addr[RM];
 #pragma unroll
-  for (int i = 0; i < RM; i++) {
-    const int e = lo + i;
-    addr[i] = (e < a.st_lo ? e : e + a.st_shift) * TX + b;
-    t[i] = (e < hi) ? lds[addr[i]] : mk<T>(0, 0);
-  }
-  // terms L j scale t_j (the top one halved), summed by parity
+  for (int i = 0; i < RM; i++) t[i] = lds[lo + i < hi ? at(lo + i) : b];
+  const cpx<T> tt = lds[at(N - 1)];
+  // terms L j scale t_j, summed by parity
   double2 x[RM];
   double v[4] = {0, 0, 0, 0};  // even re, even im, odd re, odd im
 #pragma unroll
   for (int i = RM - 1; i >= 0; i--) {
     const int j = lo + i;
-    double f = (j < hi) ? L * (double)j : 0.0;
-    if (j == N - 1) f *= 0.5;
-    x[i] = make_double2(f * ((double)t[i].x * scale), f * ((double)t[i].y * scale));
-    if (j & 1) { v[2] += x[i].x; v[3] += x[i].y; }
-    else { v[0] += x[i].x; v[1] += x[i].y; }
+    const double f = j < hi ? L * (double)j : 0.0;
+    // a position past the last row adds nothing, whatever its stand-in holds
+    x[i] = j < hi ? make_double2(f * ((double)t[i].x * scale), f * ((double)t[i].y * scale)) : make_double2(0, 0);
+    v[2 * (i & 1)] += x[i].x;
+    v[2 * (i & 1) + 1] += x[i].y;
   }
   // inclusive suffix over the chunks of this wave (lanes TX apart)
   double s[4];
@@ -1034,30 +1036,33 @@ __device__ __forceinline__ void cheby_tile(cpx<T>* lds, double* wt, const ColArg
 #pragma unroll
     for (int k = 0; k < 4; k++) wt[(w * TX + b) * 4 + k] = s[k];
   __syncthreads();
-  double cr[4];
+  // the carry: the top term (halved), then the later chunks
+  const double ft = 0.5 * (L * (double)(N - 1));
+  const double2 top = make_double2(ft * ((double)tt.x * scale), ft * ((double)tt.y * scale));
+  const bool odd = (N - 1) & 1;
+  double cr[4] = {odd ? 0.0 : top.x, odd ? 0.0 : top.y, odd ? top.x : 0.0, odd ? top.y : 0.0};
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const double nx = __shfl_down(s[k], TX, 64);
-    cr[k] = c + 1 < CW ? nx : 0.0;
-  }
-#pragma unroll
-  for (int u = 1; u < NW; u++)
+  for (int u = NW - 1; u > 0; u--)
     if (u > w)
 #pragma unroll
       for (int k = 0; k < 4; k++) cr[k] += wt[(u * TX + b) * 4 + k];
-  double2 ev = make_double2(cr[0], cr[1]), od = make_double2(cr[2], cr[3]);
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const double nx = __shfl_down(s[k], TX, 64);
+    cr[k] += c + 1 < CW ? nx : 0.0;
+  }
+  double2 sum[2] = {make_double2(cr[0], cr[1]), make_double2(cr[2], cr[3])};  // even, odd rows above
   cpx<T>* oc = out + (long long)b * a.si_out;
 #pragma unroll
   for (int i = RM - 1; i >= 0; i--) {
     const int r = lo + i;
-    if (r < hi) {
-      double2 d = (r & 1) ? ev : od;
-      if (r == 0) { d.x *= 0.5; d.y *= 0.5; }
-      if (b < nb) oc[(long long)r * a.sl_out] = mk<T>((T)d.x, (T)d.y);
-      if (r & 1) { od.x += x[i].x; od.y += x[i].y; }
-      else { ev.x += x[i].x; ev.y += x[i].y; }
-    }
+    double2 d = sum[1 - (i & 1)];
+    if (i == 0 && r == 0) { d.x *= 0.5; d.y *= 0.5; }
+    if (r < hi && b < nb) oc[(long long)r * a.sl_out] = mk<T>((T)d.x, (T)d.y);
+    sum[i & 1].x += x[i].x;
+    sum[i & 1].y += x[i].y;
   }
+  if (q == P - 1 && b < nb) oc[(long long)(N - 1) * a.sl_out] = mk<T>((T)0, (T)0);
 }
 
 // Column transforms through an LDS load/store pass: DCT-I / DST-I
@@ -1126,7 +1131,7 @@ __global__ __launch_bounds__(NT, W) void k_col_ct(ColArgs a) {
   if constexpr (64 % TX == 0 && NT % 64 == 0) {
     if (a.cheby) {
       // the recurrence stores the output rows itself
-      cheby_tile<T, TX, NT>(lds, (double*)(g_smem + a.cheby_off), a, out, nb);
+      cheby_tile<T, TX, NT, cheby_rows<RL_N<RL>::value, NT / TX>>(lds, (double*)(g_smem + a.cheby_off), a, out, nb);
       return;
     }
   }
@@ -2413,8 +2418,7 @@ bool launch_col(const ColSpec& c, hipStream_t st) {
     const long long nwg = (long long)a.tiles * c.n_outer;
     if (nwg > 0x7fffffffLL) throw Error{"grid too large", -1};
     size_t b2 = bytes;
-    if (c.cheby && c.kind == COL_DCT1 && 64 % TX == 0 && ct->NTC % 64 == 0 &&
-        (c.nst + ct->NTC / TX - 1) / (ct->NTC / TX) <= kChebyRM) {
+    if (c.cheby && c.kind == COL_DCT1 && 64 % TX == 0 && ct->NTC % 64 == 0 && c.nst >= 2) {
       // per-wave FP64 sums of the fused recurrence behind the tile
       a.cheby = 1;
       a.cheby_off = (int)round16((long long)bytes);
