@@ -52,17 +52,6 @@ __device__ __forceinline__ int tile_of(int rev, int xcd = 1) {
   return rev ? (int)gridDim.x - 1 - t : t;
 }
 
-// copy the twiddle table into LDS behind the data tile
-template <class T, int NT>
-__device__ __forceinline__ const typename TwT<T>::type* stage_twiddles(unsigned char* smem, size_t off,
-                                                                      const typename TwT<T>::type* tw,
-                                                                      int count) {
-  typedef typename TwT<T>::type TwL;
-  TwL* tl = (TwL*)(smem + off);
-  for (int i = threadIdx.x; i < count; i += NT) tl[i] = tw[i];
-  return tl;
-}
-
 // ---------------------------------------------------------------------------
 // X kernels
 // ---------------------------------------------------------------------------
@@ -136,17 +125,10 @@ struct ColArgs {
 // time, so twiddle reads are LDS reads).  Addresses are a wave-uniform 64-bit
 // tile base plus 32-bit byte offsets (the host checks that they fit).
 // ---------------------------------------------------------------------------
-template <class T, int NT, bool TWL>
-__device__ __forceinline__ const typename TwT<T>::type* ct_twiddles(const void* tw, int off, int count) {
-  typedef typename TwT<T>::type TwL;
-  if constexpr (TWL) return stage_twiddles<T, NT>(g_smem, off, (const TwL*)tw, count);
-  else return (const TwL*)tw;
-}
-
 // X r2c of the row pairs pair0 .. pair0+B-1 (nr <= 2B rows exist) through
 // the LDS tile `lds`
-template <class T, int B, int NT, class RL, bool XT>
-__device__ __forceinline__ void x_r2c_ct_tile(cpx<T>* lds, const typename TwT<T>::type* tw, const XArgs& a,
+template <class T, int B, int NT, class RL, bool XT, class Tw>
+__device__ __forceinline__ void x_r2c_ct_tile(cpx<T>* lds, const Tw& tw, const XArgs& a,
                                               long long pin, long long pair0, int nr) {
   constexpr int N = RL_N<RL>::value;
   constexpr int BP = B + 1;
@@ -176,8 +158,9 @@ __device__ __forceinline__ void x_r2c_ct_tile(cpx<T>* lds, const typename TwT<T>
       if (((B * N) % NT == 0) || q < B * N) lds[(q % N) * BP + q / N] = mk<T>(xa[i], xb[i]);
     }
   }
+  tw.put();
   __syncthreads();
-  run_fft_ct<T, true, B, BP, NT>(lds, tw, RL{});
+  run_fft_ct<T, true, B, BP, NT>(lds, tw.table(), RL{});
   char* out = (char*)a.out + 2 * pair0 * a.so_row * (long long)sizeof(cpx<T>);
   const unsigned so = (unsigned)(a.so_row * sizeof(cpx<T>));
   const T h = (T)0.5;
@@ -244,7 +227,7 @@ __device__ __forceinline__ void x_r2c_ct_tile(cpx<T>* lds, const typename TwT<T>
 template <class T, int B, int NT, class RL, int W, bool TWL, bool XT>
 __global__ __launch_bounds__(NT, W) void k_x_r2c_ct(XArgs a) {
   cpx<T>* lds = (cpx<T>*)g_smem;
-  const auto* tw = ct_twiddles<T, NT, TWL>(a.tw, a.tw_off, a.L.twcount);
+  const CtTw<T, NT, TWL, RL> tw(a.tw, g_smem, a.tw_off);
   const long long pair0 = (long long)tile_of(a.rev) * B;
   // rows of this tile (2B unless it is the last one)
   const int nr = (int)(a.nrows - 2 * pair0 < 2 * B ? a.nrows - 2 * pair0 : 2 * B);
@@ -252,8 +235,8 @@ __global__ __launch_bounds__(NT, W) void k_x_r2c_ct(XArgs a) {
 }
 
 // X c2r of the row pairs pair0 .. pair0+B-1 (nr <= 2B rows exist)
-template <class T, int B, int NT, class RL, bool XT>
-__device__ __forceinline__ void x_c2r_ct_tile(cpx<T>* lds, const typename TwT<T>::type* tw, const XArgs& a,
+template <class T, int B, int NT, class RL, bool XT, class Tw>
+__device__ __forceinline__ void x_c2r_ct_tile(cpx<T>* lds, const Tw& tw, const XArgs& a,
                                               long long pair0, long long pout, int nr) {
   constexpr int N = RL_N<RL>::value;
   constexpr int BP = B + 1;
@@ -356,8 +339,9 @@ __device__ __forceinline__ void x_c2r_ct_tile(cpx<T>* lds, const typename TwT<T>
       }
     }
   }
+  tw.put();
   __syncthreads();
-  run_fft_ct<T, false, B, BP, NT>(lds, tw, RL{});
+  run_fft_ct<T, false, B, BP, NT>(lds, tw.table(), RL{});
   char* out = (char*)a.out + 2 * pout * a.so_row * (long long)sizeof(T);
   const unsigned so = (unsigned)(a.so_row * sizeof(T));
   // a compile-time trip count and the full-tile test outside the loop, so
@@ -383,7 +367,7 @@ __device__ __forceinline__ void x_c2r_ct_tile(cpx<T>* lds, const typename TwT<T>
 template <class T, int B, int NT, class RL, int W, bool TWL, bool XT>
 __global__ __launch_bounds__(NT, W) void k_x_c2r_ct(XArgs a) {
   cpx<T>* lds = (cpx<T>*)g_smem;
-  const auto* tw = ct_twiddles<T, NT, TWL>(a.tw, a.tw_off, a.L.twcount);
+  const CtTw<T, NT, TWL, RL> tw(a.tw, g_smem, a.tw_off);
   const long long pair0 = (long long)tile_of(a.rev) * B;
   const int nr = (int)(a.nrows - 2 * pair0 < 2 * B ? a.nrows - 2 * pair0 : 2 * B);
   x_c2r_ct_tile<T, B, NT, RL, XT>(lds, tw, a, pair0, pair0, nr);
@@ -699,21 +683,26 @@ struct PlaneGeom {
   static constexpr long long DATA = X_BYTES + Y_BYTES;
 };
 
+// the two tables, one after the other behind the tiles (one when NX == NY)
 template <class T, class RLX, class RLY, int NT>
-__device__ __forceinline__ void plane_twiddles(const PlaneArgs& a, const typename TwT<T>::type** tx,
-                                               const typename TwT<T>::type** ty) {
+struct PlaneTw {
   typedef PlaneGeom<T, RLX, RLY> G;
   typedef typename TwT<T>::type TwL;
-  TwL* t = (TwL*)(g_smem + G::DATA);
-  for (int i = threadIdx.x; i < a.ntwx; i += NT) t[i] = ((const TwL*)a.twx)[i];
-  *tx = t;
-  if (a.twy == a.twx) {
-    *ty = t;
-  } else {
-    for (int i = threadIdx.x; i < a.ntwy; i += NT) t[a.ntwx + i] = ((const TwL*)a.twy)[i];
-    *ty = t + a.ntwx;
+  static constexpr bool SAME = std::is_same<RLX, RLY>::value;
+  CtTw<T, NT, true, RLX> x;
+  CtTw<T, NT, !SAME, RLY> y;
+  __device__ __forceinline__ PlaneTw(const PlaneArgs& a)
+      : x(a.twx, g_smem, (int)G::DATA), y(a.twy, g_smem, (int)G::DATA + a.ntwx * (int)sizeof(TwL)) {}
+  __device__ __forceinline__ void put() const {
+    x.put();
+    y.put();
   }
-}
+  __device__ __forceinline__ const TwL* tx() const { return x.table(); }
+  __device__ __forceinline__ const TwL* ty() const {
+    if constexpr (SAME) return x.table();
+    else return y.table();
+  }
+};
 
 // forward: X r2c (two-for-one, as k_x_r2c_ct) and Y forward of plane
 // blockIdx.x: real rows of NX (row stride NX) -> half-spectrum rows of NX/2+1
@@ -723,8 +712,7 @@ __global__ __launch_bounds__(NT) void k_xy_plane_fwd(PlaneArgs a) {
   constexpr int NX = G::NX, NY = G::NY, BX = G::BX, BPX = G::BPX, H = G::H;
   cpx<T>* lx = (cpx<T>*)g_smem;
   cpx<T>* ly = (cpx<T>*)(g_smem + G::X_BYTES);
-  const typename TwT<T>::type *tx, *ty;
-  plane_twiddles<T, RLX, RLY, NT>(a, &tx, &ty);
+  const PlaneTw<T, RLX, RLY, NT> tw(a);
   const T* in = (const T*)a.in + (long long)blockIdx.x * NX * NY;
   {
     // compile-time trip counts: every load of the plane issued before the
@@ -745,8 +733,9 @@ __global__ __launch_bounds__(NT) void k_xy_plane_fwd(PlaneArgs a) {
       if ((BX * NX) % NT == 0 || q < BX * NX) lx[(q % NX) * BPX + q / NX] = mk<T>(xa[i], xb[i]);
     }
   }
+  tw.put();
   __syncthreads();
-  run_fft_ct<T, true, BX, BPX, NT>(lx, tx, RLX{});
+  run_fft_ct<T, true, BX, BPX, NT>(lx, tw.tx(), RLX{});
   const T h = (T)0.5;
   for (int q = threadIdx.x; q < BX * H; q += NT) {
     const int b = q / H, k = q % H;
@@ -755,7 +744,7 @@ __global__ __launch_bounds__(NT) void k_xy_plane_fwd(PlaneArgs a) {
     ly[(2 * b + 1) * H + k] = mk<T>((zk.y + zn.y) * h, (zn.x - zk.x) * h);
   }
   __syncthreads();
-  run_fft_ct<T, true, H, H, NT>(ly, ty, RLY{});
+  run_fft_ct<T, true, H, H, NT>(ly, tw.ty(), RLY{});
   cpx<T>* out = (cpx<T>*)a.out + (long long)blockIdx.x * H * NY;
   constexpr int LQ = (NY * H + NT - 1) / NT;
   cpx<T> v[LQ];
@@ -779,8 +768,7 @@ __global__ __launch_bounds__(NT) void k_yx_plane_bwd(PlaneArgs a) {
   constexpr int NX = G::NX, NY = G::NY, BX = G::BX, BPX = G::BPX, H = G::H;
   cpx<T>* lx = (cpx<T>*)g_smem;
   cpx<T>* ly = (cpx<T>*)(g_smem + G::X_BYTES);
-  const typename TwT<T>::type *tx, *ty;
-  plane_twiddles<T, RLX, RLY, NT>(a, &tx, &ty);
+  const PlaneTw<T, RLX, RLY, NT> tw(a);
   const cpx<T>* in = (const cpx<T>*)a.in + (long long)blockIdx.x * H * NY;
   {
     // every load of the plane issued before the LDS writes
@@ -797,8 +785,9 @@ __global__ __launch_bounds__(NT) void k_yx_plane_bwd(PlaneArgs a) {
       if ((NY * H) % NT == 0 || q < NY * H) ly[q] = v[i];
     }
   }
+  tw.put();
   __syncthreads();
-  run_fft_ct<T, false, H, H, NT>(ly, ty, RLY{});
+  run_fft_ct<T, false, H, H, NT>(ly, tw.ty(), RLY{});
   for (int q = threadIdx.x; q < BX * H; q += NT) {
     const int b = q / H, k = q % H;
     cpx<T> A = ly[(2 * b) * H + k], Bv = ly[(2 * b + 1) * H + k];
@@ -808,7 +797,7 @@ __global__ __launch_bounds__(NT) void k_yx_plane_bwd(PlaneArgs a) {
     lx[(k == 0 ? 0 : NX - k) * BPX + b] = mk<T>(A.x + Bv.y, Bv.x - A.y);
   }
   __syncthreads();
-  run_fft_ct<T, false, BX, BPX, NT>(lx, tx, RLX{});
+  run_fft_ct<T, false, BX, BPX, NT>(lx, tw.tx(), RLX{});
   T* out = (T*)a.out + (long long)blockIdx.x * NX * NY;
   constexpr int LI = (BX * NX + NT - 1) / NT;
   cpx<T> z[LI];
@@ -868,8 +857,7 @@ __device__ __forceinline__ ColIO col_io(const ColArgs& a, long long c0, int nb) 
 template <class T, bool FWD, int TX, int NT, class RL, int W, bool TWL, bool PR, class Off>
 __global__ __launch_bounds__(NT, W) void k_colio_ct(ColArgs a) {
   cpx<T>* lds = (cpx<T>*)g_smem;
-  // the twiddle staging is completed by the barrier at the end of the first stage
-  const auto* tw = ct_twiddles<T, NT, TWL>(a.tw, a.tw_off, a.L.twcount);
+  const CtTw<T, NT, TWL, RL> tw(a.tw, g_smem, a.tw_off);
   const long long ncol = (long long)a.n_inner * a.n_outer;
   const long long c0 = (long long)tile_of(a.rev, a.xcd) * TX;
   const int nb = (int)(ncol - c0 < TX ? ncol - c0 : TX);
@@ -912,8 +900,7 @@ __global__ __launch_bounds__(NT, W) void k_colio_pipe(ColArgs a) {
   constexpr int N = RL_N<RL>::value;
   constexpr bool TB = is_tab<Off>, SP = std::is_same<Off, TabSep>::value;
   cpx<T>* lds = (cpx<T>*)g_smem;
-  // the twiddle staging is completed by the barrier at the end of the first stage
-  const auto* tw = ct_twiddles<T, NT, TWL>(a.tw, a.tw_off, a.L.twcount);
+  const CtTw<T, NT, TWL, RL> tw(a.tw, g_smem, a.tw_off);
   const long long ncol = (long long)a.n_inner * a.n_outer;
   const int ntiles = (int)((ncol + TX - 1) / TX);
   // this XCD's tiles [lo, lo + cnt) and workgroups (dispatch order: all of
@@ -1072,7 +1059,7 @@ __device__ __forceinline__ void cheby_tile(cpx<T>* lds, double* wt, const ColArg
 template <class T, bool FWD, int TX, int NT, class RL, int W, bool TWL>
 __global__ __launch_bounds__(NT, W) void k_col_ct(ColArgs a) {
   cpx<T>* lds = (cpx<T>*)g_smem;
-  const auto* tw = ct_twiddles<T, NT, TWL>(a.tw, a.tw_off, a.L.twcount);
+  const CtTw<T, NT, TWL, RL> tw(a.tw, g_smem, a.tw_off);
   const int t = tile_of(a.rev, a.xcd);
   const int o = t / a.tiles;
   const int ti = t - o * a.tiles;
@@ -1109,7 +1096,10 @@ __global__ __launch_bounds__(NT, W) void k_col_ct(ColArgs a) {
     for (int u = 0; u < LU; u++)
       if (dst[u] >= 0) lds[dst[u]] = v[u];
   }
-  if (!a.mirror) __syncthreads();
+  if (!a.mirror) {
+    tw.put();
+    __syncthreads();
+  }
   if (a.kind == COL_DCT1 && !a.mirror) {
     const int m = a.L.n;
     for (int q = threadIdx.x; q < TX * (m - a.nld); q += NT) {
@@ -1127,7 +1117,7 @@ __global__ __launch_bounds__(NT, W) void k_col_ct(ColArgs a) {
     for (int b = threadIdx.x; b < TX; b += NT) lds[b] = mk<T>(0, 0);
     __syncthreads();
   }
-  if (a.kind != COL_COPY && !a.mirror) run_fft_ct<T, FWD, TX, TX, NT>(lds, tw, RL{});
+  if (a.kind != COL_COPY && !a.mirror) run_fft_ct<T, FWD, TX, TX, NT>(lds, tw.table(), RL{});
   if constexpr (64 % TX == 0 && NT % 64 == 0) {
     if (a.cheby) {
       // the recurrence stores the output rows itself
@@ -1153,7 +1143,7 @@ __global__ __launch_bounds__(NT, W) void k_col_ct(ColArgs a) {
 template <class T, bool FWD, bool IN, int TX, int NT, class RL, int W, bool TWL>
 __global__ __launch_bounds__(NT, W) void k_collf_ct(ColArgs a) {
   cpx<T>* lds = (cpx<T>*)g_smem;
-  const auto* tw = ct_twiddles<T, NT, TWL>(a.tw, a.tw_off, a.L.twcount);
+  const CtTw<T, NT, TWL, RL> tw(a.tw, g_smem, a.tw_off);
   const long long ncol = (long long)a.n_inner * a.n_outer;
   const long long c0 = (long long)tile_of(a.rev, a.xcd) * TX;
   const int nb = (int)(ncol - c0 < TX ? ncol - c0 : TX);
@@ -1169,7 +1159,7 @@ __global__ __launch_bounds__(NT, W) void k_collf_ct(ColArgs a) {
 template <class T, int TX, int NT, class RL, int W, bool TWL>
 __global__ __launch_bounds__(NT, W) void k_zsolve_ct(ColArgs a, double scale, int nxh, int ny) {
   cpx<T>* lds = (cpx<T>*)g_smem;
-  const auto* tw = ct_twiddles<T, NT, TWL>(a.tw, a.tw_off, a.L.twcount);
+  const CtTw<T, NT, TWL, RL> tw(a.tw, g_smem, a.tw_off);
   const long long ncol = a.n_inner;
   const long long c0 = (long long)tile_of(a.rev, a.xcd) * TX;
   const int nb = (int)(ncol - c0 < TX ? ncol - c0 : TX);
@@ -1208,7 +1198,7 @@ struct GrpArgs {
 template <class T, bool R2C, int B, int NT, class RL, int W, bool TWL>
 __global__ __launch_bounds__(NT, W) void k_x_grp(XArgs a, GrpArgs g) {
   cpx<T>* lds = (cpx<T>*)g_smem;
-  const auto* tw = ct_twiddles<T, NT, TWL>(a.tw, a.tw_off, a.L.twcount);
+  const CtTw<T, NT, TWL, RL> tw(a.tw, g_smem, a.tw_off);
   const int t = xcd_tile(blockIdx.x, gridDim.x);
   const int r = g.tile_req[t];
   const GrpDesc d = g.d[r];
@@ -1224,7 +1214,7 @@ __global__ __launch_bounds__(NT, W) void k_x_grp(XArgs a, GrpArgs g) {
 template <class T, bool FWD, int TX, int NT, class RL, int W, bool TWL>
 __global__ __launch_bounds__(NT, W) void k_col_grp(ColArgs a, GrpArgs g) {
   cpx<T>* lds = (cpx<T>*)g_smem;
-  const auto* tw = ct_twiddles<T, NT, TWL>(a.tw, a.tw_off, a.L.twcount);
+  const CtTw<T, NT, TWL, RL> tw(a.tw, g_smem, a.tw_off);
   const int t = xcd_tile(blockIdx.x, gridDim.x);
   const int r = g.tile_req[t];
   const GrpDesc d = g.d[r];
@@ -1243,7 +1233,7 @@ __global__ __launch_bounds__(NT, W) void k_col_grp(ColArgs a, GrpArgs g) {
 template <class T, int TX, int NT, class RL, int W, bool TWL>
 __global__ __launch_bounds__(NT, W) void k_zs_grp(ColArgs a, GrpArgs g) {
   cpx<T>* lds = (cpx<T>*)g_smem;
-  const auto* tw = ct_twiddles<T, NT, TWL>(a.tw, a.tw_off, a.L.twcount);
+  const CtTw<T, NT, TWL, RL> tw(a.tw, g_smem, a.tw_off);
   const int t = xcd_tile(blockIdx.x, gridDim.x);
   const int r = g.tile_req[t];
   const GrpDesc d = g.d[r];

@@ -138,6 +138,62 @@ __device__ __forceinline__ void run_fft_ct(cpx<T>* lds, const typename TwT<T>::t
   stages_ct<T, FWD, N, B, BP, NT, 1, 0, Rs...>(lds, tw);
 }
 
+// Twiddle table entries used by a radix list (all stages after the first).
+template <int... Rs>
+struct TwCount;
+template <int R0, int... Rs>
+struct TwCount<R0, Rs...> {
+  template <int Ns, int R, int... Rest>
+  static constexpr int tail() {
+    if constexpr (sizeof...(Rest) == 0) return Ns * (R - 1);
+    else return Ns * (R - 1) + tail<Ns * R, Rest...>();
+  }
+  static constexpr int value() {
+    if constexpr (sizeof...(Rs) == 0) return 0;
+    else return tail<R0, Rs...>();
+  }
+};
+
+// The twiddle table of a workgroup, in LDS (L) or where it is.  Its loads are
+// issued here, ahead of the tile's, and written to LDS by put() when the
+// tile's first stage is done, so that a workgroup waits for memory once and
+// not twice before its first stage.
+template <class T, int NT, bool L, class RL>
+struct CtTw;
+template <class T, int NT, bool L, int... Rs>
+struct CtTw<T, NT, L, RList<Rs...>> {
+  typedef typename TwT<T>::type TwL;
+  static constexpr int COUNT = TwCount<Rs...>::value(), K = L ? (COUNT + NT - 1) / NT : 1;
+  const TwL* src;
+  TwL* dst;
+  TwL v[K];
+  __device__ __forceinline__ CtTw(const void* tw, unsigned char* smem, int off) {
+    src = (const TwL*)tw;
+    dst = (TwL*)(smem + off);
+    if constexpr (L) {
+#pragma unroll
+      for (int i = 0; i < K; i++) {
+        const int e = threadIdx.x + i * NT;
+        v[i] = src[e < COUNT ? e : 0];
+      }
+    }
+  }
+  // before the barrier that ends the first stage
+  __device__ __forceinline__ void put() const {
+    if constexpr (L) {
+#pragma unroll
+      for (int i = 0; i < K; i++) {
+        const int e = threadIdx.x + i * NT;
+        if (e < COUNT) dst[e] = v[i];
+      }
+    }
+  }
+  __device__ __forceinline__ const TwL* table() const {
+    if constexpr (L) return dst;
+    else return src;
+  }
+};
+
 // ---------------------------------------------------------------------------
 // Column transforms with the first stage fed straight from global memory and
 // the last stage stored straight to global memory (one LDS round trip fewer
@@ -262,9 +318,10 @@ __device__ __forceinline__ void stage0_put(cpx<T>* lds, Stage0Regs<T, R, N, B, N
 // results into the LDS tile (the loads as stage0_load, written out here so
 // that every load of the tile is issued back to back: composed of the two
 // steps, the compiler interleaved them with address arithmetic and waited
-// before the last one)
-template <class T, int R, bool FWD, int N, int B, int NT, bool PR, class Off, class Row, int BP = B>
-__device__ __forceinline__ void stage0_global(cpx<T>* lds, const ColIO& io) {
+// before the last one).  pre() runs before the barrier: it writes what the later
+// stages read from LDS and was loaded ahead of the tile (CtTw).
+template <class T, int R, bool FWD, int N, int B, int NT, bool PR, class Off, class Row, int BP = B, class Pre>
+__device__ __forceinline__ void stage0_global(cpx<T>* lds, const ColIO& io, Pre pre) {
   static_assert(NT % B == 0, "one column per thread");
   constexpr bool TB = is_tab<Off>;
   typedef Stage0<R, N, B, NT> S;
@@ -309,6 +366,7 @@ __device__ __forceinline__ void stage0_global(cpx<T>* lds, const ColIO& io) {
       for (int r = 0; r < R; r++) lds[lds_at<B, BP>(j * R + r, b)] = v[m][r];
     }
   }
+  pre();
   __syncthreads();
 }
 
@@ -385,13 +443,12 @@ __device__ __forceinline__ void mid_and_last(cpx<T>* lds, const typename TwT<T>:
   }
 }
 
-template <class T, bool FWD, int B, int NT, bool PR, class Off, int R0, int... Rs>
-__device__ __forceinline__ void run_fft_io(cpx<T>* lds, const typename TwT<T>::type* tw, const ColIO& io,
-                                           RList<R0, Rs...>) {
+template <class T, bool FWD, int B, int NT, bool PR, class Off, class Tw, int R0, int... Rs>
+__device__ __forceinline__ void run_fft_io(cpx<T>* lds, const Tw& ctw, const ColIO& io, RList<R0, Rs...>) {
   static_assert(sizeof...(Rs) >= 1, "at least two stages");
   constexpr int N = R0 * RProd<Rs...>::value;
-  stage0_global<T, R0, FWD, N, B, NT, PR, Off, RowRev<Rs...>>(lds, io);
-  mid_and_last<T, FWD, N, B, B, NT, R0, 0, PR, Off, true, false, Rs...>(lds, tw, io);
+  stage0_global<T, R0, FWD, N, B, NT, PR, Off, RowRev<Rs...>>(lds, io, [&] { ctw.put(); });
+  mid_and_last<T, FWD, N, B, B, NT, R0, 0, PR, Off, true, false, Rs...>(lds, ctw.table(), io);
 }
 
 // run_fft_io over the tiles t0, t0 + dt, ... below t1 of one workgroup: the
@@ -401,9 +458,9 @@ __device__ __forceinline__ void run_fft_io(cpx<T>* lds, const typename TwT<T>::t
 // code: the memory counter retires in order, so it then waits for the loads
 // only and the stores drain during the next tile.  make_io(t) gives tile t's
 // addressing (lanes past the last column clamped).
-template <class T, bool FWD, int B, int NT, class Off, class MakeIO, int R0, int... Rs>
-__device__ __forceinline__ void run_fft_io_pipe(cpx<T>* lds, const typename TwT<T>::type* tw, int t0, int t1,
-                                                int dt, MakeIO make_io, RList<R0, Rs...>) {
+template <class T, bool FWD, int B, int NT, class Off, class Tw, class MakeIO, int R0, int... Rs>
+__device__ __forceinline__ void run_fft_io_pipe(cpx<T>* lds, const Tw& ctw, int t0, int t1, int dt, MakeIO make_io,
+                                                RList<R0, Rs...>) {
   static_assert(sizeof...(Rs) >= 1, "at least two stages");
   constexpr int N = R0 * RProd<Rs...>::value;
   if (t0 >= t1) return;
@@ -411,6 +468,8 @@ __device__ __forceinline__ void run_fft_io_pipe(cpx<T>* lds, const typename TwT<
   ColIO io = make_io(t0);
   int tid = threadIdx.x;
   stage0_load<T, R0, N, B, NT, Off, RowRev<Rs...>>(rg, io, tid);
+  ctw.put();
+  const auto* tw = ctw.table();
   stage0_put<T, R0, FWD, N, B, NT>(lds, rg, tid);
   for (int t = t0 + dt; t < t1; t += dt) {
     // the thread index is opaque in the loop: hoisted out of it, the LDS and
@@ -435,31 +494,30 @@ __device__ __forceinline__ void run_fft_io_pipe(cpx<T>* lds, const typename TwT<
 // Forward FFT of a tile whose first stage is fed from global memory (with
 // the PR row maps, e.g. a DCT-I mirror) and whose result stays in the LDS
 // tile (natural order, element e of column b at lds[e*B + b]).
-template <class T, int B, int NT, class Off, int R0, int... Rs>
-__device__ __forceinline__ void run_fft_in_io(cpx<T>* lds, const typename TwT<T>::type* tw, const ColIO& io,
-                                              RList<R0, Rs...>) {
+template <class T, int B, int NT, class Off, class Tw, int R0, int... Rs>
+__device__ __forceinline__ void run_fft_in_io(cpx<T>* lds, const Tw& ctw, const ColIO& io, RList<R0, Rs...>) {
   static_assert(sizeof...(Rs) >= 1, "at least two stages");
   constexpr int N = R0 * RProd<Rs...>::value;
-  stage0_global<T, R0, true, N, B, NT, true, Off, RowRev<Rs...>>(lds, io);
-  stages_ip<T, true, N, B, B, NT, R0, 0, Rs...>(lds, tw);
+  stage0_global<T, R0, true, N, B, NT, true, Off, RowRev<Rs...>>(lds, io, [&] { ctw.put(); });
+  stages_ip<T, true, N, B, B, NT, R0, 0, Rs...>(lds, ctw.table());
 }
 
 // Table-addressed rows (Off = TabRows or TabAll) with the row tables staged in LDS at
 // `tl` (n int2): the load table before the first stage, the store table
 // after it, so every table read is an LDS read.
-template <class T, bool FWD, int B, int NT, class Off, int R0, int... Rs>
-__device__ __forceinline__ void run_fft_io_tab(cpx<T>* lds, int2* tl, const typename TwT<T>::type* tw, ColIO io,
-                                               const int2* ltab, const int2* stab, RList<R0, Rs...>) {
+template <class T, bool FWD, int B, int NT, class Off, class Tw, int R0, int... Rs>
+__device__ __forceinline__ void run_fft_io_tab(cpx<T>* lds, int2* tl, const Tw& ctw, ColIO io, const int2* ltab,
+                                               const int2* stab, RList<R0, Rs...>) {
   static_assert(sizeof...(Rs) >= 1, "at least two stages");
   constexpr int N = R0 * RProd<Rs...>::value;
   for (int i = threadIdx.x; i < N; i += NT) tl[i] = ltab[i];
   __syncthreads();
   io.ltab = tl;
-  stage0_global<T, R0, FWD, N, B, NT, false, Off, RowRev<Rs...>>(lds, io);
+  stage0_global<T, R0, FWD, N, B, NT, false, Off, RowRev<Rs...>>(lds, io, [&] { ctw.put(); });
   for (int i = threadIdx.x; i < N; i += NT) tl[i] = stab[i];
   __syncthreads();
   io.stab = tl;
-  mid_and_last<T, FWD, N, B, B, NT, R0, 0, false, Off, true, false, Rs...>(lds, tw, io);
+  mid_and_last<T, FWD, N, B, B, NT, R0, 0, false, Off, true, false, Rs...>(lds, ctw.table(), io);
 }
 
 // Spectral solve along the column: forward FFT, per-mode multiply by
@@ -470,12 +528,13 @@ struct SolveCtx {
   double scale;
 };
 
-template <class T, int B, int NT, int R0, int... Rs>
-__device__ __forceinline__ void run_fft_solve(cpx<T>* lds, const typename TwT<T>::type* tw, const ColIO& io,
-                                              long long i0, const SolveCtx& sc, RList<R0, Rs...>) {
+template <class T, int B, int NT, class Tw, int R0, int... Rs>
+__device__ __forceinline__ void run_fft_solve(cpx<T>* lds, const Tw& ctw, const ColIO& io, long long i0,
+                                              const SolveCtx& sc, RList<R0, Rs...>) {
   static_assert(sizeof...(Rs) >= 1, "at least two stages");
   constexpr int N = R0 * RProd<Rs...>::value;
-  stage0_global<T, R0, true, N, B, NT, false, unsigned, RowRev<Rs...>>(lds, io);
+  stage0_global<T, R0, true, N, B, NT, false, unsigned, RowRev<Rs...>>(lds, io, [&] { ctw.put(); });
+  const auto* tw = ctw.table();
   stages_ip<T, true, N, B, B, NT, R0, 0, Rs...>(lds, tw);
   for (int q = threadIdx.x; q < B * N; q += NT) {
     const int e = q / B, b = q % B;
@@ -498,8 +557,8 @@ __device__ __forceinline__ void run_fft_solve(cpx<T>* lds, const typename TwT<T>
 // 256 and 1024 a workgroup per CU: 256^3 82.4 us against 74.6 us of the kernel
 // that met bank conflicts).  colb[b]:
 // byte offset of column b of the length-fastest side from the tile's first.
-template <class T, bool FWD, int B, int NT, bool IN, int R0, int... Rs>
-__device__ __forceinline__ void run_fft_lenfast(cpx<T>* lds, const typename TwT<T>::type* tw, const ColIO& io,
+template <class T, bool FWD, int B, int NT, bool IN, class Tw, int R0, int... Rs>
+__device__ __forceinline__ void run_fft_lenfast(cpx<T>* lds, const Tw& ctw, const ColIO& io,
                                                 const unsigned long long* colb, RList<R0, Rs...>) {
   static_assert(sizeof...(Rs) >= 1, "at least two stages");
   constexpr int N = R0 * RProd<Rs...>::value, BP = 0;
@@ -521,11 +580,12 @@ __device__ __forceinline__ void run_fft_lenfast(cpx<T>* lds, const typename TwT<
       const int q = threadIdx.x + u * NT;
       if ((B * N) % NT == 0 || q < B * N) lds[lds_at<B, BP>(q % N, q / N)] = v[u];
     }
+    ctw.put();
     __syncthreads();
-    mid_and_last<T, FWD, N, B, BP, NT, 1, 0, false, unsigned, false, false, R0, Rs...>(lds, tw, io);
+    mid_and_last<T, FWD, N, B, BP, NT, 1, 0, false, unsigned, false, false, R0, Rs...>(lds, ctw.table(), io);
   } else {
-    stage0_global<T, R0, FWD, N, B, NT, false, unsigned, RowRev<Rs...>, BP>(lds, io);
-    stages_ip<T, FWD, N, B, BP, NT, R0, 0, Rs...>(lds, tw);
+    stage0_global<T, R0, FWD, N, B, NT, false, unsigned, RowRev<Rs...>, BP>(lds, io, [&] { ctw.put(); });
+    stages_ip<T, FWD, N, B, BP, NT, R0, 0, Rs...>(lds, ctw.table());
 #pragma unroll
     for (int u = 0; u < LI; u++) {
       const int q = threadIdx.x + u * NT, b = q / N, p = q % N;
@@ -536,22 +596,6 @@ __device__ __forceinline__ void run_fft_lenfast(cpx<T>* lds, const typename TwT<
     }
   }
 }
-
-// Twiddle table entries used by a radix list (all stages after the first).
-template <int... Rs>
-struct TwCount;
-template <int R0, int... Rs>
-struct TwCount<R0, Rs...> {
-  template <int Ns, int R, int... Rest>
-  static constexpr int tail() {
-    if constexpr (sizeof...(Rest) == 0) return Ns * (R - 1);
-    else return Ns * (R - 1) + tail<Ns * R, Rest...>();
-  }
-  static constexpr int value() {
-    if constexpr (sizeof...(Rs) == 0) return 0;
-    else return tail<R0, Rs...>();
-  }
-};
 
 }  // namespace p3amd
 
