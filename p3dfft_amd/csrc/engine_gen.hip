@@ -194,15 +194,21 @@ __device__ __forceinline__ void gen_prime(cpx<T>* lds, const GenDesc& L, const G
   __syncthreads();
 }
 
-// an in-place stage over the tile; b: this thread's sequence, jt, js: its
+// An in-place stage over the tile.  PM: the schedule has a prime stage; the
+// others are compiled without it, whose registers (FP32 X kernels 96-109
+// against 80) cost every stage a wave per SIMD.  200-point FP32 X r2c of a
+// 200x300x250 box 39.7 -> 28.6 us, 1000-point FP64 of 1000x100x90 45.0 -> 41.6.
+// b: this thread's sequence, jt, js: its
 // first butterfly and their stride
-template <class T, bool FWD, bool DIF>
+template <class T, bool FWD, bool DIF, bool PM>
 __device__ __forceinline__ void gen_mid(cpx<T>* lds, const GenDesc& L, int s, const GenTile& t, int B, unsigned mB,
                                         int b, int jt, int js, const typename TwT<T>::type* tw) {
   const GenStage st = L.st[s];
-  if (st.R > kGenMaxRadix) {
-    gen_prime<T, FWD, DIF>(lds, L, st, t, B, mB, tw);
-    return;
+  if constexpr (PM) {
+    if (st.R > kGenMaxRadix) {
+      gen_prime<T, FWD, DIF>(lds, L, st, t, B, mB, tw);
+      return;
+    }
   }
   const int nj = gdiv(L.n, st.mR, st.R), SP = gen_stride(t, st);
   with_radix(st.R, [&](auto rc) {
@@ -232,16 +238,21 @@ __device__ __forceinline__ void gen_mid(cpx<T>* lds, const GenDesc& L, int s, co
 
 extern __shared__ __align__(16) unsigned char gen_smem[];
 
-// the twiddle table, copied into LDS behind the tile where it fits (complete
-// at the next barrier)
-template <class T>
-__device__ __forceinline__ const typename TwT<T>::type* gen_twiddles(const void* tw, int in_lds, int off, int count) {
+// the twiddle table, copied into LDS behind the tile where it fits (TL;
+// complete at the next barrier).  A compile-time choice: with one pointer for
+// either place the stages read it through the flat path (300-point FP32
+// columns of a 200x300x250 box 31.6 us so, 29.8 us now).
+template <class T, bool TL>
+__device__ __forceinline__ const typename TwT<T>::type* gen_twiddles(const void* tw, int off, int count) {
   typedef typename TwT<T>::type TwL;
   const TwL* g = (const TwL*)tw;
-  if (!in_lds) return g;
-  TwL* l = (TwL*)(gen_smem + off);
-  for (int i = threadIdx.x; i < count; i += blockDim.x) l[i] = g[i];
-  return l;
+  if constexpr (TL) {
+    TwL* l = (TwL*)(gen_smem + off);
+    for (int i = threadIdx.x; i < count; i += blockDim.x) l[i] = g[i];
+    return l;
+  } else {
+    return g;
+  }
 }
 
 // workgroup id -> tile: each XCD (id mod 8) owns a contiguous range
@@ -303,12 +314,12 @@ __device__ __forceinline__ cpx<T> gen_out(const GColArgs& a, cpx<T> v) {
 // MAP: pruned rows, DCT-I / DST-I extensions.  LF: 0 rows on both sides, 1 the
 // input is length-fastest (decimation in frequency), 2 the output is.  Off: the
 // type of the byte offsets from the tile's first column.
-template <class T, bool FWD, bool MAP, int LF, class Off>
+template <class T, bool FWD, bool MAP, int LF, class Off, bool TL, bool PM>
 __global__ __launch_bounds__(1024) void k_gcol(GColArgs a) {
   typedef cpx<T> C;
   constexpr long long E = sizeof(C);
   C* lds = (C*)gen_smem;
-  const auto* tw = gen_twiddles<T>(a.tw, a.tw_lds, a.tw_off, a.L.twcount);
+  const auto* tw = gen_twiddles<T, TL>(a.tw, a.tw_off, a.L.twcount);
   const int B = 1 << a.lB, NT = blockDim.x, S = a.L.nst;
   const unsigned mB = a.lB ? 1u << (32 - a.lB) : 0u;
   const int b = threadIdx.x & (B - 1), jt = threadIdx.x >> a.lB, js = NT >> a.lB;
@@ -359,7 +370,7 @@ __global__ __launch_bounds__(1024) void k_gcol(GColArgs a) {
       lds[e * a.t.BP + bb] = neg ? mk<T>(-v.x, -v.y) : v;
     }
     __syncthreads();
-    for (int s = S - 1; s > 0; s--) gen_mid<T, FWD, true>(lds, a.L, s, a.t, B, mB, b, jt, js, tw);
+    for (int s = S - 1; s > 0; s--) gen_mid<T, FWD, true, PM>(lds, a.L, s, a.t, B, mB, b, jt, js, tw);
     with_radix(s0.R, [&](auto rc) {
       constexpr int R = decltype(rc)::value;
       for (int j = jt; j < n0; j += js) {
@@ -408,7 +419,7 @@ __global__ __launch_bounds__(1024) void k_gcol(GColArgs a) {
   if (S == 1 && LF == 0) return;
   __syncthreads();
   const int last = LF == 2 ? S : S - 1;
-  for (int s = 1; s < last; s++) gen_mid<T, FWD, false>(lds, a.L, s, a.t, B, mB, b, jt, js, tw);
+  for (int s = 1; s < last; s++) gen_mid<T, FWD, false, PM>(lds, a.L, s, a.t, B, mB, b, jt, js, tw);
   if constexpr (LF == 2) {
     unsigned long long* colb = (unsigned long long*)(gen_smem + a.tw_off - kColTab);
     if (threadIdx.x < B) colb[threadIdx.x] = (unsigned long long)lout;
@@ -494,11 +505,11 @@ struct GXArgs {
 
 // r2c: stage 0 reads the rows (lanes along the row), in-place stages, and the
 // two half spectra separated from the natural-order result as they are stored
-template <class T>
+template <class T, bool TL, bool PM>
 __global__ __launch_bounds__(1024) void k_gx_r2c(GXArgs a) {
   typedef cpx<T> C;
   C* lds = (C*)gen_smem;
-  const auto* tw = gen_twiddles<T>(a.tw, a.tw_lds, a.tw_off, a.L.twcount);
+  const auto* tw = gen_twiddles<T, TL>(a.tw, a.tw_off, a.L.twcount);
   const int B = 1 << a.lB, NT = blockDim.x, S = a.L.nst, n = a.L.n;
   const long long pair0 = (long long)gen_tile_of(a.rev, 1) * B;
   const int nr = (int)(a.nrows - 2 * pair0 < 2 * B ? a.nrows - 2 * pair0 : 2 * B);
@@ -540,7 +551,7 @@ __global__ __launch_bounds__(1024) void k_gx_r2c(GXArgs a) {
   const int b0 = threadIdx.x & (B - 1), jt = threadIdx.x >> a.lB, js = NT >> a.lB;
   const unsigned mB = a.lB ? 1u << (32 - a.lB) : 0u;
   for (int s = 1; s < S; s++)
-    gen_mid<T, true, false>(lds, a.L, s, a.t, B, mB, b0, jt, js, tw);
+    gen_mid<T, true, false, PM>(lds, a.L, s, a.t, B, mB, b0, jt, js, tw);
   char* out = (char*)a.out + 2 * pair0 * a.so_row * (long long)sizeof(C);
   const unsigned so = (unsigned)(a.so_row * sizeof(C));
   const T h = (T)0.5;
@@ -555,34 +566,53 @@ __global__ __launch_bounds__(1024) void k_gx_r2c(GXArgs a) {
 
 // c2r: the mirror image: natural order in, decimation in frequency, stage 0
 // stores the rows
-template <class T>
+template <class T, bool TL, bool PM>
 __global__ __launch_bounds__(1024) void k_gx_c2r(GXArgs a) {
   typedef cpx<T> C;
   C* lds = (C*)gen_smem;
-  const auto* tw = gen_twiddles<T>(a.tw, a.tw_lds, a.tw_off, a.L.twcount);
+  const auto* tw = gen_twiddles<T, TL>(a.tw, a.tw_off, a.L.twcount);
   const int B = 1 << a.lB, NT = blockDim.x, S = a.L.nst, n = a.L.n, K = n / 2 + 1;
   const long long pair0 = (long long)gen_tile_of(a.rev, 1) * B;
   const int nr = (int)(a.nrows - 2 * pair0 < 2 * B ? a.nrows - 2 * pair0 : 2 * B);
   const char* in = (const char*)a.in + 2 * pair0 * a.si_row * (long long)sizeof(C);
   const unsigned si = (unsigned)(a.si_row * sizeof(C));
-  for (int q = threadIdx.x; q < B * K; q += NT) {
-    const int b = fdiv(q, a.dnk), k = q - b * K;
-    const bool oka = k < a.nk && 2 * b < nr, okb = k < a.nk && 2 * b + 1 < nr;
-    const unsigned off = (unsigned)(2 * b) * si + (unsigned)k * (unsigned)sizeof(C);
-    C A = *(const C*)(in + (oka ? off : 0u)), Bv = *(const C*)(in + (okb ? off + si : 0u));
-    if (!oka) A = mk<T>(0, 0);
-    if (!okb) Bv = mk<T>(0, 0);
-    // FFTW c2r: the imaginary parts of k = 0 and k = n/2 (n even) do not
-    // contribute; there both forms are the same value
-    if (k == 0 || 2 * k == n) { A.y = 0; Bv.y = 0; }
-    lds[k * a.t.BP + b] = mk<T>(A.x - Bv.y, A.y + Bv.x);
-    lds[(k == 0 ? 0 : n - k) * a.t.BP + b] = mk<T>(A.x + Bv.y, Bv.x - A.y);
+  // the loads of LU items in flight at a time before their LDS writes (200x300x250
+  // FP32, without the prime stage: 37.4 -> 31.3 us)
+  constexpr int LU = 4;
+  for (int q0 = threadIdx.x; q0 < B * K; q0 += LU * NT) {
+    C A[LU], Bv[LU];
+    int bb[LU], kk[LU];
+#pragma unroll
+    for (int u = 0; u < LU; u++) {
+      const int q = q0 + u * NT;
+      const int b = bb[u] = q < B * K ? fdiv(q, a.dnk) : B;
+      const int k = kk[u] = q - b * K;
+      // items outside the tile or past the valid modes read its first element
+      // and are zeroed, so no load sits under a branch
+      const bool oka = q < B * K && k < a.nk && 2 * b < nr, okb = oka && 2 * b + 1 < nr;
+      const unsigned off = (unsigned)(2 * b) * si + (unsigned)k * (unsigned)sizeof(C);
+      A[u] = *(const C*)(in + (oka ? off : 0u));
+      Bv[u] = *(const C*)(in + (okb ? off + si : 0u));
+      if (!oka) A[u] = mk<T>(0, 0);
+      if (!okb) Bv[u] = mk<T>(0, 0);
+      // FFTW c2r: the imaginary parts of k = 0 and k = n/2 (n even) do not
+      // contribute; there both forms are the same value
+      if (k == 0 || 2 * k == n) { A[u].y = 0; Bv[u].y = 0; }
+    }
+#pragma unroll
+    for (int u = 0; u < LU; u++) {
+      if (bb[u] < B) {
+        const int b = bb[u], k = kk[u];
+        lds[k * a.t.BP + b] = mk<T>(A[u].x - Bv[u].y, A[u].y + Bv[u].x);
+        lds[(k == 0 ? 0 : n - k) * a.t.BP + b] = mk<T>(A[u].x + Bv[u].y, Bv[u].x - A[u].y);
+      }
+    }
   }
   __syncthreads();
   const int b0 = threadIdx.x & (B - 1), jt = threadIdx.x >> a.lB, js = NT >> a.lB;
   const unsigned mB = a.lB ? 1u << (32 - a.lB) : 0u;
   for (int s = S - 1; s > 0; s--)
-    gen_mid<T, false, true>(lds, a.L, s, a.t, B, mB, b0, jt, js, tw);
+    gen_mid<T, false, true, PM>(lds, a.L, s, a.t, B, mB, b0, jt, js, tw);
   char* out = (char*)a.out + 2 * pair0 * a.so_row * (long long)sizeof(T);
   const unsigned so = (unsigned)(a.so_row * sizeof(T));
   const GenStage s0 = a.L.st[0];
@@ -741,9 +771,23 @@ static bool has_prime_stage(const Len1D& L) {
   return false;
 }
 
+// f(TL, PM): the twiddle table in LDS, the schedule with a prime stage
+template <class F>
+static void with_variant(bool tl, bool pm, F f) {
+  if (tl) {
+    if (pm) f(std::true_type{}, std::true_type{});
+    else f(std::true_type{}, std::false_type{});
+  } else {
+    if (pm) f(std::false_type{}, std::true_type{});
+    else f(std::false_type{}, std::false_type{});
+  }
+}
+
 template <bool FWD, bool MAP, int LF, class Off>
-static void go_col(const GColArgs& a, unsigned g, int nt, size_t bytes, hipStream_t st) {
-  k_gcol<real_t, FWD, MAP, LF, Off><<<g, nt, bytes, st>>>(a);
+static void go_col(const GColArgs& a, bool pm, unsigned g, int nt, size_t bytes, hipStream_t st) {
+  with_variant(a.tw_lds != 0, pm, [&](auto tl, auto pr) {
+    k_gcol<real_t, FWD, MAP, LF, Off, tl.value, pr.value><<<g, nt, bytes, st>>>(a);
+  });
 }
 
 void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, hipStream_t st) {
@@ -806,6 +850,7 @@ void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, hipStream_t st) {
   const size_t bytes = place_twiddles(data, *L, &a.tw_lds, &a.tw_off);
   if (bytes > kLdsMax) throw Error{"column transform does not fit in LDS", -1};
   const int nt = pick_threads(*L, B, bytes, nwg);
+  const bool pm = has_prime_stage(*L);
   const bool fwd = c.fwd || c.kind == COL_DCT1 || c.kind == COL_DST1;
   const bool ld_id = c.nld == m && (c.ld_lo >= m || (c.ld_hi <= c.ld_lo && c.ld_shift == 0));
   const bool st_id = c.nst == m && (c.st_lo >= m || c.st_shift == 0);
@@ -819,17 +864,17 @@ void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, hipStream_t st) {
   typedef unsigned long long U64;
   const unsigned g = (unsigned)nwg;
   if (fwd) {
-    if (lf_in) go_col<true, true, 1, U64>(a, g, nt, bytes, st);
-    else if (lf_out) go_col<true, true, 2, U64>(a, g, nt, bytes, st);
-    else if (!fits) go_col<true, true, 0, U64>(a, g, nt, bytes, st);
-    else if (map) go_col<true, true, 0, U32>(a, g, nt, bytes, st);
-    else go_col<true, false, 0, U32>(a, g, nt, bytes, st);
+    if (lf_in) go_col<true, true, 1, U64>(a, pm, g, nt, bytes, st);
+    else if (lf_out) go_col<true, true, 2, U64>(a, pm, g, nt, bytes, st);
+    else if (!fits) go_col<true, true, 0, U64>(a, pm, g, nt, bytes, st);
+    else if (map) go_col<true, true, 0, U32>(a, pm, g, nt, bytes, st);
+    else go_col<true, false, 0, U32>(a, pm, g, nt, bytes, st);
   } else {
-    if (lf_in) go_col<false, true, 1, U64>(a, g, nt, bytes, st);
-    else if (lf_out) go_col<false, true, 2, U64>(a, g, nt, bytes, st);
-    else if (!fits) go_col<false, true, 0, U64>(a, g, nt, bytes, st);
-    else if (map) go_col<false, true, 0, U32>(a, g, nt, bytes, st);
-    else go_col<false, false, 0, U32>(a, g, nt, bytes, st);
+    if (lf_in) go_col<false, true, 1, U64>(a, pm, g, nt, bytes, st);
+    else if (lf_out) go_col<false, true, 2, U64>(a, pm, g, nt, bytes, st);
+    else if (!fits) go_col<false, true, 0, U64>(a, pm, g, nt, bytes, st);
+    else if (map) go_col<false, true, 0, U32>(a, pm, g, nt, bytes, st);
+    else go_col<false, false, 0, U32>(a, pm, g, nt, bytes, st);
   }
   check_hip(hipGetLastError(), "k_gcol launch");
 }
@@ -869,7 +914,9 @@ void gen_launch_x_r2c(const Len1D& L, const real_t* in, cplx_t* out, long long n
   int nt;
   unsigned g;
   const size_t bytes = x_tile(a, L, nrows, std::max(si_row, so_row), &nt, &g);
-  k_gx_r2c<real_t><<<g, nt, bytes, st>>>(a);
+  with_variant(a.tw_lds != 0, has_prime_stage(L), [&](auto tl, auto pm) {
+    k_gx_r2c<real_t, tl.value, pm.value><<<g, nt, bytes, st>>>(a);
+  });
   check_hip(hipGetLastError(), "k_gx_r2c launch");
 }
 
@@ -883,7 +930,9 @@ void gen_launch_x_c2r(const Len1D& L, const cplx_t* in, real_t* out, long long n
   int nt;
   unsigned g;
   const size_t bytes = x_tile(a, L, nrows, std::max(si_row, so_row), &nt, &g);
-  k_gx_c2r<real_t><<<g, nt, bytes, st>>>(a);
+  with_variant(a.tw_lds != 0, has_prime_stage(L), [&](auto tl, auto pm) {
+    k_gx_c2r<real_t, tl.value, pm.value><<<g, nt, bytes, st>>>(a);
+  });
   check_hip(hipGetLastError(), "k_gx_c2r launch");
 }
 
@@ -892,24 +941,28 @@ static void allow_big_lds(K kernel) {
   (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax);
   (void)hipGetLastError();  // a refused attribute leaves the default limit, not a pending error
 }
-template <bool FWD>
+template <bool FWD, bool TL, bool PM>
 static void prep_dir() {
   typedef unsigned U32;
   typedef unsigned long long U64;
-  allow_big_lds(k_gcol<real_t, FWD, false, 0, U32>);
-  allow_big_lds(k_gcol<real_t, FWD, true, 0, U32>);
-  allow_big_lds(k_gcol<real_t, FWD, true, 0, U64>);
-  allow_big_lds(k_gcol<real_t, FWD, true, 1, U64>);
-  allow_big_lds(k_gcol<real_t, FWD, true, 2, U64>);
+  allow_big_lds(k_gcol<real_t, FWD, false, 0, U32, TL, PM>);
+  allow_big_lds(k_gcol<real_t, FWD, true, 0, U32, TL, PM>);
+  allow_big_lds(k_gcol<real_t, FWD, true, 0, U64, TL, PM>);
+  allow_big_lds(k_gcol<real_t, FWD, true, 1, U64, TL, PM>);
+  allow_big_lds(k_gcol<real_t, FWD, true, 2, U64, TL, PM>);
+  if (FWD) allow_big_lds(k_gx_r2c<real_t, TL, PM>);
+  else allow_big_lds(k_gx_c2r<real_t, TL, PM>);
 }
 void gen_prep_kernels() {
   static std::once_flag once;
   std::call_once(once, [] {
-    prep_dir<true>();
-    prep_dir<false>();
+    for (int tl = 0; tl < 2; tl++)
+      for (int pm = 0; pm < 2; pm++)
+        with_variant(tl != 0, pm != 0, [](auto t, auto p) {
+          prep_dir<true, t.value, p.value>();
+          prep_dir<false, t.value, p.value>();
+        });
     allow_big_lds(k_gcopy<real_t>);
-    allow_big_lds(k_gx_r2c<real_t>);
-    allow_big_lds(k_gx_c2r<real_t>);
   });
 }
 
