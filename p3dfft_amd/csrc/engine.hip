@@ -126,48 +126,34 @@ struct ColArgs {
 // tile base plus 32-bit byte offsets (the host checks that they fit).
 // ---------------------------------------------------------------------------
 // X r2c of the row pairs pair0 .. pair0+B-1 (nr <= 2B rows exist) through
-// the LDS tile `lds`
+// the LDS tile `lds`.  Bound by the latencies of a tile's serial phases, then
+// by HBM: the first stage from the loads and the others in place take 6 LDS
+// accesses per value and 3 barriers for three radices, where a loaded tile and
+// autosort stages took 8 and 7.  With the smaller tiles of ct_x_pairs, r2c /
+// c2r FP32 512^3 215 / 204 -> 200 / 196 us (5.4 TB/s), 384^3 90 / 83 ->
+// 82 / 82, 2048x128x128 58 / 58 -> 50 / 50; FP64 384^3 183 / 164 ->
+// 161 / 154, 2048x128x128 137 / 124 -> 101 / 96.
 template <class T, int B, int NT, class RL, bool XT, class Tw>
 __device__ __forceinline__ void x_r2c_ct_tile(cpx<T>* lds, const Tw& tw, const XArgs& a,
                                               long long pin, long long pair0, int nr) {
   constexpr int N = RL_N<RL>::value;
-  constexpr int BP = B + 1;
+  typedef XLay<T, B, RL> Lay;
   const char* in = (const char*)a.in + 2 * pin * a.si_row * (long long)sizeof(T);
   const unsigned si = (unsigned)(a.si_row * sizeof(T));
-  {
-    // issue every load of the tile before the LDS writes
-    constexpr int LI = (B * N + NT - 1) / NT;
-    T xa[LI], xb[LI];
-#pragma unroll
-    for (int i = 0; i < LI; i++) {
-      const int q = threadIdx.x + i * NT;
-      const int b = q / N, j = q % N;
-      const bool ok = ((B * N) % NT == 0) || q < B * N;
-      // out-of-range items load the tile's first element (always valid) and
-      // are zeroed, so no load sits under a branch
-      const bool oka = ok && 2 * b < nr, okb = ok && 2 * b + 1 < nr;
-      const unsigned o = (unsigned)(2 * b) * si + (unsigned)j * (unsigned)sizeof(T);
-      const T va = *(const T*)(in + (oka ? o : 0u));
-      const T vb = *(const T*)(in + (okb ? o + si : 0u));
-      xa[i] = oka ? va : (T)0;
-      xb[i] = okb ? vb : (T)0;
-    }
-#pragma unroll
-    for (int i = 0; i < LI; i++) {
-      const int q = threadIdx.x + i * NT;
-      if (((B * N) % NT == 0) || q < B * N) lds[(q % N) * BP + q / N] = mk<T>(xa[i], xb[i]);
-    }
-  }
-  tw.put();
-  __syncthreads();
-  run_fft_ct<T, true, B, BP, NT>(lds, tw.table(), RL{});
+  // rows past the last one read the tile's first element (always valid) and
+  // are zeroed, so no load sits under a branch
+  auto row = [&](int rw, int e) {
+    const T u = *(const T*)(in + (rw < nr ? (unsigned)rw * si + (unsigned)e * (unsigned)sizeof(T) : 0u));
+    return rw < nr ? u : (T)0;
+  };
+  x_fft_fwd<T, Lay, B, NT>(lds, tw, row, RL{});
   char* out = (char*)a.out + 2 * pair0 * a.so_row * (long long)sizeof(cpx<T>);
   const unsigned so = (unsigned)(a.so_row * sizeof(cpx<T>));
   const T h = (T)0.5;
   const bool full = nr == 2 * B;  // uniform: no per-store row guard
   // separation of mode k of pair b and its stores (FULL: no row guard)
   auto put = [&](int b, int k, auto fl) {
-    const cpx<T> zk = lds[k * BP + b], zn = lds[(k == 0 ? 0 : N - k) * BP + b];
+    const cpx<T> zk = lds[Lay::at(k) + b], zn = lds[Lay::at(k == 0 ? 0 : N - k) + b];
     const unsigned o = (unsigned)(2 * b) * so + (unsigned)k * (unsigned)sizeof(cpx<T>);
     const cpx<T> ya = mk<T>((zk.x + zn.x) * h, (zk.y - zn.y) * h), yb = mk<T>((zk.y + zn.y) * h, (zn.x - zk.x) * h);
     if (decltype(fl)::value || 2 * b < nr) *(cpx<T>*)(out + o) = ya;
@@ -192,7 +178,7 @@ __device__ __forceinline__ void x_r2c_ct_tile(cpx<T>* lds, const Tw& tw, const X
       const int q = threadIdx.x + i * NT;
       if (q < B * a.nxo) {
         const int b = fdiv(q, a.dnxo), k = q - b * a.nxo;
-        const cpx<T> zk = lds[k * BP + b], zn = lds[(k == 0 ? 0 : N - k) * BP + b];
+        const cpx<T> zk = lds[Lay::at(k) + b], zn = lds[Lay::at(k == 0 ? 0 : N - k) + b];
         const cpx<T> ya = mk<T>((zk.x + zn.x) * h, (zk.y - zn.y) * h), yb = mk<T>((zk.y + zn.y) * h, (zn.x - zk.x) * h);
         const long long r = 2 * (pair0 + b);
         cpx<T>* oc = (cpx<T>*)a.out;
@@ -239,7 +225,7 @@ template <class T, int B, int NT, class RL, bool XT, class Tw>
 __device__ __forceinline__ void x_c2r_ct_tile(cpx<T>* lds, const Tw& tw, const XArgs& a,
                                               long long pair0, long long pout, int nr) {
   constexpr int N = RL_N<RL>::value;
-  constexpr int BP = B + 1;
+  typedef XLay<T, B, RL> Lay;
   constexpr int H = N / 2;
   const char* in = (const char*)a.in + 2 * pair0 * a.si_row * (long long)sizeof(cpx<T>);
   const unsigned si = (unsigned)(a.si_row * sizeof(cpx<T>));
@@ -276,12 +262,12 @@ __device__ __forceinline__ void x_c2r_ct_tile(cpx<T>* lds, const Tw& tw, const X
         const int b = q / H, k = q % H;
         cpx<T> A = va[i], Bv = vb[i];
         if (k == 0) { A.y = 0; Bv.y = 0; }
-        lds[k * BP + b] = mk<T>(A.x - Bv.y, A.y + Bv.x);
-        lds[(k == 0 ? 0 : N - k) * BP + b] = mk<T>(A.x + Bv.y, Bv.x - A.y);
+        lds[Lay::at(k) + b] = mk<T>(A.x - Bv.y, A.y + Bv.x);
+        lds[Lay::at(k == 0 ? 0 : N - k) + b] = mk<T>(A.x + Bv.y, Bv.x - A.y);
       }
     }
     // Nyquist: Im of A and B ignored, Z[N/2] = Re A + i Re B
-    if (threadIdx.x < B) lds[H * BP + threadIdx.x] = mk<T>(na.x, nb.x);
+    if (threadIdx.x < B) lds[Lay::at(H) + threadIdx.x] = mk<T>(na.x, nb.x);
   } else {
     // each input element k <= N/2 is loaded once and gives Z[k] and Z[N-k]
     // (Z = A + iB of the two Hermitian half spectra)
@@ -334,31 +320,21 @@ __device__ __forceinline__ void x_c2r_ct_tile(cpx<T>* lds, const Tw& tw, const X
         if (k == 0 || 2 * k == N) { A.y = 0; Bv.y = 0; }
         // at k = 0 and k = N/2 both forms are the same value: the second
         // write repeats the first (row 0 stands in for row N)
-        lds[k * BP + b] = mk<T>(A.x - Bv.y, A.y + Bv.x);
-        lds[(k == 0 ? 0 : N - k) * BP + b] = mk<T>(A.x + Bv.y, Bv.x - A.y);
+        lds[Lay::at(k) + b] = mk<T>(A.x - Bv.y, A.y + Bv.x);
+        lds[Lay::at(k == 0 ? 0 : N - k) + b] = mk<T>(A.x + Bv.y, Bv.x - A.y);
       }
     }
   }
   tw.put();
   __syncthreads();
-  run_fft_ct<T, false, B, BP, NT>(lds, tw.table(), RL{});
   char* out = (char*)a.out + 2 * pout * a.so_row * (long long)sizeof(T);
   const unsigned so = (unsigned)(a.so_row * sizeof(T));
-  // a compile-time trip count and the full-tile test outside the loop, so
-  // that the LDS reads of all items can be issued ahead of their stores
-  constexpr int LS = (B * N + NT - 1) / NT;
   auto store_all = [&](auto full) {
-#pragma unroll
-    for (int i = 0; i < LS; i++) {
-      const int q = threadIdx.x + i * NT;
-      if ((B * N) % NT == 0 || q < B * N) {
-        const int b = q / N, j = q % N;
-        const cpx<T> z = lds[j * BP + b];
-        const unsigned o = (unsigned)(2 * b) * so + (unsigned)j * (unsigned)sizeof(T);
-        if (decltype(full)::value || 2 * b < nr) *(T*)(out + o) = z.x;
-        if (decltype(full)::value || 2 * b + 1 < nr) *(T*)(out + o + so) = z.y;
-      }
-    }
+    x_fft_bwd<T, Lay, B, NT>(lds, tw.table(), [&](int b, int e, cpx<T> z) {
+      const unsigned o = (unsigned)(2 * b) * so + (unsigned)e * (unsigned)sizeof(T);
+      if (decltype(full)::value || 2 * b < nr) *(T*)(out + o) = z.x;
+      if (decltype(full)::value || 2 * b + 1 < nr) *(T*)(out + o + so) = z.y;
+    }, RL{});
   };
   if (nr == 2 * B) store_all(std::true_type{});  // uniform: no per-store row guard
   else store_all(std::false_type{});
@@ -661,9 +637,12 @@ __global__ __launch_bounds__(256) void k_x_c2r_w512(XArgs a, const typename TwT<
 // more than the plane's data movement, so fusing X and Y saves one launch and
 // one HBM round trip per direction.  NX, NY are compile-time lengths with
 // specialised radix schedules RLX, RLY (the twiddle tables of those lengths).
-// LDS: the X tile (NY/2 row pairs of length NX, element e of pair b at
-// lx[e*(NY/2+1) + b]), then the Y tile (NX/2+1 columns of length NY, element
-// y of column k at ly[y*(NX/2+1) + k]), then both twiddle tables.
+// LDS: the X tile (NY/2 row pairs of length NX, XLay), then the Y tile
+// (NX/2+1 columns of length NY, position p of column k at ly[p*(NX/2+1) + k]),
+// then both twiddle tables.  A plane is one workgroup's serial chain of
+// stages, so what counts is barriers and LDS passes: the outer stages read and
+// write HBM, the first forward Y stage takes the separated rows from the X
+// tile, the others run in place.
 // ---------------------------------------------------------------------------
 struct PlaneArgs {
   const void* in;
@@ -676,9 +655,10 @@ struct PlaneArgs {
 template <class T, class RLX, class RLY>
 struct PlaneGeom {
   static constexpr int NX = RL_N<RLX>::value, NY = RL_N<RLY>::value;
-  static constexpr int BX = NY / 2, BPX = BX + 1;  // row pairs, padded
+  static constexpr int BX = NY / 2;                // row pairs
   static constexpr int H = NX / 2 + 1;             // columns of the half spectrum
-  static constexpr long long X_BYTES = (long long)NX * BPX * sizeof(cpx<T>);
+  typedef XLay<T, BX, RLX> Lay;
+  static constexpr long long X_BYTES = (Lay::BYTES + 15) / 16 * 16;
   static constexpr long long Y_BYTES = (long long)NY * H * sizeof(cpx<T>);
   static constexpr long long DATA = X_BYTES + Y_BYTES;
 };
@@ -697,67 +677,89 @@ struct PlaneTw {
     x.put();
     y.put();
   }
-  __device__ __forceinline__ const TwL* tx() const { return x.table(); }
+  __device__ __forceinline__ const TwL* table() const { return x.table(); }
   __device__ __forceinline__ const TwL* ty() const {
     if constexpr (SAME) return x.table();
     else return y.table();
   }
 };
 
+// the stages of a plane's Y transform from Ns on, in place, the last to st
+template <class T, bool FWD, int N, int H, int NT, int Ns, int Off, class ST, int R, int... Rest>
+__device__ __forceinline__ void plane_y_rest(cpx<T>* ly, const typename TwT<T>::type* tw, ST st, RList<R, Rest...>) {
+  if constexpr (sizeof...(Rest) > 0) {
+    stage_ip<T, R, FWD, N, H, H, NT, Ns, Off>(ly, tw);
+    plane_y_rest<T, FWD, N, H, NT, Ns * R, Off + Ns * (R - 1)>(ly, tw, st, RList<Rest...>{});
+  } else {
+    constexpr int total = H * Ns, IT = (total + NT - 1) / NT;
+#pragma unroll
+    for (int m = 0; m < IT; m++) {
+      const int it = threadIdx.x + m * NT;
+      if (total % NT == 0 || it < total) {
+        const int j = it / H, k = it % H;
+        cpx<T> v[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) v[r] = ly[(j + r * Ns) * H + k];
+        const typename TwT<T>::type* w = tw + Off + j * (R - 1);
+#pragma unroll
+        for (int r = 1; r < R; r++) v[r] = twmul<FWD>(v[r], w[r - 1]);
+        dft<R, FWD>(v);
+#pragma unroll
+        for (int r = 0; r < R; r++) st(j + r * Ns, k, v[r]);
+      }
+    }
+  }
+}
+
+// the Y transform of a plane: the first stage's value of row y, column k from
+// ld(y, k), the last stage's to st(y, k, v) (the tile itself if it reads ly)
+template <class T, bool FWD, int H, int NT, class LD, class PRE, class ST, int R0, int... Rs>
+__device__ __forceinline__ void plane_y(cpx<T>* ly, const typename TwT<T>::type* tw, LD ld, PRE pre, ST st,
+                                        RList<R0, Rs...>) {
+  constexpr int N = R0 * RProd<Rs...>::value, nR = N / R0, total = H * nR, IT = (total + NT - 1) / NT;
+  cpx<T> v[IT][R0];
+#pragma unroll
+  for (int m = 0; m < IT; m++) {
+    const int it = threadIdx.x + m * NT;
+    const int q = total % NT == 0 || it < total ? it : 0;
+    const int y = RowRev<Rs...>::at(q / H), k = q % H;
+#pragma unroll
+    for (int r = 0; r < R0; r++) v[m][r] = ld(y + r * nR, k);
+  }
+#pragma unroll
+  for (int m = 0; m < IT; m++) {
+    const int it = threadIdx.x + m * NT;
+    if (total % NT == 0 || it < total) {
+      dft<R0, FWD>(v[m]);
+#pragma unroll
+      for (int r = 0; r < R0; r++) ly[(it / H * R0 + r) * H + it % H] = v[m][r];
+    }
+  }
+  pre();
+  __syncthreads();
+  plane_y_rest<T, FWD, N, H, NT, R0, 0>(ly, tw, st, RList<Rs...>{});
+}
 // forward: X r2c (two-for-one, as k_x_r2c_ct) and Y forward of plane
 // blockIdx.x: real rows of NX (row stride NX) -> half-spectrum rows of NX/2+1
 template <class T, class RLX, class RLY, int NT>
 __global__ __launch_bounds__(NT) void k_xy_plane_fwd(PlaneArgs a) {
   typedef PlaneGeom<T, RLX, RLY> G;
-  constexpr int NX = G::NX, NY = G::NY, BX = G::BX, BPX = G::BPX, H = G::H;
+  typedef typename G::Lay Lay;
+  constexpr int NX = G::NX, NY = G::NY, BX = G::BX, H = G::H;
   cpx<T>* lx = (cpx<T>*)g_smem;
   cpx<T>* ly = (cpx<T>*)(g_smem + G::X_BYTES);
   const PlaneTw<T, RLX, RLY, NT> tw(a);
   const T* in = (const T*)a.in + (long long)blockIdx.x * NX * NY;
-  {
-    // compile-time trip counts: every load of the plane issued before the
-    // LDS writes (items past the plane read element 0 and are not written)
-    constexpr int LI = (BX * NX + NT - 1) / NT;
-    T xa[LI], xb[LI];
-#pragma unroll
-    for (int i = 0; i < LI; i++) {
-      const int q = threadIdx.x + i * NT;
-      const bool ok = (BX * NX) % NT == 0 || q < BX * NX;
-      const int b = q / NX, j = q % NX;
-      xa[i] = in[ok ? 2 * b * NX + j : 0];
-      xb[i] = in[ok ? (2 * b + 1) * NX + j : 0];
-    }
-#pragma unroll
-    for (int i = 0; i < LI; i++) {
-      const int q = threadIdx.x + i * NT;
-      if ((BX * NX) % NT == 0 || q < BX * NX) lx[(q % NX) * BPX + q / NX] = mk<T>(xa[i], xb[i]);
-    }
-  }
-  tw.put();
-  __syncthreads();
-  run_fft_ct<T, true, BX, BPX, NT>(lx, tw.tx(), RLX{});
-  const T h = (T)0.5;
-  for (int q = threadIdx.x; q < BX * H; q += NT) {
-    const int b = q / H, k = q % H;
-    const cpx<T> zk = lx[k * BPX + b], zn = lx[(k == 0 ? 0 : NX - k) * BPX + b];
-    ly[(2 * b) * H + k] = mk<T>((zk.x + zn.x) * h, (zk.y - zn.y) * h);
-    ly[(2 * b + 1) * H + k] = mk<T>((zk.y + zn.y) * h, (zn.x - zk.x) * h);
-  }
-  __syncthreads();
-  run_fft_ct<T, true, H, H, NT>(ly, tw.ty(), RLY{});
+  x_fft_fwd<T, Lay, BX, NT>(lx, tw, [&](int row, int e) { return in[row * NX + e]; }, RLX{});
   cpx<T>* out = (cpx<T>*)a.out + (long long)blockIdx.x * H * NY;
-  constexpr int LQ = (NY * H + NT - 1) / NT;
-  cpx<T> v[LQ];
-#pragma unroll
-  for (int i = 0; i < LQ; i++) {
-    const int q = threadIdx.x + i * NT;
-    v[i] = ly[(NY * H) % NT == 0 || q < NY * H ? q : 0];
-  }
-#pragma unroll
-  for (int i = 0; i < LQ; i++) {
-    const int q = threadIdx.x + i * NT;
-    if ((NY * H) % NT == 0 || q < NY * H) out[q] = v[i];
-  }
+  const T h = (T)0.5;
+  plane_y<T, true, H, NT>(
+      ly, tw.ty(),
+      [&](int y, int k) {
+        const cpx<T> zk = lx[Lay::at(k) + y / 2], zn = lx[Lay::at(k == 0 ? 0 : NX - k) + y / 2];
+        return y % 2 ? mk<T>((zk.y + zn.y) * h, (zn.x - zk.x) * h) : mk<T>((zk.x + zn.x) * h, (zk.y - zn.y) * h);
+      },
+      [] {}, [&](int y, int k, cpx<T> v) { out[y * H + k] = v; }, RLY{});
 }
 
 // backward: Y backward and X c2r (as k_x_c2r_ct: Im of the DC and Nyquist
@@ -765,57 +767,30 @@ __global__ __launch_bounds__(NT) void k_xy_plane_fwd(PlaneArgs a) {
 template <class T, class RLX, class RLY, int NT>
 __global__ __launch_bounds__(NT) void k_yx_plane_bwd(PlaneArgs a) {
   typedef PlaneGeom<T, RLX, RLY> G;
-  constexpr int NX = G::NX, NY = G::NY, BX = G::BX, BPX = G::BPX, H = G::H;
+  typedef typename G::Lay Lay;
+  constexpr int NX = G::NX, NY = G::NY, BX = G::BX, H = G::H;
   cpx<T>* lx = (cpx<T>*)g_smem;
   cpx<T>* ly = (cpx<T>*)(g_smem + G::X_BYTES);
   const PlaneTw<T, RLX, RLY, NT> tw(a);
   const cpx<T>* in = (const cpx<T>*)a.in + (long long)blockIdx.x * H * NY;
-  {
-    // every load of the plane issued before the LDS writes
-    constexpr int LQ = (NY * H + NT - 1) / NT;
-    cpx<T> v[LQ];
-#pragma unroll
-    for (int i = 0; i < LQ; i++) {
-      const int q = threadIdx.x + i * NT;
-      v[i] = in[(NY * H) % NT == 0 || q < NY * H ? q : 0];
-    }
-#pragma unroll
-    for (int i = 0; i < LQ; i++) {
-      const int q = threadIdx.x + i * NT;
-      if ((NY * H) % NT == 0 || q < NY * H) ly[q] = v[i];
-    }
-  }
-  tw.put();
+  plane_y<T, false, H, NT>(
+      ly, tw.ty(), [&](int y, int k) { return in[y * H + k]; }, [&] { tw.put(); },
+      [&](int y, int k, cpx<T> v) { ly[y * H + k] = v; }, RLY{});
   __syncthreads();
-  run_fft_ct<T, false, H, H, NT>(ly, tw.ty(), RLY{});
   for (int q = threadIdx.x; q < BX * H; q += NT) {
     const int b = q / H, k = q % H;
     cpx<T> A = ly[(2 * b) * H + k], Bv = ly[(2 * b + 1) * H + k];
     if (k == 0 || 2 * k == NX) { A.y = 0; Bv.y = 0; }
     // at k = 0 and k = NX/2 both forms are the same value
-    lx[k * BPX + b] = mk<T>(A.x - Bv.y, A.y + Bv.x);
-    lx[(k == 0 ? 0 : NX - k) * BPX + b] = mk<T>(A.x + Bv.y, Bv.x - A.y);
+    lx[Lay::at(k) + b] = mk<T>(A.x - Bv.y, A.y + Bv.x);
+    lx[Lay::at(k == 0 ? 0 : NX - k) + b] = mk<T>(A.x + Bv.y, Bv.x - A.y);
   }
   __syncthreads();
-  run_fft_ct<T, false, BX, BPX, NT>(lx, tw.tx(), RLX{});
   T* out = (T*)a.out + (long long)blockIdx.x * NX * NY;
-  constexpr int LI = (BX * NX + NT - 1) / NT;
-  cpx<T> z[LI];
-#pragma unroll
-  for (int i = 0; i < LI; i++) {
-    const int q = threadIdx.x + i * NT;
-    const bool ok = (BX * NX) % NT == 0 || q < BX * NX;
-    z[i] = lx[ok ? (q % NX) * BPX + q / NX : 0];
-  }
-#pragma unroll
-  for (int i = 0; i < LI; i++) {
-    const int q = threadIdx.x + i * NT;
-    if ((BX * NX) % NT == 0 || q < BX * NX) {
-      const int b = q / NX, j = q % NX;
-      out[2 * b * NX + j] = z[i].x;
-      out[(2 * b + 1) * NX + j] = z[i].y;
-    }
-  }
+  x_fft_bwd<T, Lay, BX, NT>(lx, tw.table(), [&](int b, int e, cpx<T> z) {
+    out[2 * b * NX + e] = z.x;
+    out[(2 * b + 1) * NX + e] = z.y;
+  }, RLX{});
 }
 
 // Tile of B consecutive columns c0 .. c0+B-1 of the flattened (outer, inner)
@@ -1662,28 +1637,24 @@ constexpr int ct_waves(long long lds_bytes, int nt) {
   const long long w = wg * (nt / 64) / 4;
   return w < 1 ? 1 : (w > 4 ? 4 : (int)w);  // at least 128 registers per lane
 }
-// X kernels: up to 16 row pairs per tile, 16 complex values per thread, at
-// most 512 threads and an 80 KiB padded tile (two workgroups per CU)
-#ifndef P3DFFT_X_EPT
-#define P3DFFT_X_EPT 16
-#endif
-#ifndef P3DFFT_X_NT_MAX
-#define P3DFFT_X_NT_MAX 512
-#endif
-constexpr int kEPTx = P3DFFT_X_EPT;
+// X kernels: up to 16 row pairs per tile and tiles of at most 32 KiB, so that
+// four workgroups of a CU are in different phases, 8 complex values per thread
+// (one butterfly of the first radix).  With 64 KiB and 16 values, FP32 r2c /
+// c2r of 512^3 took 213 / 201 us against 203 / 200 us, 384^3 85 / 84 against
+// 81 / 81, 1024x256x128 52 / 51 against 44 / 43; FP64 256^3 43 / 43 against
+// 41 / 42, 1024x256x128 110 / 102 against 109 / 94.
+constexpr int kEPTx = 8;
 constexpr int ct_x_pairs(int N) {
   int b = 16;
-  while (b > 1 && (b * N > P3DFFT_X_NT_MAX * kEPTx || (long long)(b + 1) * N * (long long)sizeof(cplx_t) > 80 * 1024))
-    b /= 2;
+  while (b > 1 && (long long)b * N * (long long)sizeof(cplx_t) > 32 * 1024) b /= 2;
   return b;
 }
-// a tile that gives fewer than P3DFFT_X_NT_MAX threads at kEPTx values each
-// takes up to twice the threads at half the values: more waves per CU where
-// the LDS allows few workgroups
-constexpr int ct_nt_x(int elems) {
-  int nt = (elems / kEPTx + 63) / 64 * 64;
-  if (nt < P3DFFT_X_NT_MAX) nt = (elems / (kEPTx / 2) + 63) / 64 * 64;
-  return nt < 64 ? 64 : (nt > P3DFFT_X_NT_MAX ? P3DFFT_X_NT_MAX : nt);
+// a full tile takes 512 threads in either precision: in FP64 the loads and the
+// separation spread over twice the threads of the butterflies
+constexpr int ct_nt_x(int b, int N) {
+  if ((long long)b * N * (long long)sizeof(cplx_t) > 24 * 1024) return 512;
+  const int nt = (b * N / kEPTx + 63) / 64 * 64;
+  return nt;
 }
 
 // Twiddles of a specialised length sit in LDS behind the data tile when the
@@ -1699,6 +1670,7 @@ struct CtInfo {
   bool pipe;            // the column tile takes more than half the LDS: k_colio_pipe exists
   bool twl_pipe_tab;    // twiddles in LDS in the table-addressed k_colio_pipe
   long long twb;        // twiddle table bytes
+  long long x_bytes;    // X tile bytes
   void (*col)(bool, const ColArgs&, unsigned, size_t, hipStream_t);
   void (*colio)(bool, bool, bool, const ColArgs&, unsigned, size_t, hipStream_t);
   void (*colpipe)(bool, bool, const ColArgs&, unsigned, size_t, hipStream_t);
@@ -1731,10 +1703,10 @@ struct CtLen {
   static constexpr int TX = ct_col_tx(N);
   static constexpr int NTC = ct_nt_ept(TX * N, EPTC);
   static constexpr int BX = ct_x_pairs(N);
-  static constexpr int NTX = ct_nt_x(BX * N);
+  static constexpr int NTX = ct_nt_x(BX, N);
   static constexpr long long TWB = (long long)TwCount<Rs...>::value() * sizeof(Tw);
   static constexpr long long DC = round16((long long)TX * N * sizeof(cplx_t));
-  static constexpr long long DX = round16((long long)(BX + 1) * N * sizeof(cplx_t));
+  static constexpr long long DX = round16(XLay<real_t, BX, RL>::BYTES);
   // twiddles in LDS behind the column tile: when both fit in kCtLdsTw (two
   // workgroups per CU), or when the tile alone takes more than that (one
   // workgroup per CU either way) and both fit in the LDS
@@ -1884,7 +1856,7 @@ struct CtLen {
     const int rs[] = {Rs...};
     c.nr = (int)sizeof...(Rs);
     for (int i = 0; i < c.nr; i++) c.radix[i] = rs[i];
-    c.twl_col = TWLC; c.twl_x = TWLX; c.twl_tab = TWLT; c.twb = TWB;
+    c.twl_col = TWLC; c.twl_x = TWLX; c.twl_tab = TWLT; c.twb = TWB; c.x_bytes = DX;
     c.pipe = PIPE; c.twl_pipe_tab = TWLP; c.twl_lf = TWLF; c.collf = &collf;
     c.col = &col; c.colio = &colio; c.colpipe = &colpipe; c.xr2c = &xr2c; c.xc2r = &xc2r; c.zsolve = &zsolve; c.prep = &prep;
     c.xgrp = &xgrp; c.cgrp = &cgrp; c.zgrp = &zgrp;
@@ -1996,7 +1968,7 @@ static bool x_setup_ct(XArgs& a, const Len1D& L, const CtInfo& c, long long nrow
   a.B = c.BX;
   a.L = CtLenArg{L.d.n, L.d.twcount};
   a.tw = L.tw;
-  *bytes = ct_lds((size_t)(c.BX + 1) * L.d.n * sizeof(cplx_t), c.twl_x, c, &a.tw_lds, &a.tw_off);
+  *bytes = ct_lds((size_t)c.x_bytes, c.twl_x, c, &a.tw_lds, &a.tw_off);
   const long long g = (pairs + c.BX - 1) / c.BX;
   if (g > 0x7fffffffLL) throw Error{"grid too large", -1};
   *nwg = (unsigned)g;
@@ -2116,7 +2088,8 @@ void launch_x_c2r(const cplx_t* in, real_t* out, long long nrows, long long si_r
 // instantiated below; mode 0 off, 1 wherever they apply, 2 (default) on the
 // grids where they measured faster: up to 2^22 points, and at least 64 planes
 // unless the planes are 64 x 64 or smaller (one workgroup per plane).
-// Measured on MI355X, eager fwd+bwd, separate passes -> plane kernels (us):
+// Measured on MI355X, eager fwd+bwd, separate passes -> plane kernels (us),
+// before both took the in-place X tile (64^3 FP64 19.8 -> 18.9 since):
 // FP64 32^3 27.2 -> 14.0, 64^3 24.8 -> 19.8, 64x64x256 47.6 -> 33.9,
 // 128x64x64 33.2 -> 29.8; FP32 64x64x256 33.5 -> 23.7, 128^3 48.1 -> 40.8,
 // 128x128x64 32.9 -> 32.1, but 128x128x32 26.5 -> 28.2.
@@ -2128,8 +2101,8 @@ struct PlaneLen {
   typedef PlaneGeom<real_t, RLX, RLY> G;
   // four threads per butterfly of the first X stage (up to 1024): the loads,
   // the separation and the stores spread over all of them, the butterflies
-  // over a quarter (64^3 FP64 fwd+bwd 22.4 -> 19.8 us against one thread
-  // per butterfly)
+  // over a quarter (64^3 FP64 r2c / c2r 6.8 / 6.4 us, 7.8 / 7.3 us with one
+  // thread per butterfly)
   static constexpr int NT0 = G::BX * G::NX / 8 * 4;
   static constexpr int NT = NT0 < 64 ? 64 : (NT0 > 1024 ? 1024 : (NT0 + 63) / 64 * 64);
   static void prep() {
@@ -2576,7 +2549,7 @@ GroupBatch* group_batch_create(int mode, int n, const int* shapes, real_t* const
         a.B = ct->BX;
         a.L = CtLenArg{L.d.n, L.d.twcount};
         a.tw = L.tw;
-        h.s.bytes = ct_lds((size_t)(ct->BX + 1) * len * sizeof(cplx_t), ct->twl_x, *ct, &a.tw_lds, &a.tw_off);
+        h.s.bytes = ct_lds((size_t)ct->x_bytes, ct->twl_x, *ct, &a.tw_lds, &a.tw_off);
       } else {
         ColArgs& a = h.s.ca;
         a.kind = COL_C2C;

@@ -125,6 +125,175 @@ struct RowRev {
   static __device__ __forceinline__ int at(int j) { return step<Rs...>(j, 0); }
 };
 
+// the inverse: the butterfly of the first stage that holds input row e < N/R0
+template <int R, int... Rest>
+struct RowInv {
+  static __device__ __forceinline__ int at(int e) {
+    if constexpr (sizeof...(Rest) == 0) return e;
+    else return e / RProd<Rest...>::value + R * RowInv<Rest...>::at(e % RProd<Rest...>::value);
+  }
+};
+
+// LDS tile of the X kernels: B row pairs, position p of pair b at
+// lds[at(p) + b].  The tile is reached by lanes along the pairs (middle
+// stages), along neighbouring positions (separation) and along neighbouring
+// blocks of the digit-reversed order (first stage): where a row of the tile is
+// at most half the banks wide, one element more every 4 positions and 3 more
+// every R0 R1 keep all three within twice the conflict-free cycles, else a
+// padded row and one element more every R0 R1.
+template <class T, int B, class RL>
+struct XLay;
+template <class T, int B, int R0, int R1, int... Rs>
+struct XLay<T, B, RList<R0, R1, Rs...>> {
+  static constexpr int N = RProd<R0, R1, Rs...>::value;
+  static constexpr bool HALF = B * sizeof(cpx<T>) <= 128;
+  static constexpr int BP = HALF ? B : B + 1, D = HALF ? 4 : N, S2 = HALF ? 3 : 1;
+  static_assert(!HALF || R0 % 4 == 0, "blocks of whole skews");
+  static __device__ __host__ constexpr int at(int p) { return p * BP + p / D + p / (R0 * R1) * S2; }
+  static constexpr long long BYTES = (long long)(at(N - 1) + B) * (long long)sizeof(cpx<T>);
+};
+
+// an in-place stage of the X tile (as stage_ip), decimation in time (the
+// twiddles before the butterfly) or in frequency (after it)
+template <class T, int R, bool FWD, bool DIF, class Lay, int B, int NT, int Ns, int Off>
+__device__ __forceinline__ void x_stage_ip(cpx<T>* lds, const typename TwT<T>::type* tw) {
+  constexpr int total = B * (Lay::N / R);
+  constexpr int IT = (total + NT - 1) / NT;
+#pragma unroll
+  for (int m = 0; m < IT; m++) {
+    const int it = threadIdx.x + m * NT;
+    if ((total % NT) == 0 || it < total) {
+      const int j = it / B, b = it % B;
+      const int k = j % Ns;
+      cpx<T>* p = lds + Lay::at((j - k) * R + k) + b;
+      cpx<T> v[R];
+#pragma unroll
+      for (int r = 0; r < R; r++) v[r] = p[Lay::at(r * Ns)];
+      const typename TwT<T>::type* w = tw + Off + k * (R - 1);
+      if constexpr (Ns > 1 && !DIF) {
+#pragma unroll
+        for (int r = 1; r < R; r++) v[r] = twmul<FWD>(v[r], w[r - 1]);
+      }
+      dft<R, FWD>(v);
+      if constexpr (Ns > 1 && DIF) {
+#pragma unroll
+        for (int r = 1; r < R; r++) v[r] = twmul<FWD>(v[r], w[r - 1]);
+      }
+#pragma unroll
+      for (int r = 0; r < R; r++) p[Lay::at(r * Ns)] = v[r];
+    }
+  }
+  __syncthreads();
+}
+
+// the stages after the first: upwards in time, downwards in frequency
+template <class T, bool FWD, bool DIF, class Lay, int B, int NT, int Ns, int Off, int R, int... Rest>
+__device__ __forceinline__ void x_stages_ip(cpx<T>* lds, const typename TwT<T>::type* tw) {
+  if constexpr (!DIF) x_stage_ip<T, R, FWD, DIF, Lay, B, NT, Ns, Off>(lds, tw);
+  if constexpr (sizeof...(Rest) > 0)
+    x_stages_ip<T, FWD, DIF, Lay, B, NT, Ns * R, Off + Ns * (R - 1), Rest...>(lds, tw);
+  if constexpr (DIF) x_stage_ip<T, R, FWD, DIF, Lay, B, NT, Ns, Off>(lds, tw);
+}
+
+// r2c: two real rows per complex sequence, ld(row, e) element e of a row of
+// the tile.  The first stage reads the rows itself, lanes along N/R0 elements,
+// where those are at least 32 bytes; shorter ones are read row by row into
+// the tile's digit-reversed order first.  The other stages run in place.
+template <class T, class Lay, int B, int NT, class Tw, class LD, int R0, int... Rs>
+__device__ __forceinline__ void x_fft_fwd(cpx<T>* lds, const Tw& ctw, LD ld, RList<R0, Rs...>) {
+  constexpr int N = Lay::N, nR = N / R0;
+  if constexpr (nR * sizeof(T) >= 32) {
+    constexpr int total = B * nR, IT = (total + NT - 1) / NT;
+    cpx<T> v[IT][R0];
+#pragma unroll
+    for (int m = 0; m < IT; m++) {
+      const int it = threadIdx.x + m * NT;
+      const bool ok = (total % NT) == 0 || it < total;
+      const int b = ok ? it / nR : 0, e = it % nR;
+#pragma unroll
+      for (int r = 0; r < R0; r++) {
+        v[m][r].x = ld(2 * b, e + r * nR);
+        v[m][r].y = ld(2 * b + 1, e + r * nR);
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < IT; m++) {
+      const int it = threadIdx.x + m * NT;
+      if ((total % NT) == 0 || it < total) {
+        const int b = it / nR, e = it % nR;
+        dft<R0, true>(v[m]);
+        cpx<T>* p = lds + Lay::at(RowInv<Rs...>::at(e) * R0) + b;
+#pragma unroll
+        for (int r = 0; r < R0; r++) p[Lay::at(r)] = v[m][r];
+      }
+    }
+    ctw.put();
+    __syncthreads();
+  } else {
+    constexpr int LI = (B * N + NT - 1) / NT;
+    cpx<T> v[LI];
+#pragma unroll
+    for (int i = 0; i < LI; i++) {
+      const int q = threadIdx.x + i * NT;
+      const bool ok = (B * N) % NT == 0 || q < B * N;
+      const int b = ok ? q / N : 0, e = q % N;
+      v[i].x = ld(2 * b, e);
+      v[i].y = ld(2 * b + 1, e);
+    }
+#pragma unroll
+    for (int i = 0; i < LI; i++) {
+      const int q = threadIdx.x + i * NT;
+      if ((B * N) % NT == 0 || q < B * N) {
+        const int e = q % N;
+        lds[Lay::at(RowInv<Rs...>::at(e % nR) * R0 + e / nR) + q / N] = v[i];
+      }
+    }
+    ctw.put();
+    __syncthreads();
+    x_stage_ip<T, R0, true, false, Lay, B, NT, 1, 0>(lds, ctw.table());
+  }
+  x_stages_ip<T, true, false, Lay, B, NT, R0, 0, Rs...>(lds, ctw.table());
+}
+
+// c2r, the mirror image: natural order in the tile, the stages downwards in
+// place, the first radix last; st(pair, e, z) stores element e of a pair's
+// rows.  From the last stage itself where N/R0 elements are at least 64 bytes:
+// below (FP32, 48 points) the short runs of the stores cost more than the
+// pass through the tile.
+template <class T, class Lay, int B, int NT, class ST, int R0, int... Rs>
+__device__ __forceinline__ void x_fft_bwd(cpx<T>* lds, const typename TwT<T>::type* tw, ST st, RList<R0, Rs...>) {
+  constexpr int N = Lay::N, nR = N / R0;
+  x_stages_ip<T, false, true, Lay, B, NT, R0, 0, Rs...>(lds, tw);
+  if constexpr (nR * sizeof(T) >= 64) {
+    constexpr int total = B * nR, IT = (total + NT - 1) / NT;
+#pragma unroll
+    for (int m = 0; m < IT; m++) {
+      const int it = threadIdx.x + m * NT;
+      if ((total % NT) == 0 || it < total) {
+        const int b = it / nR, e = it % nR;
+        const cpx<T>* p = lds + Lay::at(RowInv<Rs...>::at(e) * R0) + b;
+        cpx<T> v[R0];
+#pragma unroll
+        for (int r = 0; r < R0; r++) v[r] = p[Lay::at(r)];
+        dft<R0, false>(v);
+#pragma unroll
+        for (int r = 0; r < R0; r++) st(b, e + r * nR, v[r]);
+      }
+    }
+  } else {
+    x_stage_ip<T, R0, false, true, Lay, B, NT, 1, 0>(lds, tw);
+    constexpr int LI = (B * N + NT - 1) / NT;
+#pragma unroll
+    for (int i = 0; i < LI; i++) {
+      const int q = threadIdx.x + i * NT;
+      if ((B * N) % NT == 0 || q < B * N) {
+        const int e = q % N;
+        st(q / N, e, lds[Lay::at(RowInv<Rs...>::at(e % nR) * R0 + e / nR) + q / N]);
+      }
+    }
+  }
+}
+
 template <class T, bool FWD, int N, int B, int BP, int NT, int Ns, int Off, int R, int... Rest>
 __device__ __forceinline__ void stages_ct(cpx<T>* lds, const typename TwT<T>::type* tw) {
   stage_ct<T, R, FWD, N, B, BP, NT, Ns, Off>(lds, tw);
