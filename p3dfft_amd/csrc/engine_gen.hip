@@ -494,7 +494,7 @@ struct GXArgs {
   void* out;
   long long nrows, si_row, so_row;
   int nk;         // r2c: kept modes; c2r: valid input modes
-  int lB, lBL;    // log2 of the row pairs per tile, and of those side by side in a wave
+  int lB;         // log2 of the row pairs per tile
   FDiv dnk, dn0;  // divide by the modes, by n / R_0
   GenTile t;
   GenDesc L;
@@ -504,7 +504,12 @@ struct GXArgs {
 };
 
 // r2c: stage 0 reads the rows (lanes along the row), in-place stages, and the
-// two half spectra separated from the natural-order result as they are stored
+// two half spectra separated from the natural-order result as they are stored.
+// Bound by the latencies of a tile's serial phases and the run-time index
+// arithmetic.  Lanes along one row throughout: 16 lanes along each of 4 rows met
+// fewer LDS conflicts, but their short runs cost more on the memory side: FP64
+// 200x300x250 r2c / c2r 51 / 70 -> 46 / 49 us (5.0 TB/s), FP32 30 / 34 ->
+// 28 / 31 us.
 template <class T, bool TL, bool PM>
 __global__ __launch_bounds__(1024) void k_gx_r2c(GXArgs a) {
   typedef cpx<T> C;
@@ -520,8 +525,7 @@ __global__ __launch_bounds__(1024) void k_gx_r2c(GXArgs a) {
   with_radix(s0.R, [&](auto rc) {
     constexpr int R = decltype(rc)::value;
     for (int it = threadIdx.x; it < B * n0; it += NT) {
-      const int u = it >> a.lBL, bh = fdiv(u, a.dn0), e0 = u - bh * n0;
-      const int b = (it & ((1 << a.lBL) - 1)) + (bh << a.lBL);
+      const int b = fdiv(it, a.dn0), e0 = it - b * n0;
       const bool oka = 2 * b < nr, okb = 2 * b + 1 < nr;
       // rows past the last one read the tile's first row and are zeroed
       const char* pa = in + ((oka ? (unsigned)(2 * b) * si : 0u) + (unsigned)e0 * (unsigned)sizeof(T));
@@ -620,8 +624,7 @@ __global__ __launch_bounds__(1024) void k_gx_c2r(GXArgs a) {
   with_radix(s0.R, [&](auto rc) {
     constexpr int R = decltype(rc)::value;
     for (int it = threadIdx.x; it < B * n0; it += NT) {
-      const int u = it >> a.lBL, bh = fdiv(u, a.dn0), e0 = u - bh * n0;
-      const int b = (it & ((1 << a.lBL) - 1)) + (bh << a.lBL);
+      const int b = fdiv(it, a.dn0), e0 = it - b * n0;
       C v[R];
       const C* p = lds + gen_unrev(a.L, e0) * a.t.P0 + b;
 #pragma unroll
@@ -884,10 +887,14 @@ static size_t x_tile(GXArgs& a, const Len1D& L, long long nrows, long long row, 
   const long long pairs = (nrows + 1) / 2, E = sizeof(cplx_t);
   const int n = L.gd.n;
   int B = 16;
-  while (B > 1 && ((long long)n * (B + 1) * E > L.tile_bytes || (2LL * B + 1) * row * E >= (1LL << 32))) B /= 2;
+  // FP64 tiles of at most 40 KiB (four workgroups per CU in different phases;
+  // a prime stage wants the pairs): r2c / c2r 600x128x200 61 / 74 -> 48 / 50 us,
+  // 720x240x200 155 / 165 -> 139 / 130.  FP32 measured no gain (1500x64x100 28
+  // -> 29), its tiles hold twice the values per byte in flight.
+  const long long lim = sizeof(real_t) == 8 && !has_prime_stage(L) ? std::min(L.tile_bytes, 40 * 1024) : L.tile_bytes;
+  while (B > 1 && ((long long)n * (B + 1) * E > lim || (2LL * B + 1) * row * E >= (1LL << 32))) B /= 2;
   while (B > 2 && (pairs + B - 1) / B < 512) B /= 2;
   a.lB = log2i(B);
-  a.lBL = std::min(2, a.lB);
   a.t.BP = B > 1 ? B + 1 : 1;
   a.t.R0 = L.gd.radix[0];
   a.t.mR0 = magic(a.t.R0);
