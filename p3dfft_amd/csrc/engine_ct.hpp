@@ -1,12 +1,14 @@
-// engine_ct.hpp -- compile-time specialised Stockham engine.
+// engine_ct.hpp -- compile-time specialised engine.
 //
 // For the transform lengths the workloads use, the radix schedule, the tile
 // width and the thread count are template parameters, so every index
 // computation of a stage folds to shifts and constant multiplies and the
-// per-thread register arrays have fixed size.  The LDS tile holds B sequences
-// with element e of sequence b at lds[e*BP + b]; BP = B+1 pads each row so that
-// both the sequence-fastest accesses of the stages and the element-fastest
-// accesses of row loads avoid bank conflicts.  Stage twiddles use the same
+// per-thread register arrays have fixed size.  The LDS tile holds B sequences,
+// element e of sequence b at lds[e*B + b] (columns), in rotated rows (lds_at:
+// length-fastest columns) or in skewed ones (XLay: rows along X), each laid out
+// so that the accesses along the sequences and along the elements both avoid
+// bank conflicts.  The stages run in place wherever one side is addressed by
+// row, and so can be digit-reversed at no cost.  Stage twiddles use the same
 // table layout as the run-time engine (stage 0 has none; stage s holds
 // Ns*(R-1) entries W_{Ns R}^{k r}, k < Ns, r = 1..R-1).
 #pragma once

@@ -1,7 +1,7 @@
 // engine_gen.hip -- gfx950 kernels for transform lengths whose radix schedule
 // is a run-time value.
 //
-// A length n = R_0 R_1 ... R_{S-1} (radices up to 16, the composite ones as
+// A length n = R_0 R_1 ... R_{S-1} (radices up to 10, the composite ones as
 // prime-factor butterflies in registers) is run in place over an LDS tile of
 // B sequences.  Position p of the tile is written in mixed radix with R_0 the
 // fastest digit; stage s combines the R_s values a stride Ns = R_0 ... R_{s-1}
@@ -18,13 +18,17 @@
 // (or writes) global memory itself, one 128-byte row segment per value, and
 // the reversal is one division per butterfly.
 //
-// A prime radix above 16 runs as a stage over LDS by the symmetric pairs
+// A prime radix above 10 runs as a stage over LDS by the symmetric pairs
 // v_i +- v_{R-i} (half the multiplications of the direct sum), its outputs
 // held in registers across a barrier.
 //
 // What bounds the passes: with 128-byte row segments they move each byte once
-// per pass and run at 3-5 TB/s; the rest is the instruction issue of the
-// butterflies and the compensated twiddles.
+// per pass and run at 4-5.5 TB/s; the rest is the instruction issue of the
+// butterflies, the compensated twiddles and the run-time index arithmetic.
+// Against a tile loaded to LDS, autosort stages and a direct sum for every
+// prime: FP32 200x300x250 columns of 300 points 97 -> 30 us, of 250 102 -> 28,
+// X r2c of 200 54 -> 28; FP64 1000x100x90 columns of 100 points 85 -> 26 us, of
+// 90 100 -> 27, X r2c of 1000 80 -> 38.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -66,13 +70,11 @@ struct GenTile {
 
 template <class F>
 __device__ __forceinline__ void with_radix(int R, F f) {
-#define P3_CASE(N)                                                            \
-  case N:                                                                     \
-    if constexpr (N <= kGenMaxRadix) f(std::integral_constant<int, N>{});     \
-    break;
+#define P3_CASE(N) case N: f(std::integral_constant<int, N>{}); break;
+  static_assert(kGenMaxRadix == 10, "one case per radix");
   switch (R) {
     P3_CASE(1) P3_CASE(2) P3_CASE(3) P3_CASE(4) P3_CASE(5) P3_CASE(6) P3_CASE(7) P3_CASE(8)
-    P3_CASE(9) P3_CASE(10) P3_CASE(11) P3_CASE(12) P3_CASE(13) P3_CASE(14) P3_CASE(15) P3_CASE(16)
+    P3_CASE(9) P3_CASE(10)
     default: break;
   }
 #undef P3_CASE
@@ -111,7 +113,7 @@ __device__ __forceinline__ int gen_stride(const GenTile& t, const GenStage& st) 
   return gdiv(st.Ns, t.mR0, t.R0) * t.P0;
 }
 
-// a stage with a prime radix above 16: outputs by symmetric pairs
+// a stage with a prime radix above kGenMaxRadix: outputs by symmetric pairs
 constexpr int kPrimeItems = 8;
 template <class T, bool FWD, bool DIF>
 __device__ __forceinline__ void gen_prime(cpx<T>* lds, const GenDesc& L, const GenStage& st, const GenTile& t, int B,
@@ -651,8 +653,8 @@ __global__ __launch_bounds__(1024) void k_gx_c2r(GXArgs a) {
 // twiddles, addresses and LDS accesses per value, in units of one FP32
 // instruction: the schedule with the smallest sum is taken
 static double radix_cost(int r) {
-  static const double c[17] = {0, 0, 4, 12, 16, 34, 36, 66, 56, 90, 88, 160, 96, 220, 160, 162, 170};
-  return r <= 16 ? c[r] / r : 8.0 * r;
+  static const double c[kGenMaxRadix + 1] = {0, 0, 4, 12, 16, 34, 36, 66, 56, 90, 88};
+  return c[r] / r;
 }
 constexpr double kStageCost = 16;
 
@@ -739,8 +741,9 @@ static size_t place_twiddles(size_t data, const Len1D& L, int* tw_lds, int* tw_o
 
 // threads of a workgroup: the count that finishes most tiles per unit of
 // time, a butterfly of radix R counted as R + 3 and a CU as holding as many
-// workgroups as the LDS, 16 waves (128 registers per lane) and the number of
-// tiles allow
+// workgroups as the LDS, 16 waves (128 registers per lane; 24 in FP32, whose
+// kernels need 80, measured slower: 240-point columns of 320x240x160 24.0 ->
+// 26.1 us) and the number of tiles allow
 static int pick_threads(const Len1D& L, int B, size_t lds, long long tiles) {
   double best = -1;
   int bn = 64;

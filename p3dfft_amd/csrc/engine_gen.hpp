@@ -6,17 +6,16 @@
 
 namespace p3amd {
 
-// the radix schedule of a length: factors of at most 16 where the length has
-// such a form, a prime above 16 otherwise stands between two factors (1 if
-// there is none), since the first and the last stage hold a whole butterfly
-// in registers
+// the radix schedule of a length: factors of at most kGenMaxRadix where the
+// length has such a form, a larger prime otherwise stands between two factors
+// (1 if there is none), since the first and the last stage hold a whole
+// butterfly in registers
 std::vector<int> gen_factors(int n);
 // the same for factors in a given order (a plan-time candidate)
 std::vector<int> gen_wrap(const std::vector<int>& f);
-#ifndef P3_RM
-#define P3_RM 10
-#endif
-constexpr int kGenMaxRadix = P3_RM;
+// the largest radix held in registers: with radices up to 16 the kernels with
+// row maps need 544 to 880 bytes of scratch per lane, with 10 none
+constexpr int kGenMaxRadix = 10;
 inline bool gen_in_registers(int r) { return r <= kGenMaxRadix; }
 // a prime radix above that (the specialised schedules also hold 16)
 inline bool gen_is_prime_stage(int r) { return r > kGenMaxRadix && r % 2 == 1; }

@@ -1,10 +1,11 @@
 // fft_device.hpp -- device-side building blocks of the gfx950 FFT engine.
 //
 // Complex numbers are (re, im) pairs of float or double.  A transform of length
-// n = r_0 r_1 ... r_{S-1} is run as S Stockham autosort stages over data held
-// in LDS; each stage reads R values per butterfly into registers, applies the
-// stage twiddles, runs a length-R DFT in registers and writes the results to
-// their autosorted position.  Twiddles are FP64-generated tables; the FP32
+// n = r_0 r_1 ... r_{S-1} is run as S stages over data held in LDS; each stage
+// reads R values per butterfly into registers, applies the stage twiddles, runs
+// a length-R DFT in registers and writes the results in place (positions in
+// mixed radix, one side digit-reversed) or, where both sides are in natural
+// order, to their autosorted position.  Twiddles are FP64-generated tables; the FP32
 // engine stores each twiddle as a hi+lo pair of floats and multiplies with
 // both (compensated twiddle multiply).
 #pragma once
@@ -176,26 +177,13 @@ __device__ __forceinline__ void dft5(cpx<T>* v) {
   v[3] = sub(m2, n2);
 }
 
-// odd-prime DFTs by the pairwise (a_p +- a_{P-p}) form; tables hold
+// odd-prime DFT (of 7) by the pairwise (a_p +- a_{P-p}) form; tables hold
 // cos(2 pi j/P), sin(2 pi j/P) for j = 1..(P-1)/2.
 template <int P> struct PrimeTab;
 template <> struct PrimeTab<7> {
   static constexpr double c[4] = {1.0, 0.6234898018587336, -0.22252093395631434, -0.900968867902419};
   static constexpr double s[4] = {0.0, 0.7818314824680298, 0.9749279121818236, 0.43388373911755823};
 };
-template <> struct PrimeTab<11> {
-  static constexpr double c[6] = {1.0, 0.8412535328311812, 0.41541501300188644, -0.142314838273285,
-                                  -0.654860733945285, -0.9594929736144974};
-  static constexpr double s[6] = {0.0, 0.5406408174555976, 0.9096319953545183, 0.9898214418809328,
-                                  0.7557495743542583, 0.28173255684142967};
-};
-template <> struct PrimeTab<13> {
-  static constexpr double c[7] = {1.0, 0.8854560256532099, 0.5680647467311559, 0.120536680255323,
-                                  -0.35460488704253545, -0.7485107481711012, -0.970941817426052};
-  static constexpr double s[7] = {0.0, 0.4647231720437685, 0.8229838658936564, 0.992708874098054,
-                                  0.9350162426854148, 0.6631226582407952, 0.23931566428755768};
-};
-
 template <int P, bool FWD, class T>
 __device__ __forceinline__ void dftp(cpx<T>* v) {
   constexpr int H = (P - 1) / 2;
@@ -303,8 +291,6 @@ __device__ __forceinline__ void dft(cpx<T>* v) {
   else if constexpr (R == 9) dft9<FWD>(v);
   else if constexpr (R == 10) dft_pfa<2, 5, FWD>(v);
   else if constexpr (R == 12) dft_pfa<4, 3, FWD>(v);
-  else if constexpr (R == 14) dft_pfa<2, 7, FWD>(v);
-  else if constexpr (R == 15) dft_pfa<3, 5, FWD>(v);
   else if constexpr (R == 16) dft16<FWD>(v);
   else dftp<R, FWD>(v);
 }
