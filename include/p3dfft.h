@@ -307,6 +307,14 @@ void p3dfft_amd_set_plan_mode(int mode);
 int p3dfft_amd_plan_report(char *buf, int len);
 /* default plans again (no active setup and no live Poisson graph) */
 int p3dfft_amd_reset_plans(void);
+/* The launch shape the kernels with run-time radix schedules take for n <= 8192
+ * points (host only, no GPU call): form 0 columns read and written by rows, 1
+ * columns with a length-fastest (STRIDE1) side, 2 rows along X; count columns
+ * or rows.  tile_bytes and segment as a plan has them (defaults 65536, 128).
+ * Sequences per workgroup, threads (0: none can hold the tile) and LDS bytes
+ * (at most 163840 can be launched).  Returns 0, or -1 for another n. */
+int p3dfft_amd_run_time_tile(int n, int form, long long count, int tile_bytes, int segment, int *sequences,
+                             int *threads, size_t *lds);
 /* sizeof(p3dfft_real) of this build: 8 or 4. */
 int p3dfft_amd_precision(void);
 

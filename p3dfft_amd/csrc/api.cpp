@@ -1318,6 +1318,17 @@ int p3dfft_amd_reset_plans(void) {
   }
 }
 
+int p3dfft_amd_run_time_tile(int n, int form, long long count, int tile_bytes, int segment, int* sequences,
+                             int* threads, size_t* lds) {
+  try {
+    run_time_tile(n, form, count, tile_bytes, segment, sequences, threads, lds);
+    return 0;
+  } catch (const Error& e) {
+    set_error(e.msg);
+    return -1;
+  }
+}
+
 // Stream capture of the library's asynchronous (_dev) calls into a HIP
 // graph: every transform issues kernel launches only (kernel attributes are
 // set when a length is planned and the work buffers exist from setup), so a

@@ -1490,10 +1490,10 @@ static tw_t* gen_table(const std::vector<int2>& idx) {
 
 std::vector<int> default_factors(int n) { return has_ct_schedule(n) ? ct_factors(n) : gen_factors(n); }
 
-// stage descriptor of the radix schedule f and its FP64-generated twiddle
+// stage descriptor of the radix schedule f and the entries of its twiddle
 // table: stage s > 0 has W_{Ns R}^{k r}, k < Ns, r = 1..R-1, a prime stage of
 // the run-time kernels also W_R^j, j < R
-static LenDesc build_desc(int n, const std::vector<int>& f, tw_t** tw) {
+static LenDesc describe(int n, const std::vector<int>& f, std::vector<int2>& idx) {
   LenDesc d;
   std::memset(&d, 0, sizeof(d));
   d.n = n;
@@ -1501,7 +1501,6 @@ static LenDesc build_desc(int n, const std::vector<int>& f, tw_t** tw) {
   for (int r : f) prod *= r;
   if (prod != n) throw Error{"radix schedule does not multiply to the length", -1};
   if ((int)f.size() > kMaxStages) throw Error{"transform length has too many factors", -1};
-  std::vector<int2> idx;
   int ns = 1;
   for (size_t s = 0; s < f.size(); s++) {
     const int R = f[s];
@@ -1517,8 +1516,21 @@ static LenDesc build_desc(int n, const std::vector<int>& f, tw_t** tw) {
   }
   d.nst = (int)f.size();
   d.twcount = (int)idx.size();
+  return d;
+}
+
+// the same with the table on the device
+static LenDesc build_desc(int n, const std::vector<int>& f, tw_t** tw) {
+  std::vector<int2> idx;
+  const LenDesc d = describe(n, f, idx);
   *tw = gen_table(idx);
   return d;
+}
+
+void run_time_tile(int n, int form, long long count, int tile_bytes, int seg, int* seqs, int* threads, size_t* lds) {
+  if (n < 1 || n > max_len()) throw Error{"the run-time kernels take lengths up to " + std::to_string(max_len()), -1};
+  std::vector<int2> idx;
+  gen_tile_shape(describe(n, gen_factors(n), idx), form, count, tile_bytes, seg, seqs, threads, lds);
 }
 
 // plan of length n with the radix schedule f: the specialised kernels' (and

@@ -58,6 +58,9 @@ void set_len_plan(int n, const std::vector<int>& factors, bool ct_ok, int tile_b
 bool len_has_ct(int n);
 // "radix 8x8x8, specialised" / "radix 5x5x5x8, generic, tile 64 KiB, segment 128 B"
 std::string len_describe(int n);
+// launch shape of the run-time kernels' default schedule of a length, host only
+// (gen_tile_shape; throws where the length is out of their range)
+void run_time_tile(int n, int form, long long count, int tile_bytes, int seg, int* seqs, int* threads, size_t* lds);
 
 // Largest transform length the engine runs in one workgroup.
 int max_len();

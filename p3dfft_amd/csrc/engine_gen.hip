@@ -732,10 +732,10 @@ static int log2i(int x) {
 
 // LDS bytes of a tile of `data` bytes and its twiddle table, which joins the
 // tile where that leaves room for as many workgroups per CU or at least two
-static size_t place_twiddles(size_t data, const Len1D& L, int* tw_lds, int* tw_off) {
-  const size_t off = (data + 15) & ~(size_t)15, twb = (size_t)L.gd.twcount * sizeof(Tw);
+static size_t place_twiddles(size_t data, const LenDesc& d, int* tw_lds, int* tw_off) {
+  const size_t off = (data + 15) & ~(size_t)15, twb = (size_t)d.twcount * sizeof(Tw);
   *tw_off = (int)off;
-  *tw_lds = L.gd.twcount > 0 && (off + twb <= 80 * 1024 || (off > 80 * 1024 && off + twb <= kLdsMax)) ? 1 : 0;
+  *tw_lds = d.twcount > 0 && (off + twb <= 80 * 1024 || (off > 80 * 1024 && off + twb <= kLdsMax)) ? 1 : 0;
   return *tw_lds ? off + twb : off;
 }
 
@@ -743,18 +743,18 @@ static size_t place_twiddles(size_t data, const Len1D& L, int* tw_lds, int* tw_o
 // time, a butterfly of radix R counted as R + 3 and a CU as holding as many
 // workgroups as the LDS, 16 waves (128 registers per lane; 24 in FP32, whose
 // kernels need 80, measured slower: 240-point columns of 320x240x160 24.0 ->
-// 26.1 us) and the number of tiles allow
-static int pick_threads(const Len1D& L, int B, size_t lds, long long tiles) {
+// 26.1 us) and the number of tiles allow; 0 where no count holds the tile
+static int pick_threads(const LenDesc& d, int B, size_t lds, long long tiles) {
   double best = -1;
-  int bn = 64;
+  int bn = 0;
   for (int nt = 64; nt <= 1024; nt += 64) {
     long long wg = std::min<long long>((long long)(kLdsMax / std::max<size_t>(lds, 1)), 1024 / nt);
     wg = std::max<long long>(1, std::min<long long>(wg, (tiles + 255) / 256));
     double t = 0;
     bool ok = true;
-    for (int s = 0; s < L.gd.nst; s++) {
-      const int R = L.gd.radix[s];
-      const long long nb = (long long)B * (L.gd.n / R);
+    for (int s = 0; s < d.nst; s++) {
+      const int R = d.radix[s];
+      const long long nb = (long long)B * (d.n / R);
       if (gen_in_registers(R)) {
         t += (double)((nb + nt - 1) / nt) * (R + 3);
       } else {
@@ -767,14 +767,67 @@ static int pick_threads(const Len1D& L, int B, size_t lds, long long tiles) {
     const double rate = (double)wg / t;
     if (rate > best * 1.02) { best = rate; bn = nt; }
   }
-  if (best < 0) throw Error{"transform tile exceeds the 1024-thread workgroup capacity", -1};
   return bn;
 }
 
-static bool has_prime_stage(const Len1D& L) {
-  for (int s = 0; s < L.gd.nst; s++)
-    if (!gen_in_registers(L.gd.radix[s])) return true;
+static bool has_prime_stage(const LenDesc& d) {
+  for (int s = 0; s < d.nst; s++)
+    if (!gen_in_registers(d.radix[s])) return true;
   return false;
+}
+
+// the tile of a launch: sequences, threads, LDS bytes and the layout
+struct TileChoice {
+  int B, nt;
+  size_t bytes;
+  GenTile t;
+  int tw_lds, tw_off;
+};
+
+// column tile of m rows (d: the schedule, null: rows are copied): a 128-byte
+// row segment (plan-time measurement may choose another) while the tile stays
+// within the plan's bytes, segments of 64 bytes as long as the tile fits at
+// all; halved while there is not a tile for every CU
+static TileChoice col_tile(const LenDesc* d, int m, bool lf, long long ncol, int tile_bytes, int seg) {
+  const long long E = sizeof(cplx_t);
+  const int R0 = d ? d->radix[0] : 1;
+  // LDS bytes of a tile of b columns, sk elements between its blocks
+  auto data_of = [&](int b, int sk) {
+    const size_t x = (size_t)(((long long)m * (lf && b > 1 ? b + 1 : b) + (long long)(m / R0) * sk) * E);
+    return lf && d ? ((x + 15) & ~(size_t)15) + kColTab : x;
+  };
+  auto above_want = [&](int b) {
+    return ((long long)m * (lf && b > 1 ? b + 1 : b) + b) * E + 256 > (long long)tile_bytes + tile_bytes / 8;
+  };
+  int B = 1;
+  while (B * 2 * E <= seg) B *= 2;
+  while (B > 1 && ((above_want(B) && B * E > 64) || data_of(B, 0) > kLdsMax)) B /= 2;
+  // a prime stage holds its outputs in registers, kPrimeItems pairs a thread
+  while (B > 1 && d && has_prime_stage(*d) && (long long)B * m > 1024LL * (2 * kPrimeItems - 1)) B /= 2;
+  while (B * E > 32 && (ncol + B - 1) / B < 256) B /= 2;
+  // fewer columns than one LDS access covers: blocks an odd multiple of B
+  // apart, where the LDS has room for that.  Where it has not, the whole
+  // segment counts for more than the bank conflicts: without the skew against
+  // half the columns with it, FP64 2400 points x 4096 columns 79 / 73 us (4.0
+  // TB/s) against 107 / 94, 5000 x 2048 108 / 88 against 166 / 141; FP32 42 / 42
+  // against 51 / 52, 50 / 50 against 74 / 74
+  int skew = !lf && B * E < 128 && R0 % 2 == 0 ? B : 0;
+  if (data_of(B, skew) > kLdsMax) skew = 0;
+  const size_t data = data_of(B, skew);
+  TileChoice c;
+  c.B = B;
+  c.t.BP = lf && B > 1 ? B + 1 : B;
+  c.t.R0 = R0;
+  c.t.mR0 = magic(R0);
+  c.t.skew = skew;
+  c.t.P0 = R0 * c.t.BP + skew;
+  c.tw_lds = c.tw_off = c.nt = 0;
+  c.bytes = data;
+  if (d) {
+    c.bytes = place_twiddles(data, *d, &c.tw_lds, &c.tw_off);
+    c.nt = pick_threads(*d, B, c.bytes, (ncol + B - 1) / B);
+  }
+  return c;
 }
 
 // f(TL, PM): the twiddle table in LDS, the schedule with a prime stage
@@ -816,35 +869,18 @@ void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, hipStream_t st) {
   const bool lf = lf_in || lf_out;
   const int m = L ? L->gd.n : c.nld;
   const long long E = sizeof(cplx_t);
-  // columns per tile: a 128-byte row segment (plan-time measurement may choose
-  // another) while the tile stays within the plan's bytes, segments of 64
-  // bytes as long as the tile fits at all; halved while there is not a tile
-  // for every CU
-  const long long want = L ? L->tile_bytes : 64 * 1024;
-  int B = 1;
-  while (B * 2 * E <= (L ? L->col_seg : 128)) B *= 2;
-  auto bytes_of = [&](int b) { return ((long long)m * (lf && b > 1 ? b + 1 : b) + b) * E + 256; };
-  while (B > 1 && ((bytes_of(B) > want + want / 8 && B * E > 64) || bytes_of(B) > (long long)kLdsMax)) B /= 2;
-  // a prime stage holds its outputs in registers, kPrimeItems pairs a thread
-  while (B > 1 && L && has_prime_stage(*L) && (long long)B * m > 1024LL * (2 * kPrimeItems - 1)) B /= 2;
-  while (B * E > 32 && (ncol + B - 1) / B < 256) B /= 2;
+  const TileChoice tc =
+      L ? col_tile(&L->gd, m, lf, ncol, L->tile_bytes, L->col_seg) : col_tile(nullptr, m, lf, ncol, 64 * 1024, 128);
+  const int B = tc.B;
   a.lB = log2i(B);
-  const bool cross = lf && B > 1;
-  a.t.BP = cross ? B + 1 : B;
-  const int R0 = L ? L->gd.radix[0] : 1;
-  a.t.R0 = R0;
-  a.t.mR0 = magic(R0);
-  // fewer columns than one LDS access covers: blocks an odd multiple of B apart
-  a.t.skew = !lf && B * E < 128 && R0 % 2 == 0 ? B : 0;
-  a.t.P0 = R0 * a.t.BP + a.t.skew;
+  a.t = tc.t;
   const long long nwg = (ncol + B - 1) / B;
   if (nwg > 0x7fffffffLL) throw Error{"grid too large", -1};
-  size_t data = (size_t)((long long)m * a.t.BP + (long long)(m / R0) * a.t.skew) * E;
   if (!L) {
-    if (data > kLdsMax) throw Error{"column copy does not fit in LDS", -1};
+    if (tc.bytes > kLdsMax) throw Error{"column copy does not fit in LDS", -1};
     a.dld = make_fdiv(c.nld);
     a.dst = make_fdiv(c.nst);
-    k_gcopy<real_t><<<(unsigned)nwg, 256, data, st>>>(a);
+    k_gcopy<real_t><<<(unsigned)nwg, 256, tc.bytes, st>>>(a);
     check_hip(hipGetLastError(), "k_gcopy launch");
     return;
   }
@@ -852,11 +888,12 @@ void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, hipStream_t st) {
   a.tw = L->gtw;
   a.dld = make_fdiv(m);
   a.dst = make_fdiv(std::max(c.nst, 1));
-  if (lf) data = ((data + 15) & ~(size_t)15) + kColTab;
-  const size_t bytes = place_twiddles(data, *L, &a.tw_lds, &a.tw_off);
+  a.tw_lds = tc.tw_lds; a.tw_off = tc.tw_off;
+  const size_t bytes = tc.bytes;
   if (bytes > kLdsMax) throw Error{"column transform does not fit in LDS", -1};
-  const int nt = pick_threads(*L, B, bytes, nwg);
-  const bool pm = has_prime_stage(*L);
+  const int nt = tc.nt;
+  if (!nt) throw Error{"transform tile exceeds the 1024-thread workgroup capacity", -1};
+  const bool pm = has_prime_stage(L->gd);
   const bool fwd = c.fwd || c.kind == COL_DCT1 || c.kind == COL_DST1;
   const bool ld_id = c.nld == m && (c.ld_lo >= m || (c.ld_hi <= c.ld_lo && c.ld_shift == 0));
   const bool st_id = c.nst == m && (c.st_lo >= m || c.st_shift == 0);
@@ -885,33 +922,57 @@ void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, hipStream_t st) {
   check_hip(hipGetLastError(), "k_gcol launch");
 }
 
-// tile of the X kernels; returns the LDS bytes
-static size_t x_tile(GXArgs& a, const Len1D& L, long long nrows, long long row, int* nt, unsigned* nwg) {
+// tile of the X kernels, rows of at most `row` elements apart
+static TileChoice x_row_tile(const LenDesc& d, long long nrows, long long row, int tile_bytes) {
   const long long pairs = (nrows + 1) / 2, E = sizeof(cplx_t);
-  const int n = L.gd.n;
+  const int n = d.n;
   int B = 16;
   // FP64 tiles of at most 40 KiB (four workgroups per CU in different phases;
   // a prime stage wants the pairs): r2c / c2r 600x128x200 61 / 74 -> 48 / 50 us,
   // 720x240x200 155 / 165 -> 139 / 130.  FP32 measured no gain (1500x64x100 28
   // -> 29), its tiles hold twice the values per byte in flight.
-  const long long lim = sizeof(real_t) == 8 && !has_prime_stage(L) ? std::min(L.tile_bytes, 40 * 1024) : L.tile_bytes;
+  const long long lim = sizeof(real_t) == 8 && !has_prime_stage(d) ? std::min(tile_bytes, 40 * 1024) : tile_bytes;
   while (B > 1 && ((long long)n * (B + 1) * E > lim || (2LL * B + 1) * row * E >= (1LL << 32))) B /= 2;
   while (B > 2 && (pairs + B - 1) / B < 512) B /= 2;
-  a.lB = log2i(B);
-  a.t.BP = B > 1 ? B + 1 : 1;
-  a.t.R0 = L.gd.radix[0];
-  a.t.mR0 = magic(a.t.R0);
-  a.t.P0 = a.t.R0 * a.t.BP;
+  TileChoice c;
+  c.B = B;
+  c.t.BP = B > 1 ? B + 1 : 1;
+  c.t.R0 = d.radix[0];
+  c.t.mR0 = magic(c.t.R0);
+  c.t.skew = 0;
+  c.t.P0 = c.t.R0 * c.t.BP;
+  c.bytes = place_twiddles((size_t)n * c.t.BP * E, d, &c.tw_lds, &c.tw_off);
+  c.nt = pick_threads(d, B, c.bytes, (pairs + B - 1) / B);
+  return c;
+}
+
+// the same for a launch; returns the LDS bytes
+static size_t x_tile(GXArgs& a, const Len1D& L, long long nrows, long long row, int* nt, unsigned* nwg) {
+  const TileChoice c = x_row_tile(L.gd, nrows, row, L.tile_bytes);
+  a.lB = log2i(c.B);
+  a.t = c.t;
   a.L = make_desc(L);
   a.tw = L.gtw;
-  a.dn0 = make_fdiv(n / a.t.R0);
-  const size_t bytes = place_twiddles((size_t)n * a.t.BP * E, L, &a.tw_lds, &a.tw_off);
-  if (bytes > kLdsMax) throw Error{"X transform does not fit in LDS", -1};
-  const long long g = (pairs + B - 1) / B;
+  a.dn0 = make_fdiv(L.gd.n / c.t.R0);
+  a.tw_lds = c.tw_lds; a.tw_off = c.tw_off;
+  if (c.bytes > kLdsMax) throw Error{"X transform does not fit in LDS", -1};
+  if (!c.nt) throw Error{"transform tile exceeds the 1024-thread workgroup capacity", -1};
+  const long long g = ((nrows + 1) / 2 + c.B - 1) / c.B;
   if (g > 0x7fffffffLL) throw Error{"grid too large", -1};
   *nwg = (unsigned)g;
-  *nt = pick_threads(L, B, bytes, g);
-  return bytes;
+  *nt = c.nt;
+  return c.bytes;
+}
+
+// launch shape of a length (host only): form 0 rows on both sides, 1 a
+// length-fastest side, 2 rows along X
+void gen_tile_shape(const LenDesc& d, int form, long long count, int tile_bytes, int seg, int* seqs, int* threads,
+                    size_t* lds) {
+  const TileChoice c = form == 2 ? x_row_tile(d, count, d.n + 2, tile_bytes)
+                                 : col_tile(&d, d.n, form == 1, count, tile_bytes, seg);
+  *seqs = c.B;
+  *threads = c.nt;
+  *lds = c.bytes;
 }
 
 void gen_launch_x_r2c(const Len1D& L, const real_t* in, cplx_t* out, long long nrows, long long si_row,
@@ -924,7 +985,7 @@ void gen_launch_x_r2c(const Len1D& L, const real_t* in, cplx_t* out, long long n
   int nt;
   unsigned g;
   const size_t bytes = x_tile(a, L, nrows, std::max(si_row, so_row), &nt, &g);
-  with_variant(a.tw_lds != 0, has_prime_stage(L), [&](auto tl, auto pm) {
+  with_variant(a.tw_lds != 0, has_prime_stage(L.gd), [&](auto tl, auto pm) {
     k_gx_r2c<real_t, tl.value, pm.value><<<g, nt, bytes, st>>>(a);
   });
   check_hip(hipGetLastError(), "k_gx_r2c launch");
@@ -940,7 +1001,7 @@ void gen_launch_x_c2r(const Len1D& L, const cplx_t* in, real_t* out, long long n
   int nt;
   unsigned g;
   const size_t bytes = x_tile(a, L, nrows, std::max(si_row, so_row), &nt, &g);
-  with_variant(a.tw_lds != 0, has_prime_stage(L), [&](auto tl, auto pm) {
+  with_variant(a.tw_lds != 0, has_prime_stage(L.gd), [&](auto tl, auto pm) {
     k_gx_c2r<real_t, tl.value, pm.value><<<g, nt, bytes, st>>>(a);
   });
   check_hip(hipGetLastError(), "k_gx_c2r launch");

@@ -1,0 +1,42 @@
+"""Run-time-schedule column passes whose tile is near what a workgroup holds: the
+widest tile fills the LDS without room for the skew of its blocks, with enough
+columns for whole row segments, and the Chebyshev axis whose extension has such a
+length.  Against the FP64 oracle, tolerances as test_gpu_parity.py."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import TOL, cheby_tol, lib_setup, oplan, rel
+
+pytestmark = pytest.mark.gpu
+
+
+def check(precision, shape):
+    nx, ny, nz = shape
+    a = np.random.default_rng(ny + nz).standard_normal((nz, ny, nx))
+    o = oplan(nx, ny, nz)
+    ref = o.ftran_r2c(a, "fft")
+    with lib_setup(precision, nx, ny, nz) as P:
+        assert rel(P.ftran_r2c(a, "fft"), ref) < TOL[precision]
+        assert rel(P.btran_c2r(ref, "tff"), o.btran_c2r(ref, "tff")[0]) < TOL[precision]
+
+
+@pytest.mark.parametrize("precision", [8, 4])
+@pytest.mark.parametrize("n", [1714, 2400, 2500, 5000])
+def test_no_room_for_the_skew(precision, n):
+    check(precision, (2, n, 1056))  # 2112 columns
+
+
+@pytest.mark.parametrize("precision", [8, 4])
+def test_no_room_for_the_skew_few_columns(precision):
+    check(precision, (6, 4800, 3))
+    check(precision, (6, 3, 5000))
+
+
+@pytest.mark.parametrize("precision", [8, 4])
+def test_chebyshev_extension(precision):
+    """nz = 1251: the even extension has 2500 points"""
+    nx, ny, nz = 2, 1056, 1251
+    a = np.random.default_rng(5).standard_normal((nz, ny, nx))
+    ref = oplan(nx, ny, nz).cheby(a, 2.0)
+    with lib_setup(precision, nx, ny, nz) as P:
+        assert rel(P.cheby(a, 2.0), ref) < cheby_tol(precision, nz, 2.0)

@@ -1,0 +1,39 @@
+"""CPU: the launch shapes of the run-time-schedule kernels.  Every length a
+workgroup takes has one that the hardware holds, whatever the view: rows on both
+sides, a length-fastest side, rows along X; one column, few and very many."""
+import ctypes
+
+import pytest
+
+import p3dfft_amd
+
+LDS = 160 * 1024
+MAX_LEN = 8192
+COUNTS = (1, 700, 3000, 100000)
+
+
+def shapes(precision, form, tile, seg):
+    L = p3dfft_amd.load(precision)
+    s, t, b = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
+    for n in range(1, MAX_LEN + 1):
+        for c in COUNTS:
+            assert L.p3dfft_amd_run_time_tile(n, form, c, tile, seg, ctypes.byref(s), ctypes.byref(t),
+                                              ctypes.byref(b)) == 0
+            yield n, c, s.value, t.value, b.value
+
+
+@pytest.mark.parametrize("precision", [8, 4])
+@pytest.mark.parametrize("tile,seg", [(65536, 128), (32768, 64), (131072, 256)])
+@pytest.mark.parametrize("form", [0, 1, 2])
+def test_every_length_fits_the_lds(precision, form, tile, seg):
+    bad = [(n, c, b) for n, c, s, t, b in shapes(precision, form, tile, seg) if b > LDS or s < 1]
+    assert not bad, (len(bad), bad[:10])
+
+
+@pytest.mark.parametrize("precision", [8, 4])
+def test_other_lengths_are_refused(precision):
+    L = p3dfft_amd.load(precision)
+    s, t, b = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
+    for n in (0, MAX_LEN + 1):
+        assert L.p3dfft_amd_run_time_tile(n, 0, 1, 65536, 128, ctypes.byref(s), ctypes.byref(t), ctypes.byref(b)) == -1
+    L.p3dfft_amd_clear_error()
