@@ -739,6 +739,18 @@ static size_t place_twiddles(size_t data, const LenDesc& d, int* tw_lds, int* tw
   return *tw_lds ? off + twb : off;
 }
 
+// (butterfly, pair) items of a prime stage of B sequences, whose outputs a
+// workgroup holds in registers, kPrimeItems a thread
+static long long prime_items(const LenDesc& d, int s, int B) {
+  const int R = d.radix[s];
+  return (long long)B * (d.n / R) * ((R + 1) / 2);
+}
+static bool prime_stages_fit(const LenDesc& d, int B) {
+  for (int s = 0; s < d.nst; s++)
+    if (!gen_in_registers(d.radix[s]) && prime_items(d, s, B) > 1024LL * kPrimeItems) return false;
+  return true;
+}
+
 // threads of a workgroup: the count that finishes most tiles per unit of
 // time, a butterfly of radix R counted as R + 3 and a CU as holding as many
 // workgroups as the LDS, 16 waves (128 registers per lane; 24 in FP32, whose
@@ -758,7 +770,7 @@ static int pick_threads(const LenDesc& d, int B, size_t lds, long long tiles) {
       if (gen_in_registers(R)) {
         t += (double)((nb + nt - 1) / nt) * (R + 3);
       } else {
-        const long long items = nb * ((R + 1) / 2);
+        const long long items = prime_items(d, s, B);
         if (items > (long long)nt * kPrimeItems) ok = false;
         t += (double)((items + nt - 1) / nt) * 2 * R;
       }
@@ -802,8 +814,7 @@ static TileChoice col_tile(const LenDesc* d, int m, bool lf, long long ncol, int
   int B = 1;
   while (B * 2 * E <= seg) B *= 2;
   while (B > 1 && ((above_want(B) && B * E > 64) || data_of(B, 0) > kLdsMax)) B /= 2;
-  // a prime stage holds its outputs in registers, kPrimeItems pairs a thread
-  while (B > 1 && d && has_prime_stage(*d) && (long long)B * m > 1024LL * (2 * kPrimeItems - 1)) B /= 2;
+  while (B > 1 && d && !prime_stages_fit(*d, B)) B /= 2;
   while (B * E > 32 && (ncol + B - 1) / B < 256) B /= 2;
   // fewer columns than one LDS access covers: blocks an odd multiple of B
   // apart, where the LDS has room for that.  Where it has not, the whole
@@ -933,6 +944,7 @@ static TileChoice x_row_tile(const LenDesc& d, long long nrows, long long row, i
   // -> 29), its tiles hold twice the values per byte in flight.
   const long long lim = sizeof(real_t) == 8 && !has_prime_stage(d) ? std::min(tile_bytes, 40 * 1024) : tile_bytes;
   while (B > 1 && ((long long)n * (B + 1) * E > lim || (2LL * B + 1) * row * E >= (1LL << 32))) B /= 2;
+  while (B > 1 && !prime_stages_fit(d, B)) B /= 2;
   while (B > 2 && (pairs + B - 1) / B < 512) B /= 2;
   TileChoice c;
   c.B = B;

@@ -1,7 +1,7 @@
 """Run-time-schedule column passes whose tile is near what a workgroup holds: the
-widest tile fills the LDS without room for the skew of its blocks, with enough
-columns for whole row segments, and the Chebyshev axis whose extension has such a
-length.  Against the FP64 oracle, tolerances as test_gpu_parity.py."""
+widest tile fills the LDS without room for the skew of its blocks, or a prime
+stage fills the registers, with enough columns for whole row segments, and the
+Chebyshev axis whose extension has such a length.  Against the FP64 oracle, tolerances as test_gpu_parity.py."""
 import numpy as np
 import pytest
 
@@ -24,6 +24,13 @@ def check(precision, shape):
 @pytest.mark.parametrize("n", [1714, 2400, 2500, 5000])
 def test_no_room_for_the_skew(precision, n):
     check(precision, (2, n, 1056))  # 2112 columns
+
+
+@pytest.mark.parametrize("shape", [(2, 1881, 1056), (2, 1911, 1056), (6, 3762, 3), (6, 3, 3773), (2, 1, 7513)])
+def test_prime_stage_registers(shape):
+    """Prime stages of 11 and 13 just above what the threads of a workgroup hold
+    at the widest tile of FP32"""
+    check(4, shape)
 
 
 @pytest.mark.parametrize("precision", [8, 4])

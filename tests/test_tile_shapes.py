@@ -31,6 +31,15 @@ def test_every_length_fits_the_lds(precision, form, tile, seg):
 
 
 @pytest.mark.parametrize("precision", [8, 4])
+@pytest.mark.parametrize("tile,seg", [(65536, 128), (131072, 256)])
+@pytest.mark.parametrize("form", [0, 1, 2])
+def test_every_length_has_threads(precision, form, tile, seg):
+    """A prime stage holds its outputs in the registers of at most 1024 threads."""
+    bad = [(n, c, s) for n, c, s, t, b in shapes(precision, form, tile, seg) if not (0 < t <= 1024 and t % 64 == 0)]
+    assert not bad, (len(bad), bad[:10])
+
+
+@pytest.mark.parametrize("precision", [8, 4])
 def test_other_lengths_are_refused(precision):
     L = p3dfft_amd.load(precision)
     s, t, b = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
