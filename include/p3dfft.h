@@ -260,7 +260,7 @@ void p3dfft_amd_set_specialised(int on);
  * orders, so each pass starts on data the previous one wrote last (still in
  * the last-level cache); 0: every pass walks forward. Results are identical. */
 void p3dfft_amd_set_tile_order(int alternate);
-/* 1: the specialised column kernels use 64-bit element offsets even where
+/* 1: the column kernels use 64-bit element offsets even where
  * 32-bit ones fit (default 0; views over 4 GiB always use 64-bit offsets). */
 void p3dfft_amd_set_wide_offsets(int on);
 /* Tile order of the column passes over one contiguous inner axis (the Z
@@ -311,10 +311,11 @@ int p3dfft_amd_reset_plans(void);
  * points (host only, no GPU call): form 0 columns read and written by rows, 1
  * columns with a length-fastest (STRIDE1) side, 2 rows along X; count columns
  * or rows.  tile_bytes and segment as a plan has them (defaults 65536, 128).
- * Sequences per workgroup, threads (0: none can hold the tile) and LDS bytes
- * (at most 163840 can be launched).  Returns 0, or -1 for another n. */
+ * Sequences per workgroup, threads (0: none can hold the tile), LDS bytes
+ * (at most 163840 can be launched) and the bytes of an element offset (form 0:
+ * of `count` contiguous columns).  Returns 0, or -1 for another n. */
 int p3dfft_amd_run_time_tile(int n, int form, long long count, int tile_bytes, int segment, int *sequences,
-                             int *threads, size_t *lds);
+                             int *threads, size_t *lds, int *offset_bytes);
 /* sizeof(p3dfft_real) of this build: 8 or 4. */
 int p3dfft_amd_precision(void);
 

@@ -95,7 +95,7 @@ def load(precision=8):
     L.p3dfft_amd_set_x_into_out.argtypes = [ctypes.c_int]
     L.p3dfft_amd_set_plan_mode.argtypes = [ctypes.c_int]
     L.p3dfft_amd_run_time_tile.argtypes = [ctypes.c_int, ctypes.c_int, _ll, ctypes.c_int, ctypes.c_int, _ip, _ip,
-                                           ctypes.POINTER(ctypes.c_size_t)]
+                                           ctypes.POINTER(ctypes.c_size_t), _ip]
     L.p3dfft_amd_run_time_tile.restype = ctypes.c_int
     L.p3dfft_amd_batch_create.argtypes = [ctypes.c_int, ctypes.c_int, _vp, _vp, _vp, ctypes.POINTER(_vp)]
     L.p3dfft_amd_batch_create.restype = ctypes.c_int

@@ -1319,9 +1319,9 @@ int p3dfft_amd_reset_plans(void) {
 }
 
 int p3dfft_amd_run_time_tile(int n, int form, long long count, int tile_bytes, int segment, int* sequences,
-                             int* threads, size_t* lds) {
+                             int* threads, size_t* lds, int* offset_bytes) {
   try {
-    run_time_tile(n, form, count, tile_bytes, segment, sequences, threads, lds);
+    run_time_tile(n, form, count, tile_bytes, segment, sequences, threads, lds, offset_bytes);
     return 0;
   } catch (const Error& e) {
     set_error(e.msg);

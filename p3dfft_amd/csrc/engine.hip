@@ -1471,6 +1471,7 @@ static std::map<int, Len1D> g_lens;
 static std::vector<tw_t*> g_retired_tw;
 static void prep_kernels(const Len1D& L);
 static bool has_ct_schedule(int n);
+static bool g_wide_offsets = false;
 
 // the device table of the twiddles exp(-2 pi i x / y), one per entry
 static tw_t* gen_table(const std::vector<int2>& idx) {
@@ -1527,10 +1528,12 @@ static LenDesc build_desc(int n, const std::vector<int>& f, tw_t** tw) {
   return d;
 }
 
-void run_time_tile(int n, int form, long long count, int tile_bytes, int seg, int* seqs, int* threads, size_t* lds) {
+void run_time_tile(int n, int form, long long count, int tile_bytes, int seg, int* seqs, int* threads, size_t* lds,
+                   int* offset_bytes) {
   if (n < 1 || n > max_len()) throw Error{"the run-time kernels take lengths up to " + std::to_string(max_len()), -1};
   std::vector<int2> idx;
-  gen_tile_shape(describe(n, gen_factors(n), idx), form, count, tile_bytes, seg, seqs, threads, lds);
+  gen_tile_shape(describe(n, gen_factors(n), idx), form, count, tile_bytes, seg, g_wide_offsets, seqs, threads, lds,
+                 offset_bytes);
 }
 
 // plan of length n with the radix schedule f: the specialised kernels' (and
@@ -1933,7 +1936,6 @@ static void prep_kernels(const Len1D& L) {
 static bool g_use_ct = true;
 static bool g_alt_order = true;
 static int g_flat_order = 2;  // 0 XCD-aware, 1 dispatch order, 2 by shape
-static bool g_wide_offsets = false;
 static bool g_dct_direct = true;
 void set_dct_direct(bool on) { g_dct_direct = on; }
 void set_wide_offsets(bool on) { g_wide_offsets = on; }
@@ -2417,7 +2419,7 @@ bool launch_col(const ColSpec& c, hipStream_t st) {
     check_hip(hipGetLastError(), "k_col_ct launch");
     return a.cheby != 0;
   }
-  gen_launch_col(L, c, a.xcd, st);
+  gen_launch_col(L, c, a.xcd, g_wide_offsets, st);
   return false;
 }
 

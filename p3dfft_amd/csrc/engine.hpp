@@ -60,7 +60,8 @@ bool len_has_ct(int n);
 std::string len_describe(int n);
 // launch shape of the run-time kernels' default schedule of a length, host only
 // (gen_tile_shape; throws where the length is out of their range)
-void run_time_tile(int n, int form, long long count, int tile_bytes, int seg, int* seqs, int* threads, size_t* lds);
+void run_time_tile(int n, int form, long long count, int tile_bytes, int seg, int* seqs, int* threads, size_t* lds,
+                   int* offset_bytes);
 
 // Largest transform length the engine runs in one workgroup.
 int max_len();

@@ -315,7 +315,10 @@ __device__ __forceinline__ cpx<T> gen_out(const GColArgs& a, cpx<T> v) {
 
 // MAP: pruned rows, DCT-I / DST-I extensions.  LF: 0 rows on both sides, 1 the
 // input is length-fastest (decimation in frequency), 2 the output is.  Off: the
-// type of the byte offsets from the tile's first column.
+// type of the byte offsets from the tile's first column.  Rows without maps have
+// a form of either width, so that a view of 4 GiB gives the bits of a smaller one
+// (the form with maps contracts its products differently) and is not slowed by
+// the maps' arithmetic.
 template <class T, bool FWD, bool MAP, int LF, class Off, bool TL, bool PM>
 __global__ __launch_bounds__(1024) void k_gcol(GColArgs a) {
   typedef cpx<T> C;
@@ -841,6 +844,16 @@ static TileChoice col_tile(const LenDesc* d, int m, bool lf, long long ncol, int
   return c;
 }
 
+// the byte offsets of a tile of B columns from its first column stay below 2^32
+static bool offsets_fit(const ColSpec& c, int B) {
+  const long long nout = B / std::max(c.n_inner, 1) + 2;
+  auto fits = [&](long long si, long long sl, long long so) {
+    return (nout * so + (long long)c.n_inner * si + (long long)(std::max(c.nld, c.nst) + 1) * sl) *
+               (long long)sizeof(cplx_t) < (1LL << 32);
+  };
+  return fits(c.si_in, c.sl_in, c.so_in) && fits(c.si_out, c.sl_out, c.so_out);
+}
+
 // f(TL, PM): the twiddle table in LDS, the schedule with a prime stage
 template <class F>
 static void with_variant(bool tl, bool pm, F f) {
@@ -860,7 +873,7 @@ static void go_col(const GColArgs& a, bool pm, unsigned g, int nt, size_t bytes,
   });
 }
 
-void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, hipStream_t st) {
+void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, bool wide, hipStream_t st) {
   const long long ncol = (long long)c.n_inner * c.n_outer;
   if (ncol > 0x7fffffffLL) throw Error{"grid too large", -1};
   GColArgs a;
@@ -879,7 +892,6 @@ void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, hipStream_t st) {
   const bool lf_in = c.sl_in == 1 && c.si_in != 1, lf_out = c.sl_out == 1 && c.si_out != 1;
   const bool lf = lf_in || lf_out;
   const int m = L ? L->gd.n : c.nld;
-  const long long E = sizeof(cplx_t);
   const TileChoice tc =
       L ? col_tile(&L->gd, m, lf, ncol, L->tile_bytes, L->col_seg) : col_tile(nullptr, m, lf, ncol, 64 * 1024, 128);
   const int B = tc.B;
@@ -909,24 +921,22 @@ void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, hipStream_t st) {
   const bool ld_id = c.nld == m && (c.ld_lo >= m || (c.ld_hi <= c.ld_lo && c.ld_shift == 0));
   const bool st_id = c.nst == m && (c.st_lo >= m || c.st_shift == 0);
   const bool map = c.kind != COL_C2C || !(ld_id && st_id);
-  const long long nout = B / std::max(c.n_inner, 1) + 2;
-  auto span = [&](long long si, long long sl, long long so) {
-    return (nout * so + (long long)c.n_inner * si + (long long)(std::max(c.nld, c.nst) + 1) * sl) * E;
-  };
-  const bool fits = span(c.si_in, c.sl_in, c.so_in) < (1LL << 32) && span(c.si_out, c.sl_out, c.so_out) < (1LL << 32);
+  const bool fits = !wide && offsets_fit(c, B);
   typedef unsigned U32;
   typedef unsigned long long U64;
   const unsigned g = (unsigned)nwg;
   if (fwd) {
     if (lf_in) go_col<true, true, 1, U64>(a, pm, g, nt, bytes, st);
     else if (lf_out) go_col<true, true, 2, U64>(a, pm, g, nt, bytes, st);
-    else if (!fits) go_col<true, true, 0, U64>(a, pm, g, nt, bytes, st);
+    else if (!fits && map) go_col<true, true, 0, U64>(a, pm, g, nt, bytes, st);
+    else if (!fits) go_col<true, false, 0, U64>(a, pm, g, nt, bytes, st);
     else if (map) go_col<true, true, 0, U32>(a, pm, g, nt, bytes, st);
     else go_col<true, false, 0, U32>(a, pm, g, nt, bytes, st);
   } else {
     if (lf_in) go_col<false, true, 1, U64>(a, pm, g, nt, bytes, st);
     else if (lf_out) go_col<false, true, 2, U64>(a, pm, g, nt, bytes, st);
-    else if (!fits) go_col<false, true, 0, U64>(a, pm, g, nt, bytes, st);
+    else if (!fits && map) go_col<false, true, 0, U64>(a, pm, g, nt, bytes, st);
+    else if (!fits) go_col<false, false, 0, U64>(a, pm, g, nt, bytes, st);
     else if (map) go_col<false, true, 0, U32>(a, pm, g, nt, bytes, st);
     else go_col<false, false, 0, U32>(a, pm, g, nt, bytes, st);
   }
@@ -978,13 +988,20 @@ static size_t x_tile(GXArgs& a, const Len1D& L, long long nrows, long long row, 
 
 // launch shape of a length (host only): form 0 rows on both sides, 1 a
 // length-fastest side, 2 rows along X
-void gen_tile_shape(const LenDesc& d, int form, long long count, int tile_bytes, int seg, int* seqs, int* threads,
-                    size_t* lds) {
+void gen_tile_shape(const LenDesc& d, int form, long long count, int tile_bytes, int seg, bool wide, int* seqs,
+                    int* threads, size_t* lds, int* offset_bytes) {
   const TileChoice c = form == 2 ? x_row_tile(d, count, d.n + 2, tile_bytes)
                                  : col_tile(&d, d.n, form == 1, count, tile_bytes, seg);
   *seqs = c.B;
   *threads = c.nt;
   *lds = c.bytes;
+  ColSpec v{};
+  v.n_inner = (int)std::min<long long>(count, 0x7fffffff);
+  v.n_outer = 1;
+  v.si_in = v.si_out = 1;
+  v.sl_in = v.sl_out = count;
+  v.nld = v.nst = d.n;
+  *offset_bytes = form == 2 || (form == 0 && !wide && offsets_fit(v, c.B)) ? 4 : 8;
 }
 
 void gen_launch_x_r2c(const Len1D& L, const real_t* in, cplx_t* out, long long nrows, long long si_row,
@@ -1030,6 +1047,7 @@ static void prep_dir() {
   typedef unsigned long long U64;
   allow_big_lds(k_gcol<real_t, FWD, false, 0, U32, TL, PM>);
   allow_big_lds(k_gcol<real_t, FWD, true, 0, U32, TL, PM>);
+  allow_big_lds(k_gcol<real_t, FWD, false, 0, U64, TL, PM>);
   allow_big_lds(k_gcol<real_t, FWD, true, 0, U64, TL, PM>);
   allow_big_lds(k_gcol<real_t, FWD, true, 1, U64, TL, PM>);
   allow_big_lds(k_gcol<real_t, FWD, true, 2, U64, TL, PM>);

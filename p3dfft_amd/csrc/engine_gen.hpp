@@ -25,13 +25,15 @@ void gen_launch_x_r2c(const Len1D& L, const real_t* in, cplx_t* out, long long n
                       long long so_row, int nxo, bool rev, hipStream_t st);
 void gen_launch_x_c2r(const Len1D& L, const cplx_t* in, real_t* out, long long nrows, long long si_row,
                       long long so_row, int nxi, bool rev, hipStream_t st);
-// L: the plan of the transform length (null: COL_COPY)
-void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, hipStream_t st);
+// L: the plan of the transform length (null: COL_COPY); wide: 64-bit offsets
+// even where 32-bit ones fit
+void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, bool wide, hipStream_t st);
 // the launch shape of a schedule (host only): sequences per tile, threads (0:
 // no count holds the tile) and LDS bytes of `count` columns (form 0 rows on both
-// sides, 1 a length-fastest side) or rows along X (form 2)
-void gen_tile_shape(const LenDesc& d, int form, long long count, int tile_bytes, int seg, int* seqs, int* threads,
-                    size_t* lds);
+// sides, 1 a length-fastest side) or rows along X (form 2), and the width of the
+// offsets into such contiguous columns or rows
+void gen_tile_shape(const LenDesc& d, int form, long long count, int tile_bytes, int seg, bool wide, int* seqs,
+                    int* threads, size_t* lds, int* offset_bytes);
 // raise the kernels' dynamic-LDS limits (once, when a length is planned)
 void gen_prep_kernels();
 

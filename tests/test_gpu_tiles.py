@@ -47,3 +47,25 @@ def test_chebyshev_extension(precision):
     ref = oplan(nx, ny, nz).cheby(a, 2.0)
     with lib_setup(precision, nx, ny, nz) as P:
         assert rel(P.cheby(a, 2.0), ref) < cheby_tol(precision, nz, 2.0)
+
+
+@pytest.mark.parametrize("precision", [8, 4])
+@pytest.mark.parametrize("shape,cut", [((30, 50, 21), (None, None, None)), ((30, 50, 21), (20, 30, 15)),
+                                       ((22, 77, 100), (None, 50, 64))])
+def test_wide_offsets_with_maps(precision, shape, cut):
+    """The 64-bit-offset form of the row-addressed kernel against the 32-bit
+    one: plain rows, pruned rows, DCT-I and DST-I extensions.  Identical bits."""
+    nx, ny, nz = shape
+    a = np.random.default_rng(nz).standard_normal((nz, ny, nx))
+    res = []
+    for wide in (0, 1):
+        with lib_setup(precision, nx, ny, nz, *cut, ow=False) as P:
+            P.lib.p3dfft_amd_set_wide_offsets(wide)
+            try:
+                for z in "tcs":
+                    s = P.ftran_r2c(a, "ff" + z)
+                    res.append((s, P.btran_c2r(s, z + "ff")))
+            finally:
+                P.lib.p3dfft_amd_set_wide_offsets(0)
+    for (s0, b0), (s1, b1) in zip(res[:3], res[3:]):
+        assert np.array_equal(s0, s1) and np.array_equal(b0, b1)

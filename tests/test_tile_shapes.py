@@ -14,11 +14,11 @@ COUNTS = (1, 700, 3000, 100000)
 
 def shapes(precision, form, tile, seg):
     L = p3dfft_amd.load(precision)
-    s, t, b = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
+    s, t, b, o = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t(), ctypes.c_int()
     for n in range(1, MAX_LEN + 1):
         for c in COUNTS:
             assert L.p3dfft_amd_run_time_tile(n, form, c, tile, seg, ctypes.byref(s), ctypes.byref(t),
-                                              ctypes.byref(b)) == 0
+                                              ctypes.byref(b), ctypes.byref(o)) == 0
             yield n, c, s.value, t.value, b.value
 
 
@@ -40,9 +40,30 @@ def test_every_length_has_threads(precision, form, tile, seg):
 
 
 @pytest.mark.parametrize("precision", [8, 4])
+def test_wide_offsets_reach_the_run_time_kernels(precision):
+    """64-bit offsets above 4 GiB, and everywhere under the switch that the tests
+    of that form use."""
+    L = p3dfft_amd.load(precision)
+    s, t, b, o = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t(), ctypes.c_int()
+
+    def width(n, count):
+        assert L.p3dfft_amd_run_time_tile(n, 0, count, 65536, 128, ctypes.byref(s), ctypes.byref(t), ctypes.byref(b),
+                                          ctypes.byref(o)) == 0
+        return o.value
+    try:
+        assert width(300, 1000) == 4
+        assert width(1000, 1000 * 1000) == 8
+        L.p3dfft_amd_set_wide_offsets(1)
+        assert width(300, 1000) == 8
+    finally:
+        L.p3dfft_amd_set_wide_offsets(0)
+
+
+@pytest.mark.parametrize("precision", [8, 4])
 def test_other_lengths_are_refused(precision):
     L = p3dfft_amd.load(precision)
-    s, t, b = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
+    s, t, b, o = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t(), ctypes.c_int()
     for n in (0, MAX_LEN + 1):
-        assert L.p3dfft_amd_run_time_tile(n, 0, 1, 65536, 128, ctypes.byref(s), ctypes.byref(t), ctypes.byref(b)) == -1
+        assert L.p3dfft_amd_run_time_tile(n, 0, 1, 65536, 128, ctypes.byref(s), ctypes.byref(t), ctypes.byref(b),
+                                          ctypes.byref(o)) == -1
     L.p3dfft_amd_clear_error()
