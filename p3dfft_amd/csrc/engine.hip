@@ -1447,12 +1447,15 @@ static std::vector<int> ct_factors(int n) {
   if (n == 2048) return {16, 16, 8};
   // one stage fewer through a composite radix (X and column passes of 2^25
   // points, us): 48 FP32 X 12.8 / 12.4 -> 12.2 / 11.5, 96 FP64 X 33.5 / 33.7 ->
-  // 32.9 / 33.3, 384 FP32 X 23.9 / 24.0 -> 23.1 / 23.3, FP64 Y 37.7 -> 36.5;
+  // 32.9 / 33.3; the six passes of 384^3 FP32 498 -> 475, FP64 1050 -> 990 (with
+  // the in-place tiles; 8 8 6 takes 473 and 1022, but its second radix 8 scales an
+  // FP32 round trip by another -8e-9 per axis: 384^3 2.4e-7 -> 2.5e-7 from 64
+  // bits, 4 8 12 2.3e-7);
   // the like for 160 (16 10), 192 (12 16), 128 (16 8), 320 (16 5 4) and 1024
   // (16 8 8) gains in one precision what it loses in the other
   if (n == 48) return {8, 6};
   if (n == 96) return {8, 12};
-  if (n == 384) return {8, 8, 6};
+  if (n == 384) return {4, 8, 12};
   std::vector<int> f;
   int m = n, a = 0;
   while (m % 2 == 0) { m /= 2; a++; }
@@ -1885,7 +1888,7 @@ static const std::map<int, CtInfo>& ct_table() {
       {32, CtLen<8, 4>::info()},       {48, CtLen<8, 6>::info()},    {64, CtLen<8, 8>::info()},
       {96, CtLen<8, 12>::info()},    {128, CtLen<8, 4, 4>::info()},   {160, CtLen<8, 4, 5>::info()},
       {192, CtLen<8, 8, 3>::info()},   {256, CtLen<8, 8, 4>::info()},   {320, CtLen<8, 8, 5>::info()},
-      {384, CtLen<8, 8, 6>::info()}, {512, CtLen<8, 8, 8>::info()},  {1024, CtLen<8, 8, 4, 4>::info()},
+      {384, CtLen<4, 8, 12>::info()}, {512, CtLen<8, 8, 8>::info()},  {1024, CtLen<8, 8, 4, 4>::info()},
       {2048, CtLen<16, 16, 8>::info()}};
   return tab;
 }
