@@ -298,9 +298,9 @@ void p3dfft_amd_set_x_into_out(int on);
 /* Plan mode for the next p3dfft_setup (counterpart of the reference's
  * FFTW_MEASURE planning, build/fft_spec.F90:101-108).  0 (default): the
  * default plan of every length.  1: the setup times candidate plans of each
- * transform length on its own grid (specialised kernels; generic kernels with
- * 32/64/128 KiB tiles and 64/128/256-byte column segments; other radix
- * orders) and the schedule switches, and keeps the fastest.  Measured plans
+ * transform length on its own grid (specialised kernels; run-time-schedule kernels
+ * with their default, 32, 64 and 128 KiB tiles and 64/128/256-byte column
+ * segments; other radix orders) and the schedule switches, and keeps the fastest.  Measured plans
  * persist for the process; results stay within each precision's tolerance. */
 void p3dfft_amd_set_plan_mode(int mode);
 /* the last measurement's choices as text; returns the full length */
@@ -310,7 +310,8 @@ int p3dfft_amd_reset_plans(void);
 /* The launch shape the kernels with run-time radix schedules take for n <= 8192
  * points (host only, no GPU call): form 0 columns read and written by rows, 1
  * columns with a length-fastest (STRIDE1) side, 2 rows along X; count columns
- * or rows.  tile_bytes and segment as a plan has them (defaults 65536, 128).
+ * or rows.  tile_bytes (0: the kernels' default) and segment (128) as a plan has
+ * them.
  * Sequences per workgroup, threads (0: none can hold the tile), LDS bytes
  * (at most 163840 can be launched) and the bytes of an element offset (form 0:
  * of `count` contiguous columns).  Returns 0, or -1 for another n. */

@@ -751,14 +751,19 @@ static void measure_plans(State& S) {
     };
     std::vector<Cand> cands;
     const std::vector<int> f0 = default_factors(n);
-    if (len_has_ct(n)) cands.push_back({f0, true, 64 * 1024, 128});
+    if (len_has_ct(n)) cands.push_back({f0, true, 0, 128});
+    // the run-time kernels' schedule (the specialised one may have radices that
+    // they lack): their default tiles (in FP32 64 KiB), other sizes, other orders
+    const std::vector<int> fr = run_time_factors(n);
+    cands.push_back({fr, false, 0, 128});
     for (int tile : {32 * 1024, 64 * 1024, 128 * 1024})
-      for (int seg : {64, 128, 256}) cands.push_back({f0, false, tile, seg});
-    std::vector<int> f1(f0.rbegin(), f0.rend());
-    if (f1 != f0) cands.push_back({f1, false, 64 * 1024, 128});
-    std::vector<int> f2 = f0;
+      for (int seg : {64, 128, 256})
+        if (sizeof(real_t) == 8 || tile != 64 * 1024 || seg != 128) cands.push_back({fr, false, tile, seg});
+    std::vector<int> f1(fr.rbegin(), fr.rend());
+    if (f1 != fr) cands.push_back({f1, false, 0, 128});
+    std::vector<int> f2 = fr;
     std::sort(f2.begin(), f2.end());
-    if (f2 != f0 && f2 != f1) cands.push_back({f2, false, 64 * 1024, 128});
+    if (f2 != fr && f2 != f1) cands.push_back({f2, false, 0, 128});
     double best = 1e30;
     size_t bi = 0;
     for (size_t i = 0; i < cands.size(); i++) {

@@ -1494,6 +1494,18 @@ static tw_t* gen_table(const std::vector<int2>& idx) {
 
 std::vector<int> default_factors(int n) { return has_ct_schedule(n) ? ct_factors(n) : gen_factors(n); }
 
+// the run-time kernels take the schedule f of a length
+static bool runs_at_run_time(int n, const std::vector<int>& f) {
+  for (int r : f)
+    if (!gen_in_registers(r) && !gen_is_prime_stage(r)) return false;
+  return !f.empty() && (!has_ct_schedule(n) || gen_wrap(f) == f);
+}
+
+std::vector<int> run_time_factors(int n) {
+  const std::vector<int> f = default_factors(n);
+  return runs_at_run_time(n, f) ? f : gen_factors(n);
+}
+
 // stage descriptor of the radix schedule f and the entries of its twiddle
 // table: stage s > 0 has W_{Ns R}^{k r}, k < Ns, r = 1..R-1, a prime stage of
 // the run-time kernels also W_R^j, j < R
@@ -1545,12 +1557,9 @@ static Len1D build_len(int n, const std::vector<int>& f0) {
   Len1D L;
   const std::vector<int> f = has_ct_schedule(n) ? f0 : gen_wrap(f0);
   L.d = build_desc(n, f, &L.tw);
-  bool runtime = !f.empty();
-  for (int r : f) runtime = runtime && (gen_in_registers(r) || gen_is_prime_stage(r));
-  if (runtime && has_ct_schedule(n)) runtime = gen_wrap(f) == f;
   L.gtw = L.tw;
   L.gd = L.d;
-  if (!runtime) L.gd = build_desc(n, gen_factors(n), &L.gtw);
+  if (!runs_at_run_time(n, f)) L.gd = build_desc(n, gen_factors(n), &L.gtw);
   if (n == 512) {
     // the wave kernels' table W_512^e
     std::vector<int2> fidx(n);
@@ -1917,7 +1926,8 @@ std::string len_describe(int n) {
     return r;
   };
   if (find_ct(L)) return radices(L.d) + ", specialised";
-  return radices(L.gd) + ", run-time, tile " + std::to_string(L.tile_bytes / 1024) + " KiB, segment " +
+  return radices(L.gd) + ", run-time, " +
+         (L.tile_bytes ? "tile " + std::to_string(L.tile_bytes / 1024) + " KiB" : "default tile") + ", segment " +
          std::to_string(L.col_seg) + " B";
 }
 

@@ -39,10 +39,10 @@ struct Len1D {
   tw_t* gtw = nullptr;
   tw_t* twf = nullptr; // W_n^e, e < n, for the wave kernels of n = 512
   // plan choices (plan-time measurement may change them): specialised
-  // kernels allowed; data bytes per tile and bytes of adjacent columns per
-  // row segment of the run-time-generic kernels
+  // kernels allowed; data bytes per tile (0: the kernels' own default) and bytes
+  // of adjacent columns per row segment of the run-time-generic kernels
   bool ct_ok = true;
-  int tile_bytes = 64 * 1024;
+  int tile_bytes = 0;
   int col_seg = 128;
 };
 
@@ -51,7 +51,9 @@ const Len1D& get_len(int n);
 void free_lens();
 // the default radix schedule of a length
 std::vector<int> default_factors(int n);
-// replace the plan of length n (radix schedule and tile choices); the device
+// the same for the run-time kernels
+std::vector<int> run_time_factors(int n);
+// replace the plan of length n (radix schedule and tile choices, Len1D); the device
 // is synchronised before the old twiddle table is freed
 void set_len_plan(int n, const std::vector<int>& factors, bool ct_ok, int tile_bytes, int col_seg);
 // a specialised kernel set exists for length n with its default schedule

@@ -801,10 +801,11 @@ struct TileChoice {
 
 // column tile of m rows (d: the schedule, null: rows are copied): a 128-byte
 // row segment (plan-time measurement may choose another) while the tile stays
-// within the plan's bytes, segments of 64 bytes as long as the tile fits at
-// all; halved while there is not a tile for every CU
-static TileChoice col_tile(const LenDesc* d, int m, bool lf, long long ncol, int tile_bytes, int seg) {
+// within the plan's bytes (0: 64 KiB), segments of 64 bytes as long as the tile
+// fits at all; halved while there is not a tile for every CU
+static TileChoice col_tile(const LenDesc* d, int m, bool lf, long long ncol, int plan_bytes, int seg) {
   const long long E = sizeof(cplx_t);
+  const int tile_bytes = plan_bytes ? plan_bytes : 64 * 1024;
   const int R0 = d ? d->radix[0] : 1;
   // LDS bytes of a tile of b columns, sk elements between its blocks
   auto data_of = [&](int b, int sk) {
@@ -893,7 +894,7 @@ void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, bool wide, hipStr
   const bool lf = lf_in || lf_out;
   const int m = L ? L->gd.n : c.nld;
   const TileChoice tc =
-      L ? col_tile(&L->gd, m, lf, ncol, L->tile_bytes, L->col_seg) : col_tile(nullptr, m, lf, ncol, 64 * 1024, 128);
+      L ? col_tile(&L->gd, m, lf, ncol, L->tile_bytes, L->col_seg) : col_tile(nullptr, m, lf, ncol, 0, 128);
   const int B = tc.B;
   a.lB = log2i(B);
   a.t = tc.t;
@@ -944,15 +945,16 @@ void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, bool wide, hipStr
 }
 
 // tile of the X kernels, rows of at most `row` elements apart
-static TileChoice x_row_tile(const LenDesc& d, long long nrows, long long row, int tile_bytes) {
+static TileChoice x_row_tile(const LenDesc& d, long long nrows, long long row, int plan_bytes) {
   const long long pairs = (nrows + 1) / 2, E = sizeof(cplx_t);
   const int n = d.n;
   int B = 16;
-  // FP64 tiles of at most 40 KiB (four workgroups per CU in different phases;
-  // a prime stage wants the pairs): r2c / c2r 600x128x200 61 / 74 -> 48 / 50 us,
+  // the plan's bytes, by default 64 KiB, in FP64 40 KiB (four workgroups per CU in
+  // different phases; a prime stage wants the pairs): r2c / c2r 600x128x200 61 / 74 -> 48 / 50 us,
   // 720x240x200 155 / 165 -> 139 / 130.  FP32 measured no gain (1500x64x100 28
   // -> 29), its tiles hold twice the values per byte in flight.
-  const long long lim = sizeof(real_t) == 8 && !has_prime_stage(d) ? std::min(tile_bytes, 40 * 1024) : tile_bytes;
+  const long long def = sizeof(real_t) == 8 && !has_prime_stage(d) ? 40 * 1024 : 64 * 1024;
+  const long long lim = plan_bytes ? plan_bytes : def;
   while (B > 1 && ((long long)n * (B + 1) * E > lim || (2LL * B + 1) * row * E >= (1LL << 32))) B /= 2;
   while (B > 1 && !prime_stages_fit(d, B)) B /= 2;
   while (B > 2 && (pairs + B - 1) / B < 512) B /= 2;

@@ -23,7 +23,7 @@ def shapes(precision, form, tile, seg):
 
 
 @pytest.mark.parametrize("precision", [8, 4])
-@pytest.mark.parametrize("tile,seg", [(65536, 128), (32768, 64), (131072, 256)])
+@pytest.mark.parametrize("tile,seg", [(0, 128), (32768, 64), (131072, 256)])
 @pytest.mark.parametrize("form", [0, 1, 2])
 def test_every_length_fits_the_lds(precision, form, tile, seg):
     bad = [(n, c, b) for n, c, s, t, b in shapes(precision, form, tile, seg) if b > LDS or s < 1]
@@ -31,7 +31,7 @@ def test_every_length_fits_the_lds(precision, form, tile, seg):
 
 
 @pytest.mark.parametrize("precision", [8, 4])
-@pytest.mark.parametrize("tile,seg", [(65536, 128), (131072, 256)])
+@pytest.mark.parametrize("tile,seg", [(0, 128), (131072, 256)])
 @pytest.mark.parametrize("form", [0, 1, 2])
 def test_every_length_has_threads(precision, form, tile, seg):
     """A prime stage holds its outputs in the registers of at most 1024 threads."""
@@ -57,6 +57,21 @@ def test_wide_offsets_reach_the_run_time_kernels(precision):
         assert width(300, 1000) == 8
     finally:
         L.p3dfft_amd_set_wide_offsets(0)
+
+
+@pytest.mark.parametrize("precision", [8, 4])
+@pytest.mark.parametrize("form", [0, 2])
+def test_plan_tile_sizes_reach_the_kernels(precision, form):
+    """The tile sizes that a measured setup times are different tiles."""
+    L = p3dfft_amd.load(precision)
+    t, b, o = ctypes.c_int(), ctypes.c_size_t(), ctypes.c_int()
+    got = []
+    for tile in (32768, 65536, 131072):
+        s = ctypes.c_int()
+        assert L.p3dfft_amd_run_time_tile(500, form, 1000000, tile, 256, ctypes.byref(s), ctypes.byref(t),
+                                          ctypes.byref(b), ctypes.byref(o)) == 0
+        got.append(s.value)
+    assert got[0] < got[1] < got[2], got
 
 
 @pytest.mark.parametrize("precision", [8, 4])
