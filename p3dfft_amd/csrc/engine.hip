@@ -55,21 +55,13 @@ __device__ __forceinline__ int tile_of(int rev, int xcd = 1) {
 // ---------------------------------------------------------------------------
 // X kernels
 // ---------------------------------------------------------------------------
-// a length as the specialised kernels see it
-struct CtLenArg {
-  int n, twcount;
-};
-
 struct XArgs {
   const void* in;
   void* out;
   long long nrows, si_row, so_row;
   int nxo;     // r2c: kept modes; c2r: valid input modes
-  int B;       // row pairs per workgroup
   FDiv dnxo;
-  CtLenArg L;
   const void* tw;
-  int tw_lds;  // twiddles staged in LDS
   int tw_off;  // byte offset of the staged twiddles
   int rev;     // walk the tiles from the last one
   // table-addressed rows (share mode): mode k of row r at element
@@ -87,16 +79,14 @@ struct ColArgs {
   void* out;
   long long si_in, sl_in, so_in, si_out, sl_out, so_out;
   int n_inner, n_outer, tiles;
-  int TX;
-  FDiv dTX;
   int kind;
   int nld, ld_lo, ld_hi, ld_shift;
   int nst, st_lo, st_shift;
   int ld_lenfast, st_lenfast;
   FDiv dnld, dnst;
-  CtLenArg L;
+  int n;  // transform length
   const void* tw;
-  int tw_lds, tw_off;
+  int tw_off;
   int rev;  // walk the tiles from the last one
   // XCD-aware tile order (tiles that share cache lines at their edges run in
   // one XCD's L2); 0: dispatch order, for views whose tiles never share a
@@ -649,7 +639,7 @@ struct PlaneArgs {
   void* out;
   const void* twx;  // twiddles of NX, of NY (the same table when NX == NY)
   const void* twy;
-  int ntwx, ntwy;   // entries
+  int ntwx;         // entries of twx
 };
 
 template <class T, class RLX, class RLY>
@@ -1028,9 +1018,9 @@ __device__ __forceinline__ void cheby_tile(cpx<T>* lds, double* wt, const ColArg
 }
 
 // Column transforms through an LDS load/store pass: DCT-I / DST-I
-// extensions, length-fastest ("STRIDE1") views, copies, and views whose
-// offsets do not fit the 32-bit form.  Loads are issued LU at a time per
-// thread before their LDS stores (several loads in flight per thread).
+// extensions, length-fastest ("STRIDE1") views and views whose offsets do not
+// fit the 32-bit form.  Loads are issued LU at a time per thread before their LDS
+// stores (several loads in flight per thread).
 template <class T, bool FWD, int TX, int NT, class RL, int W, bool TWL>
 __global__ __launch_bounds__(NT, W) void k_col_ct(ColArgs a) {
   cpx<T>* lds = (cpx<T>*)g_smem;
@@ -1076,14 +1066,14 @@ __global__ __launch_bounds__(NT, W) void k_col_ct(ColArgs a) {
     __syncthreads();
   }
   if (a.kind == COL_DCT1 && !a.mirror) {
-    const int m = a.L.n;
+    const int m = a.n;
     for (int q = threadIdx.x; q < TX * (m - a.nld); q += NT) {
       const int r = q / TX, b = q % TX, e = a.nld + r;
       lds[e * TX + b] = lds[(m - e) * TX + b];
     }
     __syncthreads();
   } else if (a.kind == COL_DST1) {
-    const int m = a.L.n;
+    const int m = a.n;
     for (int q = threadIdx.x; q < TX * (m - a.nld - 1); q += NT) {
       const int r = q / TX, b = q % TX, e = a.nld + 1 + r;
       if (e == a.nld + 1) lds[e * TX + b] = mk<T>(0, 0);
@@ -1092,7 +1082,7 @@ __global__ __launch_bounds__(NT, W) void k_col_ct(ColArgs a) {
     for (int b = threadIdx.x; b < TX; b += NT) lds[b] = mk<T>(0, 0);
     __syncthreads();
   }
-  if (a.kind != COL_COPY && !a.mirror) run_fft_ct<T, FWD, TX, TX, NT>(lds, tw.table(), RL{});
+  if (!a.mirror) run_fft_ct<T, FWD, TX, TX, NT>(lds, tw.table(), RL{});
   if constexpr (64 % TX == 0 && NT % 64 == 0) {
     if (a.cheby) {
       // the recurrence stores the output rows itself
@@ -1140,7 +1130,7 @@ __global__ __launch_bounds__(NT, W) void k_zsolve_ct(ColArgs a, double scale, in
   const int nb = (int)(ncol - c0 < TX ? ncol - c0 : TX);
   const ColIO io = col_io<T, TX>(a, c0, nb);
   SolveCtx sc;
-  sc.nxh = nxh; sc.ny = ny; sc.nz = a.L.n; sc.scale = scale;
+  sc.nxh = nxh; sc.ny = ny; sc.nz = a.n; sc.scale = scale;
   run_fft_solve<T, TX, NT>(lds, tw, io, c0, sc, RL{});
 }
 
@@ -1222,7 +1212,7 @@ __global__ __launch_bounds__(NT, W) void k_zs_grp(ColArgs a, GrpArgs g) {
   const int nb = (int)(ncol - c0 < TX ? ncol - c0 : TX);
   const ColIO io = col_io<T, TX>(a, c0, nb);
   SolveCtx sc;
-  sc.nxh = d.nxh; sc.ny = d.ny; sc.nz = a.L.n; sc.scale = d.scale;
+  sc.nxh = d.nxh; sc.ny = d.ny; sc.nz = a.n; sc.scale = d.scale;
   run_fft_solve<T, TX, NT>(lds, tw, io, c0, sc, RL{});
 }
 
@@ -1979,9 +1969,8 @@ bool tile_order_alternate() { return g_alt_order; }
 void set_specialised(bool on) { g_use_ct = on; }
 
 // LDS bytes of a specialised tile of `data` bytes; sets the twiddle placement
-static size_t ct_lds(size_t data, bool twl, const CtInfo& c, int* tw_lds, int* tw_off) {
+static size_t ct_lds(size_t data, bool twl, const CtInfo& c, int* tw_off) {
   const size_t d16 = (size_t)round16((long long)data);
-  *tw_lds = twl ? 1 : 0;
   *tw_off = twl ? (int)d16 : 0;
   return twl ? d16 + (size_t)c.twb : data;
 }
@@ -1992,10 +1981,8 @@ static bool x_setup_ct(XArgs& a, const Len1D& L, const CtInfo& c, long long nrow
   const long long span = (2LL * c.BX + 1) * std::max(si_row, so_row) * (long long)sizeof(cplx_t);
   if (span >= (1LL << 32)) return false;
   const long long pairs = (nrows + 1) / 2;
-  a.B = c.BX;
-  a.L = CtLenArg{L.d.n, L.d.twcount};
   a.tw = L.tw;
-  *bytes = ct_lds((size_t)c.x_bytes, c.twl_x, c, &a.tw_lds, &a.tw_off);
+  *bytes = ct_lds((size_t)c.x_bytes, c.twl_x, c, &a.tw_off);
   const long long g = (pairs + c.BX - 1) / c.BX;
   if (g > 0x7fffffffLL) throw Error{"grid too large", -1};
   *nwg = (unsigned)g;
@@ -2203,7 +2190,7 @@ void launch_xy_plane(bool fwd, const void* in, void* out, int nx, int ny, int nz
   PlaneArgs a;
   a.in = in; a.out = out;
   a.twx = Lx.tw; a.twy = Ly.tw;
-  a.ntwx = Lx.d.twcount; a.ntwy = nx == ny ? 0 : Ly.d.twcount;
+  a.ntwx = Lx.d.twcount;
   p->go(fwd, a, nz, plane_bytes(*p, Lx, Ly), st);
   check_hip(hipGetLastError(), fwd ? "k_xy_plane_fwd launch" : "k_yx_plane_bwd launch");
 }
@@ -2284,20 +2271,18 @@ bool launch_col_tab(const ColSpec& c, const int2* ltab, const int2* stab, bool a
   a.rev = c.rev ? 1 : 0;
   a.xcd = 1;  // table-addressed rows: tiles share lines across peer blocks
   const int TX = ct->TX;
-  a.TX = TX;
-  a.dTX = make_fdiv(TX);
   a.tiles = (c.n_inner + TX - 1) / TX;
-  a.L = CtLenArg{L.d.n, L.d.twcount};
+  a.n = L.d.n;
   a.tw = L.tw;
   if (g_col_pipe && ct->pipe && sep.ok && sep.r0 == ct->radix[0] && sep.rl == ct->radix[ct->nr - 1]) {
     a.sep = sep;
-    const size_t pb = ct_lds((size_t)TX * c.n * sizeof(cplx_t), ct->twl_col, *ct, &a.tw_lds, &a.tw_off);
+    const size_t pb = ct_lds((size_t)TX * c.n * sizeof(cplx_t), ct->twl_col, *ct, &a.tw_off);
     ct->colpipe(c.fwd, true, a, pipe_grid(ncol), pb, st);
     check_hip(hipGetLastError(), "k_colio_pipe (separable table) launch");
     return true;
   }
   if (g_col_pipe && ct->pipe) {
-    size_t pb = ct_lds((size_t)TX * c.n * sizeof(cplx_t), ct->twl_pipe_tab, *ct, &a.tw_lds, &a.tw_off);
+    size_t pb = ct_lds((size_t)TX * c.n * sizeof(cplx_t), ct->twl_pipe_tab, *ct, &a.tw_off);
     a.tab_off = (int)round16((long long)pb);
     pb = (size_t)a.tab_off + 2 * (size_t)c.n * sizeof(int2);
     if (pb <= kLdsMax) {
@@ -2306,7 +2291,7 @@ bool launch_col_tab(const ColSpec& c, const int2* ltab, const int2* stab, bool a
       return true;
     }
   }
-  size_t bytes = ct_lds((size_t)TX * c.n * sizeof(cplx_t), ct->twl_tab, *ct, &a.tw_lds, &a.tw_off);
+  size_t bytes = ct_lds((size_t)TX * c.n * sizeof(cplx_t), ct->twl_tab, *ct, &a.tw_off);
   a.tab_off = (int)round16((long long)bytes);
   bytes = (size_t)a.tab_off + (size_t)c.n * sizeof(int2);
   if (bytes > kLdsMax) return false;
@@ -2360,12 +2345,10 @@ bool launch_col(const ColSpec& c, hipStream_t st) {
   const bool fwd = c.fwd || c.kind == COL_DCT1 || c.kind == COL_DST1;
   if (const CtInfo* ct = (L && g_use_ct) ? find_ct(*L) : nullptr) {
     const int TX = ct->TX;
-    a.TX = TX;
-    a.dTX = make_fdiv(TX);
     a.tiles = (c.n_inner + TX - 1) / TX;
-    a.L = CtLenArg{L->d.n, L->d.twcount};
+    a.n = L->d.n;
     a.tw = L->tw;
-    const size_t bytes = ct_lds((size_t)TX * rows * sizeof(cplx_t), ct->twl_col, *ct, &a.tw_lds, &a.tw_off);
+    const size_t bytes = ct_lds((size_t)TX * rows * sizeof(cplx_t), ct->twl_col, *ct, &a.tw_off);
     if (bytes > kLdsMax) throw Error{"column transform does not fit in LDS", -1};
     const long long ncol = (long long)c.n_inner * c.n_outer;
     if (ncol > 0x7fffffffLL) throw Error{"grid too large", -1};
@@ -2395,7 +2378,7 @@ bool launch_col(const ColSpec& c, hipStream_t st) {
         col_side_fits32(c, !a.ld_lenfast, TX, rows) && !g_wide_offsets) {
       size_t lf = (size_t)round16((long long)TX * nfft * (long long)sizeof(cplx_t));
       a.tab_off = (int)lf;
-      lf = ct_lds(lf + 8 * (size_t)(TX + TX % 2), ct->twl_lf, *ct, &a.tw_lds, &a.tw_off);
+      lf = ct_lds(lf + 8 * (size_t)(TX + TX % 2), ct->twl_lf, *ct, &a.tw_off);
       if (lf <= kLdsMax) {
         a.xcd = flat_dispatch_order(c) ? 0 : 1;
         ct->collf(fwd, a.ld_lenfast != 0, a, (unsigned)((ncol + TX - 1) / TX), lf, st);
@@ -2449,12 +2432,11 @@ bool launch_zsolve(cplx_t* spec, int nxh, int ny, int nz, double scale, hipStrea
   a.n_inner = (int)ninner; a.n_outer = 1;
   a.kind = COL_C2C;
   const int TX = ct->TX;
-  a.TX = TX;
   a.tiles = (int)((ninner + TX - 1) / TX);
-  a.L = CtLenArg{L.d.n, L.d.twcount};
+  a.n = L.d.n;
   a.tw = L.tw;
   if ((ninner + (long long)nz * ninner + TX) * (long long)sizeof(cplx_t) >= (1LL << 32)) return false;
-  const size_t bytes = ct_lds((size_t)TX * nz * sizeof(cplx_t), ct->twl_col, *ct, &a.tw_lds, &a.tw_off);
+  const size_t bytes = ct_lds((size_t)TX * nz * sizeof(cplx_t), ct->twl_col, *ct, &a.tw_off);
   if (bytes > kLdsMax) return false;
   ct->zsolve(a, scale, nxh, ny, (unsigned)a.tiles, bytes, st);
   check_hip(hipGetLastError(), "k_zsolve_ct launch");
@@ -2573,18 +2555,14 @@ GroupBatch* group_batch_create(int mode, int n, const int* shapes, real_t* const
         a.so_row = kind == 0 ? nxh : len;
         a.nxo = nxh;
         a.dnxo = make_fdiv(nxh);
-        a.B = ct->BX;
-        a.L = CtLenArg{L.d.n, L.d.twcount};
         a.tw = L.tw;
-        h.s.bytes = ct_lds((size_t)ct->x_bytes, ct->twl_x, *ct, &a.tw_lds, &a.tw_off);
+        h.s.bytes = ct_lds((size_t)ct->x_bytes, ct->twl_x, *ct, &a.tw_off);
       } else {
         ColArgs& a = h.s.ca;
         a.kind = COL_C2C;
-        a.TX = ct->TX;
-        a.dTX = make_fdiv(ct->TX);
-        a.L = CtLenArg{L.d.n, L.d.twcount};
+        a.n = L.d.n;
         a.tw = L.tw;
-        h.s.bytes = ct_lds((size_t)ct->TX * len * sizeof(cplx_t), ct->twl_col, *ct, &a.tw_lds, &a.tw_off);
+        h.s.bytes = ct_lds((size_t)ct->TX * len * sizeof(cplx_t), ct->twl_col, *ct, &a.tw_off);
       }
       if (h.s.bytes > kLdsMax) throw Error{"grouped pass does not fit in LDS", -1};
       hs.push_back(std::move(h));

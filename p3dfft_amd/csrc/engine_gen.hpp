@@ -14,7 +14,8 @@ std::vector<int> gen_factors(int n);
 // the same for factors in a given order (a plan-time candidate)
 std::vector<int> gen_wrap(const std::vector<int>& f);
 // the largest radix held in registers: with radices up to 16 the kernels with
-// row maps need 544 to 880 bytes of scratch per lane, with 10 none
+// row maps need 544 to 880 bytes of scratch per lane, with 10 none (the FP64
+// kernels with a length-fastest side 68 bytes, spilled scalar registers)
 constexpr int kGenMaxRadix = 10;
 inline bool gen_in_registers(int r) { return r <= kGenMaxRadix; }
 // a prime radix above that (the specialised schedules also hold 16)
