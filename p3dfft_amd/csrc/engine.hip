@@ -1497,8 +1497,8 @@ std::vector<int> run_time_factors(int n) {
 }
 
 // stage descriptor of the radix schedule f and the entries of its twiddle
-// table: stage s > 0 has W_{Ns R}^{k r}, k < Ns, r = 1..R-1, a prime stage of
-// the run-time kernels also W_R^j, j < R
+// table: stage s > 0 has W_{Ns R}^{k r}, k < Ns, r = 1..R-1, a prime stage over
+// LDS of the run-time kernels also W_R^j, j < R
 static LenDesc describe(int n, const std::vector<int>& f, std::vector<int2>& idx) {
   LenDesc d;
   std::memset(&d, 0, sizeof(d));
@@ -1516,7 +1516,7 @@ static LenDesc describe(int n, const std::vector<int>& f, std::vector<int2>& idx
     if (s > 0)
       for (int k = 0; k < ns; k++)
         for (int r = 1; r < R; r++) idx.push_back(make_int2(k * r, ns * R));
-    if (gen_is_prime_stage(R))
+    if (gen_over_lds(R))
       for (int j = 0; j < R; j++) idx.push_back(make_int2(j, R));
     ns *= R;
   }

@@ -18,9 +18,10 @@
 // (or writes) global memory itself, one 128-byte row segment per value, and
 // the reversal is one division per butterfly.
 //
-// A prime radix above 10 runs as a stage over LDS by the symmetric pairs
-// v_i +- v_{R-i} (half the multiplications of the direct sum), its outputs
-// held in registers across a barrier.
+// 11 and 13 points run as such a butterfly too, by the symmetric pairs
+// v_i +- v_{R-i} (half the multiplications of the direct sum).  A larger prime
+// radix runs as a stage over LDS by those pairs, its outputs held in registers
+// across a barrier.
 //
 // What bounds the passes: with 128-byte row segments they move each byte once
 // per pass and run at 4-5.5 TB/s; the rest is the instruction issue of the
@@ -113,7 +114,79 @@ __device__ __forceinline__ int gen_stride(const GenTile& t, const GenStage& st) 
   return gdiv(st.Ns, t.mR0, t.R0) * t.P0;
 }
 
-// a stage with a prime radix above kGenMaxRadix: outputs by symmetric pairs
+// a butterfly of 11 or 13 points in place, its positions SP apart: the sums and
+// differences of the symmetric pairs in registers, each pair of outputs written
+// as soon as it is summed, so 13 FP64 points hold 13 values and not 26.  One
+// barrier and 2 R LDS accesses a butterfly: 25600 columns of 143 points 35 us in
+// FP64 and 28 us in FP32 (3.4 and 2.1 TB/s), 4096 of 2197 points 95 and 60 us; with
+// the pairs' sums over LDS (gen_prime) 90 and 47, 170 and 142 us, slower than a
+// direct radix 11 or 13 of autosort stages (77 and 43, 240 and 115 us).
+template <int R>
+struct PrimeConst;
+template <>
+struct PrimeConst<11> {
+  static constexpr double c[6] = {1.0, 0.84125353283118116886, 0.41541501300188642553, -0.14231483827328514044,
+                                  -0.65486073394528506406, -0.95949297361449738989};
+  static constexpr double s[6] = {0.0, 0.54064081745559758211, 0.90963199535451837141, 0.98982144188093273238,
+                                  0.75574957435425828377, 0.28173255684142969771};
+};
+template <>
+struct PrimeConst<13> {
+  static constexpr double c[7] = {1.0, 0.88545602565320989590, 0.56806474673115580251, 0.12053668025532305335,
+                                  -0.35460488704253562597, -0.74851074817110109863, -0.97094181742605202716};
+  static constexpr double s[7] = {0.0, 0.46472317204376854566, 0.82298386589365639458, 0.99270887409805399280,
+                                  0.93501624268541482344, 0.66312265824079520238, 0.23931566428755776715};
+};
+
+// a + x * k, the constant hi + lo in FP32
+template <class T>
+__device__ __forceinline__ cpx<T> fma_const(cpx<T> x, double k, cpx<T> a) {
+  if constexpr (sizeof(T) == 4) {
+    const float h = (float)k, l = (float)(k - (double)h);
+    return mk<T>(fmaf(x.x, h, fmaf(x.x, l, a.x)), fmaf(x.y, h, fmaf(x.y, l, a.y)));
+  } else {
+    return mk<T>(fma(x.x, k, a.x), fma(x.y, k, a.y));
+  }
+}
+
+template <class T, bool FWD, bool DIF, int R>
+__device__ __forceinline__ void gen_reg_prime(cpx<T>* p, int SP, const typename TwT<T>::type* w) {
+  constexpr int H = (R - 1) / 2;
+  const cpx<T> v0 = p[0];
+  cpx<T> s[H], d[H], y0 = v0;
+#pragma unroll
+  for (int i = 0; i < H; i++) {
+    cpx<T> u = p[(i + 1) * SP], v = p[(R - 1 - i) * SP];
+    if constexpr (!DIF) {
+      u = twmul<FWD>(u, w[i]);
+      v = twmul<FWD>(v, w[R - 2 - i]);
+    }
+    s[i] = add(u, v);
+    d[i] = sub(u, v);
+    y0 = add(y0, s[i]);
+  }
+  p[0] = y0;
+#pragma unroll
+  for (int q = 1; q <= H; q++) {
+    cpx<T> c = v0, e = mk<T>(0, 0);
+#pragma unroll
+    for (int i = 0; i < H; i++) {
+      const int m = (i + 1) * q % R;
+      c = fma_const(s[i], PrimeConst<R>::c[m <= H ? m : R - m], c);
+      e = fma_const(d[i], m <= H ? PrimeConst<R>::s[m] : -PrimeConst<R>::s[R - m], e);
+    }
+    e = rot<FWD>(e);
+    cpx<T> a = add(c, e), b = sub(c, e);
+    if constexpr (DIF) {
+      a = twmul<FWD>(a, w[q - 1]);
+      b = twmul<FWD>(b, w[R - 1 - q]);
+    }
+    p[q * SP] = a;
+    p[(R - q) * SP] = b;
+  }
+}
+
+// a stage with a larger prime radix: outputs by symmetric pairs over LDS
 constexpr int kPrimeItems = 8;
 template <class T, bool FWD, bool DIF>
 __device__ __forceinline__ void gen_prime(cpx<T>* lds, const GenDesc& L, const GenStage& st, const GenTile& t, int B,
@@ -207,12 +280,25 @@ __device__ __forceinline__ void gen_mid(cpx<T>* lds, const GenDesc& L, int s, co
                                         int b, int jt, int js, const typename TwT<T>::type* tw) {
   const GenStage st = L.st[s];
   if constexpr (PM) {
-    if (st.R > kGenMaxRadix) {
+    if (st.R > kGenRegPrime) {
       gen_prime<T, FWD, DIF>(lds, L, st, t, B, mB, tw);
       return;
     }
   }
   const int nj = gdiv(L.n, st.mR, st.R), SP = gen_stride(t, st);
+  if constexpr (PM) {
+    if (st.R > kGenMaxRadix) {
+      for (int j = jt; j < nj; j += js) {
+        const int g = gdiv(j, st.mNs, st.Ns), k = j - g * st.Ns;
+        cpx<T>* p = lds + gen_base(t, st, g, k, SP) + b;
+        const typename TwT<T>::type* w = tw + st.tw + k * (st.R - 1);
+        if (st.R == 11) gen_reg_prime<T, FWD, DIF, 11>(p, SP, w);
+        else gen_reg_prime<T, FWD, DIF, 13>(p, SP, w);
+      }
+      __syncthreads();
+      return;
+    }
+  }
   with_radix(st.R, [&](auto rc) {
     constexpr int R = decltype(rc)::value;
     for (int j = jt; j < nj; j += js) {
@@ -750,7 +836,7 @@ static long long prime_items(const LenDesc& d, int s, int B) {
 }
 static bool prime_stages_fit(const LenDesc& d, int B) {
   for (int s = 0; s < d.nst; s++)
-    if (!gen_in_registers(d.radix[s]) && prime_items(d, s, B) > 1024LL * kPrimeItems) return false;
+    if (gen_over_lds(d.radix[s]) && prime_items(d, s, B) > 1024LL * kPrimeItems) return false;
   return true;
 }
 
@@ -770,8 +856,9 @@ static int pick_threads(const LenDesc& d, int B, size_t lds, long long tiles) {
     for (int s = 0; s < d.nst; s++) {
       const int R = d.radix[s];
       const long long nb = (long long)B * (d.n / R);
-      if (gen_in_registers(R)) {
-        t += (double)((nb + nt - 1) / nt) * (R + 3);
+      if (!gen_over_lds(R)) {
+        // (11 and 13 points by pairs: about as many operations as two of their size)
+        t += (double)((nb + nt - 1) / nt) * (gen_in_registers(R) ? R + 3 : 2 * R);
       } else {
         const long long items = prime_items(d, s, B);
         if (items > (long long)nt * kPrimeItems) ok = false;

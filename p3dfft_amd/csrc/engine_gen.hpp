@@ -18,8 +18,12 @@ std::vector<int> gen_wrap(const std::vector<int>& f);
 // kernels with a length-fastest side 68 bytes, spilled scalar registers)
 constexpr int kGenMaxRadix = 10;
 inline bool gen_in_registers(int r) { return r <= kGenMaxRadix; }
-// a prime radix above that (the specialised schedules also hold 16)
+// a prime radix above that (the specialised schedules also hold 16), never first
+// or last; up to kGenRegPrime the pairs of a butterfly sit in registers, above
+// they are summed over LDS
+constexpr int kGenRegPrime = 13;
 inline bool gen_is_prime_stage(int r) { return r > kGenMaxRadix && r % 2 == 1; }
+inline bool gen_over_lds(int r) { return r > kGenRegPrime && r % 2 == 1; }
 
 // the launchers of engine.hpp for these kernels
 void gen_launch_x_r2c(const Len1D& L, const real_t* in, cplx_t* out, long long nrows, long long si_row,

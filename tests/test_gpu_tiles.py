@@ -40,6 +40,23 @@ def test_no_room_for_the_skew_few_columns(precision):
 
 
 @pytest.mark.parametrize("precision", [8, 4])
+@pytest.mark.parametrize("n", [26, 169, 286, 2197])
+def test_stages_of_11_and_13(precision, n):
+    """In registers: alone, between factors, several in a row; decimation in time
+    (rows) and in frequency (X c2r, length-fastest input), a row map."""
+    for shape, cut, stride1 in (((n, 3, 4), None, False), ((4, n, 300), None, False), ((10, 7, n), None, True),
+                                ((10, 6, n), 2 * (n // 3), True), ((10, n, 4), 2 * (n // 3), False)):
+        nx, ny, nz = shape
+        c = (None, None, cut) if stride1 else (None, cut, None)
+        a = np.random.default_rng(n).standard_normal((nz, ny, nx))
+        o = oplan(nx, ny, nz, *c, stride1=stride1)
+        ref = o.ftran_r2c(a, "fft")
+        with lib_setup(precision, nx, ny, nz, *c, stride1=stride1) as P:
+            assert rel(P.ftran_r2c(a, "fft"), ref) < TOL[precision]
+            assert rel(P.btran_c2r(ref, "tff"), o.btran_c2r(ref, "tff")[0]) < TOL[precision]
+
+
+@pytest.mark.parametrize("precision", [8, 4])
 def test_chebyshev_extension(precision):
     """nz = 1251: the even extension has 2500 points"""
     nx, ny, nz = 2, 1056, 1251

@@ -74,6 +74,20 @@ def test_plan_tile_sizes_reach_the_kernels(precision, form):
     assert got[0] < got[1] < got[2], got
 
 
+@pytest.mark.parametrize("n,like", [(3773, 3780), (1859, 1875), (946, 960)])
+def test_11_and_13_points_are_register_stages(n, like):
+    """They take as many FP32 columns as a length of small factors, and are not
+    held back by what a prime stage over LDS can hold."""
+    L = p3dfft_amd.load(4)
+    s, t, b, o = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t(), ctypes.c_int()
+    got = []
+    for m in (n, like):
+        assert L.p3dfft_amd_run_time_tile(m, 0, 100000, 131072, 256, ctypes.byref(s), ctypes.byref(t),
+                                          ctypes.byref(b), ctypes.byref(o)) == 0
+        got.append(s.value)
+    assert got[0] == got[1], got
+
+
 @pytest.mark.parametrize("precision", [8, 4])
 def test_other_lengths_are_refused(precision):
     L = p3dfft_amd.load(precision)
