@@ -586,7 +586,7 @@ struct GXArgs {
   long long nrows, si_row, so_row;
   int nk;         // r2c: kept modes; c2r: valid input modes
   int lB;         // log2 of the row pairs per tile
-  FDiv dnk, dn0;  // divide by the modes, by n / R_0
+  FDiv dnk, dn0;  // divide by the modes, by n / R_0 (c2r of one stage: by n)
   GenTile t;
   GenDesc L;
   const void* tw;
@@ -711,6 +711,29 @@ __global__ __launch_bounds__(1024) void k_gx_c2r(GXArgs a) {
   char* out = (char*)a.out + 2 * pair0 * a.so_row * (long long)sizeof(T);
   const unsigned so = (unsigned)(a.so_row * sizeof(T));
   const GenStage s0 = a.L.st[0];
+  if (S == 1) {
+    // rows of one butterfly: stored by it, the lanes would write a value each of
+    // 64 rows at a time (2^23 points in rows of 8, FP32 45 us, through the tile
+    // 15 us; of 7 41 and 14.5)
+    with_radix(s0.R, [&](auto rc) {
+      constexpr int R = decltype(rc)::value;
+      for (int b = threadIdx.x; b < B; b += NT) {
+        C v[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) v[r] = lds[r * a.t.BP + b];
+        dft<R, false>(v);
+#pragma unroll
+        for (int r = 0; r < R; r++) lds[r * a.t.BP + b] = v[r];
+      }
+    });
+    __syncthreads();
+    for (int q = threadIdx.x; q < nr * n; q += NT) {
+      const int row = fdiv(q, a.dn0), e = q - row * n;
+      const C z = lds[e * a.t.BP + (row >> 1)];
+      *(T*)(out + ((unsigned)row * so + (unsigned)e * (unsigned)sizeof(T))) = row & 1 ? z.y : z.x;
+    }
+    return;
+  }
   const int n0 = gdiv(n, s0.mR, s0.R);
   with_radix(s0.R, [&](auto rc) {
     constexpr int R = decltype(rc)::value;
@@ -1036,6 +1059,11 @@ static TileChoice x_row_tile(const LenDesc& d, long long nrows, long long row, i
   const long long pairs = (nrows + 1) / 2, E = sizeof(cplx_t);
   const int n = d.n;
   int B = 16;
+  // short rows: tiles of more than 256 values, below which the launch of the
+  // workgroups bounds the pass, up to 64 pairs (the lanes along them divide every
+  // workgroup).  Not from 16 points on: FP32 c2r of 2^23 points in rows of 16 takes
+  // 20.6 us with 16 pairs, 22.6 with 32; of 11 31 and 22 us
+  while (B < 64 && 2LL * B * n < 512) B *= 2;
   // the plan's bytes, by default 64 KiB, in FP64 40 KiB (four workgroups per CU in
   // different phases; a prime stage wants the pairs): r2c / c2r 600x128x200 61 / 74 -> 48 / 50 us,
   // 720x240x200 155 / 165 -> 139 / 130.  FP32 measured no gain (1500x64x100 28
@@ -1119,6 +1147,7 @@ void gen_launch_x_c2r(const Len1D& L, const cplx_t* in, real_t* out, long long n
   int nt;
   unsigned g;
   const size_t bytes = x_tile(a, L, nrows, std::max(si_row, so_row), &nt, &g);
+  if (L.gd.nst == 1) a.dn0 = make_fdiv(L.gd.n);
   with_variant(a.tw_lds != 0, has_prime_stage(L.gd), [&](auto tl, auto pm) {
     k_gx_c2r<real_t, tl.value, pm.value><<<g, nt, bytes, st>>>(a);
   });

@@ -57,6 +57,22 @@ def test_stages_of_11_and_13(precision, n):
 
 
 @pytest.mark.parametrize("precision", [8, 4])
+@pytest.mark.parametrize("n", range(1, 16))
+def test_short_rows(precision, n):
+    """Rows of one stage (up to 10 points) and just above along X, in wide tiles
+    of which the last is partial and holds an odd row; pruned modes."""
+    for ny, nz, cut in ((5, 7, None), (201, 331, None), (6, 9, 2 * ((n + 1) // 3))):
+        if cut == 0:
+            continue
+        a = np.random.default_rng(n).standard_normal((nz, ny, n))
+        o = oplan(n, ny, nz, cut)
+        ref = o.ftran_r2c(a, "fft")
+        with lib_setup(precision, n, ny, nz, cut) as P:
+            assert rel(P.ftran_r2c(a, "fft"), ref) < TOL[precision]
+            assert rel(P.btran_c2r(ref, "tff"), o.btran_c2r(ref, "tff")[0]) < TOL[precision]
+
+
+@pytest.mark.parametrize("precision", [8, 4])
 def test_chebyshev_extension(precision):
     """nz = 1251: the even extension has 2500 points"""
     nx, ny, nz = 2, 1056, 1251

@@ -89,6 +89,18 @@ def test_11_and_13_points_are_register_stages(n, like):
 
 
 @pytest.mark.parametrize("precision", [8, 4])
+def test_short_rows_fill_a_tile(precision):
+    """Many short rows along X: a tile holds 256 values and more, and its row pairs
+    divide every workgroup."""
+    L = p3dfft_amd.load(precision)
+    s, t, b, o = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t(), ctypes.c_int()
+    for n in range(4, 40):
+        assert L.p3dfft_amd_run_time_tile(n, 2, 1000000, 0, 128, ctypes.byref(s), ctypes.byref(t), ctypes.byref(b),
+                                          ctypes.byref(o)) == 0
+        assert s.value * n >= 256 and t.value % s.value == 0, (n, s.value, t.value)
+
+
+@pytest.mark.parametrize("precision", [8, 4])
 def test_other_lengths_are_refused(precision):
     L = p3dfft_amd.load(precision)
     s, t, b, o = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t(), ctypes.c_int()
