@@ -309,8 +309,8 @@ int p3dfft_amd_plan_report(char *buf, int len);
 int p3dfft_amd_reset_plans(void);
 /* The launch shape the kernels with run-time radix schedules take for n <= 8192
  * points (host only, no GPU call): form 0 columns read and written by rows, 1
- * columns with a length-fastest (STRIDE1) side, 2 rows along X; count columns
- * or rows.  tile_bytes (0: the kernels' default) and segment (128) as a plan has
+ * columns with a length-fastest (STRIDE1) side, 2 rows along X, 3 and 4 as 0 and 1
+ * for columns that are copied (op 'n'); count columns or rows.  tile_bytes (0: the kernels' default) and segment (128) as a plan has
  * them.
  * Sequences per workgroup, threads (0: none can hold the tile), LDS bytes
  * (at most 163840 can be launched) and the bytes of an element offset (form 0:

@@ -544,7 +544,7 @@ __global__ __launch_bounds__(1024) void k_gcol(GColArgs a) {
 // through an LDS tile so that both sides are read and written along their
 // contiguous index
 template <class T>
-__global__ __launch_bounds__(256) void k_gcopy(GColArgs a) {
+__global__ __launch_bounds__(1024) void k_gcopy(GColArgs a) {
   typedef cpx<T> C;
   C* lds = (C*)gen_smem;
   const int B = 1 << a.lB, NT = blockDim.x;
@@ -946,8 +946,13 @@ static TileChoice col_tile(const LenDesc* d, int m, bool lf, long long ncol, int
   c.t.mR0 = magic(R0);
   c.t.skew = skew;
   c.t.P0 = R0 * c.t.BP + skew;
-  c.tw_lds = c.tw_off = c.nt = 0;
+  c.tw_lds = c.tw_off = 0;
   c.bytes = data;
+  // a copy has a tile or two per CU in flight and waits for its loads: four values
+  // a thread (FP32 with op 'n', forward / backward: 3 fields of 3x192x2149,
+  // length-fastest, 95 / 90 us with 256 threads, 51 / 50 so; 2 of 256x32x564, 176
+  // modes kept, 66 / 61 -> 46 / 47; with sixteen a thread 63 / 61 and 50 / 49)
+  c.nt = (int)std::max<long long>(64, std::min<long long>(1024, ((long long)m * B + 255) / 256 * 64));
   if (d) {
     c.bytes = place_twiddles(data, *d, &c.tw_lds, &c.tw_off);
     c.nt = pick_threads(*d, B, c.bytes, (ncol + B - 1) / B);
@@ -1014,7 +1019,7 @@ void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, bool wide, hipStr
     if (tc.bytes > kLdsMax) throw Error{"column copy does not fit in LDS", -1};
     a.dld = make_fdiv(c.nld);
     a.dst = make_fdiv(c.nst);
-    k_gcopy<real_t><<<(unsigned)nwg, 256, tc.bytes, st>>>(a);
+    k_gcopy<real_t><<<(unsigned)nwg, tc.nt, tc.bytes, st>>>(a);
     check_hip(hipGetLastError(), "k_gcopy launch");
     return;
   }
@@ -1104,11 +1109,12 @@ static size_t x_tile(GXArgs& a, const Len1D& L, long long nrows, long long row, 
 }
 
 // launch shape of a length (host only): form 0 rows on both sides, 1 a
-// length-fastest side, 2 rows along X
+// length-fastest side, 2 rows along X, 3 and 4 as 0 and 1 of rows that are copied
 void gen_tile_shape(const LenDesc& d, int form, long long count, int tile_bytes, int seg, bool wide, int* seqs,
                     int* threads, size_t* lds, int* offset_bytes) {
-  const TileChoice c = form == 2 ? x_row_tile(d, count, d.n + 2, tile_bytes)
-                                 : col_tile(&d, d.n, form == 1, count, tile_bytes, seg);
+  const TileChoice c = form == 2   ? x_row_tile(d, count, d.n + 2, tile_bytes)
+                       : form >= 3 ? col_tile(nullptr, d.n, form == 4, count, 0, 128)
+                                   : col_tile(&d, d.n, form == 1, count, tile_bytes, seg);
   *seqs = c.B;
   *threads = c.nt;
   *lds = c.bytes;

@@ -35,8 +35,8 @@ void gen_launch_x_c2r(const Len1D& L, const cplx_t* in, real_t* out, long long n
 void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, bool wide, hipStream_t st);
 // the launch shape of a schedule (host only): sequences per tile, threads (0:
 // no count holds the tile) and LDS bytes of `count` columns (form 0 rows on both
-// sides, 1 a length-fastest side) or rows along X (form 2), and the width of the
-// offsets into such contiguous columns or rows
+// sides, 1 a length-fastest side; 3 and 4 the same of copied rows) or rows along X
+// (form 2), and the width of the offsets into such contiguous columns or rows
 void gen_tile_shape(const LenDesc& d, int form, long long count, int tile_bytes, int seg, bool wide, int* seqs,
                     int* threads, size_t* lds, int* offset_bytes);
 // raise the kernels' dynamic-LDS limits (once, when a length is planned)

@@ -101,6 +101,15 @@ def test_short_rows_fill_a_tile(precision):
 
 
 @pytest.mark.parametrize("precision", [8, 4])
+@pytest.mark.parametrize("form", [3, 4])
+def test_copies_have_loads_in_flight(precision, form):
+    """Op 'n': at most four values a thread, up to the largest workgroup."""
+    for n, c, s, t, b in shapes(precision, form, 0, 128):
+        assert 0 < b <= LDS and t % 64 == 0 and t <= 1024, (n, c, s, t, b)
+        assert t == 1024 or 4 * t >= n * s, (n, c, s, t)
+
+
+@pytest.mark.parametrize("precision", [8, 4])
 def test_other_lengths_are_refused(precision):
     L = p3dfft_amd.load(precision)
     s, t, b, o = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t(), ctypes.c_int()
