@@ -855,9 +855,14 @@ struct PipeRows<RList<R0, Rs...>, TX, NT> {
 // workgroup per CU: gridDim.x workgroups, the 8 XCDs (workgroup w on XCD
 // w mod 8) each owning a contiguous range of tiles that its workgroups
 // share out round robin (a.xcd; else workgroup w takes tiles w, w + G, ...)
-// in whole rounds, the columns left after those as one round of narrower tiles,
-// and each workgroup keeping its next tile's loads in flight while the
-// current tile computes.  The row tables (TabRows, TabAll) are the
+// in whole rounds, the columns left after those as one round of narrower tiles
+// where these are at most half as wide, and each workgroup keeping its next tile's
+// loads in flight while the current tile computes.  Z of 2048 points forward /
+// backward, narrower tiles against full ones: FP32 768 columns 17.5 / 15.1 us
+// against 15.0 / 11.9, 1792 17.8 / 17.5 against 15.5 / 14.6, 2304 22.4 / 21.6
+// against 23.4 / 22.6, 3840 27.4 / 27.7 against 25.4 / 26.0; FP64 256 15.1 / 16.2
+// against 12.2 / 13.3, 1408 21.4 / 22.2 against 23.6 / 24.2, 1664 24.5 / 25.8
+// against 23.7 / 24.8.  The row tables (TabRows, TabAll) are the
 // same for every tile and stay in LDS, load table then store table, at
 // tab_off.
 template <class T, bool FWD, int TX, int NT, class RL, int W, bool TWL, class Off>
@@ -883,7 +888,10 @@ __global__ __launch_bounds__(NT, W) void k_colio_pipe(ColArgs a) {
   const long long tail_end = (long long)(lo + cnt - (a.rev ? nfull : 0)) * TX;
   const int tail = (int)((tail_end < ncol ? tail_end : ncol) - tail0);
   constexpr int WMIN = sizeof(cpx<T>) < 16 ? 16 / (int)sizeof(cpx<T>) : 1;  // at least 16 bytes of a row
-  const int wt0 = (tail + nslot - 1) / nslot, wt = wt0 < WMIN ? WMIN : wt0;
+  // (no whole round, or a remainder of more than half a tile each: full tiles on
+  // fewer workgroups, whose row segments are whole lines)
+  const int wt0 = (tail + nslot - 1) / nslot;
+  const int wt = nfull == 0 || 2 * wt0 > TX ? TX : (wt0 < WMIN ? WMIN : wt0);
   const int nt = nfull + (tail > 0 ? (tail + wt - 1) / wt : 0);
   int2* tl = (int2*)(g_smem + a.tab_off);
   if constexpr (TB) {

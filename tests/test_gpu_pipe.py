@@ -26,6 +26,20 @@ def test_narrow_last_round(precision, n):
 
 
 @pytest.mark.parametrize("precision", [8, 4])
+@pytest.mark.parametrize("n", [(34, 47, 2048), (34, 2048, 200), (34, 200, 2048), (2, 1, 2048)])
+def test_full_last_round(precision, n):
+    """846 columns (no whole round), 3600 (a remainder of three quarters of a round
+    and more) and 2: full tiles, the last one partial"""
+    nx, ny, nz = n
+    a = np.random.default_rng(ny).standard_normal((nz, ny, nx))
+    ref = np.fft.rfftn(a)
+    with lib_setup(precision, nx, ny, nz) as P:
+        s = P.ftran_r2c(a)
+        assert rel(s, ref) < TOL[precision]
+        assert rel(P.btran_c2r(s, "tff"), a * nx * ny * nz) < TOL[precision] * 10
+
+
+@pytest.mark.parametrize("precision", [8, 4])
 @pytest.mark.parametrize("dims", [(2, 4), (3, 2)])
 def test_peer_blocks(precision, dims):
     nx, ny, nz = 18, 2048, 16
