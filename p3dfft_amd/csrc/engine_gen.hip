@@ -269,24 +269,30 @@ __device__ __forceinline__ void gen_prime(cpx<T>* lds, const GenDesc& L, const G
   __syncthreads();
 }
 
-// An in-place stage over the tile.  PM: the schedule has a prime stage; the
-// others are compiled without it, whose registers (FP32 X kernels 96-109
-// against 80) cost every stage a wave per SIMD.  200-point FP32 X r2c of a
-// 200x300x250 box 39.7 -> 28.6 us, 1000-point FP64 of 1000x100x90 45.0 -> 41.6.
-// b: this thread's sequence, jt, js: its
+// The prime stages of a schedule: none, over LDS only (all of them above
+// kGenRegPrime), or some in registers.  Each is compiled apart: the registers of a
+// stage over LDS (FP32 X kernels 96-109 against 80) cost every stage a wave per
+// SIMD (200-point FP32 X r2c of a 200x300x250 box 39.7 -> 28.6 us without,
+// 1000-point FP64 of 1000x100x90 45.0 -> 41.6), and 11 and 13 points in registers
+// beside it 8 to 48 bytes of scratch in FP64 (X r2c / c2r of 2^22 points in rows
+// of 57 31.7 / 29.7 us with, 28.2 / 27.1 without, c2r in rows of 1360 34.0
+// and 28.0; FP32, 2^23 points in columns of 127, 101 and 94).
+enum { kPrimeNone = 0, kPrimeLds = 1, kPrimeAny = 2 };
+
+// An in-place stage over the tile.  b: this thread's sequence, jt, js: its
 // first butterfly and their stride
-template <class T, bool FWD, bool DIF, bool PM>
+template <class T, bool FWD, bool DIF, int PM>
 __device__ __forceinline__ void gen_mid(cpx<T>* lds, const GenDesc& L, int s, const GenTile& t, int B, unsigned mB,
                                         int b, int jt, int js, const typename TwT<T>::type* tw) {
   const GenStage st = L.st[s];
-  if constexpr (PM) {
+  if constexpr (PM != kPrimeNone) {
     if (st.R > kGenRegPrime) {
       gen_prime<T, FWD, DIF>(lds, L, st, t, B, mB, tw);
       return;
     }
   }
   const int nj = gdiv(L.n, st.mR, st.R), SP = gen_stride(t, st);
-  if constexpr (PM) {
+  if constexpr (PM == kPrimeAny) {
     if (st.R > kGenMaxRadix) {
       for (int j = jt; j < nj; j += js) {
         const int g = gdiv(j, st.mNs, st.Ns), k = j - g * st.Ns;
@@ -405,7 +411,7 @@ __device__ __forceinline__ cpx<T> gen_out(const GColArgs& a, cpx<T> v) {
 // a form of either width, so that a view of 4 GiB gives the bits of a smaller one
 // (the form with maps contracts its products differently) and is not slowed by
 // the maps' arithmetic.
-template <class T, bool FWD, bool MAP, int LF, class Off, bool TL, bool PM>
+template <class T, bool FWD, bool MAP, int LF, class Off, bool TL, int PM>
 __global__ __launch_bounds__(1024) void k_gcol(GColArgs a) {
   typedef cpx<T> C;
   constexpr long long E = sizeof(C);
@@ -601,7 +607,7 @@ struct GXArgs {
 // fewer LDS conflicts, but their short runs cost more on the memory side: FP64
 // 200x300x250 r2c / c2r 51 / 70 -> 46 / 49 us (5.0 TB/s), FP32 30 / 34 ->
 // 28 / 31 us.
-template <class T, bool TL, bool PM>
+template <class T, bool TL, int PM>
 __global__ __launch_bounds__(1024) void k_gx_r2c(GXArgs a) {
   typedef cpx<T> C;
   C* lds = (C*)gen_smem;
@@ -661,7 +667,7 @@ __global__ __launch_bounds__(1024) void k_gx_r2c(GXArgs a) {
 
 // c2r: the mirror image: natural order in, decimation in frequency, stage 0
 // stores the rows
-template <class T, bool TL, bool PM>
+template <class T, bool TL, int PM>
 __global__ __launch_bounds__(1024) void k_gx_c2r(GXArgs a) {
   typedef cpx<T> C;
   C* lds = (C*)gen_smem;
@@ -895,10 +901,11 @@ static int pick_threads(const LenDesc& d, int B, size_t lds, long long tiles) {
   return bn;
 }
 
-static bool has_prime_stage(const LenDesc& d) {
+static int prime_stages(const LenDesc& d) {
+  int k = kPrimeNone;
   for (int s = 0; s < d.nst; s++)
-    if (!gen_in_registers(d.radix[s])) return true;
-  return false;
+    if (!gen_in_registers(d.radix[s])) k = std::max(k, gen_over_lds(d.radix[s]) ? (int)kPrimeLds : (int)kPrimeAny);
+  return k;
 }
 
 // the tile of a launch: sequences, threads, LDS bytes and the layout
@@ -970,20 +977,20 @@ static bool offsets_fit(const ColSpec& c, int B) {
   return fits(c.si_in, c.sl_in, c.so_in) && fits(c.si_out, c.sl_out, c.so_out);
 }
 
-// f(TL, PM): the twiddle table in LDS, the schedule with a prime stage
+// f(TL, PM): the twiddle table in LDS, the schedule's prime stages
 template <class F>
-static void with_variant(bool tl, bool pm, F f) {
-  if (tl) {
-    if (pm) f(std::true_type{}, std::true_type{});
-    else f(std::true_type{}, std::false_type{});
-  } else {
-    if (pm) f(std::false_type{}, std::true_type{});
-    else f(std::false_type{}, std::false_type{});
-  }
+static void with_variant(bool tl, int pm, F f) {
+  auto with_tl = [&](auto t) {
+    if (pm == kPrimeAny) f(t, std::integral_constant<int, kPrimeAny>{});
+    else if (pm == kPrimeLds) f(t, std::integral_constant<int, kPrimeLds>{});
+    else f(t, std::integral_constant<int, kPrimeNone>{});
+  };
+  if (tl) with_tl(std::true_type{});
+  else with_tl(std::false_type{});
 }
 
 template <bool FWD, bool MAP, int LF, class Off>
-static void go_col(const GColArgs& a, bool pm, unsigned g, int nt, size_t bytes, hipStream_t st) {
+static void go_col(const GColArgs& a, int pm, unsigned g, int nt, size_t bytes, hipStream_t st) {
   with_variant(a.tw_lds != 0, pm, [&](auto tl, auto pr) {
     k_gcol<real_t, FWD, MAP, LF, Off, tl.value, pr.value><<<g, nt, bytes, st>>>(a);
   });
@@ -1032,7 +1039,7 @@ void gen_launch_col(const Len1D* L, const ColSpec& c, int xcd, bool wide, hipStr
   if (bytes > kLdsMax) throw Error{"column transform does not fit in LDS", -1};
   const int nt = tc.nt;
   if (!nt) throw Error{"transform tile exceeds the 1024-thread workgroup capacity", -1};
-  const bool pm = has_prime_stage(L->gd);
+  const int pm = prime_stages(L->gd);
   const bool fwd = c.fwd || c.kind == COL_DCT1 || c.kind == COL_DST1;
   const bool ld_id = c.nld == m && (c.ld_lo >= m || (c.ld_hi <= c.ld_lo && c.ld_shift == 0));
   const bool st_id = c.nst == m && (c.st_lo >= m || c.st_shift == 0);
@@ -1073,7 +1080,7 @@ static TileChoice x_row_tile(const LenDesc& d, long long nrows, long long row, i
   // different phases; a prime stage wants the pairs): r2c / c2r 600x128x200 61 / 74 -> 48 / 50 us,
   // 720x240x200 155 / 165 -> 139 / 130.  FP32 measured no gain (1500x64x100 28
   // -> 29), its tiles hold twice the values per byte in flight.
-  const long long def = sizeof(real_t) == 8 && !has_prime_stage(d) ? 40 * 1024 : 64 * 1024;
+  const long long def = sizeof(real_t) == 8 && prime_stages(d) == kPrimeNone ? 40 * 1024 : 64 * 1024;
   const long long lim = plan_bytes ? plan_bytes : def;
   while (B > 1 && ((long long)n * (B + 1) * E > lim || (2LL * B + 1) * row * E >= (1LL << 32))) B /= 2;
   while (B > 1 && !prime_stages_fit(d, B)) B /= 2;
@@ -1137,7 +1144,7 @@ void gen_launch_x_r2c(const Len1D& L, const real_t* in, cplx_t* out, long long n
   int nt;
   unsigned g;
   const size_t bytes = x_tile(a, L, nrows, std::max(si_row, so_row), &nt, &g);
-  with_variant(a.tw_lds != 0, has_prime_stage(L.gd), [&](auto tl, auto pm) {
+  with_variant(a.tw_lds != 0, prime_stages(L.gd), [&](auto tl, auto pm) {
     k_gx_r2c<real_t, tl.value, pm.value><<<g, nt, bytes, st>>>(a);
   });
   check_hip(hipGetLastError(), "k_gx_r2c launch");
@@ -1154,7 +1161,7 @@ void gen_launch_x_c2r(const Len1D& L, const cplx_t* in, real_t* out, long long n
   unsigned g;
   const size_t bytes = x_tile(a, L, nrows, std::max(si_row, so_row), &nt, &g);
   if (L.gd.nst == 1) a.dn0 = make_fdiv(L.gd.n);
-  with_variant(a.tw_lds != 0, has_prime_stage(L.gd), [&](auto tl, auto pm) {
+  with_variant(a.tw_lds != 0, prime_stages(L.gd), [&](auto tl, auto pm) {
     k_gx_c2r<real_t, tl.value, pm.value><<<g, nt, bytes, st>>>(a);
   });
   check_hip(hipGetLastError(), "k_gx_c2r launch");
@@ -1165,7 +1172,7 @@ static void allow_big_lds(K kernel) {
   (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax);
   (void)hipGetLastError();  // a refused attribute leaves the default limit, not a pending error
 }
-template <bool FWD, bool TL, bool PM>
+template <bool FWD, bool TL, int PM>
 static void prep_dir() {
   typedef unsigned U32;
   typedef unsigned long long U64;
@@ -1182,8 +1189,8 @@ void gen_prep_kernels() {
   static std::once_flag once;
   std::call_once(once, [] {
     for (int tl = 0; tl < 2; tl++)
-      for (int pm = 0; pm < 2; pm++)
-        with_variant(tl != 0, pm != 0, [](auto t, auto p) {
+      for (int pm : {kPrimeNone, kPrimeLds, kPrimeAny})
+        with_variant(tl != 0, pm, [](auto t, auto p) {
           prep_dir<true, t.value, p.value>();
           prep_dir<false, t.value, p.value>();
         });

@@ -57,6 +57,15 @@ def test_stages_of_11_and_13(precision, n):
 
 
 @pytest.mark.parametrize("precision", [8, 4])
+@pytest.mark.parametrize("n", [187, 221, 266, 2431])
+def test_stages_of_both_kinds(precision, n):
+    """11 and 13 points in registers beside larger primes over LDS, and larger ones
+    alone, along each axis"""
+    for shape in ((n, 3, 4), (4, n, 300), (10, 7, n)):
+        check(precision, shape)
+
+
+@pytest.mark.parametrize("precision", [8, 4])
 @pytest.mark.parametrize("n", range(1, 16))
 def test_short_rows(precision, n):
     """Rows of one stage (up to 10 points) and just above along X, in wide tiles
