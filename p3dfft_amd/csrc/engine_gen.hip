@@ -958,8 +958,10 @@ static TileChoice col_tile(const LenDesc* d, int m, bool lf, long long ncol, int
   // a copy has a tile or two per CU in flight and waits for its loads: four values
   // a thread (FP32 with op 'n', forward / backward: 3 fields of 3x192x2149,
   // length-fastest, 95 / 90 us with 256 threads, 51 / 50 so; 2 of 256x32x564, 176
-  // modes kept, 66 / 61 -> 46 / 47; with sixteen a thread 63 / 61 and 50 / 49)
-  c.nt = (int)std::max<long long>(64, std::min<long long>(1024, ((long long)m * B + 255) / 256 * 64));
+  // modes kept, 66 / 61 -> 46 / 47; with sixteen a thread 63 / 61 and 50 / 49), and
+  // at least 256 threads (FP64 forward 192x22x32, 21 modes kept, 14.2 us, 15.7 with
+  // 64)
+  c.nt = (int)std::max<long long>(256, std::min<long long>(1024, ((long long)m * B + 255) / 256 * 64));
   if (d) {
     c.bytes = place_twiddles(data, *d, &c.tw_lds, &c.tw_off);
     c.nt = pick_threads(*d, B, c.bytes, (ncol + B - 1) / B);
