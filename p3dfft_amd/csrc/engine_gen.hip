@@ -24,8 +24,11 @@
 // across a barrier.
 //
 // What bounds the passes: with 128-byte row segments they move each byte once
-// per pass and run at 4-5.5 TB/s; the rest is the instruction issue of the
-// butterflies, the compensated twiddles and the run-time index arithmetic.
+// per pass and run at 4-5.5 TB/s.  Counters of 200x300x250 FP32 / 1000x100x90
+// FP64: 48-63% / 26-33% of the VALU slots busy (butterflies, compensated
+// twiddles, run-time index arithmetic), the waves waiting for half of their
+// cycles, 1-4% of them for LDS: the latencies of a tile's serial phases, and in
+// FP32 the instruction issue beside them.
 // Against a tile loaded to LDS, autosort stages and a direct sum for every
 // prime: FP32 200x300x250 columns of 300 points 97 -> 30 us, of 250 102 -> 28,
 // X r2c of 200 54 -> 28; FP64 1000x100x90 columns of 100 points 85 -> 26 us, of
@@ -602,11 +605,10 @@ struct GXArgs {
 
 // r2c: stage 0 reads the rows (lanes along the row), in-place stages, and the
 // two half spectra separated from the natural-order result as they are stored.
-// Bound by the latencies of a tile's serial phases and the run-time index
-// arithmetic.  Lanes along one row throughout: 16 lanes along each of 4 rows met
-// fewer LDS conflicts, but their short runs cost more on the memory side: FP64
-// 200x300x250 r2c / c2r 51 / 70 -> 46 / 49 us (5.0 TB/s), FP32 30 / 34 ->
-// 28 / 31 us.
+// Bound by the latencies of a tile's serial phases (see the top of the file).
+// Lanes along one row throughout: 16 lanes along each of 4 rows met fewer LDS
+// conflicts, but their short runs cost more on the memory side: FP64 200x300x250
+// r2c / c2r 51 / 70 -> 46 / 49 us (5.0 TB/s), FP32 30 / 34 -> 28 / 31 us.
 template <class T, bool TL, int PM>
 __global__ __launch_bounds__(1024) void k_gx_r2c(GXArgs a) {
   typedef cpx<T> C;
